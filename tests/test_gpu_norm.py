@@ -82,6 +82,22 @@ def test_rms_norm_types_strides_and_in_place(gpu):
     assert rel_l2(call(gpu, big, w, 1e-6), want_norm(big, w, 1e-6)) <= 1e-6
 
 
+@pytest.mark.parametrize("k", [8, 2040, 2049, 4104, 6144, 6152, 14337])
+@pytest.mark.parametrize("pad", [0, 3])
+def test_rms_norm_pieces_of_a_row(gpu, k, pad):
+    # a thread holds pieces of 8 columns: rows that end inside a piece or just past a round of 256 pieces (2048 columns), rows of more
+    # pieces than the registers hold (above 6144), rows that 16-byte loads may not touch (an odd stride); magnitudes at which the
+    # quotient by the reciprocal gives way to the plain division (rms outside 2^-60 .. 2^60)
+    rng = np.random.default_rng(k + pad)
+    x = rng.standard_normal((3, k)).astype(np.float32)
+    w = rng.standard_normal(k).astype(np.float32)
+    for scale, eps in ((1.0, 1e-6), (1e-20, 0.0)) + (((2e18, 1e-6),) if k == 8 else ()):
+        xs = (x * np.float32(scale)).astype(np.float32)
+        # (8 squares of up to (3 * 2e18)^2 stay below 3.4e38; squares of 1e-40 and below are f32 subnormals, 2^-149 each against 1e-40: 1e-5; else a few f32 ulps)
+        bar = 1e-6 if scale >= 1.0 else 2e-3
+        assert rel_l2(call(gpu, xs, w, eps, ldx=k + pad, ldy=k + pad, mem=capi.MEM_DEVICE), want_norm(xs, w, eps)) <= bar, scale
+
+
 def test_rms_norm_errors(gpu):
     L, ctx = gpu.L, gpu.ctx
     x = np.zeros((2, 8), np.float32)

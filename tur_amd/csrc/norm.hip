@@ -15,21 +15,71 @@ template <int XT> __device__ inline float ld_elem(const void *x, int64_t i) {
     return (float)h;
 }
 
-// the workgroup's part of sqrt(mean(x^2) + eps): s = what thread t added up of the squares of columns t, t + 256, ... (explicit
-// fused multiply-adds in that order), then the waves their lanes and the workgroup its four waves - one fixed order, shared by
-// the kernels below so that they agree to the bit
+// Both kernels take a row in pieces of 8 neighbouring columns: thread t of a row's 256 holds the pieces t, t + 256, ... (PER of them
+// in registers), loaded and stored 16 bytes at a time where the row allows it.  Bound by latency at decode sizes (one row is one
+// chain load -> sum -> barrier -> divide -> store in a launch of 4 us) and by the memory system at prompt sizes.  With one element per load
+// (2 bytes of a bf16 row) the chain of 16 loads per thread was the kernel: 8 rows of 4096 bf16 columns took 10.5 us, now 4.0 - 4.7.
+
+// eight columns of a row from column col0 on, +0 past k
+template <int XT> __device__ inline void ld_piece(const void *x, int64_t row_off, int64_t col0, int64_t k, bool vec, float (&v)[8]) {
+    if (vec && col0 + 8 <= k) {
+        const uint8_t *p = (const uint8_t *)x + (row_off + col0) * (XT == TURQ_ACT_F32 ? 4 : 2);
+        if constexpr (XT == TURQ_ACT_F32) {
+            const float4v lo = ((const float4v *)p)[0], hi = ((const float4v *)p)[1];
+            v[0] = lo.x, v[1] = lo.y, v[2] = lo.z, v[3] = lo.w, v[4] = hi.x, v[5] = hi.y, v[6] = hi.z, v[7] = hi.w;
+        } else {
+            const uint4v u = *(const uint4v *)p;
+            const uint32_t wd[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if constexpr (XT == TURQ_ACT_BF16) {
+                    v[2 * j] = __uint_as_float(wd[j] << 16);
+                    v[2 * j + 1] = __uint_as_float(wd[j] & 0xFFFF0000u);
+                } else {
+                    const half2v hh = as_half2(wd[j]);
+                    v[2 * j] = (float)hh.x;
+                    v[2 * j + 1] = (float)hh.y;
+                }
+            }
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = col0 + e < k ? ld_elem<XT>(x, row_off + col0 + e) : 0.0f;
+    }
+}
+
+__device__ inline bool vec_row(const void *p, int64_t ld, int elem_bytes) {
+    return ((uintptr_t)p & 15) == 0 && ((ld * elem_bytes) & 15) == 0;
+}
+
+// sqrt(mean(x^2) + eps) of the row that a group of four waves holds: s = what a thread added up of the squares of its columns
+// (explicit fused multiply-adds, piece by piece), then the waves their lanes and the group its four waves - one fixed order, shared
+// by the kernels below so that they agree to the bit.  part: four floats of the row's group.  Every thread of the workgroup calls it.
 __device__ inline float rms_of(float s, int64_t k, float eps, float *part) {
-    const int tid = threadIdx.x;
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) s += __shfl_xor(s, off, 64);
-    if ((tid & 63) == 0) part[tid >> 6] = s;
+    if ((threadIdx.x & 63) == 0) part[(threadIdx.x >> 6) & 3] = s;
     __syncthreads();
     const float total = (part[0] + part[1]) + (part[2] + part[3]);
     return sqrtf(total / (float)k + eps);
 }
 
-// one workgroup of 256 threads per row; a thread keeps up to PER of the row's elements in registers between the two passes
-// (rows of up to 256 * PER elements are read once, so y may be x whatever the two element types), longer rows are read again
+// v / rms for many v against one rms, to the last bit: with r = 1 / rms correctly rounded, q = v * r corrected once by its own
+// remainder is the correctly rounded quotient (P. Markstein, "Computation of elementary functions on the IBM RISC System/6000",
+// 1990) as long as nothing over- or underflows on the way.  No |v| of a row exceeds sqrt(k) * rms, so only the range of rms matters:
+// rows whose rms is an infinity, a NaN or outside a generous range take the plain division.
+struct RowDiv {
+    float rms, r;
+    bool plain;
+    __device__ explicit RowDiv(float d) : rms(d), r(1.0f / d), plain(!(d > 0x1p-60f && d < 0x1p60f)) {}
+    __device__ float operator()(float v) const {
+        const float q = v * r;
+        return __builtin_expect(plain, 0) ? v / rms : __builtin_fmaf(__builtin_fmaf(-q, rms, v), r, q);
+    }
+};
+
+// one workgroup of 256 threads per row; rows of up to 2048 * PER elements are read once (so y may be x whatever the two element
+// types), longer rows are read again
 template <int XT, int YT, int PER>
 __global__ void __launch_bounds__(256) rms_norm_kernel(const void *__restrict__ x, int64_t k, int64_t ldx, const float *__restrict__ w,
                                                        float eps, void *__restrict__ y, int64_t ldy) {
@@ -37,62 +87,116 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(const void *__restrict__ 
     const int tid = threadIdx.x;
     const int64_t row = blockIdx.x;
     const int64_t xo = row * ldx, yo = row * ldy;
-    float v[PER];
+    const bool vx = vec_row(x, ldx, XT == TURQ_ACT_F32 ? 4 : 2), vy = vec_row(y, ldy, YT == TURQ_ACT_F32 ? 4 : 2);
+    const bool vw = ((uintptr_t)w & 15) == 0;
+    float v[PER][8];
     float s = 0.0f;
 #pragma unroll
     for (int j = 0; j < PER; j++) {
-        const int64_t c = (int64_t)j * 256 + tid;
-        v[j] = c < k ? ld_elem<XT>(x, xo + c) : 0.0f;
-        s = __builtin_fmaf(v[j], v[j], s);  // (columns past k add +0: the sum is that of the columns that exist)
+        const int64_t col0 = ((int64_t)j * 256 + tid) * 8;
+        ld_piece<XT>(x, xo, col0, k, vx, v[j]);
     }
-    for (int64_t c = (int64_t)PER * 256 + tid; c < k; c += 256) {
-        const float t = ld_elem<XT>(x, xo + c);
-        s = __builtin_fmaf(t, t, s);
-    }
-    const float rms = rms_of(s, k, eps, part);
 #pragma unroll
-    for (int j = 0; j < PER; j++) {
-        const int64_t c = (int64_t)j * 256 + tid;
-        if (c < k) turq_store_out<YT>(y, yo + c, v[j] / rms * w[c]);
+    for (int j = 0; j < PER; j++)
+#pragma unroll
+        for (int e = 0; e < 8; e++) s = __builtin_fmaf(v[j][e], v[j][e], s);  // (columns past k add +0: the sum is that of the columns that exist)
+    for (int64_t col0 = ((int64_t)PER * 256 + tid) * 8; col0 < k; col0 += 2048) {
+        float t[8];
+        ld_piece<XT>(x, xo, col0, k, vx, t);
+#pragma unroll
+        for (int e = 0; e < 8; e++) s = __builtin_fmaf(t[e], t[e], s);
     }
-    for (int64_t c = (int64_t)PER * 256 + tid; c < k; c += 256) turq_store_out<YT>(y, yo + c, ld_elem<XT>(x, xo + c) / rms * w[c]);
+    const RowDiv div(rms_of(s, k, eps, part));
+    auto store = [&](int64_t col0, const float (&t)[8]) {
+        if (col0 >= k) return;
+        float wv[8], o[8];
+        ld_piece<TURQ_ACT_F32>(w, 0, col0, k, vw, wv);
+#pragma unroll
+        for (int e = 0; e < 8; e++) o[e] = div(t[e]) * wv[e];
+        if (vy && col0 + 8 <= k) {
+            uint32_t bad = 0;
+#pragma unroll
+            for (int e = 0; e < 8; e++) turq_note_accum(o[e], turq_finite_limit(YT), bad);
+            turq_note_flush(bad);
+            uint8_t *p = (uint8_t *)y + (yo + col0) * (YT == TURQ_ACT_F32 ? 4 : 2);
+            if constexpr (YT == TURQ_ACT_F32) {
+                ((float4v *)p)[0] = float4v{o[0], o[1], o[2], o[3]};
+                ((float4v *)p)[1] = float4v{o[4], o[5], o[6], o[7]};
+            } else if constexpr (YT == TURQ_ACT_BF16) {
+                *(uint4v *)p = uint4v{turq_f2bf_x2(o[0], o[1]), turq_f2bf_x2(o[2], o[3]), turq_f2bf_x2(o[4], o[5]), turq_f2bf_x2(o[6], o[7])};
+            } else {
+                half8v h;
+#pragma unroll
+                for (int e = 0; e < 8; e++) h[e] = (_Float16)o[e];
+                *(half8v *)p = h;
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                if (col0 + e < k) turq_store_out<YT>(y, yo + col0 + e, o[e]);
+        }
+    };
+#pragma unroll
+    for (int j = 0; j < PER; j++) store(((int64_t)j * 256 + tid) * 8, v[j]);
+    for (int64_t col0 = ((int64_t)PER * 256 + tid) * 8; col0 < k; col0 += 2048) {
+        float t[8];
+        ld_piece<XT>(x, xo, col0, k, vx, t);
+        store(col0, t);
+    }
 }
 
 // The same rows written straight into the fragments of the prefill GEMM (the order act_prep32_kernel writes, see there): what
 // rms_norm_kernel with an f32 output followed by that kernel would leave - the same sums in the same order, the same one rounding
-// to f16 - without the launch and the round trip in between.  One workgroup per row of the 32-row m-tiles (rows past m: zeros);
-// thread t holds the pieces of 8 columns t, t + 256, ... (PER of them: k <= 2048 * PER); the sub-block sums of the fragments
-// (32 columns) are added up between the four neighbouring lanes that hold a sub-block.
+// to f16 - without the launch and the round trip in between.  A workgroup takes kPrepRows neighbouring rows of a 32-row m-tile
+// (rows past m: zeros), 256 threads each: a fragment block holds 16 bytes of each row next to each other, and rows that are
+// written by one workgroup meet in one cache line of one L2 (with a row per workgroup every 128-byte line was written in eight pieces
+// from eight XCDs; 4096 bf16 columns: 2048 rows 34.7 -> 12.5 us, 512 rows 15 -> 7, 77 rows 10.4 -> 5.6).  A thread keeps its PER pieces of 8 columns in registers between the two passes (k <= 2048 * PER); the
+// sub-block sums of the fragments (32 columns) are added up between the four neighbouring lanes that hold a sub-block.
+constexpr int kPrepRows = 4;
 template <int XT, bool Q8, int PER>
-__global__ void __launch_bounds__(256) rms_norm_prep32_kernel(const void *__restrict__ x, int64_t m, int64_t k, int64_t ldx,
-                                                              const float *__restrict__ w, float eps, int64_t ntc, half8v *__restrict__ frags) {
-    __shared__ float part[4];
-    const int tid = threadIdx.x;
-    const int64_t row = blockIdx.x;
+__global__ void __launch_bounds__(256 * kPrepRows) rms_norm_prep32_kernel(const void *__restrict__ x, int64_t m, int64_t k, int64_t ldx,
+                                                                          const float *__restrict__ w, float eps, int64_t ntc,
+                                                                          half8v *__restrict__ frags) {
+    __shared__ float part[kPrepRows][4];
+    const int tid = threadIdx.x & 255, sub = threadIdx.x >> 8;
+    // workgroups of one XCD (blockIdx % 8) take neighbouring rows
+    const int nwg = (int)gridDim.x;
+    const int lid = (nwg & 7) == 0 ? ((int)blockIdx.x & 7) * (nwg >> 3) + ((int)blockIdx.x >> 3) : (int)blockIdx.x;
+    const int64_t row = (int64_t)lid * kPrepRows + sub;
     const int64_t mt = row >> 5;
     const int r = (int)(row & 31);
     const bool live = row < m;
     const int64_t xo = row * ldx;
-    float s = 0.0f;  // the row's sum of squares, added up as rms_norm_kernel adds it up
-    if (live)
-        for (int64_t c = tid; c < k; c += 256) {
-            const float t = ld_elem<XT>(x, xo + c);
-            s = __builtin_fmaf(t, t, s);
-        }
-    const float rms = rms_of(s, k, eps, part);
+    const bool vx = vec_row(x, ldx, XT == TURQ_ACT_F32 ? 4 : 2), vw = ((uintptr_t)w & 15) == 0;
+    float v[PER][8];
+    float s = 0.0f;
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        const int64_t col0 = ((int64_t)j * 256 + tid) * 8;
+        ld_piece<XT>(x, xo, col0, live ? k : 0, vx, v[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < PER; j++)
+#pragma unroll
+        for (int e = 0; e < 8; e++) s = __builtin_fmaf(v[j][e], v[j][e], s);
+    const RowDiv div(rms_of(s, k, eps, part[sub]));
 #pragma unroll
     for (int j = 0; j < PER; j++) {
         const int64_t piece = (int64_t)j * 256 + tid, col0 = piece * 8;
         if (col0 >= k) continue;  // (k is a multiple of 256: whole pieces, and whole groups of four lanes)
+        float wv[8];
+        ld_piece<TURQ_ACT_F32>(w, 0, col0, k, vw, wv);
         half8v h;
         float sum = 0.0f;
+        uint32_t bad = 0;
 #pragma unroll
         for (int e = 0; e < 8; e++) {
-            const float f = live ? ld_elem<XT>(x, xo + col0 + e) / rms * w[col0 + e] : 0.0f;
-            turq_note_result<TURQ_ACT_F16>(f);
+            const float f = live ? div(v[j][e]) * wv[e] : 0.0f;
+            turq_note_accum(f, turq_finite_limit(TURQ_ACT_F16), bad);
             h[e] = (_Float16)f;
             sum += (float)h[e];
         }
+        turq_note_flush(bad);
         const int64_t b = piece >> 5;
         const int cc = (int)(piece & 31);
         half8v *dst = frags + (mt * ntc + b) * (17 * 64);
@@ -113,8 +217,9 @@ __global__ void __launch_bounds__(256) rms_norm_prep32_kernel(const void *__rest
 
 template <int XT, int YT>
 hipError_t launch2(const void *x, int64_t m, int64_t k, int64_t ldx, const float *w, float eps, void *y, int64_t ldy, hipStream_t s) {
-    if (k <= 4 * 256) rms_norm_kernel<XT, YT, 4><<<(unsigned)m, 256, 0, s>>>(x, k, ldx, w, eps, y, ldy);
-    else rms_norm_kernel<XT, YT, 16><<<(unsigned)m, 256, 0, s>>>(x, k, ldx, w, eps, y, ldy);
+    if (k <= 2048) rms_norm_kernel<XT, YT, 1><<<(unsigned)m, 256, 0, s>>>(x, k, ldx, w, eps, y, ldy);
+    else if (k <= 2 * 2048) rms_norm_kernel<XT, YT, 2><<<(unsigned)m, 256, 0, s>>>(x, k, ldx, w, eps, y, ldy);
+    else rms_norm_kernel<XT, YT, 3><<<(unsigned)m, 256, 0, s>>>(x, k, ldx, w, eps, y, ldy);
     return hipGetLastError();
 }
 
@@ -148,13 +253,15 @@ hipError_t turq_launch_rms_norm_prep32(int dtype, const void *x, int x_dtype, in
     if (m == 0 || k == 0) return hipSuccess;
     if (k % 256 != 0 || k > 16384 || m > (1 << 26)) return hipErrorInvalidValue;
     const int64_t ntc = k / 256;
-    const unsigned grid = (unsigned)(((m + 31) / 32) * 32);
+    const unsigned grid = (unsigned)(((m + 31) / 32) * (32 / kPrepRows));
     const bool q8 = dtype == TURQ_Q8_0;
 #define TURQ_NP32(XT, PER)                                                                                                           \
-    if (q8) rms_norm_prep32_kernel<XT, true, PER><<<grid, 256, 0, stream>>>(x, m, k, ldx, weight, eps, ntc, (half8v *)frags);       \
-    else rms_norm_prep32_kernel<XT, false, PER><<<grid, 256, 0, stream>>>(x, m, k, ldx, weight, eps, ntc, (half8v *)frags)
+    if (q8) rms_norm_prep32_kernel<XT, true, PER><<<grid, 256 * kPrepRows, 0, stream>>>(x, m, k, ldx, weight, eps, ntc, (half8v *)frags);       \
+    else rms_norm_prep32_kernel<XT, false, PER><<<grid, 256 * kPrepRows, 0, stream>>>(x, m, k, ldx, weight, eps, ntc, (half8v *)frags)
 #define TURQ_NP32_X(XT)                                  \
-    if (k <= 2048 * 2) { TURQ_NP32(XT, 2); }             \
+    if (k <= 2048) { TURQ_NP32(XT, 1); }                 \
+    else if (k <= 2048 * 2) { TURQ_NP32(XT, 2); }        \
+    else if (k <= 2048 * 3) { TURQ_NP32(XT, 3); }        \
     else if (k <= 2048 * 6) { TURQ_NP32(XT, 6); }        \
     else { TURQ_NP32(XT, 8); }                           \
     break
