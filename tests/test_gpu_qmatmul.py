@@ -756,3 +756,35 @@ def test_prefill_tile_shapes(switch, value):
                           os.path.join(root, "tests", "test_gpu_fullsize.py")],
                          cwd=root, env=env, capture_output=True, text=True, timeout=280)
     assert out.returncode == 0, out.stdout[-3000:] + out.stderr[-1000:]
+
+
+# The kernel whose waves split the columns picks its tile (in 32 x 32 units, rows x columns) from the launch; the small matrices of the
+# tests above take the smallest one, so they run once more with each of the others forced: ragged rows and columns at every tile's
+# edges, super-blocks fewer than waves and not a multiple of them, every format, biases, several weights in one launch.
+@pytest.mark.parametrize("tile", ["21", "31", "22", "32", "23", "42"])
+def test_prefill_column_split_tile_shapes(tile):
+    import os
+    import subprocess
+    import sys
+
+    env = dict(os.environ, TURQ_GEMM_COLS=tile)
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    out = subprocess.run([sys.executable, "-m", "pytest", "-q", "-x", "-m", "gpu", "-k", "(prefill or more_rows) and not tile_shapes and not forced",
+                          "-p", "no:cacheprovider", os.path.join(root, "tests", "test_gpu_qmatmul.py")],
+                         cwd=root, env=env, capture_output=True, text=True, timeout=280)
+    assert out.returncode == 0, out.stdout[-3000:] + out.stderr[-1000:]
+
+
+@pytest.mark.parametrize("dt", [Q4_K, Q5_K, Q6_K, Q8_0])
+@pytest.mark.parametrize("n,k,m", [(31, 256, 33), (33, 768, 65), (97, 1280, 96), (160, 2304, 129)])
+def test_prefill_column_split_edges(gpu, dt, n, k, m):
+    # rows and columns one short of, one past and on the 32 x 32 tiles; one, three, five and nine super-blocks for four waves.
+    # The bound of the prefill kernels: weights d * sc rounded to f16, twice 2^-11 of each product.
+    raw = synth.random_weight(dt, n, k, seed=n + k)
+    w = gpu.upload(dt, n, k, raw, capi.LAYOUT_TILED)
+    x = synth.random_activation(m, k, seed=m, bf16=True)
+    want = orc.matmul_dequant(dt, x, raw, n, k)
+    got = gpu.qmatmul(w, x, n, k)
+    assert rel_l2(got, want) <= 1e-3
+    assert np.array_equal(got, gpu.qmatmul(w, x, n, k))
+    gpu.release(w)

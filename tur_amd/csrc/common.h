@@ -201,7 +201,7 @@ hipError_t turq_launch_gemv_simple(int dtype, const void *w, int64_t n, int64_t 
 // per translation unit whose kernels store results: adds the current device's count of non-finite results to *sum (mfma_common.h)
 #define TURQ_NONFINITE_UNITS(X)                                                                                                   \
     X(turq_nonfinite_gemv_mfma) X(turq_nonfinite_gemv_row1) X(turq_nonfinite_gemv_cs) X(turq_nonfinite_gemv_cs_staged_f32)         \
-    X(turq_nonfinite_gemv_cs_staged_bf16) X(turq_nonfinite_gemv_cs_staged_f16) X(turq_nonfinite_gemm_mfma)                        \
+    X(turq_nonfinite_gemv_cs_staged_bf16) X(turq_nonfinite_gemv_cs_staged_f16) X(turq_nonfinite_gemm_mfma) X(turq_nonfinite_gemm_cols) \
     X(turq_nonfinite_gemv_simple) X(turq_nonfinite_act_mul) X(turq_nonfinite_wide) X(turq_nonfinite_norm) X(turq_nonfinite_act_prep)
 #define TURQ_DECLARE_NONFINITE(fn) hipError_t fn(unsigned long long *sum, int reset);
 TURQ_NONFINITE_UNITS(TURQ_DECLARE_NONFINITE)

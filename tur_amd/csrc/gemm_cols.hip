@@ -1,0 +1,426 @@
+// Quantized matmul for prompt chunks whose tiles, one workgroup each, would leave the machine waiting: the columns (k) of a tile are
+// shared out over the WAVES of its workgroup instead of its rows.
+//
+// Every wave holds the whole workgroup tile - MT x NT MFMA tiles of 32 x 32 - and walks its own super-blocks (256 columns): the
+// activation fragments (prepared in 32-row A order by act_prep32_kernel and its relatives) and the packed weights come straight
+// into registers, a lane's 16 bytes at a time, each 1 KiB instruction reading one contiguous KiB of fragments.  Nothing a wave
+// reads is read by another wave of the workgroup, so there is no LDS and no barrier in the loop; the waves' sums meet in the LDS once
+// at the end, in a fixed order.  Against gemm_kq_kernel (gemm_mfma.hip), whose waves share a ring of stages in the LDS: that one moves
+// fewer bytes per flop and is the better kernel where its launch fills the machine for many super-blocks, but each of its stage
+// boundaries waits for copies that left one stage earlier, which is what a launch of few tiles spends its time on.
+//
+// Loads of a wave return in order, so a weight load that comes from HBM holds up every fragment load issued after it.  The weights of
+// super-block b + 1 are therefore requested together, behind the fragments of the last stage of b: the first loads that are waited for
+// behind them belong to super-block b + 1 itself.
+#include <hip/hip_ext.h>
+
+#include "gemm_formats.h"
+#include "tuning.h"
+
+namespace {
+
+constexpr int kMaxGroup = 4;
+struct ColsGroup {
+    const uint8_t *w[kMaxGroup];
+    void *y[kMaxGroup];
+    const float *bias[kMaxGroup];
+    int64_t n[kMaxGroup], ldy[kMaxGroup];
+    float wscale[kMaxGroup];
+    int first[kMaxGroup];  // first n-block of the weight
+    int count, second;     // weights from `second` on are of the kernel's second format
+};
+
+// a lane's packed weights of one 32-row tile and one super-block, as the loads deliver them
+template <int DT> struct WBlk;
+// loads: `t` the lane's 16-row tile (scalar base + lane offset `o`), slot = r16 + 32 * g32
+__device__ inline uint4v ld16(const uint8_t *base, uint32_t o) { return *(const uint4v *)(base + o); }
+
+template <> struct WBlk<TURQ_Q4_K> {
+    uint4v q[4], hd;
+    __device__ void load(const uint8_t *p, uint32_t o, uint32_t r16, uint32_t slot) {
+        using F = TiledFmt<TURQ_Q4_K>;
+        hd = ld16(p, o + F::kHDR + 16u * r16);
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++) q[ks] = ld16(p, o + 16u * slot + (uint32_t)((ks & 1) * 1024 + (ks >> 1) * 256));
+    }
+    __device__ GFmt<TURQ_Q4_K>::Hdr hdr() const { return {hd}; }
+    template <int KS> __device__ GFmt<TURQ_Q4_K>::Stage stage() const { return {q[KS]}; }
+};
+template <> struct WBlk<TURQ_Q5_K> {
+    uint4v q[4], hd;
+    uint2v hh[2];
+    __device__ void load(const uint8_t *p, uint32_t o, uint32_t r16, uint32_t slot) {
+        using F = TiledFmt<TURQ_Q5_K>;
+        hd = ld16(p, o + F::kHDR + 16u * r16);
+#pragma unroll
+        for (int s = 0; s < 2; s++) hh[s] = *(const uint2v *)(p + (o + F::kQH + 8u * slot + (uint32_t)(s * 128)));
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++) q[ks] = ld16(p, o + 16u * slot + (uint32_t)((ks & 1) * 1024 + (ks >> 1) * 256));
+    }
+    __device__ GFmt<TURQ_Q5_K>::Hdr hdr() const { return {hd}; }
+    template <int KS> __device__ GFmt<TURQ_Q5_K>::Stage stage() const { return {q[KS], hh[KS >> 1]}; }
+};
+template <> struct WBlk<TURQ_Q6_K> {
+    uint4v ql[4], qh[2];
+    uint32_t sc0, sc1, d16;
+    __device__ void load(const uint8_t *p, uint32_t o, uint32_t r16, uint32_t slot) {
+        using F = TiledFmt<TURQ_Q6_K>;
+        sc0 = *(const uint32_t *)(p + (o + F::kSC + 4u * slot));
+        sc1 = *(const uint32_t *)(p + (o + F::kSC + 4u * slot + 64u));
+        d16 = *(const uint16_t *)(p + (o + F::kD + 2u * r16));
+#pragma unroll
+        for (int s = 0; s < 2; s++) qh[s] = ld16(p, o + F::kQH + 16u * slot + (uint32_t)(s * 256));
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++) ql[ks] = ld16(p, o + 16u * slot + (uint32_t)((ks & 1) * 1024 + (ks >> 1) * 256));
+    }
+    __device__ GFmt<TURQ_Q6_K>::Hdr hdr() const { return {sc0, sc1, d16}; }
+    template <int KS> __device__ GFmt<TURQ_Q6_K>::Stage stage() const { return {ql[KS], qh[KS >> 1]}; }
+};
+template <> struct WBlk<TURQ_Q8_0> {
+    uint4v a[4], b[4], dd;
+    __device__ void load(const uint8_t *p, uint32_t o, uint32_t r16, uint32_t slot) {
+        using F = TiledFmt<TURQ_Q8_0>;
+        dd = ld16(p, o + F::kD + 16u * r16);
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++) {
+            a[ks] = ld16(p, o + 16u * slot + (uint32_t)(ks * 1024));
+            b[ks] = ld16(p, o + 16u * slot + (uint32_t)(ks * 1024 + 256));
+        }
+    }
+    __device__ GFmt<TURQ_Q8_0>::Hdr hdr() const { return {dd}; }
+    template <int KS> __device__ GFmt<TURQ_Q8_0>::Stage stage() const { return {a[KS], b[KS]}; }
+};
+
+template <int MT> struct AStage { half8v f[MT][4]; };
+
+// 16-byte groups (4 neighbouring rows of one column) of a 32 x 32 tile
+constexpr int kGroups = 256;
+// Four waves in every tile shape, and one stage of fragments in flight besides the one being used.  The sums of a result are then the
+// same numbers in the same order whatever the tile (a weight alone and in a launch with others agree to the bit).  Eight waves were up
+// to 7 % faster on the 64-row tile and spill on the larger ones; three stages in flight measured 1 - 8 % slower than one (registers).
+constexpr int W = 4, RA = 2;
+// The waves meet in rounds of T tiles, T x 16 KiB of LDS.
+template <int MT, int NT> struct Meet {
+    static constexpr int T = MT * NT < 4 ? MT * NT : 4;
+    static constexpr int ROUNDS = (MT * NT + T - 1) / T;
+    static constexpr int PER = T;  // groups of a round per thread
+    static constexpr int LDS = W * T * 4096;
+    static_assert(T * kGroups == PER * 64 * W, "every thread adds up the same number of groups");
+};
+
+template <int DT, int MT, int NT>
+__device__ __forceinline__ void cols_body(const ColsGroup &grp, int wi, int nb, int mb, int64_t k, const uint8_t *__restrict__ frags, int64_t m,
+                                          int yt, uint8_t *lds) {
+    using Fm = GFmt<DT>;
+    using Wb = WBlk<DT>;
+    constexpr int TB = TiledFmt<DT>::kTileBytes;
+    constexpr bool SUMS = Fm::SUMS;
+    const uint8_t *__restrict__ w = grp.w[wi];
+    const int64_t n = grp.n[wi];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n32 = lane & 31, g32 = lane >> 5, r16 = n32 & 15, tsel = n32 >> 4;
+    const int ntc = (int)(k / 256);
+    const int64_t mtiles = (m + 31) / 32;
+    const int nrt = (int)turq_tile_rows(n);
+    // this wave's super-blocks
+    const int b0 = ntc * wave / W, b1 = ntc * (wave + 1) / W;
+
+    const uint8_t *a_src[MT];  // (m-tiles past the last: the last one again, never stored)
+#pragma unroll
+    for (int i = 0; i < MT; i++) {
+        const int64_t mt = (int64_t)mb * MT + i;
+        a_src[i] = frags + ((size_t)((mt < mtiles ? mt : mtiles - 1) * ntc * 17) << 10);
+    }
+    const int tile0 = nb * NT * 2;
+    const uint8_t *w_src = w + (size_t)tile0 * ntc * TB;
+    uint32_t w_off[NT];  // the lane's 16-row tile of every 32-row tile
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+        int t = tile0 + 2 * j + tsel;
+        t = t < nrt ? t : nrt - 1;  // (row tiles past the end: the last one again, never stored)
+        w_off[j] = (uint32_t)(t - tile0) * (uint32_t)ntc * (uint32_t)TB;
+    }
+    uint32_t lane16 = 16u * (uint32_t)lane;
+    const uint32_t slot = (uint32_t)(r16 + 32 * g32);
+    const _Float16 ws = (_Float16)grp.wscale[wi];
+
+    float16v acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) acc[i][j][e] = 0.0f;
+
+    AStage<MT> ra[RA];
+    half8v sf[MT];
+    Wb wcur[NT], wnext[NT];
+    auto load_a = [&](int b, auto KS) {
+        constexpr int ks = decltype(KS)::value;
+#pragma unroll
+        for (int i = 0; i < MT; i++) {
+            const uint8_t *p = a_src[i] + ((size_t)(b * 17 + 4 * ks) << 10);
+#pragma unroll
+            for (int st = 0; st < 4; st++) ra[ks % RA].f[i][st] = __builtin_bit_cast(half8v, ld16(p, lane16 + (uint32_t)(st * 1024)));
+        }
+        if constexpr (SUMS && ks == 3) {
+#pragma unroll
+            for (int i = 0; i < MT; i++) sf[i] = __builtin_bit_cast(half8v, ld16(a_src[i] + ((size_t)(b * 17 + 16) << 10), lane16));
+        }
+    };
+    auto load_w = [&](Wb (&dst)[NT], int b) {
+        const uint8_t *p = w_src + (size_t)b * TB;
+#pragma unroll
+        for (int j = 0; j < NT; j++) dst[j].load(p, w_off[j], (uint32_t)r16, slot);
+    };
+    auto block = [&](int b, int bn, auto MORE) {
+        constexpr bool more = decltype(MORE)::value;
+        typename Fm::Consts cs[NT];
+#pragma unroll
+        for (int j = 0; j < NT; j++) cs[j] = Fm::consts(wcur[j].hdr(), g32, ws);
+        static_for<4>([&](auto KS) {
+            constexpr int ks = decltype(KS)::value, ahead = ks + RA - 1;
+            if constexpr (ahead < 4) load_a(b, std::integral_constant<int, ahead>{});
+            else if constexpr (more) load_a(bn, std::integral_constant<int, (ahead & 3)>{});
+            if constexpr (more && ks == 2) load_w(wnext, bn);
+            __builtin_amdgcn_sched_barrier(0);
+            static_for<4>([&](auto ST) {
+                constexpr int st = decltype(ST)::value;
+                half8v bop[NT];
+#pragma unroll
+                for (int j = 0; j < NT; j++) bop[j] = Fm::template operand<ks, st>(wcur[j].template stage<ks>(), cs[j]);
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+#pragma unroll
+                    for (int j = 0; j < NT; j++) acc[i][j] = mfma32x32x16(ra[ks % RA].f[i][st], bop[j], acc[i][j]);
+            });
+            if constexpr (SUMS && ks == 3) {
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+#pragma unroll
+                    for (int j = 0; j < NT; j++) acc[i][j] = mfma32x32x16(sf[i], Fm::bmin(cs[j]), acc[i][j]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        if constexpr (more) {
+#pragma unroll
+            for (int j = 0; j < NT; j++) wcur[j] = wnext[j];
+        }
+    };
+    if (b0 < b1) {
+        const int cnt = b1 - b0;
+        int b = b0;
+        load_w(wcur, b);
+        static_for<RA - 1>([&](auto KS) { load_a(b, KS); });
+        for (int i = 1; i < cnt; i++) {
+            asm volatile("" : "+v"(lane16));
+            const int bn = b + 1 == b1 ? b0 : b + 1;
+            block(b, bn, std::true_type{});
+            b = bn;
+        }
+        block(b, b, std::false_type{});
+    }
+
+    // ---- the waves meet: thread t adds up the groups t, t + 256, ... of a round's tiles ----
+    // group g of tile (i, j) is rows 8 (g / 64) + 4 (g / 32 % 2) .. + 3 of column g % 32
+    using M = Meet<MT, NT>;
+    const float inv_ws = 1.0f / grp.wscale[wi];  // (a power of two: exact)
+    const float *bias = grp.bias[wi];
+    void *y = grp.y[wi];
+    const int64_t ldy = grp.ldy[wi];
+    const int ytb = yt & 0xFF;
+    const int64_t row_g = (int64_t)mb * MT * 32 + 8 * wave + 4 * g32, col_g = (int64_t)nb * NT * 32 + n32;  // of the thread's group of tile (0, 0)
+    float4v *red = (float4v *)lds;  // [wave][tile of the round][group]
+#pragma unroll
+    for (int r = 0; r < M::ROUNDS; r++) {
+        // with TURQ_OUT_ACCUMULATE: what y holds, requested together and ahead of the round, so that it arrives under the meeting
+        float4v old[M::T];
+#pragma unroll
+        for (int t = 0; t < M::T; t++) {
+            old[t] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
+            const int tile = r * M::T + t;
+            if (tile >= MT * NT || !(yt & TURQ_OUT_ACCUMULATE)) continue;
+            const int64_t row = row_g + tile / NT * 32, col = col_g + tile % NT * 32;
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (row + e < m && col < n) {
+                    const int64_t at = (row + e) * ldy + col;
+                    old[t][e] = ytb == TURQ_ACT_F32 ? turq_load_out<TURQ_ACT_F32>(y, at)
+                              : ytb == TURQ_ACT_BF16 ? turq_load_out<TURQ_ACT_BF16>(y, at) : turq_load_out<TURQ_ACT_F16>(y, at);
+                }
+        }
+        if (r) __syncthreads();
+#pragma unroll
+        for (int t = 0; t < M::T; t++) {
+            if (r * M::T + t >= MT * NT) continue;
+            const int i = (r * M::T + t) / NT, j = (r * M::T + t) % NT;
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                red[(wave * M::T + t) * kGroups + q * 64 + lane] = float4v{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+        }
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < M::T; t++) {
+            const int tile = r * M::T + t;
+            if (tile >= MT * NT) continue;
+            float4v s = red[t * kGroups + tid];
+#pragma unroll
+            for (int v = 1; v < W; v++) s += red[(v * M::T + t) * kGroups + tid];
+            const int64_t row = row_g + tile / NT * 32, col = col_g + tile % NT * 32;
+            if (col >= n) continue;
+            const float bv = bias ? bias[col] : 0.0f;
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (row + e < m) turq_store_any(y, ytb, (row + e) * ldy + col, (s[e] * inv_ws + bv) + old[t][e]);
+        }
+    }
+}
+
+template <int DTA, int DTB, int MT, int NT>
+__global__ void __launch_bounds__(64 * W) gemm_cols_kernel(ColsGroup grp, int64_t k, const uint8_t *__restrict__ frags, int64_t m, int yt,
+                                                           int nblocks_n, int nblocks_m) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    // consecutive logical ids run on one XCD (blockIdx % 8): the m-blocks of one n-block share its packed weights in that XCD's L2
+    const int nwg = nblocks_n * nblocks_m;
+    int lid = blockIdx.x;
+    if ((nwg & 7) == 0) lid = (blockIdx.x & 7) * (nwg >> 3) + (blockIdx.x >> 3);
+    const int mb = lid % nblocks_m, nb_all = lid / nblocks_m;
+    int wi = 0;
+#pragma unroll
+    for (int i = 1; i < kMaxGroup; i++)
+        if (i < grp.count && nb_all >= grp.first[i]) wi = i;
+    const int nb = nb_all - grp.first[wi];
+    if (DTA == DTB || wi < grp.second) cols_body<DTA, MT, NT>(grp, wi, nb, mb, k, frags, m, yt, lds);
+    else cols_body<DTB, MT, NT>(grp, wi, nb, mb, k, frags, m, yt, lds);
+}
+
+template <int DTA, int DTB, int MT, int NT>
+hipError_t launch_cols(const TurqGemmWeights &ws, int second, int64_t k, const void *frags, int64_t m, int yt, hipStream_t stream,
+                       hipEvent_t ev_start, hipEvent_t ev_stop) {
+    const auto kernel = gemm_cols_kernel<DTA, DTB, MT, NT>;
+    constexpr int LDS_BYTES = Meet<MT, NT>::LDS;
+    static_assert(LDS_BYTES <= 64 * 1024, "no raised LDS limit");
+    ColsGroup grp{};
+    grp.count = ws.count;
+    grp.second = second;
+    int nbn = 0;
+    for (int i = 0; i < ws.count; i++) {
+        grp.w[i] = (const uint8_t *)ws.w[i];
+        grp.y[i] = ws.y[i];
+        grp.bias[i] = ws.bias[i];
+        grp.n[i] = ws.n[i];
+        grp.ldy[i] = ws.ldy[i];
+        grp.wscale[i] = ws.wscale[i];
+        grp.first[i] = nbn;
+        nbn += (int)((ws.n[i] + 32 * NT - 1) / (32 * NT));
+    }
+    const int nbm = (int)((m + 32 * MT - 1) / (32 * MT));
+    const dim3 grid((unsigned)(nbn * nbm)), block(64 * W);
+    if (ev_start)
+        hipExtLaunchKernelGGL(kernel, grid, block, LDS_BYTES, stream, ev_start, ev_stop, 0, grp, k, (const uint8_t *)frags, m, yt, nbn, nbm);
+    else
+        kernel<<<grid, block, LDS_BYTES, stream>>>(grp, k, (const uint8_t *)frags, m, yt, nbn, nbm);
+    return hipGetLastError();
+}
+
+template <int DTA, int DTB>
+hipError_t launch_tile(int tile, const TurqGemmWeights &ws, int second, int64_t k, const void *frags, int64_t m, int yt, hipStream_t stream,
+                       hipEvent_t ev_start, hipEvent_t ev_stop) {
+    switch (tile) {
+#define TURQ_COLS(MT, NT) \
+    case 10 * MT + NT: return launch_cols<DTA, DTB, MT, NT>(ws, second, k, frags, m, yt, stream, ev_start, ev_stop)
+        TURQ_COLS(1, 1);
+        TURQ_COLS(2, 1);
+        TURQ_COLS(3, 1);
+        TURQ_COLS(2, 2);
+        TURQ_COLS(3, 2);
+        TURQ_COLS(2, 3);
+        TURQ_COLS(4, 2);
+#undef TURQ_COLS
+    default: return hipErrorInvalidValue;
+    }
+}
+
+}  // namespace
+
+bool turq_gemm_cols_mixed(int dtype_a, int dtype_b) { return (dtype_a == TURQ_Q4_K || dtype_a == TURQ_Q5_K) && dtype_b == TURQ_Q6_K; }
+
+// The tile (10 * MT + NT) with which `count` weights of n[i] rows and k columns go through this kernel in one launch, 0 where the launch
+// is gemm_kq_kernel's; *us: roughly what it takes.
+//
+// A launch of one round over the CUs takes base + per_sb * super-blocks, fitted to launches of every format (graphs of launches over more
+// weights than the caches hold); a further round costs as much again without the launch itself, of the smallest tile, of which three workgroups
+// share a CU, three fifths of it.  So the smallest tile that makes the launch one round is the best of them.  Against gemm_kq_kernel:
+//   one or two MFMA tiles: Q6_K 1024 x 4096 at 40 .. 512 rows 14.7 .. 24.9 -> 8.2 .. 11.6 us, Q4_K 4096 x 4096 at 40 / 100 rows 19.3 / 22.8 ->
+//   9.1 / 12.1, Q6_K 4096 x 12288 33 / 43 -> 23 / 29, Q8_0 1024 x 2048 at 40 .. 700 rows 15 -> 6 .. 10;
+//   three or four: Q8_0 4096 x 4096 at 160 / 256 rows 27 -> 15.6 / 18.2, Q4_K at 256 24 -> 16, Q6_K 2048 x 6144 at 512 38 -> 25;
+//   six: from 12 super-blocks on (Q4_K 4096 x 4096 at 300 rows 23.7 -> 22.5, Q6_K 4096 x 12288 73 -> 53; with 8 super-blocks Q4_K 2048 x 2048 at
+//   600 rows 12.6 -> 13.5);
+//   eight: from 40 super-blocks on, Q6_K from 24 (512 rows, 4096 x 12288: Q4_K 66.0 -> 63.8, Q5_K 76 -> 69, Q6_K 84 -> 69; 4096 x 4096: Q4_K 26.0 -> 29.8).
+// Q8_0, whose tile in gemm_kq_kernel is the narrow 128 x 64, takes whichever kernel has the smaller estimate, in any number of rounds
+// (4096 x 12288 at 700 / 1024 / 2048 rows 142 / 160 / 300 -> 102 / 126 / 283; 4096 x 4096 at 700 53 -> 46, at 2048 it stays: 109 against 120).
+int turq_gemm_cols_tile(int dtype_a, int dtype_b, int count, const int64_t *n, int64_t k, int64_t m, int compute_units, double *us) {
+    const TurqTuning &t = turq_tuning();
+    const bool kq_forced = t.gemm_wide >= 0 || t.gemm_low >= 0 || t.gemm_split >= 0 || t.gemm_kgroups != 0 || t.gemm_grid_2x2 || t.gemm_merge >= 0;
+    if (us) *us = 0.0;
+    if (t.gemm_cols == 0 || (t.gemm_cols < 0 && kq_forced)) return 0;
+    if (!turq_dt_is_quant(dtype_a) || (dtype_b != dtype_a && !turq_gemm_cols_mixed(dtype_a, dtype_b))) return 0;
+    if (count < 1 || count > kMaxGroup || m <= 0 || k <= 0 || k % 256 != 0) return 0;
+    if (t.gemm_cols > 0) return t.gemm_cols;
+    const int64_t cus = compute_units > 0 ? compute_units : 256, ntc = k / 256;
+    static constexpr struct { int mt, nt; double base, per_sb; } kTiles[] = {{1, 1, 3.6, 0.42}, {2, 1, 4.4, 0.55}, {3, 1, 5.6, 0.62}, {2, 2, 6.2, 0.72},
+                                                                             {3, 2, 8.0, 0.95}, {2, 3, 8.0, 0.95}, {4, 2, 9.0, 1.18}};
+    const bool eight = dtype_a == TURQ_Q8_0;
+    int best = 0;
+    double best_us = eight ? turq_gemm_launch_us(dtype_a, count, n, k, m, compute_units) : 1e30;
+    for (const auto &c : kTiles) {
+        const int area = c.mt * c.nt;
+        int64_t nbn = 0;
+        for (int i = 0; i < count; i++) nbn += (n[i] + 32 * c.nt - 1) / (32 * c.nt);
+        const int64_t wgs = nbn * ((m + 32 * c.mt - 1) / (32 * c.mt));
+        if (!eight) {
+            if (wgs > (area == 1 ? cus + cus / 2 : cus)) continue;
+            if (area > 4 && ntc < (area == 6 ? 12 : dtype_a == TURQ_Q6_K ? 24 : 40)) continue;
+        }
+        const double x = (double)wgs / (double)cus;
+        const double rounds = x <= 1.0 ? 1.0 : area == 1 ? 1.0 + 0.6 * (x - 1.0) : (double)((wgs + cus - 1) / cus);
+        const double est = kTurqLaunchUs + (c.base + c.per_sb * (double)ntc - kTurqLaunchUs) * rounds;
+        if (est < best_us) {
+            best = 10 * c.mt + c.nt;
+            best_us = est;
+        }
+    }
+    if (us && best) *us = best_us;
+    return best;
+}
+
+// frags: as for turq_launch_gemm_mfma, in the order of the formats (Q8_0, or the K-quants); weights from `second` on are of dtype_b
+hipError_t turq_launch_gemm_cols(int dtype_a, int dtype_b, int second, int tile, const TurqGemmWeights &ws, int64_t k, const void *frags, int64_t m,
+                                 int y_dtype, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop) {
+    if (ws.count < 1 || ws.count > kMaxGroup || k <= 0 || k % 256 != 0 || k / 256 > (1 << 20)) return hipErrorInvalidValue;
+    int64_t n = 0;
+    for (int i = 0; i < ws.count; i++) {
+        if (ws.n[i] <= 0) return ws.count == 1 && ws.n[i] == 0 ? hipSuccess : hipErrorInvalidValue;
+        if (!(ws.wscale[i] >= 6.103515625e-5f && ws.wscale[i] <= 32768.0f)) return hipErrorInvalidValue;
+        n += ws.n[i];
+    }
+    if (m == 0) return hipSuccess;
+    if ((n / 32 + ws.count) * ((m + 31) / 32) > 0x7FFFFFFF) return hipErrorInvalidValue;
+#define TURQ_COLS_TILE(A, B) return launch_tile<A, B>(tile, ws, second, k, frags, m, y_dtype, stream, ev_start, ev_stop)
+    if (dtype_a != dtype_b && second < ws.count) {
+        if (dtype_a == TURQ_Q4_K && dtype_b == TURQ_Q6_K) TURQ_COLS_TILE(TURQ_Q4_K, TURQ_Q6_K);
+        if (dtype_a == TURQ_Q5_K && dtype_b == TURQ_Q6_K) TURQ_COLS_TILE(TURQ_Q5_K, TURQ_Q6_K);
+        return hipErrorInvalidValue;
+    }
+    switch (dtype_a) {
+    case TURQ_Q4_K: TURQ_COLS_TILE(TURQ_Q4_K, TURQ_Q4_K);
+    case TURQ_Q5_K: TURQ_COLS_TILE(TURQ_Q5_K, TURQ_Q5_K);
+    case TURQ_Q6_K: TURQ_COLS_TILE(TURQ_Q6_K, TURQ_Q6_K);
+    case TURQ_Q8_0: TURQ_COLS_TILE(TURQ_Q8_0, TURQ_Q8_0);
+    default: return hipErrorInvalidValue;
+    }
+#undef TURQ_COLS_TILE
+}
+
+TURQ_NONFINITE_READER(turq_nonfinite_gemm_cols)

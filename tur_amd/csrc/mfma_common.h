@@ -326,7 +326,14 @@ struct TurqGemmWeights {
 hipError_t turq_launch_gemm_mfma_group(int dtype, const TurqGemmWeights &ws, int64_t k, const void *frags, int64_t m, int y_dtype,
                                        int compute_units, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop,
                                        void *split_counters = nullptr, void *split_partials = nullptr, size_t split_partial_bytes = 0);
-// the workgroup tile the launch rules pick (0: no kernel for the format)
+// the kernel whose waves split the columns (gemm_cols.hip): its tile for a launch, 0 where gemm_kq_kernel takes it; the launch
+bool turq_gemm_cols_mixed(int dtype_a, int dtype_b);
+int turq_gemm_cols_tile(int dtype_a, int dtype_b, int count, const int64_t *n, int64_t k, int64_t m, int compute_units, double *us = nullptr);
+double turq_gemm_launch_us(int dtype, int count, const int64_t *n, int64_t k, int64_t m, int compute_units);
+constexpr double kTurqLaunchUs = 2.5;  // the share of a launch's time that a further round over the CUs does not pay again
+hipError_t turq_launch_gemm_cols(int dtype_a, int dtype_b, int second, int tile, const TurqGemmWeights &ws, int64_t k, const void *frags, int64_t m,
+                                 int y_dtype, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop);
+// the workgroup tile the launch rules of gemm_kq_kernel pick (0: no kernel for the format)
 int turq_gemm_form(int dtype, int64_t n, int64_t k, int64_t m, int compute_units);
 // the launch the tile rules would make for these rows: its workgroups and the share of its CU rounds it keeps busy (x the wide
 // tile's gain)

@@ -171,14 +171,15 @@ struct GemmSplit {
     void *partials[turq_ctx::kSplitSlots] = {};
     size_t bytes[turq_ctx::kSplitSlots] = {};
 };
-static int gemm_split_reserve(turq_ctx *ctx, int count, const turq_weight *const *w, int64_t m, GemmSplit *out) {
+// (skip: launches that the kernel whose waves split the columns takes, which needs none)
+static int gemm_split_reserve(turq_ctx *ctx, int count, const turq_weight *const *w, int64_t m, const bool *skip, GemmSplit *out) {
     *out = GemmSplit{};
     if (ctx->fixed_scratch || count > turq_ctx::kSplitSlots) return TURQ_OK;
     constexpr size_t kCounters = (size_t)turq_ctx::kSplitSlots * TURQ_GEMM_SPLIT_COUNTER_BYTES;
     size_t off[turq_ctx::kSplitSlots], total = kCounters;
     bool any = false;
     for (int i = 0; i < count; i++) {
-        out->bytes[i] = turq_gemm_split_scratch(w[i]->dtype, w[i]->n, w[i]->k, m, ctx->compute_units, nullptr, nullptr);
+        out->bytes[i] = skip[i] ? 0 : turq_gemm_split_scratch(w[i]->dtype, w[i]->n, w[i]->k, m, ctx->compute_units, nullptr, nullptr);
         off[i] = total;
         total += (out->bytes[i] + 255) & ~(size_t)255;
         any = any || out->bytes[i] != 0;
@@ -201,6 +202,56 @@ static int gemm_split_reserve(turq_ctx *ctx, int count, const turq_weight *const
     return TURQ_OK;
 }
 
+// the weights of one launch as the launchers take them
+static TurqGemmWeights gemm_weights(int count, const turq_weight *const *w, void *const *y, const int64_t *ldy, const float *const *bias,
+                                    const float *ws) {
+    TurqGemmWeights g{};
+    g.count = count;
+    for (int i = 0; i < count; i++) {
+        g.w[i] = w[i]->dev;
+        g.y[i] = y[i];
+        g.bias[i] = bias ? bias[i] : nullptr;
+        g.n[i] = w[i]->n;
+        g.ldy[i] = ldy[i];
+        g.wscale[i] = ws[i];
+    }
+    return g;
+}
+
+// the tile with which the first `count` weights go through gemm_cols.hip in one launch (one format, or Q4_K / Q5_K followed by
+// Q6_K), 0: not; *second: the first weight of the second format
+static int gemm_cols_tile(const turq_ctx *ctx, int count, const turq_weight *const *w, int64_t m, int *second, double *us = nullptr) {
+    int64_t n[4];
+    int s = count;
+    if (count < 1 || count > 4) return 0;
+    for (int i = 0; i < count; i++) {
+        n[i] = w[i]->n;
+        if (w[i]->dtype != w[0]->dtype && s == count) s = i;
+        if (w[i]->n <= 0 || w[i]->k != w[0]->k || w[i]->dtype != w[i < s ? 0 : s]->dtype) return 0;
+    }
+    if (second) *second = s;
+    return turq_gemm_cols_tile(w[0]->dtype, w[s < count ? s : 0]->dtype, count, n, w[0]->k, m, ctx->compute_units, us);
+}
+
+// the prefill GEMM of one weight on the fragments in ctx->act_prep, by either kernel
+static int gemm_on_frags(turq_ctx *ctx, const turq_weight *w, int64_t m, void *y, int yt, int64_t ldy, const float *bias, float wscale) {
+    int second = 1;
+    const int tile = gemm_cols_tile(ctx, 1, &w, m, &second);
+    const bool cols = tile != 0;
+    GemmSplit sp;
+    int rc = gemm_split_reserve(ctx, 1, &w, m, &cols, &sp);
+    if (rc != TURQ_OK) return rc;
+    hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    TURQ_HIP(ctx, turq_prof_next(ctx, &ev0, &ev1));
+    if (cols)
+        TURQ_HIP(ctx, turq_launch_gemm_cols(w->dtype, w->dtype, second, tile, gemm_weights(1, &w, &y, &ldy, &bias, &wscale), w->k, ctx->act_prep, m, yt,
+                                            ctx->stream, ev0, ev1));
+    else
+        TURQ_HIP(ctx, turq_launch_gemm_mfma(w->dtype, w->dev, w->n, w->k, ctx->act_prep, m, y, yt, ldy, bias, wscale, ctx->compute_units,
+                                            ctx->stream, ev0, ev1, sp.counters[0], sp.partials[0], sp.bytes[0]));
+    return TURQ_OK;
+}
+
 // CUs that the GEMM launch for [m, n] takes: its workgroups, by the launcher's choice between the 64-row tile (two of those
 // workgroups share a CU) and the 128-row tiles (one per CU; wide tiles counted as two).  Measured on the Q4_K_M layer: launches
 // of 192 workgroups next to each other help with the 64-row tile (m = 128: +4.8 %) and hurt with the 128-row tile (m = 256: -2.7 %).
@@ -211,6 +262,7 @@ static int64_t gemm_cus_taken_shape(int compute_units, int dtype, int64_t n, int
         const bool whole = form != 4 || turq_gemm_low_two_groups(n, k, m, split, compute_units);
         return whole ? tiles * split : (tiles * split + 1) / 2;
     }
+    if (dtype == TURQ_Q8_0) return ((n + 63) / 64) * ((m + 127) / 128);
     const int64_t nt = (n + 127) / 128, wgs128 = ((m + 127) / 128) * nt;
     const bool low = m <= 64 || 2 * wgs128 <= compute_units;
     if (!low) return wgs128;
@@ -227,11 +279,41 @@ static int64_t gemm_cus_taken(const turq_ctx *ctx, const turq_weight *w, int64_t
 // chosen for all the rows keeps a larger share of its rounds busy (by 5 % at least).  taken_alone: CUs one of them takes.
 static bool gemm_merge_rule(int dtype, int64_t n, int64_t k, int64_t m, int run, int compute_units, int64_t taken_alone) {
     const int64_t cus = compute_units;
-    if (run < 2 || 2 * taken_alone <= cus || !turq_dt_is_quant(dtype) || dtype == TURQ_Q8_0 || n % 256 != 0) return false;
+    if (run < 2 || 2 * taken_alone <= cus || !turq_dt_is_quant(dtype) || n % 256 != 0) return false;
     int64_t wgs_one = 0, wgs_all = 0;
     const double fill_one = turq_gemm_fill(dtype, n, k, m, compute_units, &wgs_one);
     const double fill_all = turq_gemm_fill(dtype, n * run, k, m, compute_units, &wgs_all);
     return (wgs_one < cus && wgs_all <= cus) || fill_all > 1.05 * fill_one;
+}
+
+// how many of the next `left` weights go out as one launch of gemm_kq_kernel (0: the first one alone): see where it is asked
+static int gemm_run(const turq_ctx *ctx, int left, const turq_weight *const *w, int64_t m, bool may_split) {
+    const int merge_env = turq_tuning().gemm_merge;  // 0: never, 2: every run
+    const bool no_merge = merge_env == 0, merge_all = merge_env == 2;
+    const int64_t c = gemm_cus_taken(ctx, w[0], m, may_split);
+    if (no_merge || !(2 * c > ctx->compute_units || merge_all) || !turq_dt_is_quant(w[0]->dtype) || w[0]->n % 256 != 0) return 0;
+    int run = 1;
+    while (run < left && run < 4 && w[run]->dtype == w[0]->dtype && w[run]->n == w[0]->n) run++;
+    return run >= 2 && (merge_all || gemm_merge_rule(w[0]->dtype, w[0]->n, w[0]->k, m, run, ctx->compute_units, c)) ? run : 0;
+}
+
+// what `run` neighbouring weights take as ONE launch of gemm_kq_kernel, where that is known and less than what a launch each takes; else 0.
+// cols: the weights that gemm_cols.hip would take alone
+static double gemm_run_us(const turq_ctx *ctx, int run, const turq_weight *const *w, int64_t m, const bool *cols) {
+    if (run > 4 || turq_tuning().gemm_merge >= 0 || turq_tuning().gemm_cols > 0) return 0.0;
+    int64_t n[4];
+    double apart = 0.0;
+    for (int i = 0; i < run; i++) {
+        if (w[i]->dtype != w[0]->dtype || w[i]->n <= 0 || w[i]->n % 256 != 0) return 0.0;
+        n[i] = w[i]->n;
+        double us = 0.0;
+        if (cols[i]) (void)gemm_cols_tile(ctx, 1, w + i, m, nullptr, &us);
+        else us = turq_gemm_launch_us(w[i]->dtype, 1, n + i, w[i]->k, m, ctx->compute_units);
+        if (us == 0.0) return 0.0;
+        apart += us;
+    }
+    const double us = turq_gemm_launch_us(w[0]->dtype, run, n, w[0]->k, m, ctx->compute_units);
+    return us < apart ? us : 0.0;
 }
 
 int turq_qmatmul_multi_gemm(turq_ctx *ctx, int count, const turq_weight *const *w, const void *x, int xt, int64_t m, int64_t ldx,
@@ -244,8 +326,10 @@ int turq_qmatmul_multi_gemm(turq_ctx *ctx, int count, const turq_weight *const *
         if (!gemm_takes(w[i], &ws[i])) return TURQ_OK;
     int rc = turq_ctx_reserve(ctx, &ctx->act_prep, &ctx->act_prep_cap, turq_act_prep32_bytes(m, w[0]->k));
     if (rc != TURQ_OK) return rc;
+    bool cols[16] = {};  // weights that the kernel whose waves split the columns would take alone
+    for (int i = 0; i < count; i++) cols[i] = gemm_cols_tile(ctx, 1, w + i, m, nullptr) != 0;
     GemmSplit sp;
-    rc = gemm_split_reserve(ctx, count, w, m, &sp);
+    rc = gemm_split_reserve(ctx, count, w, m, cols, &sp);
     if (rc != TURQ_OK) return rc;
     // k_proj / v_proj of a prompt chunk are launches of a quarter of the machine each.  Launches that leave half of the CUs free
     // run in groups, as many as fit the machine together (three at most): the first of a group on the context's stream, the
@@ -257,7 +341,7 @@ int turq_qmatmul_multi_gemm(turq_ctx *ctx, int count, const turq_weight *const *
     int n_small = 0;
     bool one_order = true;
     for (int i = 0; i < count; i++) {
-        n_small += 2 * gemm_cus_taken(ctx, w[i], m, sp.counters[i] != nullptr) <= cus;
+        n_small += !cols[i] && 2 * gemm_cus_taken(ctx, w[i], m, sp.counters[i] != nullptr) <= cus;
         one_order = one_order && (w[i]->dtype == TURQ_Q8_0) == (w[0]->dtype == TURQ_Q8_0);
     }
     const bool fork = !no_side && one_order && n_small >= 2 && side_ready(ctx);
@@ -266,8 +350,6 @@ int turq_qmatmul_multi_gemm(turq_ctx *ctx, int count, const turq_weight *const *
     int64_t group_cus = 0;  // CUs they take together
     int prepared = 0;       // 1: K-quant order, 2: Q8_0 order
     hipError_t e = hipSuccess;
-    const int merge_env = turq_tuning().gemm_merge;  // 0: never, 2: every run
-    const bool no_merge = merge_env == 0, merge_all = merge_env == 2;
     for (int i = 0; i < count && e == hipSuccess; i++) {
         const int order = w[i]->dtype == TURQ_Q8_0 ? 2 : 1;
         if (order != prepared) {
@@ -277,6 +359,35 @@ int turq_qmatmul_multi_gemm(turq_ctx *ctx, int count, const turq_weight *const *
             prepared = order;
         }
         hipStream_t st = ctx->stream;
+        // As many neighbouring weights as one launch takes in about one round over the CUs (q, k and v; k and v; gate and up of a small
+        // model), by either kernel: a launch of few tiles is mostly its start and its end (Q8_0 2 x 3072 x 1024 at 256 rows 21.1 -> 11.1
+        // us), and a second format costs a launch of gemm_cols.hip nothing.
+        {
+            int run = std::min(count - i, 4), tile = 0, second = 0;
+            bool kq = false;
+            for (; run >= 2; run--) {
+                double us = 0.0;
+                if ((w[i + run - 1]->dtype == TURQ_Q8_0) != (order == 2)) continue;
+                tile = gemm_cols_tile(ctx, run, w + i, m, &second, &us);
+                const double kq_us = gemm_run_us(ctx, run, w + i, m, cols + i);
+                kq = kq_us > 0.0 && (tile == 0 || kq_us < us);
+                if (tile != 0 || kq) break;
+            }
+            // (one alone: unless it goes out together with its like below)
+            if (run == 1 && cols[i] && !gemm_run(ctx, count - i, w + i, m, sp.counters[i] != nullptr)) tile = gemm_cols_tile(ctx, 1, w + i, m, &second);
+            if (tile != 0 || kq) {
+                group_n = 0;  // (closes a group of small ones)
+                const TurqGemmWeights g = gemm_weights(run, w + i, y + i, ldy + i, bias ? bias + i : nullptr, ws + i);
+                hipEvent_t ev0 = nullptr, ev1 = nullptr;
+                e = turq_prof_next(ctx, &ev0, &ev1);
+                if (e == hipSuccess)
+                    e = kq ? turq_launch_gemm_mfma_group(w[i]->dtype, g, w[i]->k, ctx->act_prep, m, yt, ctx->compute_units, st, ev0, ev1)
+                           : turq_launch_gemm_cols(w[i]->dtype, w[i + (second < run ? second : 0)]->dtype, second, tile, g, w[i]->k, ctx->act_prep, m,
+                                                   yt, st, ev0, ev1);
+                i += run - 1;
+                continue;
+            }
+        }
         const int64_t c = gemm_cus_taken(ctx, w[i], m, sp.counters[i] != nullptr);
         // Neighbouring weights of one K-quant format and one shape that each take more than half of the machine (gate and up)
         // go out as ONE launch over the rows of all of them where that fills the rounds over the CUs better: where each alone
@@ -284,30 +395,15 @@ int turq_qmatmul_multi_gemm(turq_ctx *ctx, int count, const turq_weight *const *
         // of its rounds busy (Q4_K 2 x 12288 x 4096, two launches -> one: 128 rows 50 -> 42 us, 256 rows 80 -> 67, 1024 rows
         // 257 -> 220; at 384 and 512 rows one launch is 3 % slower and the rule keeps two).  TURQ_GEMM_MERGE = 0: never, 2: every
         // such run whatever its size.
-        if (!no_merge && (2 * c > cus || merge_all) && turq_dt_is_quant(w[i]->dtype) && w[i]->dtype != TURQ_Q8_0 && w[i]->n % 256 == 0) {
-            int j = i + 1;
-            while (j < count && j - i < 4 && w[j]->dtype == w[i]->dtype && w[j]->n == w[i]->n) j++;
-            if (j - i >= 2) {
-                if (merge_all || gemm_merge_rule(w[i]->dtype, w[i]->n, w[i]->k, m, j - i, ctx->compute_units, c)) {
-                    TurqGemmWeights g{};
-                    g.count = j - i;
-                    for (int t = i; t < j; t++) {
-                        g.w[t - i] = w[t]->dev;
-                        g.y[t - i] = y[t];
-                        g.bias[t - i] = bias ? bias[t] : nullptr;
-                        g.n[t - i] = w[t]->n;
-                        g.ldy[t - i] = ldy[t];
-                        g.wscale[t - i] = ws[t];
-                    }
-                    group_n = 0;  // (such a launch closes a group of small ones)
-                    hipEvent_t ev0 = nullptr, ev1 = nullptr;
-                    e = turq_prof_next(ctx, &ev0, &ev1);
-                    if (e == hipSuccess)
-                        e = turq_launch_gemm_mfma_group(w[i]->dtype, g, w[i]->k, ctx->act_prep, m, yt, ctx->compute_units, st, ev0, ev1);
-                    i = j - 1;
-                    continue;
-                }
-            }
+        if (const int run = gemm_run(ctx, count - i, w + i, m, sp.counters[i] != nullptr)) {
+            group_n = 0;  // (such a launch closes a group of small ones)
+            hipEvent_t ev0 = nullptr, ev1 = nullptr;
+            e = turq_prof_next(ctx, &ev0, &ev1);
+            if (e == hipSuccess)
+                e = turq_launch_gemm_mfma_group(w[i]->dtype, gemm_weights(run, w + i, y + i, ldy + i, bias ? bias + i : nullptr, ws + i), w[i]->k,
+                                                ctx->act_prep, m, yt, ctx->compute_units, st, ev0, ev1);
+            i += run - 1;
+            continue;
         }
         if (fork && 2 * c <= cus) {
             if (group_n == 0 || group_n > turq_ctx::kSide || group_cus + c > cus) {
@@ -364,18 +460,6 @@ bool turq_norm_fuses(const turq_ctx *ctx, int count, const turq_weight *const *w
     return true;
 }
 
-// the prefill GEMM of one weight on fragments that already sit in ctx->act_prep
-static int gemm_on_frags(turq_ctx *ctx, const turq_weight *w, int64_t m, void *y, int yt, int64_t ldy, const float *bias, float wscale) {
-    GemmSplit sp;
-    int rc = gemm_split_reserve(ctx, 1, &w, m, &sp);
-    if (rc != TURQ_OK) return rc;
-    hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    TURQ_HIP(ctx, turq_prof_next(ctx, &ev0, &ev1));
-    TURQ_HIP(ctx, turq_launch_gemm_mfma(w->dtype, w->dev, w->n, w->k, ctx->act_prep, m, y, yt, ldy, bias, wscale, ctx->compute_units,
-                                        ctx->stream, ev0, ev1, sp.counters[0], sp.partials[0], sp.bytes[0]));
-    return TURQ_OK;
-}
-
 // `Qwen3MLP::forward` (src/models/qwen3.rs:161-167) on a prompt chunk.  The separate calls write the two products (f32), read
 // them back for SiLU(gate) * up, write that as f16, read it back for down_proj's fragment preparation: here one kernel reads
 // the two products and writes the fragments (the same f16 values, so the results are those of the separate calls bit for bit),
@@ -429,16 +513,9 @@ int turq_qmatmul_mfma(turq_ctx *ctx, const turq_weight *w, const void *x, int xt
     if (m > TURQ_GEMV_MAX_M && algo == TURQ_ALGO_GEMM) {
         int rc = turq_ctx_reserve(ctx, &ctx->act_prep, &ctx->act_prep_cap, turq_act_prep32_bytes(m, w->k));
         if (rc != TURQ_OK) return rc;
-        GemmSplit sp;
-        rc = gemm_split_reserve(ctx, 1, &w, m, &sp);
-        if (rc != TURQ_OK) return rc;
-        hipEvent_t ev0 = nullptr, ev1 = nullptr;
         if (norm) TURQ_HIP(ctx, turq_launch_rms_norm_prep32(w->dtype, x, xt, m, w->k, ldx, norm->w, norm->eps, ctx->act_prep, ctx->stream));
         else TURQ_HIP(ctx, turq_launch_act_prep32(w->dtype, x, xt, m, w->k, ldx, ctx->act_prep, ctx->stream));
-        TURQ_HIP(ctx, turq_prof_next(ctx, &ev0, &ev1));
-        TURQ_HIP(ctx, turq_launch_gemm_mfma(w->dtype, w->dev, w->n, w->k, ctx->act_prep, m, y, yt, ldy, bias, wscale, ctx->compute_units,
-                                            ctx->stream, ev0, ev1, sp.counters[0], sp.partials[0], sp.bytes[0]));
-        return TURQ_OK;
+        return gemm_on_frags(ctx, w, m, y, yt, ldy, bias, wscale);
     }
     const int nwaves = pick_waves(ctx, w->n, w->k);
     for (int64_t m0 = 0; m0 < m; m0 += TURQ_GEMV_MAX_M) {
