@@ -112,3 +112,17 @@ def test_dequantize_full_size_row_block(gpu):
     gpu.release(w)
     want = orc.dequantize(Q4_K, raw)
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("dt,n,k", [(Q4_K, 33, 768), (Q5_K, 17, 512), (Q6_K, 49, 1280), (Q8_0, 35, 96), (Q8_0, 16, 800),
+                                    (Q6_K, 15, 256), (Q8_0, 4112, 8192)])
+def test_tiling_on_the_device_matches_the_host(gpu, dt, n, k):
+    # uploads are tiled by a kernel: every byte of the tensor back through the host's inverse, ragged rows and blocks, a tensor larger than
+    # the buffer that uploads pass through; then one row through it (the kernels read the padding rows and blocks along)
+    raw = synth.random_weight(dt, n, k, seed=n + k)
+    w = gpu.upload(dt, n, k, raw, capi.LAYOUT_TILED)
+    assert np.array_equal(gpu.export(w, raw.size), np.ascontiguousarray(raw).view(np.uint8).reshape(-1))
+    x = synth.random_activation(1, k, seed=1, bf16=True)
+    want = orc.matmul_dequant(dt, x, raw, n, k)
+    assert np.linalg.norm(gpu.qmatmul(w, x, n, k) - want) <= 1e-4 * np.linalg.norm(want)
+    gpu.release(w)

@@ -9,6 +9,7 @@
 #include <cstdio>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <utility>
 #include <vector>
@@ -86,6 +87,8 @@ struct turq_ctx {
     void *stage_x = nullptr;  size_t stage_x_cap = 0;
     void *stage_y = nullptr;  size_t stage_y_cap = 0;
     void *stage_b = nullptr;  size_t stage_b_cap = 0;
+    void *stage_w = nullptr;  // turq_weight_upload: a fixed size, held by one upload at a time (stage_w_mu: uploads may come from several threads)
+    std::mutex stage_w_mu;
     void *act_prep = nullptr; size_t act_prep_cap = 0;
     void *gate_up = nullptr;  size_t gate_up_cap = 0;  // the two f32 products of turq_qmatmul_gate_up's general path
     // the wide-activation path (wide.hip): scaled f16 copy of the activations, per-row inverse scales, f32 results before rescaling
@@ -185,6 +188,8 @@ hipError_t turq_static_scratch(void **ptr, size_t *cap);
 // All are asynchronous on `stream` and return hipGetLastError() of the launch.
 hipError_t turq_launch_gather_rows(int dtype, int layout, const void *w, int64_t n, int64_t k, const uint32_t *ids, int64_t count,
                                    void *out, int out_dtype, int64_t ldo, hipStream_t stream);
+hipError_t turq_launch_tile(int dt, const void *nat, int64_t rows, int64_t k, void *tiled, uint32_t *top, hipStream_t stream);
+hipError_t turq_launch_block_scale(int dt, const void *nat, int64_t blocks, uint32_t *top, hipStream_t stream);
 hipError_t turq_launch_dequant(int dtype, int layout, const void *w, int64_t n, int64_t k, float *out,
                                hipStream_t stream);
 hipError_t turq_launch_wide_scale(const void *x, int x_dtype, int64_t m, int64_t k, int64_t ldx, void *x16, float *inv, hipStream_t stream);
