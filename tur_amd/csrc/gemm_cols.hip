@@ -93,24 +93,21 @@ template <> struct WBlk<TURQ_Q8_0> {
 
 template <int MT> struct AStage { half8v f[MT][4]; };
 
-// 16-byte groups (4 neighbouring rows of one column) of a 32 x 32 tile
-constexpr int kGroups = 256;
 // Four waves in every tile shape, and one stage of fragments in flight besides the one being used.  The sums of a result are then the
 // same numbers in the same order whatever the tile (a weight alone and in a launch with others agree to the bit).  Eight waves were up
 // to 7 % faster on the 64-row tile and spill on the larger ones; three stages in flight measured 1 - 8 % slower than one (registers).
 constexpr int W = 4, RA = 2;
-// The waves meet in rounds of T tiles, T x 16 KiB of LDS.
+// The waves meet in rounds of T tiles, rows of kPitch floats (rows r and r + 4, which a store of a wave writes, lie 16 banks apart).
+constexpr int kPitch = 36;
 template <int MT, int NT> struct Meet {
-    static constexpr int T = MT * NT < 4 ? MT * NT : 4;
+    static constexpr int T = MT * NT < 3 ? MT * NT : MT * NT == 4 || MT * NT == 8 ? 2 : 3;
     static constexpr int ROUNDS = (MT * NT + T - 1) / T;
-    static constexpr int PER = T;  // groups of a round per thread
-    static constexpr int LDS = W * T * 4096;
-    static_assert(T * kGroups == PER * 64 * W, "every thread adds up the same number of groups");
+    static constexpr int LDS = W * T * 32 * kPitch * 4;
 };
 
 template <int DT, int MT, int NT>
 __device__ __forceinline__ void cols_body(const ColsGroup &grp, int wi, int nb, int mb, int64_t k, const uint8_t *__restrict__ frags, int64_t m,
-                                          int yt, uint8_t *lds) {
+                                          int yt, int vec_out, uint8_t *lds) {
     using Fm = GFmt<DT>;
     using Wb = WBlk<DT>;
     constexpr int TB = TiledFmt<DT>::kTileBytes;
@@ -222,16 +219,19 @@ __device__ __forceinline__ void cols_body(const ColsGroup &grp, int wi, int nb, 
         block(b, b, std::false_type{});
     }
 
-    // ---- the waves meet: thread t adds up the groups t, t + 256, ... of a round's tiles ----
-    // group g of tile (i, j) is rows 8 (g / 64) + 4 (g / 32 % 2) .. + 3 of column g % 32
+    // ---- the waves meet: thread t adds up, of every tile, the four columns 4 (t % 8) .. + 3 of row t / 8 ----
+    // (stored as they lie: 16 or 8 bytes per lane.  With a lane's four values in one column, as the MFMA leaves them, the stores were 4 us of a
+    // launch of eight tiles per workgroup and 3 us of one of four)
     using M = Meet<MT, NT>;
     const float inv_ws = 1.0f / grp.wscale[wi];  // (a power of two: exact)
     const float *bias = grp.bias[wi];
     void *y = grp.y[wi];
     const int64_t ldy = grp.ldy[wi];
     const int ytb = yt & 0xFF;
-    const int64_t row_g = (int64_t)mb * MT * 32 + 8 * wave + 4 * g32, col_g = (int64_t)nb * NT * 32 + n32;  // of the thread's group of tile (0, 0)
-    float4v *red = (float4v *)lds;  // [wave][tile of the round][group]
+    const float lim = turq_finite_limit(ytb);
+    uint32_t bad = 0;
+    const int64_t row_t = (int64_t)mb * MT * 32 + (tid >> 3), col_t = (int64_t)nb * NT * 32 + 4 * (tid & 7);
+    float *red = (float *)lds;  // [wave][tile of the round][row][kPitch]
 #pragma unroll
     for (int r = 0; r < M::ROUNDS; r++) {
         // with TURQ_OUT_ACCUMULATE: what y holds, requested together and ahead of the round, so that it arrives under the meeting
@@ -241,45 +241,74 @@ __device__ __forceinline__ void cols_body(const ColsGroup &grp, int wi, int nb, 
             old[t] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
             const int tile = r * M::T + t;
             if (tile >= MT * NT || !(yt & TURQ_OUT_ACCUMULATE)) continue;
-            const int64_t row = row_g + tile / NT * 32, col = col_g + tile % NT * 32;
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                if (row + e < m && col < n) {
-                    const int64_t at = (row + e) * ldy + col;
-                    old[t][e] = ytb == TURQ_ACT_F32 ? turq_load_out<TURQ_ACT_F32>(y, at)
-                              : ytb == TURQ_ACT_BF16 ? turq_load_out<TURQ_ACT_BF16>(y, at) : turq_load_out<TURQ_ACT_F16>(y, at);
+            const int64_t row = row_t + tile / NT * 32, col = col_t + tile % NT * 32, at = row * ldy + col;
+            if (row >= m || col >= n) continue;
+            if (vec_out) {
+                if (ytb == TURQ_ACT_F32) {
+                    old[t] = *(const float4v *)((const float *)y + at);
+                } else {
+                    const uint2v u = *(const uint2v *)((const uint16_t *)y + at);
+                    if (ytb == TURQ_ACT_BF16) {
+                        old[t] = float4v{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xFFFF0000u), __uint_as_float(u.y << 16), __uint_as_float(u.y & 0xFFFF0000u)};
+                    } else {
+                        const half2v a = as_half2(u.x), c = as_half2(u.y);
+                        old[t] = float4v{(float)a.x, (float)a.y, (float)c.x, (float)c.y};
+                    }
                 }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (col + e < n)
+                        old[t][e] = ytb == TURQ_ACT_F32 ? turq_load_out<TURQ_ACT_F32>(y, at + e)
+                                  : ytb == TURQ_ACT_BF16 ? turq_load_out<TURQ_ACT_BF16>(y, at + e) : turq_load_out<TURQ_ACT_F16>(y, at + e);
+            }
         }
         if (r) __syncthreads();
 #pragma unroll
         for (int t = 0; t < M::T; t++) {
             if (r * M::T + t >= MT * NT) continue;
             const int i = (r * M::T + t) / NT, j = (r * M::T + t) % NT;
+            // lane (n32, g32), register e: row 8 (e / 4) + 4 g32 + e % 4 of column n32
 #pragma unroll
-            for (int q = 0; q < 4; q++)
-                red[(wave * M::T + t) * kGroups + q * 64 + lane] = float4v{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+            for (int e = 0; e < 16; e++) red[((wave * M::T + t) * 32 + 8 * (e >> 2) + 4 * g32 + (e & 3)) * kPitch + n32] = acc[i][j][e];
         }
         __syncthreads();
 #pragma unroll
         for (int t = 0; t < M::T; t++) {
             const int tile = r * M::T + t;
             if (tile >= MT * NT) continue;
-            float4v s = red[t * kGroups + tid];
+            const int at_lds = (t * 32 + (tid >> 3)) * kPitch + 4 * (tid & 7);
+            float4v s = *(const float4v *)(red + at_lds);
 #pragma unroll
-            for (int v = 1; v < W; v++) s += red[(v * M::T + t) * kGroups + tid];
-            const int64_t row = row_g + tile / NT * 32, col = col_g + tile % NT * 32;
-            if (col >= n) continue;
-            const float bv = bias ? bias[col] : 0.0f;
+            for (int v = 1; v < W; v++) s += *(const float4v *)(red + v * (M::T * 32 * kPitch) + at_lds);
+            const int64_t row = row_t + tile / NT * 32, col = col_t + tile % NT * 32, at = row * ldy + col;
+            if (row >= m || col >= n) continue;
+            float o[4];
 #pragma unroll
-            for (int e = 0; e < 4; e++)
-                if (row + e < m) turq_store_any(y, ytb, (row + e) * ldy + col, (s[e] * inv_ws + bv) + old[t][e]);
+            for (int e = 0; e < 4; e++) o[e] = (s[e] * inv_ws + (bias && col + e < n ? bias[col + e] : 0.0f)) + old[t][e];
+            if (vec_out) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) turq_note_accum(o[e], lim, bad);
+                if (ytb == TURQ_ACT_F32) {
+                    *(float4v *)((float *)y + at) = float4v{o[0], o[1], o[2], o[3]};
+                } else if (ytb == TURQ_ACT_BF16) {
+                    *(uint2v *)((uint16_t *)y + at) = uint2v{turq_f2bf_x2(o[0], o[1]), turq_f2bf_x2(o[2], o[3])};
+                } else {
+                    *(uint2v *)((uint16_t *)y + at) = uint2v{as_u32(half2v{(_Float16)o[0], (_Float16)o[1]}), as_u32(half2v{(_Float16)o[2], (_Float16)o[3]})};
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (col + e < n) turq_store_any(y, ytb, at + e, o[e]);
+            }
         }
     }
+    turq_note_flush(bad);
 }
 
 template <int DTA, int DTB, int MT, int NT>
 __global__ void __launch_bounds__(64 * W) gemm_cols_kernel(ColsGroup grp, int64_t k, const uint8_t *__restrict__ frags, int64_t m, int yt,
-                                                           int nblocks_n, int nblocks_m) {
+                                                           int nblocks_n, int nblocks_m, int vec_out) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     // consecutive logical ids run on one XCD (blockIdx % 8): the m-blocks of one n-block share its packed weights in that XCD's L2
     const int nwg = nblocks_n * nblocks_m;
@@ -291,8 +320,8 @@ __global__ void __launch_bounds__(64 * W) gemm_cols_kernel(ColsGroup grp, int64_
     for (int i = 1; i < kMaxGroup; i++)
         if (i < grp.count && nb_all >= grp.first[i]) wi = i;
     const int nb = nb_all - grp.first[wi];
-    if (DTA == DTB || wi < grp.second) cols_body<DTA, MT, NT>(grp, wi, nb, mb, k, frags, m, yt, lds);
-    else cols_body<DTB, MT, NT>(grp, wi, nb, mb, k, frags, m, yt, lds);
+    if (DTA == DTB || wi < grp.second) cols_body<DTA, MT, NT>(grp, wi, nb, mb, k, frags, m, yt, vec_out, lds);
+    else cols_body<DTB, MT, NT>(grp, wi, nb, mb, k, frags, m, yt, vec_out, lds);
 }
 
 template <int DTA, int DTB, int MT, int NT>
@@ -304,8 +333,10 @@ hipError_t launch_cols(const TurqGemmWeights &ws, int second, int64_t k, const v
     ColsGroup grp{};
     grp.count = ws.count;
     grp.second = second;
-    int nbn = 0;
+    const int es = (yt & 0xFF) == TURQ_ACT_F32 ? 4 : 2;
+    int nbn = 0, vec_out = 1;  // rows of y can be written four aligned columns at a time (every weight of the launch, or none)
     for (int i = 0; i < ws.count; i++) {
+        vec_out = vec_out && (uintptr_t)ws.y[i] % (4 * es) == 0 && ws.ldy[i] % 4 == 0 && ws.n[i] % 4 == 0;
         grp.w[i] = (const uint8_t *)ws.w[i];
         grp.y[i] = ws.y[i];
         grp.bias[i] = ws.bias[i];
@@ -318,9 +349,9 @@ hipError_t launch_cols(const TurqGemmWeights &ws, int second, int64_t k, const v
     const int nbm = (int)((m + 32 * MT - 1) / (32 * MT));
     const dim3 grid((unsigned)(nbn * nbm)), block(64 * W);
     if (ev_start)
-        hipExtLaunchKernelGGL(kernel, grid, block, LDS_BYTES, stream, ev_start, ev_stop, 0, grp, k, (const uint8_t *)frags, m, yt, nbn, nbm);
+        hipExtLaunchKernelGGL(kernel, grid, block, LDS_BYTES, stream, ev_start, ev_stop, 0, grp, k, (const uint8_t *)frags, m, yt, nbn, nbm, vec_out);
     else
-        kernel<<<grid, block, LDS_BYTES, stream>>>(grp, k, (const uint8_t *)frags, m, yt, nbn, nbm);
+        kernel<<<grid, block, LDS_BYTES, stream>>>(grp, k, (const uint8_t *)frags, m, yt, nbn, nbm, vec_out);
     return hipGetLastError();
 }
 
@@ -352,14 +383,14 @@ bool turq_gemm_cols_mixed(int dtype_a, int dtype_b) { return (dtype_a == TURQ_Q4
 // A launch of one round over the CUs takes base + per_sb * super-blocks, fitted to launches of every format (graphs of launches over more
 // weights than the caches hold); a further round costs as much again without the launch itself, of the smallest tile, of which three workgroups
 // share a CU, three fifths of it.  So the smallest tile that makes the launch one round is the best of them.  Against gemm_kq_kernel:
-//   one or two MFMA tiles: Q6_K 1024 x 4096 at 40 .. 512 rows 14.7 .. 24.9 -> 8.2 .. 11.6 us, Q4_K 4096 x 4096 at 40 / 100 rows 19.3 / 22.8 ->
-//   9.1 / 12.1, Q6_K 4096 x 12288 33 / 43 -> 23 / 29, Q8_0 1024 x 2048 at 40 .. 700 rows 15 -> 6 .. 10;
-//   three or four: Q8_0 4096 x 4096 at 160 / 256 rows 27 -> 15.6 / 18.2, Q4_K at 256 24 -> 16, Q6_K 2048 x 6144 at 512 38 -> 25;
-//   six: from 12 super-blocks on (Q4_K 4096 x 4096 at 300 rows 23.7 -> 22.5, Q6_K 4096 x 12288 73 -> 53; with 8 super-blocks Q4_K 2048 x 2048 at
-//   600 rows 12.6 -> 13.5);
-//   eight: from 40 super-blocks on, Q6_K from 24 (512 rows, 4096 x 12288: Q4_K 66.0 -> 63.8, Q5_K 76 -> 69, Q6_K 84 -> 69; 4096 x 4096: Q4_K 26.0 -> 29.8).
+//   one or two MFMA tiles: Q4_K 1024 x 4096 at 40 / 300 / 512 rows 13.0 / 19.0 / 19.1 -> 6.6 / 9.3 / 10.7 us, 4096 x 4096 at 40 / 100 rows 19.2 /
+//   22.6 -> 8.7 / 11.3, Q6_K 4096 x 12288 33 / 43 -> 23 / 29, Q8_0 2048 x 2048 15 -> 5.4 / 5.5;
+//   three or four: Q8_0 2048 x 2048 at 300 / 512 rows 15.4 -> 8.5 / 10.2, Q4_K 4096 x 4096 at 256 24 -> 15;
+//   six: from 12 super-blocks on (Q4_K 4096 x 4096 at 300 rows 23.4 -> 20.4, Q6_K 4096 x 12288 74 -> 51; with 4 super-blocks Q8_0 6144 x 1024
+//   at 160 rows 11.1 -> 11.7);
+//   eight: from 40 super-blocks on, Q6_K from 24 (512 rows, 4096 x 12288: Q4_K 66 -> 64, Q5_K 76 -> 69, Q6_K 81 -> 66; 4096 x 4096: Q4_K 26.3 -> 27.5).
 // Q8_0, whose tile in gemm_kq_kernel is the narrow 128 x 64, takes whichever kernel has the smaller estimate, in any number of rounds
-// (4096 x 12288 at 700 / 1024 / 2048 rows 142 / 160 / 300 -> 102 / 126 / 283; 4096 x 4096 at 700 53 -> 46, at 2048 it stays: 109 against 120).
+// (4096 x 4096 at 512 / 700 rows 31 / 53 -> 29 / 41, 4096 x 12288 at 1024 / 2048 rows 160 / 300 -> 126 / 283).
 int turq_gemm_cols_tile(int dtype_a, int dtype_b, int count, const int64_t *n, int64_t k, int64_t m, int compute_units, double *us) {
     const TurqTuning &t = turq_tuning();
     const bool kq_forced = t.gemm_wide >= 0 || t.gemm_low >= 0 || t.gemm_split >= 0 || t.gemm_kgroups != 0 || t.gemm_grid_2x2 || t.gemm_merge >= 0;
@@ -369,8 +400,8 @@ int turq_gemm_cols_tile(int dtype_a, int dtype_b, int count, const int64_t *n, i
     if (count < 1 || count > kMaxGroup || m <= 0 || k <= 0 || k % 256 != 0) return 0;
     if (t.gemm_cols > 0) return t.gemm_cols;
     const int64_t cus = compute_units > 0 ? compute_units : 256, ntc = k / 256;
-    static constexpr struct { int mt, nt; double base, per_sb; } kTiles[] = {{1, 1, 3.6, 0.42}, {2, 1, 4.4, 0.55}, {3, 1, 5.6, 0.62}, {2, 2, 6.2, 0.72},
-                                                                             {3, 2, 8.0, 0.95}, {2, 3, 8.0, 0.95}, {4, 2, 9.0, 1.18}};
+    static constexpr struct { int mt, nt; double base, per_sb; } kTiles[] = {{1, 1, 3.2, 0.40}, {2, 1, 4.0, 0.52}, {3, 1, 4.6, 0.60}, {2, 2, 5.2, 0.68},
+                                                                             {3, 2, 6.2, 0.92}, {2, 3, 6.2, 0.92}, {4, 2, 7.0, 1.20}};
     const bool eight = dtype_a == TURQ_Q8_0;
     int best = 0;
     double best_us = eight ? turq_gemm_launch_us(dtype_a, count, n, k, m, compute_units) : 1e30;
