@@ -718,6 +718,22 @@ def test_staged_rows_kernel(dts, k):
         own.close()
 
 
+# 17 .. 32 rows of more than 4096 columns: rows of f32, and rows that cannot be loaded 16 bytes at a time, are rounded to f16 rows in
+# scratch first; the same values as 16-bit rows take no scratch and give the same bits.  n = 200 ends inside a row tile, 4112 rows are
+# 257 row tiles (two per workgroup), 4608 / 9728 columns nine / nineteen pairs for eight waves.  Tolerance: f32 sums in another order.
+@pytest.mark.parametrize("dt,n,k", [(Q4_K, 200, 9728), (Q4_K, 4112, 4608), (Q5_K, 200, 4608), (Q6_K, 200, 9728), (Q6_K, 4112, 4608), (Q8_0, 4112, 4608)])
+def test_wide_rows_give_the_same_bits_in_every_type(gpu, dt, n, k):
+    raw = synth.random_weight(dt, n, k, seed=n + k)
+    w = gpu.upload(dt, n, k, raw, capi.LAYOUT_TILED)
+    for m in (17, 32):
+        x = f16_round(synth.random_activation(m, k, seed=m + k, bf16=True))
+        y = gpu.qmatmul(w, x, n, k, x_dtype=capi.ACT_F16)
+        assert rel_l2(y, orc.matmul_dequant(dt, x, raw, n, k)) <= 2e-5
+        for x_dtype, ldx in ((capi.ACT_F32, k), (capi.ACT_F32, k + 1), (capi.ACT_F16, k + 3), (capi.ACT_F16, k + 8)):
+            assert np.array_equal(gpu.qmatmul(w, x, n, k, x_dtype=x_dtype, ldx=ldx), y), (m, x_dtype, ldx)
+    gpu.release(w)
+
+
 # ... and with each of its row-tile group sizes forced (the rule takes one row tile per workgroup for matrices this small)
 @pytest.mark.parametrize("row_tiles", [2, 3, 6])
 def test_staged_rows_kernel_group_sizes(row_tiles):

@@ -101,6 +101,31 @@ hipError_t launch(int dtype, const void *x, int64_t m, int64_t k, int64_t ldx, v
     return hipGetLastError();
 }
 
+// ---- rows as f16, for the kernels that read rows (gemv_cs_staged.h): one launch of 8 columns per thread, k a multiple of 8 ----
+// Bound by the launch itself (32 x 12288: 1.5 MB in, 0.8 MB out); it stands in for the fragment preparation where the rows are f32.
+template <int XT>
+__global__ void __launch_bounds__(256) act_rows_f16_kernel(const void *__restrict__ x, int64_t pieces, int64_t per_row, int64_t ldx, half8v *__restrict__ out) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= pieces) return;
+    const int64_t at = i / per_row * ldx + i % per_row * 8;
+    float v[8];
+    const float4v *p = (const float4v *)((const float *)x + at);
+    if (XT == TURQ_ACT_F32 && ((uintptr_t)p & 15) == 0) {
+        const float4v lo = p[0], hi = p[1];
+        v[0] = lo.x, v[1] = lo.y, v[2] = lo.z, v[3] = lo.w, v[4] = hi.x, v[5] = hi.y, v[6] = hi.z, v[7] = hi.w;
+    } else {
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = ld_act<XT>(x, at + j);
+    }
+    half8v h;
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        turq_note_result<TURQ_ACT_F16>(v[j]);
+        h[j] = (_Float16)v[j];
+    }
+    out[i] = h;
+}
+
 // ---- fragments for the prefill GEMM (v_mfma_f32_32x32x16_f16) ----
 // 32-row m-tiles; per 256-column tile b there are 16 operand steps plus one group-sum step.  Lane
 // (r, g32) = r + 32 * g32 of step q holds x[32 mt + r][256 b + 128 g32 + 8 q + j], j = 0..7; step 16
@@ -201,6 +226,21 @@ hipError_t turq_launch_act_prep(int dtype, const void *x, int x_dtype, int64_t m
     case TURQ_ACT_F16: return launch<TURQ_ACT_F16>(dtype, x, m, k, ldx, frags, stream);
     default: return hipErrorInvalidValue;
     }
+}
+
+// out: [m, k] f16, rows without a gap; k a multiple of 8
+hipError_t turq_launch_act_rows_f16(const void *x, int x_dtype, int64_t m, int64_t k, int64_t ldx, void *out, hipStream_t stream) {
+    if (m == 0 || k == 0) return hipSuccess;
+    if (m < 0 || k < 0 || k % 8 != 0 || m > TURQ_GEMV_MAX_M || k > ((int64_t)1 << 31)) return hipErrorInvalidValue;
+    const int64_t per_row = k / 8, pieces = m * per_row;
+    const unsigned grid = (unsigned)((pieces + 255) / 256);
+    switch (x_dtype) {
+    case TURQ_ACT_F32: act_rows_f16_kernel<TURQ_ACT_F32><<<grid, 256, 0, stream>>>(x, pieces, per_row, ldx, (half8v *)out); break;
+    case TURQ_ACT_BF16: act_rows_f16_kernel<TURQ_ACT_BF16><<<grid, 256, 0, stream>>>(x, pieces, per_row, ldx, (half8v *)out); break;
+    case TURQ_ACT_F16: act_rows_f16_kernel<TURQ_ACT_F16><<<grid, 256, 0, stream>>>(x, pieces, per_row, ldx, (half8v *)out); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
 }
 
 hipError_t turq_launch_act_prep32(int dtype, const void *x, int x_dtype, int64_t m, int64_t k, int64_t ldx, void *frags,

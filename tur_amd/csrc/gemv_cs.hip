@@ -205,11 +205,12 @@ hipError_t turq_launch_gemv_cs_staged_f16(TURQ_STAGED_LAUNCH_ARGS);
 
 // whether the staged form has this case: formats (dtype_b = dtype_a for one format, else a K-quant pair with Q6_K second),
 // k, m and row tiles per workgroup (1, 2; 3 up to 16 rows; 6 up to 16 rows and, in the four-wave form, from 17)
-bool turq_gemv_cs_staged_takes(int dtype_a, int dtype_b, int64_t k, int64_t m, int row_tiles) {
+bool turq_gemv_cs_staged_takes(int dtype_a, int dtype_b, int x_dtype, int64_t k, int64_t m, int row_tiles) {
     if (!turq_gemv_cs_staged_waves(k) || m < 1 || m > 32) return false;
     if (dtype_a != dtype_b && !((dtype_a == TURQ_Q4_K || dtype_a == TURQ_Q5_K) && dtype_b == TURQ_Q6_K)) return false;
     if (dtype_a != TURQ_Q4_K && dtype_a != TURQ_Q5_K && dtype_a != TURQ_Q6_K && dtype_a != TURQ_Q8_0) return false;
-    if (m > 16 && row_tiles != 6 && k > 4096) return false;  // the two passes of 16 rows are only built with one pair per wave
+    // (the two passes of 16 rows of f32 are only built with one pair per wave)
+    if (m > 16 && row_tiles != 6 && k > 4096 && x_dtype == TURQ_ACT_F32) return false;
     return row_tiles == 1 || row_tiles == 2 || (row_tiles == 3 && m <= 16) || row_tiles == 6;
 }
 
@@ -222,7 +223,7 @@ hipError_t turq_launch_gemv_cs_staged(int dtype_a, int dtype_b, int count, int s
                                       const void *x, int x_dtype, int64_t ldx, int64_t m, void *const *y, int y_dtype, const int64_t *ldy,
                                       const float *const *bias, int row_tiles, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop) {
     if (count < 1 || count > kMaxMulti || second < 1 || second > count || (second == count) != (dtype_a == dtype_b) ||
-        !turq_gemv_cs_staged_takes(dtype_a, dtype_b, k, m, row_tiles))
+        !turq_gemv_cs_staged_takes(dtype_a, dtype_b, x_dtype, k, m, row_tiles))
         return hipErrorInvalidValue;
     if (!turq_yt_ok(y_dtype, true)) return hipErrorInvalidValue;
     switch (x_dtype) {

@@ -413,12 +413,12 @@ template <int MR, int RG> size_t staged_lds(int nwaves) {
     return std::max((size_t)nwaves * (MR / HV) * kXRow, (size_t)nwaves * RG * HV * 64 * sizeof(float4v));
 }
 
-// one pair per wave (up to 4096 columns) written out, anything else counted at run time; more than 16 rows are only taken on
-// up to 4096 columns
+// one pair per wave (up to 4096 columns) written out, anything else counted at run time; more than 16 rows of f32 are only taken on
+// up to 4096 columns (turq_gemv_cs_staged_takes)
 template <int DTA, int DTB, int XT, int MR, int RG>
 hipError_t staged_count(const StagedLaunch &l) {
     if (l.cnt == 1) return staged_go<gemv_cs_staged_kernel<DTA, DTB, XT, MR, RG, 1>>(staged_lds<MR, RG>(l.nwaves), l);
-    if constexpr (MR <= 16) return staged_go<gemv_cs_staged_kernel<DTA, DTB, XT, MR, RG, 0>>(staged_lds<MR, RG>(l.nwaves), l);
+    if constexpr (MR <= 16 || XT != TURQ_ACT_F32) return staged_go<gemv_cs_staged_kernel<DTA, DTB, XT, MR, RG, 0>>(staged_lds<MR, RG>(l.nwaves), l);
     return hipErrorInvalidValue;
 }
 

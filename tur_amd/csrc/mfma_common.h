@@ -233,6 +233,7 @@ __host__ __device__ inline size_t turq_act_prep32_bytes(int64_t m, int64_t k) {
 }
 
 // launchers (act_prep.hip, gemv_mfma.hip)
+hipError_t turq_launch_act_rows_f16(const void *x, int x_dtype, int64_t m, int64_t k, int64_t ldx, void *out, hipStream_t stream);
 hipError_t turq_launch_act_prep32(int dtype, const void *x, int x_dtype, int64_t m, int64_t k, int64_t ldx, void *frags,
                                   hipStream_t stream);
 hipError_t turq_launch_rms_norm_prep32(int dtype, const void *x, int x_dtype, int64_t m, int64_t k, int64_t ldx, const float *weight,
@@ -285,7 +286,7 @@ bool turq_gemv_cs_rows_ok(int row_tiles_per_group);
 hipError_t turq_launch_gemv_cs(int dtype, int count, const void *const *w_tiled, const int64_t *n, int64_t k, const void *x, int x_dtype,
                                int64_t ldx, int64_t m, void *const *y, int y_dtype, const int64_t *ldy, const float *const *bias,
                                int nwaves, int row_tiles, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop);
-bool turq_gemv_cs_staged_takes(int dtype_a, int dtype_b, int64_t k, int64_t m, int row_tiles);
+bool turq_gemv_cs_staged_takes(int dtype_a, int dtype_b, int x_dtype, int64_t k, int64_t m, int row_tiles);
 int turq_gemv_cs_staged_second_rows(int row_tiles);
 hipError_t turq_launch_gemv_cs_staged(int dtype_a, int dtype_b, int count, int second, const void *const *w_tiled, const int64_t *n,
                                       int64_t k, const void *x, int x_dtype, int64_t ldx, int64_t m, void *const *y, int y_dtype,

@@ -95,7 +95,7 @@ int cs_row_tiles(const turq_ctx *ctx, int64_t m, int64_t row_tiles, int dtype, b
 // pays for small launches, where it replaces a preparation launch and a kernel that re-reads prepared fragments: row tiles per
 // workgroup so that the launch is about one workgroup per compute unit.  0: not this call.  TURQ_CS_STAGED = 0 switches it off,
 // TURQ_CS_RG forces the group size.
-int staged_row_tiles(const turq_ctx *ctx, int dtype_a, int dtype_b, int64_t k, int64_t m, int64_t row_tiles, int64_t row_tiles_b,
+int staged_row_tiles(const turq_ctx *ctx, int dtype_a, int dtype_b, int xt, int64_t k, int64_t m, int64_t row_tiles, int64_t row_tiles_b,
                      bool aligned) {
     const TurqTuning &tune = turq_tuning();
     const int mode = tune.cs_staged, forced = tune.cs_rg, min_m = tune.cs_staged_min_m, max_m = tune.cs_staged_max_m;
@@ -110,15 +110,17 @@ int staged_row_tiles(const turq_ctx *ctx, int dtype_a, int dtype_b, int64_t k, i
         const int gb = turq_gemv_cs_staged_second_rows(g);
         if ((row_tiles - row_tiles_b + g - 1) / g + (row_tiles_b + gb - 1) / gb <= cus) rg = g;
     }
-    // more than 16 rows: on weights of up to 4096 columns (beyond, the f32 rows that every unit reads outweigh the preparation
-    // launch); up to two row tiles per unit as two passes of 16 rows, more in the four-wave form with groups of six
+    // more than 16 rows: on weights of up to 4096 columns up to two row tiles per unit as two passes of 16 rows, more in the four-wave
+    // form with groups of six; on wider ones (where the f32 rows that every unit reads would outweigh a preparation launch) the two
+    // passes on 16-bit rows.  Whole calls at 32 bf16 rows, prepared fragments -> here: Q6_K 4096 x 12288 24.6 -> 22.3 us, Q4_K 8192 x
+    // 8192 27.7 -> 21.9, Q8_0 2048 x 6144 16.4 -> 11.3; f32 rows 24.5 -> 23.7, 27.9 -> 21.8, 16.4 -> 13.1
     if (m > 16 && !forced) {
-        if (k > 4096) return 0;
+        if (k > 4096 && (xt == TURQ_ACT_F32 || row_tiles > 2 * cus)) return 0;
         if (row_tiles > 2 * cus) rg = 6;  // the four-wave form
     }
     if (forced) rg = forced;
-    while (rg > 1 && !turq_gemv_cs_staged_takes(dtype_a, dtype_b, k, m, rg)) rg = rg == 6 ? 3 : rg - 1;
-    return turq_gemv_cs_staged_takes(dtype_a, dtype_b, k, m, rg) ? rg : 0;
+    while (rg > 1 && !turq_gemv_cs_staged_takes(dtype_a, dtype_b, xt, k, m, rg)) rg = rg == 6 ? 3 : rg - 1;
+    return turq_gemv_cs_staged_takes(dtype_a, dtype_b, xt, k, m, rg) ? rg : 0;
 }
 
 // whether the prefill GEMM can take this weight (its largest packed value must fit f16), and the power of two by which the
@@ -570,7 +572,7 @@ bool turq_rows_in_chunks(const turq_ctx *ctx, int count, const turq_weight *cons
         row_tiles += turq_tile_rows(w[i]->n);
     }
     if (row_tiles <= 2 * cus) return false;
-    return staged_row_tiles(ctx, w[0]->dtype, w[0]->dtype, w[0]->k, TURQ_GEMV_MAX_M, row_tiles, 0, aligned) == 6;
+    return staged_row_tiles(ctx, w[0]->dtype, w[0]->dtype, xt, w[0]->k, TURQ_GEMV_MAX_M, row_tiles, 0, aligned) == 6;
 }
 
 int turq_qmatmul_gate_up_mfma(turq_ctx *ctx, const turq_weight *gate, const turq_weight *up, const void *x, int xt, int64_t m,
@@ -660,14 +662,14 @@ int turq_qmatmul_multi_mfma(turq_ctx *ctx, int count, const turq_weight *const *
         all_bytes += w[t]->dev_bytes;
     }
     const bool fused = use_fused(ctx, m, all_tiles, all_bytes) && aligned && !no_fuse;
-    int prepared = 0;  // fragment order currently in ctx->act_prep: 0 none, 1 K-quants, 2 Q8_0
+    int prepared = 0;  // what ctx->act_prep holds: 0 nothing, fragments in the order of 1 the K-quants, 2 Q8_0; 3 rows as f16
     int i = 0;
     while (i < count) {
         int j = i + 1;
         while (j < count && j - i < 4 && w[j]->dtype == w[i]->dtype) j++;
         // one activation row: a run of a second format joins the launch where the kernel has that pair (q, k Q4_K + v Q6_K)
         const bool no_mixed = turq_tuning().gemv_no_mixed;
-        // 5 .. 16 rows: fragments made in the kernel from the rows themselves (staged through the LDS), a second format in the
+        // 3 .. 32 rows: fragments made in the kernel from the rows themselves (staged through the LDS), a second format in the
         // same launch where the kernel has the pair
         {
             int j2 = j;
@@ -681,8 +683,17 @@ int turq_qmatmul_multi_mfma(turq_ctx *ctx, int count, const turq_weight *const *
                 for (int t = i; t < end; t++) tiles += turq_tile_rows(w[t]->n);
                 for (int t = j; t < end; t++) tiles_b += turq_tile_rows(w[t]->n);
                 const int dtb = end > j ? w[j]->dtype : w[i]->dtype;
-                const int rg = staged_row_tiles(ctx, w[i]->dtype, dtb, w[i]->k, m, tiles, tiles_b, aligned);
+                // (more than 16 wide rows of f32, or rows that cannot be loaded 16 bytes at a time: as f16 first, so that a call gives
+                // the same bits whatever type and alignment its rows have)
+                const bool as_f16 = m > 16 && w[i]->k > 4096 && (xt == TURQ_ACT_F32 || !aligned);
+                const int rg = staged_row_tiles(ctx, w[i]->dtype, dtb, as_f16 ? (int)TURQ_ACT_F16 : xt, w[i]->k, m, tiles, tiles_b, aligned || as_f16);
                 if (!rg) continue;
+                if (as_f16 && prepared != 3) {
+                    const int rc = turq_ctx_reserve(ctx, &ctx->act_prep, &ctx->act_prep_cap, turq_act_prep_bytes(w[i]->dtype, m, w[i]->k));
+                    if (rc != TURQ_OK) return rc;
+                    TURQ_HIP(ctx, turq_launch_act_rows_f16(x, xt, m, w[i]->k, ldx, ctx->act_prep, ctx->stream));
+                    prepared = 3;
+                }
                 const void *wp[4];
                 int64_t nn[4];
                 for (int t = i; t < end; t++) {
@@ -691,7 +702,8 @@ int turq_qmatmul_multi_mfma(turq_ctx *ctx, int count, const turq_weight *const *
                 }
                 hipEvent_t ev0 = nullptr, ev1 = nullptr;
                 TURQ_HIP(ctx, turq_prof_next(ctx, &ev0, &ev1));
-                TURQ_HIP(ctx, turq_launch_gemv_cs_staged(w[i]->dtype, dtb, end - i, end > j ? j - i : end - i, wp, nn, w[i]->k, x, xt, ldx, m,
+                TURQ_HIP(ctx, turq_launch_gemv_cs_staged(w[i]->dtype, dtb, end - i, end > j ? j - i : end - i, wp, nn, w[i]->k, as_f16 ? ctx->act_prep : x,
+                                                         as_f16 ? (int)TURQ_ACT_F16 : xt, as_f16 ? w[i]->k : ldx, m,
                                                          y + i, yt, ldy + i, bias ? bias + i : nullptr, rg, ctx->stream, ev0, ev1));
                 i = end;
                 break;
