@@ -67,6 +67,26 @@ def test_gate_up_matches_the_two_calls(gpu, dt, m):
     gpu.release(wu)
 
 
+# 17 .. 32 rows, staged in the kernel: one row tile of each weight per workgroup (200 rows end inside one; 4096 rows are 256 workgroups) or
+# three (8240 rows: more than two row tiles per compute unit); 512 columns are one pair of column tiles for one wave, 2048 one for each of
+# four, 4096 for each of eight.  The kernel rounds f32 rows to f16 as the caller would.  Tolerance as above.
+@pytest.mark.parametrize("dt", ALL)
+@pytest.mark.parametrize("n,k", [(200, 512), (200, 2048), (200, 4096), (4096, 512), (8240, 512)])
+def test_gate_up_up_to_32_rows_staged(gpu, dt, n, k):
+    raw_g = synth.random_weight(dt, n, k, seed=dt + n)
+    raw_u = synth.random_weight(dt, n, k, seed=dt + k)
+    wg = gpu.upload(dt, n, k, raw_g, capi.LAYOUT_TILED)
+    wu = gpu.upload(dt, n, k, raw_u, capi.LAYOUT_TILED)
+    for m in (17, 32):
+        x = f16_round(synth.random_activation(m, k, seed=m + k))
+        y = gpu.gate_up(wg, wu, x, n, k, x_dtype=capi.ACT_F16)
+        assert rel_l2(y, expected(dt, x, raw_g, raw_u, n, k)) <= 5e-5, m
+        assert np.array_equal(gpu.gate_up(wg, wu, x, n, k), y), m
+        assert rel_l2(gpu.gate_up(wg, wu, x, n, k, ldx=k + 1), y) <= 5e-5, m      # rows no kernel loads 16 bytes at a time
+    gpu.release(wg)
+    gpu.release(wu)
+
+
 @pytest.mark.parametrize("dt", [Q4_K, Q6_K])
 def test_gate_up_two_rows_on_large_weights(gpu, dt):
     # 2 x 5 MiB and more: two activation rows stay in the one-row kernel (Q4_K: one packed pair)

@@ -240,12 +240,16 @@ hipError_t turq_launch_gemv_cs_staged_gateup_bf16(TURQ_STAGED_GATEUP_ARGS);
 hipError_t turq_launch_gemv_cs_staged_gateup_f16(TURQ_STAGED_GATEUP_ARGS);
 
 // tiles per workgroup (gate and up together: 2 or 6) for n output columns on `units` compute units, 0: not this case
-// (17 .. 32 rows: the four-wave form, which has groups of 6, on up to 4096 columns)
+// (17 .. 32 rows, on up to 4096 columns: groups of 6 in the four-wave form, or of 2 as two passes where that is one round of
+// workgroups; against the preparation and the prepared-fragment kernel, whole calls at 32 f16 / f32 rows: 2 x 3072 x 1024 Q4_K 10.5 -> 7.0 /
+// 10.1 -> 7.8 us, Q6_K 10.7 -> 8.9 / 10.4 -> 9.6, 2 x 4096 x 1536 Q8_0 13.3 -> 8.1 / 13.3 -> 9.2.  In two rounds, 2 x 6912 x 2560, Q4_K
+// 16.4 -> 17.0 / 21.0 and Q6_K 19.7 -> 22.1 / 27.1; in the four-wave form on 5120 columns, 2 x 17408, Q4_K 47.5 -> 52.9)
 int turq_gemv_cs_staged_gateup_tiles(int dtype, int64_t n, int64_t k, int64_t m, int64_t units) {
     if (dtype != TURQ_Q4_K && dtype != TURQ_Q5_K && dtype != TURQ_Q6_K && dtype != TURQ_Q8_0) return 0;
     if (!turq_gemv_cs_staged_waves(k) || m < 1 || m > 32) return 0;
-    if (m > 16) return (turq_tile_rows(n) > 2 * units && k <= 4096) ? 6 : 0;
-    return turq_tile_rows(n) > 2 * units ? 6 : 2;
+    const int64_t row_tiles = turq_tile_rows(n);
+    if (m > 16 && (k > 4096 || (row_tiles > units && row_tiles <= 2 * units))) return 0;
+    return row_tiles > 2 * units ? 6 : 2;
 }
 
 // y[r][c] = silu(x[r] . gate[c] + bias_gate[c]) * (x[r] . up[c] + bias_up[c]); tiled weights of one format, n and k; m (1..32)
@@ -253,7 +257,9 @@ int turq_gemv_cs_staged_gateup_tiles(int dtype, int64_t n, int64_t k, int64_t m,
 hipError_t turq_launch_gemv_cs_staged_gateup(int dtype, const void *w_gate, const void *w_up, int64_t n, int64_t k, const void *x, int x_dtype,
                                              int64_t ldx, int64_t m, void *y, int y_dtype, int64_t ldy, const float *bias_gate,
                                              const float *bias_up, int tiles, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop) {
-    if (!turq_gemv_cs_staged_waves(k) || m < 1 || m > 32 || (tiles != 2 && tiles != 6) || (m > 16 && tiles != 6)) return hipErrorInvalidValue;
+    if (!turq_gemv_cs_staged_waves(k) || m < 1 || m > 32 || (tiles != 2 && tiles != 6) ||
+        (m > 16 && k > 4096))
+        return hipErrorInvalidValue;
     if (!turq_yt_ok(y_dtype, true)) return hipErrorInvalidValue;
     switch (x_dtype) {
     case TURQ_ACT_F32: return turq_launch_gemv_cs_staged_gateup_f32(TURQ_STAGED_GATEUP_PASS);

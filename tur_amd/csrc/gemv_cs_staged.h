@@ -453,10 +453,11 @@ hipError_t staged_rows(int rg, const StagedLaunch &l) {
 template <int DT, int XT, int MR, int RG>
 hipError_t staged_gateup_count(const StagedLaunch &l) {
     if (l.cnt == 1) return staged_go<gemv_cs_staged_gateup_kernel<DT, XT, MR, RG, 1>>(staged_lds<MR, RG>(l.nwaves), l);
-    return staged_go<gemv_cs_staged_gateup_kernel<DT, XT, MR, RG, 0>>(staged_lds<MR, RG>(l.nwaves), l);
+    if constexpr (MR <= 16) return staged_go<gemv_cs_staged_gateup_kernel<DT, XT, MR, RG, 0>>(staged_lds<MR, RG>(l.nwaves), l);
+    return hipErrorInvalidValue;
 }
 
-// tiles per workgroup (both weights together): 2 or 6; 17 .. 32 rows: 6, four waves
+// tiles per workgroup (both weights together): 2 or 6; 17 .. 32 rows: 2 in two passes, 6 in four waves
 template <int DT, int XT>
 hipError_t staged_gateup_shape(int rg, const StagedLaunch &l) {
     if (l.two) {
@@ -464,8 +465,10 @@ hipError_t staged_gateup_shape(int rg, const StagedLaunch &l) {
         if (rg != 6) return hipErrorInvalidValue;
         return l.cnt == 2 ? staged_go<gemv_cs_staged_two_gateup_kernel<DT, XT, 2>>(lds, l) : staged_go<gemv_cs_staged_two_gateup_kernel<DT, XT, 0>>(lds, l);
     }
-    if (rg == 2) return l.m <= 4 ? staged_gateup_count<DT, XT, 4, 2>(l) : l.m <= 8 ? staged_gateup_count<DT, XT, 8, 2>(l) : staged_gateup_count<DT, XT, 16, 2>(l);
-    if (rg == 6) return l.m <= 4 ? staged_gateup_count<DT, XT, 4, 6>(l) : l.m <= 8 ? staged_gateup_count<DT, XT, 8, 6>(l) : staged_gateup_count<DT, XT, 16, 6>(l);
+    if (rg == 2)
+        return l.m <= 4 ? staged_gateup_count<DT, XT, 4, 2>(l) : l.m <= 8 ? staged_gateup_count<DT, XT, 8, 2>(l)
+             : l.m <= 16 ? staged_gateup_count<DT, XT, 16, 2>(l) : staged_gateup_count<DT, XT, 32, 2>(l);
+    if (rg == 6 && l.m <= 16) return l.m <= 4 ? staged_gateup_count<DT, XT, 4, 6>(l) : l.m <= 8 ? staged_gateup_count<DT, XT, 8, 6>(l) : staged_gateup_count<DT, XT, 16, 6>(l);
     return hipErrorInvalidValue;
 }
 

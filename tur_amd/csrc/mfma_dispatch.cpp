@@ -603,7 +603,7 @@ int turq_qmatmul_gate_up_mfma(turq_ctx *ctx, const turq_weight *gate, const turq
         up->layout != TURQ_LAYOUT_TILED)
         return TURQ_OK;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    // 3 .. 16 rows: the kernel that makes its fragments from the rows themselves (no preparation launch), activation in its epilogue
+    // 3 .. 32 rows: the kernel that makes its fragments from the rows themselves (no preparation launch), activation in its epilogue
     {
         const int staged = turq_tuning().cs_staged;
         const int64_t cus = ctx->compute_units > 0 ? ctx->compute_units : 256;
