@@ -211,7 +211,7 @@ int turq_qmatmul(turq_ctx *ctx, const turq_weight *w, const void *x, int x_dtype
  * TURQ_MEM_DEVICE and TURQ_ALGO_AUTO (one exception: where turq_qmatmul gives the columns of every workgroup tile to several
  * workgroups - see there - this call runs the same kernel unsplit, the same products added in another order: within 2e-6
  * relative L2 of each other), but the prepared activation fragments of the calls that use them
- * (more than 32 rows, and 17 - 32 rows on all but small weights) live in a static device array of TURQ_NOALLOC_SCRATCH_BYTES (one copy per GPU, held until
+ * (more than 32 rows, and 17 - 32 rows on many shapes; f32 rows of more than 4096 columns as f16) live in a static device array of TURQ_NOALLOC_SCRATCH_BYTES (one copy per GPU, held until
  * the process ends) instead of the context's growable buffer: the call runs no hipMalloc / hipFree
  * and creates no stream or event.  A call that needs more is refused with TURQ_ERR_SHAPE and a
  * message that names the bytes needed: fragments take 2.25 * mpad * k bytes for up to 32 rows (mpad
@@ -227,8 +227,9 @@ int turq_qmatmul_noalloc(turq_ctx *ctx, const turq_weight *w, const void *x, int
 /* The same product for `count` weights that take the same activations: ys[i][m, n_i] = x[m, k] * W_i^T (+ biases[i]).
  * All weights must share k.  With device pointers, tiled weights and m <= 32, neighbouring weights of one format
  * go out as ONE kernel launch, and so do Q4_K or Q5_K weights followed by Q6_K ones (q, k and v of a Q4_K_M file); up to
- * 16 rows that launch is all there is (the kernel makes its MFMA operands from the activation rows themselves), with 17 - 32
- * rows on all but small weights, with activation rows that are not 16-byte aligned, and with k that is not a multiple of 512,
+ * 16 rows that launch is all there is (the kernel makes its MFMA operands from the activation rows themselves; with 17 - 32
+ * rows too on up to 8192 weight rows, f32 rows of more than 4096 columns being rounded to f16 first), with 17 - 32 rows on
+ * larger weights, with activation rows that are not 16-byte aligned, and with k that is not a multiple of 512,
  * one preparation of the activations for all the weights comes first; with more than 32 rows the
  * activations are prepared once for all the weights and each weight runs its GEMM on them (the results of the single
  * calls, bit for bit; GEMMs that leave half of the GPU free, such as k_proj and v_proj of a prompt chunk, run next to each other,
