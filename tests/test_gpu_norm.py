@@ -98,6 +98,22 @@ def test_rms_norm_pieces_of_a_row(gpu, k, pad):
         assert rel_l2(call(gpu, xs, w, eps, ldx=k + pad, ldy=k + pad, mem=capi.MEM_DEVICE), want_norm(xs, w, eps)) <= bar, scale
 
 
+def test_rms_norm_small_elements_and_signed_zeros(gpu):
+    # the squares of all but four elements vanish in the sum, which makes the root exactly 3: every other element is v / 3 to the last
+    # bit, whatever its size (quotients and remainders below the f32 range among them), and a zero keeps its sign
+    rng = np.random.default_rng(9)
+    k = 4096
+    v = (rng.uniform(1, 2, k) * 2.0 ** rng.integers(-149, -29, k) * rng.choice([-1.0, 1.0], k)).astype(np.float32)
+    v[4:200:2], v[5:200:2] = -0.0, 0.0
+    v[200:] = np.where(np.arange(200, k) % 16 == 0, np.copysign(np.float32(0), v[200:]), v[200:])
+    v[:4] = 96.0  # mean of the squares: 4 * 96^2 / 4096 = 9
+    for scale in (1.0, 0x1p-45):  # ... and a root at which every element takes the plain division
+        x = (v * np.float32(scale)).astype(np.float32).reshape(1, k)
+        want = x / (np.float32(3) * np.float32(scale))
+        y = call(gpu, x, np.ones(k, np.float32), 0.0, mem=capi.MEM_DEVICE)
+        assert np.array_equal(y.view(np.uint32), want.view(np.uint32)), scale
+
+
 def test_rms_norm_errors(gpu):
     L, ctx = gpu.L, gpu.ctx
     x = np.zeros((2, 8), np.float32)

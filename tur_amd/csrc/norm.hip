@@ -66,15 +66,15 @@ __device__ inline float rms_of(float s, int64_t k, float eps, float *part) {
 
 // v / rms for many v against one rms, to the last bit: with r = 1 / rms correctly rounded, q = v * r corrected once by its own
 // remainder is the correctly rounded quotient (P. Markstein, "Computation of elementary functions on the IBM RISC System/6000",
-// 1990) as long as nothing over- or underflows on the way.  No |v| of a row exceeds sqrt(k) * rms, so only the range of rms matters:
-// rows whose rms is an infinity, a NaN or outside a generous range take the plain division.
+// 1990) as long as nothing over- or underflows on the way.  No |v| of a row exceeds sqrt(k) * rms; from 2^-60 on, against an rms between
+// 2^-40 and 2^40, the quotient is at least 2^-100 and the remainder, a multiple of 2^-48 |v| or so, stays exact.  Smaller elements - zeros, whose
+// sign the correction would lose, among them - and rows whose rms is an infinity, a NaN or outside that range take the plain division.
 struct RowDiv {
-    float rms, r;
-    bool plain;
-    __device__ explicit RowDiv(float d) : rms(d), r(1.0f / d), plain(!(d > 0x1p-60f && d < 0x1p60f)) {}
+    float rms, r, least;  // least: the smallest |v| that is corrected (an infinity: none is)
+    __device__ explicit RowDiv(float d) : rms(d), r(1.0f / d), least(d > 0x1p-40f && d < 0x1p40f ? 0x1p-60f : __builtin_inff()) {}
     __device__ float operator()(float v) const {
         const float q = v * r;
-        return __builtin_expect(plain, 0) ? v / rms : __builtin_fmaf(__builtin_fmaf(-q, rms, v), r, q);
+        return __builtin_expect(!(__builtin_fabsf(v) >= least), 0) ? v / rms : __builtin_fmaf(__builtin_fmaf(-q, rms, v), r, q);
     }
 };
 
