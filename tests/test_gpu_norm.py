@@ -114,6 +114,18 @@ def test_rms_norm_small_elements_and_signed_zeros(gpu):
         assert np.array_equal(y.view(np.uint32), want.view(np.uint32)), scale
 
 
+@pytest.mark.parametrize("k,ldy", [(2048, 2048), (2049, 2049)])   # rows stored eight columns at a time, and element by element
+def test_rms_norm_counts_every_element_that_is_no_finite_number(gpu, k, ldy):
+    w = np.ones(k, np.float32)
+    w[16:24], w[40:43], w[k - 1] = 1e6, 1e6, 1e6   # a whole piece of eight columns, three of another, the last column
+    x = np.full((5, k), 2.0, np.float32)
+    n = ctypes.c_uint64()
+    capi.check(gpu.L.turq_ctx_nonfinite_count(gpu.ctx, ctypes.byref(n), 1), gpu.ctx)
+    call(gpu, x, w, 1e-6, y_dtype=capi.ACT_F16, mem=capi.MEM_DEVICE, ldy=ldy)
+    capi.check(gpu.L.turq_ctx_nonfinite_count(gpu.ctx, ctypes.byref(n), 1), gpu.ctx)
+    assert n.value == 5 * 12
+
+
 def test_rms_norm_errors(gpu):
     L, ctx = gpu.L, gpu.ctx
     x = np.zeros((2, 8), np.float32)

@@ -160,6 +160,17 @@ __device__ inline void turq_note_flush(uint32_t bad) {
             __hip_atomic_fetch_add(&turq_nonfinite_word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
+// ... with every one of the run counted
+template <int YT, int N> __device__ inline void turq_note_results(const float (&v)[N]) {
+    const float lim = turq_finite_limit(YT);
+    uint32_t bad = 0;
+#pragma unroll
+    for (int e = 0; e < N; e++) bad += __builtin_fabsf(v[e]) < lim ? 0u : 1u;
+    if (__builtin_expect(bad != 0, 0)) {
+        if (__hip_atomic_load(&turq_nonfinite_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < (1u << 20))
+            __hip_atomic_fetch_add(&turq_nonfinite_word, bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
 // host side of it, once per translation unit whose kernels store results: adds the current device's word to *sum (and clears it)
 #define TURQ_NONFINITE_READER(fn)                                                                      \
     hipError_t fn(unsigned long long *sum, int reset) {                                                \

@@ -114,10 +114,7 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(const void *__restrict__ 
 #pragma unroll
         for (int e = 0; e < 8; e++) o[e] = div(t[e]) * wv[e];
         if (vy && col0 + 8 <= k) {
-            uint32_t bad = 0;
-#pragma unroll
-            for (int e = 0; e < 8; e++) turq_note_accum(o[e], turq_finite_limit(YT), bad);
-            turq_note_flush(bad);
+            turq_note_results<YT>(o);
             uint8_t *p = (uint8_t *)y + (yo + col0) * (YT == TURQ_ACT_F32 ? 4 : 2);
             if constexpr (YT == TURQ_ACT_F32) {
                 ((float4v *)p)[0] = float4v{o[0], o[1], o[2], o[3]};
@@ -187,16 +184,14 @@ __global__ void __launch_bounds__(256 * kPrepRows) rms_norm_prep32_kernel(const 
         float wv[8];
         ld_piece<TURQ_ACT_F32>(w, 0, col0, k, vw, wv);
         half8v h;
-        float sum = 0.0f;
-        uint32_t bad = 0;
+        float sum = 0.0f, f[8];
 #pragma unroll
         for (int e = 0; e < 8; e++) {
-            const float f = live ? div(v[j][e]) * wv[e] : 0.0f;
-            turq_note_accum(f, turq_finite_limit(TURQ_ACT_F16), bad);
-            h[e] = (_Float16)f;
+            f[e] = live ? div(v[j][e]) * wv[e] : 0.0f;
+            h[e] = (_Float16)f[e];
             sum += (float)h[e];
         }
-        turq_note_flush(bad);
+        turq_note_results<TURQ_ACT_F16>(f);
         const int64_t b = piece >> 5;
         const int cc = (int)(piece & 31);
         half8v *dst = frags + (mt * ntc + b) * (17 * 64);
