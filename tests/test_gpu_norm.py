@@ -107,7 +107,7 @@ def test_rms_norm_small_elements_and_signed_zeros(gpu):
     v[4:200:2], v[5:200:2] = -0.0, 0.0
     v[200:] = np.where(np.arange(200, k) % 16 == 0, np.copysign(np.float32(0), v[200:]), v[200:])
     v[:4] = 96.0  # mean of the squares: 4 * 96^2 / 4096 = 9
-    for scale in (1.0, 0x1p-45):  # ... and a root at which every element takes the plain division
+    for scale in (1.0, 2.0 ** -45):  # ... and a root at which every element takes the plain division
         x = (v * np.float32(scale)).astype(np.float32).reshape(1, k)
         want = x / (np.float32(3) * np.float32(scale))
         y = call(gpu, x, np.ones(k, np.float32), 0.0, mem=capi.MEM_DEVICE)
