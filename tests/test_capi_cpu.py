@@ -218,8 +218,9 @@ def test_gguf_reader_refuses_hostile_files(tmp_path, kwargs, what):
 
 
 def test_prefill_launch_rules_on_a_256_cu_device():
-    # the launches the rules make for the matrices of a Qwen3-8B Q4_K_M layer on prompt chunks, as measured and documented:
-    # (tile, workgroups per tile, wave groups); tiles: 1 = 128 x 128, 2 = 128 x 192, 3 = 128 x 256, 4 = 64 x 128
+    # the launches the rules make for the matrices of a Qwen3-8B Q4_K_M layer (and some of a 0.6B Q8_0 one) on prompt chunks, as measured
+    # and documented: (tile, workgroups per tile, wave groups); tiles: 1 = 128 x 128, 2 = 128 x 192 (Q8_0: 128 x 64), 3 = 128 x 256, 4 = 64 x 128,
+    # 10 r + c = 32 r x 32 c of the kernel whose waves split the columns
     L = capi.lib()
     Q4_K, Q6_K = capi.Q4_K, capi.Q6_K
 
@@ -228,27 +229,30 @@ def test_prefill_launch_rules_on_a_256_cu_device():
         capi.check(L.turq_prefill_plan(dt, n, k, m, 256, ctypes.byref(t), ctypes.byref(s), ctypes.byref(g)))
         return t.value, s.value, g.value
 
-    # down_proj 4096 x 12288: low tile in 6 / 3 parts up to 128 rows, wide tile in 6 parts at 256, unsplit from 512 on
-    assert plan(Q6_K, 4096, 12288, 64) == (4, 6, 2)
-    assert plan(Q6_K, 4096, 12288, 128) == (4, 3, 2)
-    assert plan(Q6_K, 4096, 12288, 256) == (3, 6, 1)
-    assert plan(Q6_K, 4096, 12288, 512) == (4, 1, 2)
+    # down_proj 4096 x 12288: the smallest tile that makes the launch one round, six and eight MFMA tiles from 12 and 24 super-blocks on
+    assert [plan(Q6_K, 4096, 12288, m) for m in (33, 64, 96, 128, 256, 300, 512)] == [(t, 1, 1) for t in (11, 11, 11, 21, 22, 32, 42)]
     assert plan(Q6_K, 4096, 12288, 1024) == (1, 1, 1)
-    # o_proj / q_proj 4096 x 4096 and k_proj 1024 x 4096: parts only while they take at most a quarter of the CUs; eight waves
+    # o_proj / q_proj 4096 x 4096 and k_proj 1024 x 4096: eight MFMA tiles not at 16 super-blocks; there the low tile, with eight waves
     # while there is at most one workgroup per CU
-    assert plan(Q4_K, 4096, 4096, 64) == (4, 2, 2)
-    assert plan(Q4_K, 4096, 4096, 128) == (4, 1, 2)
-    assert plan(Q4_K, 1024, 4096, 128) == (4, 4, 2)
-    assert plan(Q4_K, 4096, 4096, 256) == (4, 1, 2)
+    assert [plan(Q4_K, 4096, 4096, m) for m in (64, 128, 256, 300)] == [(t, 1, 1) for t in (11, 21, 22, 32)]
     assert plan(Q4_K, 4096, 4096, 512) == (4, 1, 2)
+    assert [plan(Q4_K, 1024, 4096, m) for m in (128, 512, 1024)] == [(t, 1, 1) for t in (11, 21, 22)]
+    assert plan(Q4_K, 1024, 4096, 2048) == (4, 1, 2)
     # up_proj 12288 x 4096 alone, and gate + up as one launch (24576 rows)
-    assert plan(Q4_K, 12288, 4096, 128) == (4, 1, 2)
+    assert [plan(Q4_K, 12288, 4096, m) for m in (64, 77, 128)] == [(t, 1, 1) for t in (22, 32, 23)]
     assert plan(Q4_K, 12288, 4096, 256) == (1, 1, 1)
     assert plan(Q4_K, 12288, 4096, 512) == (2, 1, 1)
     assert plan(Q4_K, 12288, 4096, 2048) == (3, 1, 1)
+    assert plan(Q4_K, 24576, 4096, 64) == (23, 1, 1)
     assert plan(Q4_K, 24576, 4096, 128) == (1, 1, 1)
     assert plan(Q4_K, 24576, 4096, 256) == (2, 1, 1)
     assert plan(Q4_K, 24576, 4096, 1024) == (3, 1, 1)
+    # fewer super-blocks than six MFMA tiles ask for: the low tile, whose four waves hold all the columns where their number is odd
+    assert plan(Q4_K, 2048, 2048, 600) == (4, 1, 2) and plan(Q4_K, 2048, 2304, 600) == (4, 1, 1)
+    # Q8_0: whichever kernel has the smaller estimate, in any number of rounds
+    Q8_0 = capi.Q8_0
+    assert [plan(Q8_0, 3072, 1024, m)[0] for m in (256, 300, 512, 1024, 2048)] == [11, 22, 23, 23, 2]
+    assert [plan(Q8_0, 1024, 3072, m)[0] for m in (300, 512, 1024, 2048)] == [11, 21, 22, 42]
     # the LM head: more workgroups than CUs, four waves
     assert plan(Q6_K, 151936, 4096, 64) == (4, 1, 1)
     # gate_proj and up_proj (2 x 12288 x 4096) through turq_qmatmul_multi: one launch where that fills the rounds better, which the

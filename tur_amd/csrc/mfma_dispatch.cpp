@@ -843,7 +843,7 @@ extern "C" int turq_prefill_plan_multi(int dtype, int64_t n, int64_t k, int64_t 
     return TURQ_OK;
 }
 
-// which launch the rules above and in gemm_mfma.hip make for a prompt chunk (no GPU needed)
+// which launch the rules above, in gemm_cols.hip and in gemm_mfma.hip make for a prompt chunk (no GPU needed)
 extern "C" int turq_prefill_plan(int dtype, int64_t n, int64_t k, int64_t m, int compute_units, int *tile, int *split, int *wave_groups) {
     if (tile) *tile = 0;
     if (split) *split = 1;
@@ -852,6 +852,10 @@ extern "C" int turq_prefill_plan(int dtype, int64_t n, int64_t k, int64_t m, int
     if (n <= 0 || k <= 0 || k % 256 != 0 || m <= TURQ_GEMV_MAX_M || compute_units <= 0)
         return turq_fail(nullptr, TURQ_ERR_SHAPE, "turq_prefill_plan: n=%lld k=%lld m=%lld on %d compute units", (long long)n, (long long)k,
                          (long long)m, compute_units);
+    if (const int cols = turq_gemm_cols_tile(dtype, dtype, 1, &n, k, m, compute_units)) {  // gemm_cols.hip, asked first as in gemm_on_frags
+        if (tile) *tile = cols;
+        return TURQ_OK;
+    }
     int form = turq_gemm_form(dtype, n, k, m, compute_units), parts = 1, sform = 0;
     if (turq_gemm_split_scratch(dtype, n, k, m, compute_units, &sform, &parts) != 0) form = sform;
     else parts = 1;
