@@ -277,6 +277,21 @@ def test_prefill_launch_rules_on_a_256_cu_device():
     assert L.turq_prefill_plan(capi.F32, 4096, 4096, 64, 256, ctypes.byref(t), None, None) == capi.ERR_DTYPE
 
 
+@pytest.mark.parametrize("dt,row_tiles", [(capi.Q4_K, 8), (capi.Q5_K, 8), (capi.Q6_K, 8), (capi.Q8_0, 6)])
+def test_prefill_columns_beyond_32_bit_offsets(dt, row_tiles):
+    # a lane's offset to the last row tile of its workgroup has 32 bits: from the column count on where it would wrap the launch belongs to the
+    # other kernel, which refuses it (K-quants: n-blocks of eight row tiles; Q8_0: four, against at most six here)
+    L = capi.lib()
+    t = ctypes.c_int()
+
+    def cols(super_blocks):
+        capi.check(L.turq_prefill_plan(dt, 64, 256 * super_blocks, 40, 256, ctypes.byref(t), None, None))
+        return t.value > 10
+
+    top = (2**32 // row_tiles - 1) // L.turq_tiled_nbytes(dt, 16, 256)
+    assert cols(top) and not cols(top + 1) and not cols(986896) and not cols(2**20)
+
+
 
 def test_tuning_switches_are_listed_and_overrides_are_announced():
     # every environment switch of the kernel-selection rules lives in one table (tur_amd/csrc/tuning.h); a process lists what it

@@ -14,6 +14,8 @@
 // behind them belong to super-block b + 1 itself.
 #include <hip/hip_ext.h>
 
+#include <algorithm>
+
 #include "gemm_formats.h"
 #include "tuning.h"
 
@@ -373,6 +375,11 @@ hipError_t launch_tile(int tile, const TurqGemmWeights &ws, int second, int64_t 
     }
 }
 
+// bytes of one row tile's super-blocks, the larger of the two formats'
+size_t row_tile_bytes(int dtype_a, int dtype_b, int64_t k) {
+    return (size_t)(k / 256) * (size_t)std::max(turq_tile_bytes(dtype_a), turq_tile_bytes(dtype_b));
+}
+
 }  // namespace
 
 bool turq_gemm_cols_mixed(int dtype_a, int dtype_b) { return (dtype_a == TURQ_Q4_K || dtype_a == TURQ_Q5_K) && dtype_b == TURQ_Q6_K; }
@@ -398,6 +405,9 @@ int turq_gemm_cols_tile(int dtype_a, int dtype_b, int count, const int64_t *n, i
     if (t.gemm_cols == 0 || (t.gemm_cols < 0 && kq_forced)) return 0;
     if (!turq_dt_is_quant(dtype_a) || (dtype_b != dtype_a && !turq_gemm_cols_mixed(dtype_a, dtype_b))) return 0;
     if (count < 1 || count > kMaxGroup || m <= 0 || k <= 0 || k % 256 != 0) return 0;
+    // a lane's offset to the last of its 16-row tiles is 32-bit, here and in gemm_kq_kernel, whose n-blocks of eight row tiles (Q8_0: four)
+    // decide: columns that it refuses are not taken instead (six row tiles are the most of a workgroup here)
+    if (row_tile_bytes(dtype_a, dtype_b, k) >= (1ull << 32) / (dtype_a == TURQ_Q8_0 ? 6 : 8)) return 0;
     if (t.gemm_cols > 0) return t.gemm_cols;
     const int64_t cus = compute_units > 0 ? compute_units : 256, ntc = k / 256;
     static constexpr struct { int mt, nt; double base, per_sb; } kTiles[] = {{1, 1, 3.2, 0.40}, {2, 1, 4.0, 0.52}, {3, 1, 4.6, 0.60}, {2, 2, 5.2, 0.68},
@@ -437,6 +447,7 @@ hipError_t turq_launch_gemm_cols(int dtype_a, int dtype_b, int second, int tile,
         n += ws.n[i];
     }
     if (m == 0) return hipSuccess;
+    if (row_tile_bytes(dtype_a, second < ws.count ? dtype_b : dtype_a, k) * 2 * (size_t)(tile % 10) >= (1ull << 32)) return hipErrorInvalidValue;
     if ((n / 32 + ws.count) * ((m + 31) / 32) > 0x7FFFFFFF) return hipErrorInvalidValue;
 #define TURQ_COLS_TILE(A, B) return launch_tile<A, B>(tile, ws, second, k, frags, m, y_dtype, stream, ev_start, ev_stop)
     if (dtype_a != dtype_b && second < ws.count) {
