@@ -526,6 +526,31 @@ def test_multi_weight_prefill_shares_the_preparation(gpu):
         gpu.release(w)
 
 
+@pytest.mark.parametrize("dts,ns,k,ms", [
+    ((Q8_0, Q8_0, Q8_0), [2048, 1024, 1024], 1024, (300, 512, 1024)),   # q / k / v of a 0.6B model: one launch, and several
+    ((Q8_0, Q8_0), [3072, 3072], 1024, (256, 512, 2048)),               # its gate / up: one launch of either kernel
+    ((Q4_K, Q4_K, Q6_K), [4096, 1024, 1024], 4096, (200, 300, 512)),    # q / k / v of an 8B model
+    ((Q6_K, Q6_K, Q6_K), [4096, 1024, 1024], 4096, (200, 256)),
+    ((Q4_K, Q4_K), [2048, 2048], 2048, (300, 512)),                     # (from about 600 rows on: large weights of one shape, within 2e-6)
+    ((Q8_0, Q8_0), [4096, 512], 512, (400, 1100)),
+], ids=["qkv-q8_0", "gateup-q8_0", "qkv-q4km", "qkv-q6k", "pair-q4k", "uneven-q8_0"])
+def test_multi_weight_prefill_keeps_the_bits_of_the_single_calls(gpu, dts, ns, k, ms):
+    # whatever launches the rules make of several weights: each keeps the kernel that it takes alone, so the sums are the same
+    raws = [synth.random_weight(dt, n, k, seed=11 * i + n) for i, (dt, n) in enumerate(zip(dts, ns))]
+    ws = [gpu.upload(dt, n, k, raw, capi.LAYOUT_TILED) for dt, n, raw in zip(dts, ns, raws)]
+    for m in ms:
+        x = synth.random_activation(m, k, seed=m, bf16=True)
+        ys = gpu.qmatmul_multi(ws, x, ns, k, x_dtype=capi.ACT_BF16)
+        for i, (dt, n, raw, w, y) in enumerate(zip(dts, ns, raws, ws, ys)):
+            single = gpu.qmatmul_device(w, x, n, k, x_dtype=capi.ACT_BF16)
+            assert np.array_equal(y, single), (m, i, rel_l2(y, single))
+            rows = np.arange(i, n, 16)
+            sub = raw.reshape(n, -1)[rows].reshape(-1)
+            assert rel_l2(y[:, rows], orc.matmul_dequant(dt, x, sub, len(rows), k)) <= 1e-3, (m, i)
+    for w in ws:
+        gpu.release(w)
+
+
 def test_multi_weight_prefill_runs_of_one_format(gpu):
     # neighbouring weights of one K-quant format and shape (rows a multiple of 256) may go out as ONE launch of the prefill GEMM
     # whose n-blocks are dealt out to the weights; the rule only does that for weights that fill half the machine, so this test

@@ -397,7 +397,8 @@ bool turq_gemm_cols_mixed(int dtype_a, int dtype_b) { return (dtype_a == TURQ_Q4
 //   at 160 rows 11.1 -> 11.7);
 //   eight: from 40 super-blocks on, Q6_K from 24 (512 rows, 4096 x 12288: Q4_K 66 -> 64, Q5_K 76 -> 69, Q6_K 81 -> 66; 4096 x 4096: Q4_K 26.3 -> 27.5).
 // Q8_0, whose tile in gemm_kq_kernel is the narrow 128 x 64, takes whichever kernel has the smaller estimate, in any number of rounds
-// (4096 x 4096 at 512 / 700 rows 31 / 53 -> 29 / 41, 4096 x 12288 at 1024 / 2048 rows 160 / 300 -> 126 / 283).
+// (4096 x 4096 at 512 / 700 rows 31 / 53 -> 29 / 41, 4096 x 12288 at 1024 / 2048 rows 160 / 300 -> 126 / 283); several weights, each
+// of which is this kernel's, go together where that is less than one after the other.
 int turq_gemm_cols_tile(int dtype_a, int dtype_b, int count, const int64_t *n, int64_t k, int64_t m, int compute_units, double *us) {
     const TurqTuning &t = turq_tuning();
     const bool kq_forced = t.gemm_wide >= 0 || t.gemm_low >= 0 || t.gemm_split >= 0 || t.gemm_kgroups != 0 || t.gemm_grid_2x2 || t.gemm_merge >= 0;
@@ -414,7 +415,16 @@ int turq_gemm_cols_tile(int dtype_a, int dtype_b, int count, const int64_t *n, i
                                                                              {3, 2, 6.2, 0.92}, {2, 3, 6.2, 0.92}, {4, 2, 7.0, 1.20}};
     const bool eight = dtype_a == TURQ_Q8_0;
     int best = 0;
-    double best_us = eight ? turq_gemm_launch_us(dtype_a, count, n, k, m, compute_units) : 1e30;
+    double best_us = 1e30;
+    if (eight && count == 1) best_us = turq_gemm_launch_us(dtype_a, 1, n, k, m, compute_units);
+    if (eight && count > 1) {
+        best_us = 0.0;
+        for (int i = 0; i < count; i++) {
+            double alone = 0.0;
+            if (!turq_gemm_cols_tile(dtype_a, dtype_a, 1, n + i, k, m, compute_units, &alone)) return 0;
+            best_us += alone;
+        }
+    }
     for (const auto &c : kTiles) {
         const int area = c.mt * c.nt;
         int64_t nbn = 0;

@@ -222,7 +222,7 @@ static TurqGemmWeights gemm_weights(int count, const turq_weight *const *w, void
 
 // the tile with which the first `count` weights go through gemm_cols.hip in one launch (one format, or Q4_K / Q5_K followed by
 // Q6_K), 0: not; *second: the first weight of the second format
-static int gemm_cols_tile(const turq_ctx *ctx, int count, const turq_weight *const *w, int64_t m, int *second, double *us = nullptr) {
+static int gemm_cols_tile(const turq_ctx *ctx, int count, const turq_weight *const *w, int64_t m, int *second) {
     int64_t n[4];
     int s = count;
     if (count < 1 || count > 4) return 0;
@@ -232,7 +232,7 @@ static int gemm_cols_tile(const turq_ctx *ctx, int count, const turq_weight *con
         if (w[i]->n <= 0 || w[i]->k != w[0]->k || w[i]->dtype != w[i < s ? 0 : s]->dtype) return 0;
     }
     if (second) *second = s;
-    return turq_gemm_cols_tile(w[0]->dtype, w[s < count ? s : 0]->dtype, count, n, w[0]->k, m, ctx->compute_units, us);
+    return turq_gemm_cols_tile(w[0]->dtype, w[s < count ? s : 0]->dtype, count, n, w[0]->k, m, ctx->compute_units);
 }
 
 // the prefill GEMM of one weight on the fragments in ctx->act_prep, by either kernel
@@ -294,28 +294,26 @@ static int gemm_run(const turq_ctx *ctx, int left, const turq_weight *const *w, 
     const bool no_merge = merge_env == 0, merge_all = merge_env == 2;
     const int64_t c = gemm_cus_taken(ctx, w[0], m, may_split);
     if (no_merge || !(2 * c > ctx->compute_units || merge_all) || !turq_dt_is_quant(w[0]->dtype) || w[0]->n % 256 != 0) return 0;
+    if (w[0]->dtype == TURQ_Q8_0 && gemm_cols_tile(ctx, 1, w, m, nullptr) != 0) return 0;  // (bit-equal with the single calls, see there)
     int run = 1;
     while (run < left && run < 4 && w[run]->dtype == w[0]->dtype && w[run]->n == w[0]->n) run++;
     return run >= 2 && (merge_all || gemm_merge_rule(w[0]->dtype, w[0]->n, w[0]->k, m, run, ctx->compute_units, c)) ? run : 0;
 }
 
-// what `run` neighbouring weights take as ONE launch of gemm_kq_kernel, where that is known and less than what a launch each takes; else 0.
-// cols: the weights that gemm_cols.hip would take alone
-static double gemm_run_us(const turq_ctx *ctx, int run, const turq_weight *const *w, int64_t m, const bool *cols) {
-    if (run > 4 || turq_tuning().gemm_merge >= 0 || turq_tuning().gemm_cols > 0) return 0.0;
+// whether `run` neighbouring weights take less as ONE launch of gemm_kq_kernel than as a launch each, where both are known
+static bool gemm_run_pays(const turq_ctx *ctx, int run, const turq_weight *const *w, int64_t m) {
+    if (run > 4 || turq_tuning().gemm_merge >= 0 || turq_tuning().gemm_cols > 0) return false;
     int64_t n[4];
     double apart = 0.0;
     for (int i = 0; i < run; i++) {
-        if (w[i]->dtype != w[0]->dtype || w[i]->n <= 0 || w[i]->n % 256 != 0) return 0.0;
+        if (w[i]->dtype != w[0]->dtype || w[i]->n <= 0 || w[i]->n % 256 != 0) return false;
         n[i] = w[i]->n;
-        double us = 0.0;
-        if (cols[i]) (void)gemm_cols_tile(ctx, 1, w + i, m, nullptr, &us);
-        else us = turq_gemm_launch_us(w[i]->dtype, 1, n + i, w[i]->k, m, ctx->compute_units);
-        if (us == 0.0) return 0.0;
+        const double us = turq_gemm_launch_us(w[i]->dtype, 1, n + i, w[i]->k, m, ctx->compute_units);
+        if (us == 0.0) return false;
         apart += us;
     }
     const double us = turq_gemm_launch_us(w[0]->dtype, run, n, w[0]->k, m, ctx->compute_units);
-    return us < apart ? us : 0.0;
+    return us > 0.0 && us < apart;
 }
 
 int turq_qmatmul_multi_gemm(turq_ctx *ctx, int count, const turq_weight *const *w, const void *x, int xt, int64_t m, int64_t ldx,
@@ -362,17 +360,18 @@ int turq_qmatmul_multi_gemm(turq_ctx *ctx, int count, const turq_weight *const *
         }
         hipStream_t st = ctx->stream;
         // As many neighbouring weights as one launch takes in about one round over the CUs (q, k and v; k and v; gate and up of a small
-        // model), by either kernel: a launch of few tiles is mostly its start and its end (Q8_0 2 x 3072 x 1024 at 256 rows 21.1 -> 11.1
-        // us), and a second format costs a launch of gemm_cols.hip nothing.
+        // model): a launch of few tiles is mostly its start and its end (Q8_0 2 x 3072 x 1024 at 256 rows 21.1 -> 11.1 us), and a
+        // second format costs a launch of gemm_cols.hip nothing.  All by the kernel that each takes alone, whose sums do not depend on the
+        // launch: in gemm_cols.hip they are the same for every tile, in the one-round launches of gemm_kq_kernel asked here the low
+        // tile keeps its wave groups and Q8_0 has one tile.
         {
             int run = std::min(count - i, 4), tile = 0, second = 0;
             bool kq = false;
             for (; run >= 2; run--) {
-                double us = 0.0;
                 if ((w[i + run - 1]->dtype == TURQ_Q8_0) != (order == 2)) continue;
-                tile = gemm_cols_tile(ctx, run, w + i, m, &second, &us);
-                const double kq_us = gemm_run_us(ctx, run, w + i, m, cols + i);
-                kq = kq_us > 0.0 && (tile == 0 || kq_us < us);
+                const int64_t n_cols = std::count(cols + i, cols + i + run, true);
+                if (n_cols == run) tile = gemm_cols_tile(ctx, run, w + i, m, &second);
+                if (n_cols == 0) kq = gemm_run_pays(ctx, run, w + i, m);
                 if (tile != 0 || kq) break;
             }
             // (one alone: unless it goes out together with its like below)
