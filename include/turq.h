@@ -196,9 +196,9 @@ int turq_rms_norm(turq_ctx *ctx, const void *x, int x_dtype, int64_t m, int64_t 
  * y_dtype | TURQ_OUT_ACCUMULATE adds the results to y instead of overwriting it (see there).
  * Errors instead of panics for m < 0, ld too small, unsupported dtypes.  m == 0 is a no-op.
  * Device calls of 33 - 64 rows on large weights of up to 4096 columns (gate / up of an 8B model) go through the kernels of up
- * to 32 rows in two chunks.  Device calls of more than 32 rows (prompt chunks) whose workgroup tiles would leave most compute units idle - the tall
- * down_proj of a model up to about 256 rows, every matrix of a layer up to 64 - split the columns of every tile over several
- * workgroups, which meet in a scratch buffer of the context (partial tiles, at most 256 MiB per launch and 512 MiB per call; grown like the other scratch
+ * to 32 rows in two chunks.  Device calls of more than 32 rows (prompt chunks) that make few workgroup tiles share the columns of a
+ * tile out over the waves of its workgroup and, for a few tiles of K-quant weights with very many columns (from 16384 on at the earliest), over several
+ * workgroups, which meet in a scratch buffer of the context (partial tiles, 6 MiB per launch; grown like the other scratch
  * buffers: not during a graph capture).  The sums of a result are the same numbers in the same order on every call.
  * Replaces: `LinearX::forward` -> `QMatMul::forward(&Tensor)` (src/models/layers/linear.rs:19-31)
  * -> candle `CustomOp1::cpu_fwd` -> `k_quants::matmul`. */
@@ -209,7 +209,7 @@ int turq_qmatmul(turq_ctx *ctx, const turq_weight *w, const void *x, int x_dtype
  * capture, tight serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the
  * reference.  Same product, same kernels and bit-identical results as turq_qmatmul with
  * TURQ_MEM_DEVICE and TURQ_ALGO_AUTO (one exception: where turq_qmatmul gives the columns of every workgroup tile to several
- * workgroups - see there - this call runs the same kernel unsplit, the same products added in another order: within 2e-6
+ * workgroups - see there - this call shares them out over waves only, the same products added in another order: within 2e-6
  * relative L2 of each other), but the prepared activation fragments of the calls that use them
  * (more than 32 rows, and 17 - 32 rows on many shapes; f32 rows of more than 4096 columns as f16) live in a static device array of TURQ_NOALLOC_SCRATCH_BYTES (one copy per GPU, held until
  * the process ends) instead of the context's growable buffer: the call runs no hipMalloc / hipFree

@@ -247,6 +247,11 @@ def test_prefill_launch_rules_on_a_256_cu_device():
     assert plan(Q4_K, 24576, 4096, 128) == (1, 1, 1)
     assert plan(Q4_K, 24576, 4096, 256) == (2, 1, 1)
     assert plan(Q4_K, 24576, 4096, 1024) == (3, 1, 1)
+    # a few tiles of very many columns: the low tile, each given to as many workgroups as divide the super-blocks; not where the tiles are many,
+    # nor on fewer columns
+    assert [plan(Q4_K, n, 28672, 64) for n in (512, 1024, 8192)] == [(4, 8, 2), (4, 8, 2), (21, 1, 1)]
+    assert plan(Q4_K, 256, 65536, 512) == (4, 8, 2) and plan(capi.Q5_K, 1024, 28672, 128) == (4, 8, 2) and plan(Q6_K, 130, 30720, 40) == (4, 8, 1)
+    assert [plan(dt, 1024, 16384, 64) for dt in (Q4_K, Q6_K)] == [(11, 1, 1)] * 2 and plan(Q6_K, 1024, 12288, 64) == (11, 1, 1)
     # fewer super-blocks than six MFMA tiles ask for: the low tile, whose four waves hold all the columns where their number is odd
     assert plan(Q4_K, 2048, 2048, 600) == (4, 1, 2) and plan(Q4_K, 2048, 2304, 600) == (4, 1, 1)
     # Q8_0: whichever kernel has the smaller estimate, in any number of rounds
@@ -285,7 +290,8 @@ def test_prefill_columns_beyond_32_bit_offsets(dt, row_tiles):
     t = ctypes.c_int()
 
     def cols(super_blocks):
-        capi.check(L.turq_prefill_plan(dt, 64, 256 * super_blocks, 40, 256, ctypes.byref(t), None, None))
+        capi.check(L.turq_prefill_plan(dt, 12416, 256 * super_blocks, 40, 256,  # (too many tiles for a split over workgroups)
+                                       ctypes.byref(t), None, None))
         return t.value > 10
 
     top = (2**32 // row_tiles - 1) // L.turq_tiled_nbytes(dt, 16, 256)

@@ -79,7 +79,8 @@ CASES = [  # dtype, n, k, rows
     (Q4_K, 4096, 4096, (1, 2, 4, 8, 24)),       # one-row kernel (1, 2, 4 rows), rows staged in the kernel
     (Q6_K, 1040, 12288, (1, 3, 20, 32)),        # tall: prepared fragments at 17 .. 32 rows
     (Q8_0, 200, 1056, (1, 5, 40)),              # ragged Q8_0 columns: the skinny kernel in chunks at 40 rows
-    (Q4_K, 512, 8192, (70, 128)),               # prefill GEMM with its columns split over workgroups
+    (Q4_K, 512, 8192, (70, 128)),               # prefill GEMM, columns split over waves ...
+    (Q4_K, 130, 28672, (70,)),                  # ... and over workgroups
     (Q5_K, 1000, 2048, (33, 300)),              # prefill GEMM, ragged n (scalar stores) ...
     (Q6_K, 1024, 2048, (512,)),                 # ... and aligned (16-byte stores)
 ]

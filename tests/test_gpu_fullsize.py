@@ -98,8 +98,7 @@ def test_prefill_up_proj(gpu, m):
 @pytest.mark.parametrize("m", [64, 128, 256])
 def test_prefill_down_proj_split_columns(gpu, m):
     # the tall matrix of the layer (Q6_K down_proj 4096 x 12288) at prompt-chunk sizes: few workgroup tiles, so every tile's
-    # columns go to several workgroups whose partial sums meet in device memory (low tile up to 128 rows, wide tile at 256);
-    # the oracle checks every 16th weight row
+    # columns go to the waves of its workgroup (tiles of 32 x 32, 64 x 32 and 64 x 64); the oracle checks every 16th weight row
     n, k = 4096, 12288
     raw = synth.random_weight(Q6_K, n, k, seed=45)
     w = gpu.upload(Q6_K, n, k, raw, capi.LAYOUT_TILED)
@@ -139,7 +138,7 @@ def test_q4km_decoder_layer_grouped_calls(gpu, layer, m, x_dtype):
     # turq_qmatmul_multi, down_proj alone; device pointers, every output against the f32 matmul on the dequantized weights
     raws, ws = layer
     # (40 and 64 rows: gate / up in two chunks through the kernels of up to 32 rows, the others through the prefill GEMM, whose
-    # folded f16 scales cost about 3e-4; down_proj, o_proj and q / k / v with their columns split over several workgroups;
+    # folded f16 scales cost about 3e-4; down_proj, o_proj and q / k / v with their columns split over the waves;
     # 128 and 256 rows: gate and up as one GEMM launch over the rows of both)
     bf = x_dtype == capi.ACT_BF16
     bar = 2e-5 if bf and m <= 32 else 1e-3

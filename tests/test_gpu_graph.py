@@ -82,9 +82,9 @@ class Step:
                                   capi.MEM_DEVICE, capi.ALGO_AUTO), ctx)
 
 
-# (64 rows of 8192 columns: prefill launches whose tiles are split over several workgroups - their counters in device memory
+# (64 rows of 28672 columns: prefill launches whose tiles are split over several workgroups - their counters in device memory
 # must be back at zero after every replay, with no memset node in the graph)
-@pytest.mark.parametrize("m,k", [(1, 1024), (8, 1024), (64, 1024), (64, 8192)])
+@pytest.mark.parametrize("m,k", [(1, 1024), (8, 1024), (64, 1024), (64, 8192), (64, 28672)])
 def test_graph_replays_equal_the_eager_calls(gpu, m, k):
     L, ctx = gpu.L, gpu.ctx
     st = Step(gpu, m, k=k)

@@ -248,12 +248,12 @@ def test_prefill_tall_weight_f32_and_bf16(gpu, dt):
 
 
 
-# Tall-k matrices at prefill chunk sizes (down_proj: 4096 x 12288) make few workgroup tiles, so the launcher gives every tile
-# to several workgroups that each take a part of the columns and meet in device memory.  Shapes that split on a 256-CU device
-# (few tiles, many super-blocks): results against the oracle, twice in a row (the tiles' counters must be back at zero), with
-# bias, row strides, a ragged n and m, and every output type.
+# Tall-k matrices at prefill chunk sizes (down_proj: 4096 x 12288) make few workgroup tiles, so the columns of a tile are shared out
+# over its waves or, from many more columns on, over several workgroups that meet in device memory (the last two shapes on a 256-CU device:
+# shares of 14 super-blocks in two groups of waves, of 15 in one).  Results against the oracle, twice in a row (the tiles' counters must be
+# back at zero), with bias, row strides, a ragged n and m, and every output type.
 @pytest.mark.parametrize("dt", [Q4_K, Q5_K, Q6_K])
-@pytest.mark.parametrize("n,k,m", [(512, 8192, 128), (200, 6144, 70), (1024, 12288, 300), (256, 4096, 512)])
+@pytest.mark.parametrize("n,k,m", [(512, 8192, 128), (200, 6144, 70), (1024, 12288, 300), (256, 4096, 512), (300, 28672, 70), (130, 30720, 40)])
 def test_prefill_gemm_split_columns(gpu, dt, n, k, m):
     raw = synth.random_weight(dt, n, k, seed=n + m)
     x = synth.random_activation(m, k, seed=m, bf16=True)
@@ -533,7 +533,8 @@ def test_multi_weight_prefill_shares_the_preparation(gpu):
     ((Q6_K, Q6_K, Q6_K), [4096, 1024, 1024], 4096, (200, 256)),
     ((Q4_K, Q4_K), [2048, 2048], 2048, (300, 512)),                     # (from about 600 rows on: large weights of one shape, within 2e-6)
     ((Q8_0, Q8_0), [4096, 512], 512, (400, 1100)),
-], ids=["qkv-q8_0", "gateup-q8_0", "qkv-q4km", "qkv-q6k", "pair-q4k", "uneven-q8_0"])
+    ((Q4_K, Q4_K, Q6_K), [512, 512, 256], 28672, (64, 300)),            # columns split over workgroups, and not any more
+], ids=["qkv-q8_0", "gateup-q8_0", "qkv-q4km", "qkv-q6k", "pair-q4k", "uneven-q8_0", "many-columns"])
 def test_multi_weight_prefill_keeps_the_bits_of_the_single_calls(gpu, dts, ns, k, ms):
     # whatever launches the rules make of several weights: each keeps the kernel that it takes alone, so the sums are the same
     raws = [synth.random_weight(dt, n, k, seed=11 * i + n) for i, (dt, n) in enumerate(zip(dts, ns))]
@@ -778,13 +779,12 @@ def test_staged_rows_kernel_group_sizes(row_tiles):
 # that would leave CUs idle) from the problem size; the small matrices of the tests above would never reach the wide one and
 # always take the low one, so they run once more in child processes with each of the two forced and forbidden (the rule takes
 # the wide tile for some of the full-size cases), and with the columns of every tile split over 2, 4 or 8 workgroups wherever
-# that number divides the super-blocks (on the wide or the low tile), or never; and with the low tile's eight-wave form (two
+# that number divides the super-blocks (on the low tile), or never; and with the low tile's eight-wave form (two
 # groups of waves on alternate super-blocks) forbidden, and forced on every low-tile launch with an even share of super-blocks.
 @pytest.mark.parametrize("switch,value", [("TURQ_GEMM_WIDE", "1"), ("TURQ_GEMM_WIDE", "0"), ("TURQ_GEMM_LOW", "1"), ("TURQ_GEMM_LOW", "0"),
-                                          ("TURQ_GEMM_SPLIT", "0"), ("TURQ_GEMM_SPLIT+TURQ_GEMM_SPLIT_FORM", "2+3"),
-                                          ("TURQ_GEMM_SPLIT+TURQ_GEMM_SPLIT_FORM", "4+4"), ("TURQ_GEMM_SPLIT", "8"),
+                                          ("TURQ_GEMM_SPLIT", "0"), ("TURQ_GEMM_SPLIT", "2"), ("TURQ_GEMM_SPLIT", "4"), ("TURQ_GEMM_SPLIT", "8"),
                                           ("TURQ_GEMM_KGROUPS", "1"), ("TURQ_GEMM_KGROUPS+TURQ_GEMM_LOW", "2+1"),
-                                          ("TURQ_GEMM_KGROUPS+TURQ_GEMM_SPLIT+TURQ_GEMM_SPLIT_FORM", "2+2+4")])
+                                          ("TURQ_GEMM_KGROUPS+TURQ_GEMM_SPLIT", "2+2")])
 def test_prefill_tile_shapes(switch, value):
     import os
     import subprocess

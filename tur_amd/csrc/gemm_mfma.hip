@@ -50,7 +50,7 @@
 // tiles are larger (2816 / 3360 bytes), so their workgroup is 128 x 128 to keep three super-blocks of weights in the LDS.  Q8_0 (4352-byte tiles, f16 block scales, no sums term): 128 x 64, wave tile 2 x 1.
 //
 // Launches that would leave CUs idle.  Three further forms of the same loop, chosen per launch by the rules at the end of this
-// file: every tile's super-blocks shared out over several workgroups that meet in device memory (SK); the low tile with eight
+// file: the low tile's super-blocks shared out over several workgroups that meet in device memory (SK); the low tile with eight
 // waves as two groups on alternate super-blocks that meet in the LDS (KG = 2); and up to four weights of one format in one
 // launch (GemmGroup), the n-blocks dealt out to them in order.
 //
@@ -58,6 +58,7 @@
 // that a lane stores 16 contiguous bytes and a row segment is 192 (bf16, f16) or 384 (f32) bytes.
 #include <hip/hip_ext.h>
 
+#include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 #include <utility>
@@ -808,50 +809,32 @@ int turq_gemm_form(int dtype, int64_t n, int64_t k, int64_t m, int compute_units
     }
 }
 
-// ---- which launches split their columns ----
-// A launch whose tiles leave most CUs idle - the tall-k matrices of a model at prefill chunk sizes (down_proj 4096 x 12288 makes
-// 32 low tiles at 64 rows, 64 wide ones at 512), and every matrix of the layer at 64 rows - gives every tile to `split`
-// workgroups.  What the parts' meeting costs grows with the partial tiles the launch writes and reads back (m x n x 4 bytes
-// x (2 split - 1)), so the rule takes the low tile for few rows and the wide one above, and only as many parts as leave a
-// quarter of the CUs free (low tiles; a quarter of the CUs taken when k is short, and then only up to 128 rows: since the
-// low tile runs eight waves there is less to win) or fill them once (wide tiles, up to an eighth of the CUs).  Measured on MI355X, Q6_K 4096 x 12288, no split -> split: 64 rows 75 -> 35 us
-// (low, 6 parts), 128: 78 -> 47 (low, 3), 256: 82 -> 66 (wide, 6), 512: 97 -> 92 (wide, 4: within what a whole layer's step
-// varies by, not taken), 1024: none helps; Q4_K 4096 x 4096: 64 rows 28 -> 22 us (low, 4), 128: 28 -> 27 (low, 2), from 256
-// rows on none helps; 12288 x 4096: none helps; with the eight-wave low tile since: 4096 x 4096 unsplit 21.8 / 22.3 us at 64 /
-// 128 rows against 21.1 / 24.2 in 4 / 2 parts, 1024 x 4096 21.6 / 21.8 against 15.3 / 16.9 in 4 parts.  TURQ_GEMM_SPLIT = 0: never, s > 1: by s wherever s divides (with
-// TURQ_GEMM_SPLIT_FORM = 3 / 4: on the wide / low tile).
-size_t turq_gemm_split_scratch(int dtype, int64_t n, int64_t k, int64_t m, int compute_units, int *form_out, int *split_out) {
-    if (form_out) *form_out = 0;
+// ---- which launches split their columns over workgroups ----
+// Few tiles over very many columns: where gemm_cols.hip, whose four waves share out the columns of a tile, leaves most CUs idle for a
+// hundred super-blocks, every 64 x 128 tile is given to up to eight workgroups, as many as divide the super-blocks, leave each part four of them and
+// a quarter of the CUs free.  Taken where what that takes is a tenth below what gemm_cols.hip's smallest tile takes, both fitted to launches on
+// MI355X: the parts' meeting costs about 7 us and more with the partial tiles to move.  gemm_cols.hip -> here, 64 rows: Q4_K 512 x 28672 38 -> 29
+// us, 256 x 65536 80 -> 49, Q5_K 1024 x 28672 41 -> 32 (128 rows 39 -> 36); not taken: Q4_K 1024 x 16384 23.6 -> 23.3 (128 rows 22.7 -> 27.6), 512 x
+// 16384 19.7 -> 19.8, Q6_K 1024 x 12288 21.5 -> 22.8, 4096 x 12288 24 -> 35.  TURQ_GEMM_SPLIT = 0: never, s > 1: by s wherever s divides.
+size_t turq_gemm_split_scratch(int dtype, int64_t n, int64_t k, int64_t m, int compute_units, int *split_out) {
     if (split_out) *split_out = 1;
-    const int env = turq_tuning().gemm_split, env_form = turq_tuning().gemm_split_form;
+    const int env = turq_tuning().gemm_split;
     if (env == 0 || compute_units <= 0 || (dtype != TURQ_Q4_K && dtype != TURQ_Q5_K && dtype != TURQ_Q6_K)) return 0;
-    const int64_t cus = compute_units, ntc = k / 256;
-    const int64_t low_tiles = ((n + 127) / 128) * ((m + 63) / 64), wide_tiles = ((n + 255) / 256) * ((m + 127) / 128);
-    // the most parts that divide the super-blocks, leave each part at least min_sb of them and make at most max_wgs workgroups
-    auto parts = [&](int64_t tiles, int64_t max_wgs, int64_t min_sb) {
-        int best = 1;
-        for (int s = 2; s <= 8; s++)
-            if (ntc % s == 0 && ntc / s >= min_sb && tiles * s <= max_wgs) best = s;
-        return best;
-    };
-    int form = 0, split = 1;
+    const int64_t ntc = k / 256, tiles = ((n + 127) / 128) * ((m + 63) / 64);
+    int split = 1;
+    if (env <= 1 && turq_tuning().gemm_cols > 0) return 0;
     if (env > 1) {
-        form = env_form == 3 || env_form == 4 ? env_form : (m <= 128 ? 4 : 3);
         split = ntc % env == 0 ? env : 1;
     } else {
-        const bool tall = ntc >= 32;
-        split = tall || m <= 128 ? parts(low_tiles, tall ? 3 * cus / 4 : cus / 4, 4) : 1;
-        form = 4;
-        if (split == 1 && tall && 8 * wide_tiles <= cus) {
-            split = parts(wide_tiles, cus, 8);
-            form = 3;
-        }
+        for (int s = 2; s <= 8; s++)
+            if (ntc % s == 0 && ntc / s >= 4 && 4 * tiles * s <= 3 * (int64_t)compute_units) split = s;
+        const int fmt = dtype == TURQ_Q4_K ? 0 : dtype == TURQ_Q5_K ? 1 : 2;
+        static constexpr double kHere[] = {1.15, 1.30, 1.45}, kCols[] = {0.30, 0.33, 0.36};  // us per super-block
+        const double here = 12.0 + kHere[fmt] * (double)(ntc / split) + 0.05 * (double)std::max<int64_t>(0, tiles * split - 32);
+        if (!(here < 0.9 * (4.0 + kCols[fmt] * (double)ntc))) return 0;
     }
-    if (split < 2) return 0;
-    const int64_t bm = form == 4 ? 64 : 128, bn = form == 4 ? 128 : 256;
-    const size_t tiles = (size_t)(form == 4 ? low_tiles : wide_tiles), bytes = tiles * (size_t)split * (size_t)(bm * bn * 4);
-    if (tiles * 16 > kSplitCounterBytes || bytes > (256u << 20)) return 0;
-    if (form_out) *form_out = form;
+    const size_t bytes = (size_t)tiles * (size_t)split * (size_t)(64 * 128 * 4);
+    if (split < 2 || (size_t)tiles * 16 > kSplitCounterBytes || bytes > (256u << 20)) return 0;
     if (split_out) *split_out = split;
     return bytes;
 }
@@ -939,10 +922,10 @@ hipError_t turq_launch_gemm_mfma_group(int dtype, const TurqGemmWeights &ws, int
     // eight-wave one is slower (LM head at 64 rows 178 -> 196 us).  TURQ_GEMM_KGROUPS = 1: never, 2: wherever the share is even.
     auto two_groups_for = [&](int split) { return turq_gemm_low_two_groups(n, k, m, split, compute_units); };
     if (split_counters && split_partials) {
-        int sform = 0, split = 1;
-        const size_t need = turq_gemm_split_scratch(dtype, n, k, m, compute_units, &sform, &split);
+        int split = 1;
+        const size_t need = turq_gemm_split_scratch(dtype, n, k, m, compute_units, &split);
         if (need != 0 && need <= split_partial_bytes) {
-            if (sform == 4 && two_groups_for(split)) {
+            if (two_groups_for(split)) {
 #define TURQ_GEMM_SK2(DT)                                                                                                               \
     return launch_gemm<DT, 4, true, 2>(ws, k, frags, m, y_dtype, stream, ev_start, ev_stop, split, split_counters, split_partials, \
                                        split_partial_bytes)
@@ -954,16 +937,13 @@ hipError_t turq_launch_gemm_mfma_group(int dtype, const TurqGemmWeights &ws, int
                 }
 #undef TURQ_GEMM_SK2
             }
-#define TURQ_GEMM_SK(DT, F)                                                                                                           \
-    return launch_gemm<DT, F, true>(ws, k, frags, m, y_dtype, stream, ev_start, ev_stop, split, split_counters, split_partials, \
+#define TURQ_GEMM_SK(DT)                                                                                                              \
+    return launch_gemm<DT, 4, true>(ws, k, frags, m, y_dtype, stream, ev_start, ev_stop, split, split_counters, split_partials, \
                                     split_partial_bytes)
-            switch (dtype * 8 + sform) {
-            case TURQ_Q4_K * 8 + 3: TURQ_GEMM_SK(TURQ_Q4_K, 3);
-            case TURQ_Q4_K * 8 + 4: TURQ_GEMM_SK(TURQ_Q4_K, 4);
-            case TURQ_Q5_K * 8 + 3: TURQ_GEMM_SK(TURQ_Q5_K, 3);
-            case TURQ_Q5_K * 8 + 4: TURQ_GEMM_SK(TURQ_Q5_K, 4);
-            case TURQ_Q6_K * 8 + 3: TURQ_GEMM_SK(TURQ_Q6_K, 3);
-            case TURQ_Q6_K * 8 + 4: TURQ_GEMM_SK(TURQ_Q6_K, 4);
+            switch (dtype) {
+            case TURQ_Q4_K: TURQ_GEMM_SK(TURQ_Q4_K);
+            case TURQ_Q5_K: TURQ_GEMM_SK(TURQ_Q5_K);
+            case TURQ_Q6_K: TURQ_GEMM_SK(TURQ_Q6_K);
             default: break;
             }
 #undef TURQ_GEMM_SK

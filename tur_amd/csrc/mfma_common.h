@@ -351,6 +351,6 @@ int turq_gemm_form(int dtype, int64_t n, int64_t k, int64_t m, int compute_units
 // tile's gain)
 double turq_gemm_fill(int dtype, int64_t n, int64_t k, int64_t m, int compute_units, int64_t *wgs_out);
 bool turq_gemm_low_two_groups(int64_t n, int64_t k, int64_t m, int split, int compute_units);
-// bytes of partial tiles a launch of this shape wants for splitting its columns, 0 if it does not split; form_out / split_out
-// (may be null): the tile (3: wide, 4: low) and the number of parts
-size_t turq_gemm_split_scratch(int dtype, int64_t n, int64_t k, int64_t m, int compute_units, int *form_out, int *split_out);
+// bytes of partial tiles a launch of this shape wants for splitting its columns over workgroups (in the low tile), 0 if it does not split;
+// split_out (may be null): the number of parts
+size_t turq_gemm_split_scratch(int dtype, int64_t n, int64_t k, int64_t m, int compute_units, int *split_out);

@@ -181,7 +181,7 @@ static int gemm_split_reserve(turq_ctx *ctx, int count, const turq_weight *const
     size_t off[turq_ctx::kSplitSlots], total = kCounters;
     bool any = false;
     for (int i = 0; i < count; i++) {
-        out->bytes[i] = skip[i] ? 0 : turq_gemm_split_scratch(w[i]->dtype, w[i]->n, w[i]->k, m, ctx->compute_units, nullptr, nullptr);
+        out->bytes[i] = skip[i] ? 0 : turq_gemm_split_scratch(w[i]->dtype, w[i]->n, w[i]->k, m, ctx->compute_units, nullptr);
         off[i] = total;
         total += (out->bytes[i] + 255) & ~(size_t)255;
         any = any || out->bytes[i] != 0;
@@ -232,6 +232,8 @@ static int gemm_cols_tile(const turq_ctx *ctx, int count, const turq_weight *con
         if (w[i]->n <= 0 || w[i]->k != w[0]->k || w[i]->dtype != w[i < s ? 0 : s]->dtype) return 0;
     }
     if (second) *second = s;
+    // (few tiles of very many columns: gemm_kq_kernel with the columns split over workgroups, where there is scratch for their meeting)
+    if (count == 1 && !ctx->fixed_scratch && turq_gemm_split_scratch(w[0]->dtype, n[0], w[0]->k, m, ctx->compute_units, nullptr) != 0) return 0;
     return turq_gemm_cols_tile(w[0]->dtype, w[s < count ? s : 0]->dtype, count, n, w[0]->k, m, ctx->compute_units);
 }
 
@@ -258,11 +260,10 @@ static int gemm_on_frags(turq_ctx *ctx, const turq_weight *w, int64_t m, void *y
 // workgroups share a CU) and the 128-row tiles (one per CU; wide tiles counted as two).  Measured on the Q4_K_M layer: launches
 // of 192 workgroups next to each other help with the 64-row tile (m = 128: +4.8 %) and hurt with the 128-row tile (m = 256: -2.7 %).
 static int64_t gemm_cus_taken_shape(int compute_units, int dtype, int64_t n, int64_t k, int64_t m, bool may_split) {
-    int form = 0, split = 1;
-    if (may_split && turq_gemm_split_scratch(dtype, n, k, m, compute_units, &form, &split) != 0) {
-        const int64_t tiles = form == 4 ? ((n + 127) / 128) * ((m + 63) / 64) : ((n + 255) / 256) * ((m + 127) / 128);
-        const bool whole = form != 4 || turq_gemm_low_two_groups(n, k, m, split, compute_units);
-        return whole ? tiles * split : (tiles * split + 1) / 2;
+    int split = 1;
+    if (may_split && turq_gemm_split_scratch(dtype, n, k, m, compute_units, &split) != 0) {
+        const int64_t wgs = ((n + 127) / 128) * ((m + 63) / 64) * split;
+        return turq_gemm_low_two_groups(n, k, m, split, compute_units) ? wgs : (wgs + 1) / 2;
     }
     if (dtype == TURQ_Q8_0) return ((n + 63) / 64) * ((m + 127) / 128);
     const int64_t nt = (n + 127) / 128, wgs128 = ((m + 127) / 128) * nt;
@@ -282,6 +283,7 @@ static int64_t gemm_cus_taken(const turq_ctx *ctx, const turq_weight *w, int64_t
 static bool gemm_merge_rule(int dtype, int64_t n, int64_t k, int64_t m, int run, int compute_units, int64_t taken_alone) {
     const int64_t cus = compute_units;
     if (run < 2 || 2 * taken_alone <= cus || !turq_dt_is_quant(dtype) || n % 256 != 0) return false;
+    if (turq_gemm_split_scratch(dtype, n, k, m, compute_units, nullptr) != 0) return false;  // (each alone in parts: never slower than whole)
     int64_t wgs_one = 0, wgs_all = 0;
     const double fill_one = turq_gemm_fill(dtype, n, k, m, compute_units, &wgs_one);
     const double fill_all = turq_gemm_fill(dtype, n * run, k, m, compute_units, &wgs_all);
@@ -307,6 +309,7 @@ static bool gemm_run_pays(const turq_ctx *ctx, int run, const turq_weight *const
     double apart = 0.0;
     for (int i = 0; i < run; i++) {
         if (w[i]->dtype != w[0]->dtype || w[i]->n <= 0 || w[i]->n % 256 != 0) return false;
+        if (turq_gemm_split_scratch(w[i]->dtype, w[i]->n, w[i]->k, m, ctx->compute_units, nullptr) != 0) return false;
         n[i] = w[i]->n;
         const double us = turq_gemm_launch_us(w[i]->dtype, 1, n + i, w[i]->k, m, ctx->compute_units);
         if (us == 0.0) return false;
@@ -851,13 +854,13 @@ extern "C" int turq_prefill_plan(int dtype, int64_t n, int64_t k, int64_t m, int
     if (n <= 0 || k <= 0 || k % 256 != 0 || m <= TURQ_GEMV_MAX_M || compute_units <= 0)
         return turq_fail(nullptr, TURQ_ERR_SHAPE, "turq_prefill_plan: n=%lld k=%lld m=%lld on %d compute units", (long long)n, (long long)k,
                          (long long)m, compute_units);
-    if (const int cols = turq_gemm_cols_tile(dtype, dtype, 1, &n, k, m, compute_units)) {  // gemm_cols.hip, asked first as in gemm_on_frags
+    int form = turq_gemm_form(dtype, n, k, m, compute_units), parts = 1;
+    if (turq_gemm_split_scratch(dtype, n, k, m, compute_units, &parts) != 0) {  // (the order in which gemm_cols_tile asks)
+        form = 4;
+    } else if (const int cols = turq_gemm_cols_tile(dtype, dtype, 1, &n, k, m, compute_units)) {
         if (tile) *tile = cols;
         return TURQ_OK;
     }
-    int form = turq_gemm_form(dtype, n, k, m, compute_units), parts = 1, sform = 0;
-    if (turq_gemm_split_scratch(dtype, n, k, m, compute_units, &sform, &parts) != 0) form = sform;
-    else parts = 1;
     if (tile) *tile = form;
     if (split) *split = parts;
     if (wave_groups) *wave_groups = form == 4 && turq_gemm_low_two_groups(n, k, m, parts, compute_units) ? 2 : 1;

@@ -39,7 +39,6 @@
     X(gemm_wide, "TURQ_GEMM_WIDE", TRI, -1, "prefill: the wide tile 128 x 256 always (1) or never (0)")                                     \
     X(gemm_low, "TURQ_GEMM_LOW", TRI, -1, "prefill: the low tile 64 x 128 always (1) or never (0)")                                         \
     X(gemm_split, "TURQ_GEMM_SPLIT", INT, -1, "prefill: workgroups per tile that share its columns (0 / 1: never split)")                   \
-    X(gemm_split_form, "TURQ_GEMM_SPLIT_FORM", INT, 0, "prefill: tile of a forced split (3 wide, 4 low)")                                   \
     X(gemm_kgroups, "TURQ_GEMM_KGROUPS", INT, 0, "prefill low tile: 1 four waves, 2 eight waves as two groups")                             \
     X(gemm_cols, "TURQ_GEMM_COLS", INT, -1, "prefill kernel whose waves split the columns: 0 never, 11 21 31 22 32 23 42 always in that tile")  \
     X(prefetch_wgs, "TURQ_PREFETCH_WGS", INT, 0, "workgroups of turq_weight_prefetch (1 .. 4096)")                                          \
