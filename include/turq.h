@@ -371,7 +371,8 @@ int turq_read_yardstick(turq_ctx *ctx, const void *dev_ptr, size_t nbytes);
  * path, no counterpart in the reference: for tests of the rules and for tuning them on another device. */
 int turq_prefill_plan(int dtype, int64_t n, int64_t k, int64_t m, int compute_units, int *tile, int *split, int *wave_groups);
 /* ... and whether turq_qmatmul_multi sends `count` (1 .. 4) neighbouring weights of that format and shape - gate_proj and up_proj -
- * out as ONE launch over the rows of all of them (merged = 1) or as a launch each (0).  The rule compares how well the two
+ * out as ONE launch over the rows of all of them, with the tile and the kernel chosen for all the rows (merged = 1), or not (0: a launch each,
+ * or, where each makes few tiles and for Q8_0, one launch of the kernel that each takes alone).  The rule compares how well the two
  * choices fill their rounds over the device's CUs, so the answer depends on compute_units; the kernels give the same products
  * either way (another order of the f32 sums where a tile's waves split k: within 2e-6). */
 int turq_prefill_plan_multi(int dtype, int64_t n, int64_t k, int64_t m, int count, int compute_units, int *merged);

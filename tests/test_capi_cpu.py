@@ -273,6 +273,11 @@ def test_prefill_launch_rules_on_a_256_cu_device():
     # the rule counts rounds over the CUs, so a device of half the size decides differently at the same shapes
     assert [merged(12288, m, 128) for m in (64, 128, 256, 384, 512, 1024, 2048)] == [0, 1, 0, 1, 1, 0, 0]
     assert merged(1024, 2048, 128) == 1
+    # Q8_0 weights go together only in the kernel that each takes alone, whatever their size
+    g = ctypes.c_int(-1)
+    for n, k, m in ((1536, 1024, 1798), (3072, 1024, 1024), (3072, 1024, 2048), (15104, 10496, 1172)):
+        capi.check(L.turq_prefill_plan_multi(Q8_0, n, k, m, 2, 256, ctypes.byref(g)))
+        assert g.value == 0, (n, k, m)
     # arguments
     t = ctypes.c_int()
     assert L.turq_prefill_plan_multi(Q4_K, 12288, 4096, 8, 2, 256, ctypes.byref(t)) == capi.ERR_SHAPE

@@ -833,7 +833,8 @@ int turq_qmatmul_multi_mfma(turq_ctx *ctx, int count, const turq_weight *const *
     return TURQ_OK;
 }
 
-// whether turq_qmatmul_multi sends `count` neighbouring weights of this format and shape out as one prefill launch (no GPU needed)
+// whether turq_qmatmul_multi sends `count` neighbouring weights of this format and shape out as one prefill launch whose tile is chosen for
+// all the rows (no GPU needed; Q8_0 weights only go together in the kernel and the tile order that each takes alone)
 extern "C" int turq_prefill_plan_multi(int dtype, int64_t n, int64_t k, int64_t m, int count, int compute_units, int *merged) {
     if (merged) *merged = 0;
     if (!turq_dt_is_quant(dtype)) return turq_fail(nullptr, TURQ_ERR_DTYPE, "turq_prefill_plan_multi: dtype %d has no prefill kernel", dtype);
@@ -841,7 +842,7 @@ extern "C" int turq_prefill_plan_multi(int dtype, int64_t n, int64_t k, int64_t 
         return turq_fail(nullptr, TURQ_ERR_SHAPE, "turq_prefill_plan_multi: n=%lld k=%lld m=%lld count=%d on %d compute units", (long long)n,
                          (long long)k, (long long)m, count, compute_units);
     const int64_t alone = gemm_cus_taken_shape(compute_units, dtype, n, k, m, true);
-    if (merged) *merged = gemm_merge_rule(dtype, n, k, m, count, compute_units, alone) ? 1 : 0;
+    if (merged) *merged = dtype != TURQ_Q8_0 && gemm_merge_rule(dtype, n, k, m, count, compute_units, alone) ? 1 : 0;
     return TURQ_OK;
 }
 
