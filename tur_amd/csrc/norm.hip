@@ -15,7 +15,7 @@ template <int XT> __device__ inline float ld_elem(const void *x, int64_t i) {
     return (float)h;
 }
 
-// Both kernels take a row in pieces of 8 neighbouring columns: thread t of a row's 256 holds the pieces t, t + 256, ... (PER of them
+// The kernels take a row of more than 512 columns in pieces of 8 neighbouring columns: thread t of a row's 256 holds the pieces t, t + 256, ... (PER of them
 // in registers), loaded and stored 16 bytes at a time where the row allows it.  Bound by latency at decode sizes (one row is one
 // chain load -> sum -> barrier -> divide -> store in a launch of 4 us) and by the memory system at prompt sizes.  With one element per load
 // (2 bytes of a bf16 row) the chain of 16 loads per thread was the kernel: 8 rows of 4096 bf16 columns took 10.5 us, now 4.0 - 4.7.
@@ -67,19 +67,60 @@ __device__ inline float rms_of(float s, int64_t k, float eps, float *part) {
 // v / rms for many v against one rms, to the last bit: with r = 1 / rms correctly rounded, q = v * r corrected once by its own
 // remainder is the correctly rounded quotient (P. Markstein, "Computation of elementary functions on the IBM RISC System/6000",
 // 1990) as long as nothing over- or underflows on the way.  No |v| of a row exceeds sqrt(k) * rms; from 2^-60 on, against an rms between
-// 2^-40 and 2^40, the quotient is at least 2^-100 and the remainder, a multiple of 2^-48 |v| or so, stays exact.  Smaller elements - zeros, whose
-// sign the correction would lose, among them - and rows whose rms is an infinity, a NaN or outside that range take the plain division.
+// 2^-40 and 2^40, the quotient is at least 2^-100 and the remainder, a multiple of 2^-48 |v| or so, stays exact.  Pieces with a smaller element -
+// a zero, whose sign the correction would lose, among them - and rows whose rms is an infinity, a NaN or outside that range take the plain
+// division (asked once per piece: asked per element the kernel was 0.3 us longer at one row, a tenth).
 struct RowDiv {
     float rms, r, least;  // least: the smallest |v| that is corrected (an infinity: none is)
     __device__ explicit RowDiv(float d) : rms(d), r(1.0f / d), least(d > 0x1p-40f && d < 0x1p40f ? 0x1p-60f : __builtin_inff()) {}
-    __device__ float operator()(float v) const {
-        const float q = v * r;
-        return __builtin_expect(!(__builtin_fabsf(v) >= least), 0) ? v / rms : __builtin_fmaf(__builtin_fmaf(-q, rms, v), r, q);
+    __device__ void operator()(const float (&v)[8], float (&o)[8]) const {
+        bool plain = false;
+#pragma unroll
+        for (int e = 0; e < 8; e++) plain |= !(__builtin_fabsf(v[e]) >= least);
+        if (__builtin_amdgcn_ballot_w64(plain) != 0) {  // (one branch of the wave: the division gives the others the same quotients)
+#pragma unroll
+            for (int e = 0; e < 8; e++) o[e] = v[e] / rms;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float q = v[e] * r;
+                o[e] = __builtin_fmaf(__builtin_fmaf(-q, rms, v[e]), r, q);
+            }
+        }
     }
 };
 
+// rows of up to kShort columns: one workgroup of 256 threads per row, two elements t and t + 256 per thread.  A piece of eight columns per thread
+// leaves three of the four waves without any: 128 columns (the heads of q and k) at 1 / 16384 rows 2.7 / 16.0 us, here 2.2 / 11.7; from 1024
+// columns on the pieces are ahead (16384 bf16 rows 28.5 -> 20.0)
+constexpr int64_t kShort = 512;
+template <int XT> __device__ inline float short_square_sum(const void *x, int64_t xo, int64_t k, int tid, float (&v)[2]) {
+    float s = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const int64_t c = (int64_t)j * 256 + tid;
+        v[j] = c < k ? ld_elem<XT>(x, xo + c) : 0.0f;
+        s = __builtin_fmaf(v[j], v[j], s);  // (columns past k add +0)
+    }
+    return s;
+}
+template <int XT, int YT>
+__global__ void __launch_bounds__(256) rms_norm_short_kernel(const void *__restrict__ x, int64_t k, int64_t ldx, const float *__restrict__ w,
+                                                             float eps, void *__restrict__ y, int64_t ldy) {
+    __shared__ float part[4];
+    const int tid = threadIdx.x;
+    const int64_t row = blockIdx.x;
+    float v[2];
+    const float rms = rms_of(short_square_sum<XT>(x, row * ldx, k, tid, v), k, eps, part);
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const int64_t c = (int64_t)j * 256 + tid;
+        if (c < k) turq_store_out<YT>(y, row * ldy + c, v[j] / rms * w[c]);
+    }
+}
+
 // one workgroup of 256 threads per row; rows of up to 2048 * PER elements are read once (so y may be x whatever the two element
-// types), longer rows are read again
+// types), longer rows, which only PER = 3 takes, are read again
 template <int XT, int YT, int PER>
 __global__ void __launch_bounds__(256) rms_norm_kernel(const void *__restrict__ x, int64_t k, int64_t ldx, const float *__restrict__ w,
                                                        float eps, void *__restrict__ y, int64_t ldy) {
@@ -100,7 +141,7 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(const void *__restrict__ 
     for (int j = 0; j < PER; j++)
 #pragma unroll
         for (int e = 0; e < 8; e++) s = __builtin_fmaf(v[j][e], v[j][e], s);  // (columns past k add +0: the sum is that of the columns that exist)
-    for (int64_t col0 = ((int64_t)PER * 256 + tid) * 8; col0 < k; col0 += 2048) {
+    for (int64_t col0 = ((int64_t)PER * 256 + tid) * 8; PER == 3 && col0 < k; col0 += 2048) {
         float t[8];
         ld_piece<XT>(x, xo, col0, k, vx, t);
 #pragma unroll
@@ -111,8 +152,9 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(const void *__restrict__ 
         if (col0 >= k) return;
         float wv[8], o[8];
         ld_piece<TURQ_ACT_F32>(w, 0, col0, k, vw, wv);
+        div(t, o);
 #pragma unroll
-        for (int e = 0; e < 8; e++) o[e] = div(t[e]) * wv[e];
+        for (int e = 0; e < 8; e++) o[e] *= wv[e];
         if (vy && col0 + 8 <= k) {
             turq_note_results<YT>(o);
             uint8_t *p = (uint8_t *)y + (yo + col0) * (YT == TURQ_ACT_F32 ? 4 : 2);
@@ -135,7 +177,7 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(const void *__restrict__ 
     };
 #pragma unroll
     for (int j = 0; j < PER; j++) store(((int64_t)j * 256 + tid) * 8, v[j]);
-    for (int64_t col0 = ((int64_t)PER * 256 + tid) * 8; col0 < k; col0 += 2048) {
+    for (int64_t col0 = ((int64_t)PER * 256 + tid) * 8; PER == 3 && col0 < k; col0 += 2048) {
         float t[8];
         ld_piece<XT>(x, xo, col0, k, vx, t);
         store(col0, t);
@@ -172,10 +214,15 @@ __global__ void __launch_bounds__(256 * kPrepRows) rms_norm_prep32_kernel(const 
         const int64_t col0 = ((int64_t)j * 256 + tid) * 8;
         ld_piece<XT>(x, xo, col0, live ? k : 0, vx, v[j]);
     }
+    if (PER == 1 && k <= kShort) {  // (the order of rms_norm_short_kernel)
+        float sq[2];
+        s = short_square_sum<XT>(x, xo, live ? k : 0, tid, sq);
+    } else {
 #pragma unroll
-    for (int j = 0; j < PER; j++)
+        for (int j = 0; j < PER; j++)
 #pragma unroll
-        for (int e = 0; e < 8; e++) s = __builtin_fmaf(v[j][e], v[j][e], s);
+            for (int e = 0; e < 8; e++) s = __builtin_fmaf(v[j][e], v[j][e], s);
+    }
     const RowDiv div(rms_of(s, k, eps, part[sub]));
 #pragma unroll
     for (int j = 0; j < PER; j++) {
@@ -185,9 +232,10 @@ __global__ void __launch_bounds__(256 * kPrepRows) rms_norm_prep32_kernel(const 
         ld_piece<TURQ_ACT_F32>(w, 0, col0, k, vw, wv);
         half8v h;
         float sum = 0.0f, f[8];
+        div(v[j], f);
 #pragma unroll
         for (int e = 0; e < 8; e++) {
-            f[e] = live ? div(v[j][e]) * wv[e] : 0.0f;
+            f[e] = live ? f[e] * wv[e] : 0.0f;
             h[e] = (_Float16)f[e];
             sum += (float)h[e];
         }
@@ -212,7 +260,8 @@ __global__ void __launch_bounds__(256 * kPrepRows) rms_norm_prep32_kernel(const 
 
 template <int XT, int YT>
 hipError_t launch2(const void *x, int64_t m, int64_t k, int64_t ldx, const float *w, float eps, void *y, int64_t ldy, hipStream_t s) {
-    if (k <= 2048) rms_norm_kernel<XT, YT, 1><<<(unsigned)m, 256, 0, s>>>(x, k, ldx, w, eps, y, ldy);
+    if (k <= kShort) rms_norm_short_kernel<XT, YT><<<(unsigned)m, 256, 0, s>>>(x, k, ldx, w, eps, y, ldy);
+    else if (k <= 2048) rms_norm_kernel<XT, YT, 1><<<(unsigned)m, 256, 0, s>>>(x, k, ldx, w, eps, y, ldy);
     else if (k <= 2 * 2048) rms_norm_kernel<XT, YT, 2><<<(unsigned)m, 256, 0, s>>>(x, k, ldx, w, eps, y, ldy);
     else rms_norm_kernel<XT, YT, 3><<<(unsigned)m, 256, 0, s>>>(x, k, ldx, w, eps, y, ldy);
     return hipGetLastError();
