@@ -312,10 +312,11 @@ template <int DTA, int DTB, int MT, int NT>
 __global__ void __launch_bounds__(64 * W) gemm_cols_kernel(ColsGroup grp, int64_t k, const uint8_t *__restrict__ frags, int64_t m, int yt,
                                                            int nblocks_n, int nblocks_m, int vec_out) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    // consecutive logical ids run on one XCD (blockIdx % 8): the m-blocks of one n-block share its packed weights in that XCD's L2
-    const int nwg = nblocks_n * nblocks_m;
-    int lid = blockIdx.x;
-    if ((nwg & 7) == 0) lid = (blockIdx.x & 7) * (nwg >> 3) + (blockIdx.x >> 3);
+    // consecutive logical ids run on one XCD (blockIdx % 8): the m-blocks of one n-block share its packed weights in that XCD's L2.  Also where
+    // the workgroups are no multiple of 8 (the first XCDs have one more): with ids as they come there, Q8_0 18944 x 1024 at 300 rows (990
+    // workgroups) took 47.3 us instead of 41.3
+    const int nwg = nblocks_n * nblocks_m, xcd = (int)blockIdx.x & 7, extra = nwg & 7;
+    const int lid = xcd * (nwg >> 3) + (xcd < extra ? xcd : extra) + ((int)blockIdx.x >> 3);
     const int mb = lid % nblocks_m, nb_all = lid / nblocks_m;
     int wi = 0;
 #pragma unroll
@@ -387,12 +388,13 @@ bool turq_gemm_cols_mixed(int dtype_a, int dtype_b) { return (dtype_a == TURQ_Q4
 // The tile (10 * MT + NT) with which `count` weights of n[i] rows and k columns go through this kernel in one launch, 0 where the launch
 // is gemm_kq_kernel's; *us: roughly what it takes.
 //
-// A launch of one round over the CUs takes base + per_sb * super-blocks, fitted to launches of every format (graphs of launches over more
-// weights than the caches hold); a further round costs as much again without the launch itself, of the smallest tile, of which three workgroups
+// A launch of one round over the CUs takes about base + per_sb * super-blocks, one fit over launches of every format (graphs of launches over
+// more weights than the caches hold; Q4_K takes up to a quarter less, Q6_K of 32 x 32 tiles on full rounds up to a quarter more: 4096 x 12288 at 77
+// rows 35 us for 28), which serves to order the tiles and, for Q8_0, to choose between the kernels; a further round costs as much again without the launch itself, of the smallest tile, of which three workgroups
 // share a CU, three fifths of it.  So the smallest tile that makes the launch one round is the best of them.  Against gemm_kq_kernel:
 //   one or two MFMA tiles: Q4_K 1024 x 4096 at 40 / 300 / 512 rows 13.0 / 19.0 / 19.1 -> 6.6 / 9.3 / 10.7 us, 4096 x 4096 at 40 / 100 rows 19.2 /
 //   22.6 -> 8.7 / 11.3, Q6_K 4096 x 12288 33 / 43 -> 23 / 29, Q8_0 2048 x 2048 15 -> 5.4 / 5.5;
-//   three or four: Q8_0 2048 x 2048 at 300 / 512 rows 15.4 -> 8.5 / 10.2, Q4_K 4096 x 4096 at 256 24 -> 15;
+//   three or four: K-quants from two super-blocks on (Q4_K 12288 x 256 at 48 rows 8.4 -> 9.4); Q8_0 2048 x 2048 at 300 / 512 rows 15.4 -> 8.5 / 10.2, Q4_K 4096 x 4096 at 256 24 -> 15;
 //   six: from 12 super-blocks on (Q4_K 4096 x 4096 at 300 rows 23.4 -> 20.4, Q6_K 4096 x 12288 74 -> 51; with 4 super-blocks Q8_0 6144 x 1024
 //   at 160 rows 11.1 -> 11.7);
 //   eight: from 40 super-blocks on, Q6_K from 24 (512 rows, 4096 x 12288: Q4_K 66 -> 64, Q5_K 76 -> 69, Q6_K 81 -> 66; 4096 x 4096: Q4_K 26.3 -> 27.5).
@@ -432,6 +434,7 @@ int turq_gemm_cols_tile(int dtype_a, int dtype_b, int count, const int64_t *n, i
         const int64_t wgs = nbn * ((m + 32 * c.mt - 1) / (32 * c.mt));
         if (!eight) {
             if (wgs > (area == 1 ? cus + cus / 2 : cus)) continue;
+            if (area == 4 && ntc < 2) continue;
             if (area > 4 && ntc < (area == 6 ? 12 : dtype_a == TURQ_Q6_K ? 24 : 40)) continue;
         }
         const double x = (double)wgs / (double)cus;
