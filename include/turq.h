@@ -135,6 +135,8 @@ int turq_memcpy_d2h(turq_ctx *ctx, void *dst_host, const void *src_dev, size_t n
 /* Upload raw GGUF block bytes of a tensor of shape (n, k) (n output features, k input features,
  * each row = k/block consecutive blocks).  `layout` picks how it is kept in HBM.
  * Errors: unsupported dtype, k % block != 0, nbytes != turq_weight_nbytes(..).
+ * The first quantized upload allocates 32 MiB of device memory that the context keeps for later ones (without memory for it
+ * the host lays the tiles out instead).
  * Replaces: candle `gguf_file::Content::tensor(reader, name, device)` -> `QTensor` as called by
  * `QVarBuilder::get` (src/weights/gguf_varbuilder.rs:72-74) and `QMatMul::from_arc`
  * (src/models/layers/linear.rs:69). */
@@ -253,8 +255,8 @@ enum { TURQ_ACTFN_SILU = 0 };
  * act = SiLU, v / (1 + exp(-v)), computed in f32.  gate and up are two weights of one shape [n, k]; x, y, the strides, the
  * biases (NULL: none) and `mem` as in turq_qmatmul.  With device pointers, tiled weights of one format and up to 32
  * activation rows the activation and the product are applied inside the matmul kernel, which writes one output instead of
- * two: up to 16 rows that kernel is the one launch of the call, for more rows (and for the k and alignments named at
- * turq_qmatmul_multi) it follows one preparation of the activations (scratch memory of the context, which grows on demand,
+ * two: up to 16 rows, and with 17 - 32 rows on most weights of up to 4096 columns, that kernel is the one launch of the call; for the
+ * others (and for the k and alignments named at turq_qmatmul_multi) it follows one preparation of the activations (scratch memory of the context, which grows on demand,
  * never inside a graph capture).  Every other case computes the two products through turq_qmatmul_multi into scratch memory of the context and
  * combines them in one elementwise pass (with TURQ_MEM_HOST that pass runs on the host CPU, in the same f32 arithmetic: the
  * host form is for tests and one-off calls).  Errors as turq_qmatmul; gate and up of different shapes: TURQ_ERR_SHAPE; an activation other

@@ -254,6 +254,7 @@ def test_prefill_launch_rules_on_a_256_cu_device():
     assert [plan(dt, 1024, 16384, 64) for dt in (Q4_K, Q6_K)] == [(11, 1, 1)] * 2 and plan(Q6_K, 1024, 12288, 64) == (11, 1, 1)
     # fewer super-blocks than six MFMA tiles ask for: the low tile, whose four waves hold all the columns where their number is odd
     assert plan(Q4_K, 2048, 2048, 600) == (4, 1, 2) and plan(Q4_K, 2048, 2304, 600) == (4, 1, 1)
+    assert [plan(dt, n, 2816, 256) for dt, n in ((Q4_K, 5120), (capi.Q5_K, 4992))] == [(4, 1, 1)] * 2  # launches that run side by side
     # Q8_0: whichever kernel has the smaller estimate, in any number of rounds
     Q8_0 = capi.Q8_0
     assert [plan(Q8_0, 3072, 1024, m)[0] for m in (256, 300, 512, 1024, 2048)] == [11, 22, 23, 23, 2]

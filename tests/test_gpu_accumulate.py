@@ -3,9 +3,12 @@
 
 The sum is formed in f32 and rounded once to y's type, so the expected value is exact: the f32 result of the same call
 without the flag, plus what y held, rounded like y.  Every kernel family is driven through the C ABI (one row, a few rows,
-rows staged in the kernel, prepared fragments, the prefill GEMM with and without split columns, the dense and native-layout
+rows staged in the kernel, the prefill kernels in every tile, the dense and native-layout
 kernel, host pointers, wide activations, turq_mlp, turq_qmatmul_noalloc)."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -77,13 +80,16 @@ def run(gpu, w, x, n, k, y0, yt, flag, bias=None, noalloc=False, mem=capi.MEM_DE
 
 CASES = [  # dtype, n, k, rows
     (Q4_K, 4096, 4096, (1, 2, 4, 8, 24)),       # one-row kernel (1, 2, 4 rows), rows staged in the kernel
-    (Q6_K, 1040, 12288, (1, 3, 20, 32)),        # tall: prepared fragments at 17 .. 32 rows
+    (Q6_K, 1040, 12288, (1, 3, 20, 32)),        # tall: 16-bit rows staged as they are at 17 .. 32 rows
     (Q8_0, 200, 1056, (1, 5, 40)),              # ragged Q8_0 columns: the skinny kernel in chunks at 40 rows
     (Q4_K, 512, 8192, (70, 128)),               # prefill GEMM, columns split over waves ...
     (Q4_K, 130, 28672, (70,)),                  # ... and over workgroups
-    (Q5_K, 1000, 2048, (33, 300)),              # prefill GEMM, ragged n (scalar stores) ...
-    (Q6_K, 1024, 2048, (512,)),                 # ... and aligned (16-byte stores)
+    (Q5_K, 1000, 2048, (33, 300)),              # ... rows past the last tile
+    (Q6_K, 1024, 2048, (512,)),
+    (Q4_K, 999, 2048, (65, 300)),               # ... scalar stores
+    (Q8_0, 320, 1024, (100,)),
 ]
+PREFILL_CASES = " or ".join(f"{c[0]}-{c[1]}x{c[2]}" for c in CASES if max(c[3]) > 40)
 
 
 @pytest.mark.parametrize("yt", [capi.ACT_F32, capi.ACT_BF16, capi.ACT_F16], ids=["f32", "bf16", "f16"])
@@ -104,6 +110,19 @@ def test_results_are_added_to_the_output(gpu, dt, n, k, ms, yt):
         # without the flag the buffer's contents do not matter
         assert np.array_equal(run(gpu, w, x, n, k, y0, yt, 0, bias=bias, x_dtype=capi.ACT_BF16), to_type(plain, yt)), m
     gpu.release(w)
+
+
+# the matrices above are small, so the rules give them the smallest tile: once more with every tile of gemm_kq_kernel (o_proj and
+# down_proj of long prompts), and with the tiles of the column-splitting kernel whose waves meet in several rounds
+@pytest.mark.parametrize("switch,value", [("TURQ_GEMM_COLS", "0"), ("TURQ_GEMM_WIDE", "1"), ("TURQ_GEMM_LOW", "0"), ("TURQ_GEMM_KGROUPS", "1"),
+                                          ("TURQ_GEMM_COLS", "22"), ("TURQ_GEMM_COLS", "32"), ("TURQ_GEMM_COLS", "23"), ("TURQ_GEMM_COLS", "42")])
+def test_results_are_added_by_every_prefill_tile(switch, value):
+    env = dict(os.environ, **{switch: value})
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    out = subprocess.run([sys.executable, "-m", "pytest", "-q", "-x", "-m", "gpu", "-k", f"added_to_the_output and ({PREFILL_CASES})",
+                          "-p", "no:cacheprovider", os.path.join(root, "tests", "test_gpu_accumulate.py")],
+                         cwd=root, env=env, capture_output=True, text=True, timeout=280)
+    assert out.returncode == 0, out.stdout[-3000:] + out.stderr[-1000:]
 
 
 def test_other_routes(gpu):

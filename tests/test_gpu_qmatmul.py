@@ -588,32 +588,44 @@ def test_prefill_merged_runs_forced():
 
 
 def test_multi_weight_prefill_small_launches_side_by_side(gpu):
-    # q / k / v of a prompt chunk: launches that leave half of the machine free run in groups of up to three, the first on
-    # the context's stream, the others on further streams, between the shared preparation and the end of the call.  Same kernels, same inputs: bit-equal with the
-    # single calls, eagerly (twice, the buffers reused) and in a captured graph replayed with other activations.
+    # q / k / v of a prompt chunk, several weights in one launch: bit-equal with the single calls, eagerly (twice, the buffers
+    # reused) and in a captured graph replayed with other activations.
+    run_side_by_side(gpu, 1024, (Q4_K, Q4_K, Q6_K, Q5_K), [512, 128, 128, 80], (40, 130, 512, 40), 96)
+
+
+def test_multi_weight_prefill_launches_on_side_streams(gpu):
+    # launches of gemm_kq_kernel that leave half of the machine free (an odd number of super-blocks, so four waves and two workgroups
+    # per CU; too many tiles for one round of the column-splitting kernel) run in groups of up to three, the first on the context's stream,
+    # the others on further streams, between the shared preparation and the end of the call (test_capi_cpu.py pins the kernel)
+    k, ns, dts, m = 2816, [5120, 5120, 4992], (Q4_K, Q4_K, Q5_K), 256
+    run_side_by_side(gpu, k, dts, ns, (m, 250, m), m)
+
+
+def run_side_by_side(gpu, k, dts, ns, ms, m):
     L, ctx = gpu.L, gpu.ctx
-    k, dts, ns = 1024, (Q4_K, Q4_K, Q6_K, Q5_K), [512, 128, 128, 80]
+    count = len(ns)
     raws = [synth.random_weight(dt, n, k, seed=7 * i + n) for i, (dt, n) in enumerate(zip(dts, ns))]
     ws = [gpu.upload(dt, n, k, raw, capi.LAYOUT_TILED) for dt, n, raw in zip(dts, ns, raws)]
     biases = [np.random.default_rng(i).standard_normal(n).astype(np.float32) if i == 1 else None for i, n in enumerate(ns)]
-    for m in (40, 130, 512, 40):
-        x = synth.random_activation(m, k, seed=m, bf16=True)
+    for rows in ms:
+        x = synth.random_activation(rows, k, seed=rows, bf16=True)
         ys = gpu.qmatmul_multi(ws, x, ns, k, biases=biases)
         for dt, n, raw, w, y, b in zip(dts, ns, raws, ws, ys, biases):
-            assert rel_l2(y, orc.matmul_dequant(dt, x, raw, n, k) + (0 if b is None else b)) <= 1e-3, (m, dt, n)
-            assert np.array_equal(y, gpu.qmatmul(w, x, n, k, bias=b)), (m, dt, n)
+            some = np.arange(0, n, 1 + n // 512)
+            want = orc.matmul_dequant(dt, x, raw.reshape(n, -1)[some].reshape(-1), len(some), k) + (0 if b is None else b[some])
+            assert rel_l2(y[:, some], want) <= 1e-3, (rows, dt, n)
+            assert np.array_equal(y, gpu.qmatmul(w, x, n, k, bias=b)), (rows, dt, n)
 
     def dev(nbytes):
         p = ctypes.c_void_p()
         capi.check(L.turq_dev_alloc(ctx, nbytes, ctypes.byref(p)), ctx)
         return p
-    m = 96
     xd, yd = dev(m * k * 4), [dev(m * n * 4) for n in ns]
-    warr = (ctypes.c_void_p * 4)(*[w.value for w in ws])
-    yarr = (ctypes.c_void_p * 4)(*[p.value for p in yd])
-    ldys = (ctypes.c_int64 * 4)(*ns)
+    warr = (ctypes.c_void_p * count)(*[w.value for w in ws])
+    yarr = (ctypes.c_void_p * count)(*[p.value for p in yd])
+    ldys = (ctypes.c_int64 * count)(*ns)
     capi.check(L.turq_graph_begin(ctx), ctx)
-    capi.check(L.turq_qmatmul_multi(ctx, 4, warr, xd, capi.ACT_F32, m, k, yarr, capi.ACT_F32, ldys, None, capi.MEM_DEVICE,
+    capi.check(L.turq_qmatmul_multi(ctx, count, warr, xd, capi.ACT_F32, m, k, yarr, capi.ACT_F32, ldys, None, capi.MEM_DEVICE,
                                     capi.ALGO_AUTO), ctx)
     graph = ctypes.c_void_p()
     capi.check(L.turq_graph_end(ctx, ctypes.byref(graph)), ctx)

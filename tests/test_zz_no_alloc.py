@@ -39,14 +39,14 @@ def both(gpu, w, x, n, k, x_dtype, y_dtype):
 @pytest.mark.parametrize("dt,n,k,ms", [
     (capi.Q4_K, 4096, 4096, (32, 8)),       # up to 4096 columns: fragments made in the kernel from the rows themselves, no scratch
     (capi.Q6_K, 1024, 4096, (16, 3)),
-    (capi.Q6_K, 4096, 12288, (32, 20)),     # 17 .. 32 rows of 12288 columns: fragments prepared in the static array, then fewer rows
+    (capi.Q6_K, 4096, 12288, (32, 20)),     # 17 .. 32 rows of 12288 columns: 16-bit rows staged as they are
     (capi.Q4_K, 2048, 4352, (24, 17)),      # k not a multiple of 512 (17 column tiles): prepared fragments again
     (capi.Q4_K, 1024, 4096, (512, 64)),     # the prefill GEMM, then a smaller chunk
     (capi.Q5_K, 512, 2048, (200, 33)),
     (capi.Q4_K, 256, 28672, (64, 33)),      # ... whose columns turq_qmatmul splits over workgroups
     (capi.Q8_0, 3072, 1024, (48, 2)),
     (capi.Q4_K, 12288, 4096, (1, 1)),       # one row: no scratch at all
-], ids=["q4k-staged", "q6k-staged", "q6k-frag-k12288", "q4k-frag-odd-k", "q4k-gemm", "q5k-gemm", "q4k-gemm-k28672", "q8_0", "q4k-row1"])
+], ids=["q4k-staged", "q6k-staged", "q6k-staged-k12288", "q4k-frag-odd-k", "q4k-gemm", "q5k-gemm", "q4k-gemm-k28672", "q8_0", "q4k-row1"])
 def test_noalloc_equals_qmatmul_twice_in_a_row(gpu, dt, n, k, ms):
     raw = synth.random_weight(dt, n, k, seed=n + k)
     w = gpu.upload(dt, n, k, raw, capi.LAYOUT_TILED)
@@ -63,6 +63,32 @@ def test_noalloc_equals_qmatmul_twice_in_a_row(gpu, dt, n, k, ms):
             assert rel_l2(got[:, rows], orc.matmul_dequant(dt, x, sub, len(rows), k)) <= 1e-3, m
     finally:
         gpu.release(w)
+
+
+@pytest.mark.parametrize("dt,n,k", [(capi.Q6_K, 1024, 8192), (capi.Q8_0, 200, 4608)])
+def test_noalloc_wide_rows_as_f16_in_the_static_array(gpu, dt, n, k):
+    # 17 .. 32 rows of more than 4096 columns: f32 rows, and rows that 16-byte loads may not touch, are rounded to f16 into the
+    # static array first; then fewer rows, and the bits of turq_qmatmul whatever the type and the alignment
+    L, ctx = gpu.L, gpu.ctx
+    raw = synth.random_weight(dt, n, k, seed=n)
+    w = gpu.upload(dt, n, k, raw, capi.LAYOUT_TILED)
+    for m in (32, 17):
+        x = synth.random_activation(m, k, seed=m, bf16=True).astype(np.float16).astype(np.float32)
+        x = synth.from_bf16_bits(synth.to_bf16_bits(x)).reshape(m, k)
+        want = gpu.qmatmul_device(w, x, n, k, x_dtype=capi.ACT_F32)
+        assert rel_l2(want, orc.matmul_dequant(dt, x, raw, n, k)) <= 2e-5, m
+        for x_dtype, ldx in ((capi.ACT_F32, k), (capi.ACT_F32, k + 1), (capi.ACT_BF16, k), (capi.ACT_BF16, k + 1), (capi.ACT_F16, k + 3)):
+            padded = np.zeros((m, ldx), np.float32)
+            padded[:, :k] = x
+            send = (synth.to_bf16_bits(padded).reshape(m, ldx) if x_dtype == capi.ACT_BF16
+                    else padded.astype(np.float16) if x_dtype == capi.ACT_F16 else padded)
+            xd, yd = gpu.dev_buffer(send), gpu.dev_buffer(np.full((m, n), np.nan, np.float32))
+            capi.check(L.turq_qmatmul_noalloc(ctx, w, xd, x_dtype, m, ldx, yd, capi.ACT_F32, n, None), ctx)
+            got = gpu.read_back(yd, (m, n), np.float32)
+            gpu.dev_free(xd)
+            gpu.dev_free(yd)
+            assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (m, x_dtype, ldx)
+    gpu.release(w)
 
 
 def test_noalloc_refuses_what_does_not_fit(gpu):
