@@ -253,7 +253,7 @@ def test_prefill_tall_weight_f32_and_bf16(gpu, dt):
 # shares of 14 super-blocks in two groups of waves, of 15 in one).  Results against the oracle, twice in a row (the tiles' counters must be
 # back at zero), with bias, row strides, a ragged n and m, and every output type.
 @pytest.mark.parametrize("dt", [Q4_K, Q5_K, Q6_K])
-@pytest.mark.parametrize("n,k,m", [(512, 8192, 128), (200, 6144, 70), (1024, 12288, 300), (256, 4096, 512), (300, 28672, 70), (130, 30720, 40)])
+@pytest.mark.parametrize("n,k,m", [(512, 8192, 128), (200, 6144, 70), (1024, 12288, 300), (256, 4096, 512), (140, 28672, 70), (130, 30720, 40)])
 def test_prefill_gemm_split_columns(gpu, dt, n, k, m):
     raw = synth.random_weight(dt, n, k, seed=n + m)
     x = synth.random_activation(m, k, seed=m, bf16=True)
@@ -533,7 +533,7 @@ def test_multi_weight_prefill_shares_the_preparation(gpu):
     ((Q6_K, Q6_K, Q6_K), [4096, 1024, 1024], 4096, (200, 256)),
     ((Q4_K, Q4_K), [2048, 2048], 2048, (300, 512)),                     # (from about 600 rows on: large weights of one shape, within 2e-6)
     ((Q8_0, Q8_0), [4096, 512], 512, (400, 1100)),
-    ((Q4_K, Q4_K, Q6_K), [512, 512, 256], 28672, (64, 300)),            # columns split over workgroups, and not any more
+    ((Q4_K, Q4_K, Q6_K), [256, 256, 128], 28672, (64, 600)),            # columns split over workgroups, and not any more
 ], ids=["qkv-q8_0", "gateup-q8_0", "qkv-q4km", "qkv-q6k", "pair-q4k", "uneven-q8_0", "many-columns"])
 def test_multi_weight_prefill_keeps_the_bits_of_the_single_calls(gpu, dts, ns, k, ms):
     # whatever launches the rules make of several weights: each keeps the kernel that it takes alone, so the sums are the same
@@ -593,7 +593,7 @@ def test_multi_weight_prefill_small_launches_side_by_side(gpu):
     run_side_by_side(gpu, 1024, (Q4_K, Q4_K, Q6_K, Q5_K), [512, 128, 128, 80], (40, 130, 512, 40), 96)
 
 
-def test_multi_weight_prefill_launches_on_side_streams(gpu):
+def test_multi_weight_launches_on_side_streams(gpu):
     # launches of gemm_kq_kernel that leave half of the machine free (an odd number of super-blocks, so four waves and two workgroups
     # per CU; too many tiles for one round of the column-splitting kernel) run in groups of up to three, the first on the context's stream,
     # the others on further streams, between the shared preparation and the end of the call (test_capi_cpu.py pins the kernel)
