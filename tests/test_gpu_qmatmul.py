@@ -841,3 +841,35 @@ def test_prefill_column_split_edges(gpu, dt, n, k, m):
     assert rel_l2(got, want) <= 1e-3
     assert np.array_equal(got, gpu.qmatmul(w, x, n, k))
     gpu.release(w)
+
+
+def test_prefill_column_split_largest_tile():
+    # 96 x 96, the tile of gate and up together at 65 - 96 rows, on the edges of the test above
+    import os
+    import subprocess
+    import sys
+
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    out = subprocess.run([sys.executable, "-m", "pytest", "-q", "-x", "-m", "gpu", "-k", "test_prefill_column_split_edges", "-p", "no:cacheprovider",
+                          os.path.join(root, "tests", "test_gpu_qmatmul.py")],
+                         cwd=root, env=dict(os.environ, TURQ_GEMM_COLS="33"), capture_output=True, text=True, timeout=280)
+    assert out.returncode == 0, out.stdout[-3000:] + out.stderr[-1000:]
+
+
+@pytest.mark.parametrize("dt", [Q4_K, Q5_K, Q6_K, Q8_0])
+@pytest.mark.parametrize("k", [1024, 1280])
+def test_prefill_column_split_two_workgroups_per_cu(gpu, dt, k):
+    # 485 workgroups of the 64 x 64 tile, two of which share a CU in a form of the loop of its own: one super-block per wave, and two for one of
+    # the four; the bound of the prefill kernels, and the same bits as fewer rows give in another tile and form
+    import ctypes
+
+    n, m, t = 6161, 300, ctypes.c_int()
+    capi.check(gpu.L.turq_prefill_plan(dt, n, k, m, 256, ctypes.byref(t), None, None))
+    assert t.value == 22
+    raw = synth.random_weight(dt, n, k, seed=k)
+    w = gpu.upload(dt, n, k, raw, capi.LAYOUT_TILED)
+    x = synth.random_activation(m, k, seed=m, bf16=True)
+    got = gpu.qmatmul(w, x, n, k)
+    assert rel_l2(got, orc.matmul_dequant(dt, x, raw, n, k)) <= 1e-3
+    assert np.array_equal(got[:64], gpu.qmatmul(w, x[:64], n, k))
+    gpu.release(w)

@@ -9,9 +9,16 @@
 // fewer bytes per flop and is the better kernel where its launch fills the machine for many super-blocks, but each of its stage
 // boundaries waits for copies that left one stage earlier, which is what a launch of few tiles spends its time on.
 //
-// Loads of a wave return in order, so a weight load that comes from HBM holds up every fragment load issued after it.  The weights of
+// The loop exists in two forms.  Loads of a wave return in order, so a weight load that comes from HBM holds up every fragment load issued after it.  The weights of
 // super-block b + 1 are therefore requested together, behind the fragments of the last stage of b: the first loads that are waited for
-// behind them belong to super-block b + 1 itself.
+// behind them belong to super-block b + 1 itself.  That takes a second set of weight registers and two stages of fragments.  The TIGHT
+// form requests every stage of the weights of b + 1 into the registers that the same stage of b has just left, and holds one stage
+// of fragments, a step of which is requested again as soon as it is used: with it two workgroups of the 64 x 64 tile share a CU, so that one
+// computes while the other waits for its first loads or stores its results.  What bounds these launches is the issue of one wave per
+// SIMD: without any load in the loop they still take 60 - 90 % of their time, and an order of MFMAs and unpacking made by hand, deeper
+// rings and more waves of smaller tiles changed nothing.  Two workgroups per CU do: Q8_0 6144 x 1024 at 300 rows 14.1 -> 10.9 us, 4096 x 4096 at
+// 512 31.6 -> 27.2, Q4_K 24576 x 4096 at 256 84 -> 73; where there is only one workgroup per CU, the first form is ahead (Q4_K 4096 x 4096 at 77
+// rows 13.5 against 14.9).
 #include <hip/hip_ext.h>
 
 #include <algorithm>
@@ -32,18 +39,17 @@ struct ColsGroup {
     int count, second;     // weights from `second` on are of the kernel's second format
 };
 
-// a lane's packed weights of one 32-row tile and one super-block, as the loads deliver them
+// a lane's packed weights of one 32-row tile and one super-block, as the loads deliver them: the header, and the four stages in order;
+// what two stages share comes with the second of them
 template <int DT> struct WBlk;
 // loads: `t` the lane's 16-row tile (scalar base + lane offset `o`), slot = r16 + 32 * g32
 __device__ inline uint4v ld16(const uint8_t *base, uint32_t o) { return *(const uint4v *)(base + o); }
 
 template <> struct WBlk<TURQ_Q4_K> {
     uint4v q[4], hd;
-    __device__ void load(const uint8_t *p, uint32_t o, uint32_t r16, uint32_t slot) {
-        using F = TiledFmt<TURQ_Q4_K>;
-        hd = ld16(p, o + F::kHDR + 16u * r16);
-#pragma unroll
-        for (int ks = 0; ks < 4; ks++) q[ks] = ld16(p, o + 16u * slot + (uint32_t)((ks & 1) * 1024 + (ks >> 1) * 256));
+    __device__ void load_hdr(const uint8_t *p, uint32_t o, uint32_t r16, uint32_t) { hd = ld16(p, o + TiledFmt<TURQ_Q4_K>::kHDR + 16u * r16); }
+    template <int KS> __device__ void load(const uint8_t *p, uint32_t o, uint32_t slot) {
+        q[KS] = ld16(p, o + 16u * slot + (uint32_t)((KS & 1) * 1024 + (KS >> 1) * 256));
     }
     __device__ GFmt<TURQ_Q4_K>::Hdr hdr() const { return {hd}; }
     template <int KS> __device__ GFmt<TURQ_Q4_K>::Stage stage() const { return {q[KS]}; }
@@ -51,13 +57,10 @@ template <> struct WBlk<TURQ_Q4_K> {
 template <> struct WBlk<TURQ_Q5_K> {
     uint4v q[4], hd;
     uint2v hh[2];
-    __device__ void load(const uint8_t *p, uint32_t o, uint32_t r16, uint32_t slot) {
-        using F = TiledFmt<TURQ_Q5_K>;
-        hd = ld16(p, o + F::kHDR + 16u * r16);
-#pragma unroll
-        for (int s = 0; s < 2; s++) hh[s] = *(const uint2v *)(p + (o + F::kQH + 8u * slot + (uint32_t)(s * 128)));
-#pragma unroll
-        for (int ks = 0; ks < 4; ks++) q[ks] = ld16(p, o + 16u * slot + (uint32_t)((ks & 1) * 1024 + (ks >> 1) * 256));
+    __device__ void load_hdr(const uint8_t *p, uint32_t o, uint32_t r16, uint32_t) { hd = ld16(p, o + TiledFmt<TURQ_Q5_K>::kHDR + 16u * r16); }
+    template <int KS> __device__ void load(const uint8_t *p, uint32_t o, uint32_t slot) {
+        q[KS] = ld16(p, o + 16u * slot + (uint32_t)((KS & 1) * 1024 + (KS >> 1) * 256));
+        if constexpr (KS & 1) hh[KS >> 1] = *(const uint2v *)(p + (o + TiledFmt<TURQ_Q5_K>::kQH + 8u * slot + (uint32_t)((KS >> 1) * 128)));
     }
     __device__ GFmt<TURQ_Q5_K>::Hdr hdr() const { return {hd}; }
     template <int KS> __device__ GFmt<TURQ_Q5_K>::Stage stage() const { return {q[KS], hh[KS >> 1]}; }
@@ -65,29 +68,25 @@ template <> struct WBlk<TURQ_Q5_K> {
 template <> struct WBlk<TURQ_Q6_K> {
     uint4v ql[4], qh[2];
     uint32_t sc0, sc1, d16;
-    __device__ void load(const uint8_t *p, uint32_t o, uint32_t r16, uint32_t slot) {
+    __device__ void load_hdr(const uint8_t *p, uint32_t o, uint32_t r16, uint32_t slot) {
         using F = TiledFmt<TURQ_Q6_K>;
         sc0 = *(const uint32_t *)(p + (o + F::kSC + 4u * slot));
         sc1 = *(const uint32_t *)(p + (o + F::kSC + 4u * slot + 64u));
         d16 = *(const uint16_t *)(p + (o + F::kD + 2u * r16));
-#pragma unroll
-        for (int s = 0; s < 2; s++) qh[s] = ld16(p, o + F::kQH + 16u * slot + (uint32_t)(s * 256));
-#pragma unroll
-        for (int ks = 0; ks < 4; ks++) ql[ks] = ld16(p, o + 16u * slot + (uint32_t)((ks & 1) * 1024 + (ks >> 1) * 256));
+    }
+    template <int KS> __device__ void load(const uint8_t *p, uint32_t o, uint32_t slot) {
+        ql[KS] = ld16(p, o + 16u * slot + (uint32_t)((KS & 1) * 1024 + (KS >> 1) * 256));
+        if constexpr (KS & 1) qh[KS >> 1] = ld16(p, o + TiledFmt<TURQ_Q6_K>::kQH + 16u * slot + (uint32_t)((KS >> 1) * 256));
     }
     __device__ GFmt<TURQ_Q6_K>::Hdr hdr() const { return {sc0, sc1, d16}; }
     template <int KS> __device__ GFmt<TURQ_Q6_K>::Stage stage() const { return {ql[KS], qh[KS >> 1]}; }
 };
 template <> struct WBlk<TURQ_Q8_0> {
     uint4v a[4], b[4], dd;
-    __device__ void load(const uint8_t *p, uint32_t o, uint32_t r16, uint32_t slot) {
-        using F = TiledFmt<TURQ_Q8_0>;
-        dd = ld16(p, o + F::kD + 16u * r16);
-#pragma unroll
-        for (int ks = 0; ks < 4; ks++) {
-            a[ks] = ld16(p, o + 16u * slot + (uint32_t)(ks * 1024));
-            b[ks] = ld16(p, o + 16u * slot + (uint32_t)(ks * 1024 + 256));
-        }
+    __device__ void load_hdr(const uint8_t *p, uint32_t o, uint32_t r16, uint32_t) { dd = ld16(p, o + TiledFmt<TURQ_Q8_0>::kD + 16u * r16); }
+    template <int KS> __device__ void load(const uint8_t *p, uint32_t o, uint32_t slot) {
+        a[KS] = ld16(p, o + 16u * slot + (uint32_t)(KS * 1024));
+        b[KS] = ld16(p, o + 16u * slot + (uint32_t)(KS * 1024 + 256));
     }
     __device__ GFmt<TURQ_Q8_0>::Hdr hdr() const { return {dd}; }
     template <int KS> __device__ GFmt<TURQ_Q8_0>::Stage stage() const { return {a[KS], b[KS]}; }
@@ -95,7 +94,7 @@ template <> struct WBlk<TURQ_Q8_0> {
 
 template <int MT> struct AStage { half8v f[MT][4]; };
 
-// Four waves in every tile shape, and one stage of fragments in flight besides the one being used.  The sums of a result are then the
+// Four waves in every tile shape and form, and (first form) one stage of fragments in flight besides the one being used.  The sums of a result are then the
 // same numbers in the same order whatever the tile (a weight alone and in a launch with others agree to the bit).  Eight waves were up
 // to 7 % faster on the 64-row tile and spill on the larger ones; three stages in flight measured 1 - 8 % slower than one (registers).
 constexpr int W = 4, RA = 2;
@@ -107,7 +106,7 @@ template <int MT, int NT> struct Meet {
     static constexpr int LDS = W * T * 32 * kPitch * 4;
 };
 
-template <int DT, int MT, int NT>
+template <int DT, int MT, int NT, bool TIGHT>
 __device__ __forceinline__ void cols_body(const ColsGroup &grp, int wi, int nb, int mb, int64_t k, const uint8_t *__restrict__ frags, int64_t m,
                                           int yt, int vec_out, uint8_t *lds) {
     using Fm = GFmt<DT>;
@@ -129,7 +128,8 @@ __device__ __forceinline__ void cols_body(const ColsGroup &grp, int wi, int nb, 
 #pragma unroll
     for (int i = 0; i < MT; i++) {
         const int64_t mt = (int64_t)mb * MT + i;
-        a_src[i] = frags + ((size_t)((mt < mtiles ? mt : mtiles - 1) * ntc * 17) << 10);
+        const uint64_t off = ((uint64_t)((mt < mtiles ? mt : mtiles - 1) * ntc * 17)) << 10;  // (wave-uniform: kept in scalar registers)
+        a_src[i] = frags + (((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(off >> 32)) << 32) | __builtin_amdgcn_readfirstlane((uint32_t)off));
     }
     const int tile0 = nb * NT * 2;
     const uint8_t *w_src = w + (size_t)tile0 * ntc * TB;
@@ -152,73 +152,148 @@ __device__ __forceinline__ void cols_body(const ColsGroup &grp, int wi, int nb, 
 #pragma unroll
             for (int e = 0; e < 16; e++) acc[i][j][e] = 0.0f;
 
-    AStage<MT> ra[RA];
-    half8v sf[MT];
-    Wb wcur[NT], wnext[NT];
-    auto load_a = [&](int b, auto KS) {
-        constexpr int ks = decltype(KS)::value;
+    if constexpr (!TIGHT) {
+        AStage<MT> ra[RA];
+        half8v sf[MT];
+        Wb wcur[NT], wnext[NT];
+        auto load_a = [&](int b, auto KS) {
+            constexpr int ks = decltype(KS)::value;
 #pragma unroll
-        for (int i = 0; i < MT; i++) {
-            const uint8_t *p = a_src[i] + ((size_t)(b * 17 + 4 * ks) << 10);
+            for (int i = 0; i < MT; i++) {
+                const uint8_t *p = a_src[i] + ((size_t)(b * 17 + 4 * ks) << 10);
 #pragma unroll
-            for (int st = 0; st < 4; st++) ra[ks % RA].f[i][st] = __builtin_bit_cast(half8v, ld16(p, lane16 + (uint32_t)(st * 1024)));
-        }
-        if constexpr (SUMS && ks == 3) {
-#pragma unroll
-            for (int i = 0; i < MT; i++) sf[i] = __builtin_bit_cast(half8v, ld16(a_src[i] + ((size_t)(b * 17 + 16) << 10), lane16));
-        }
-    };
-    auto load_w = [&](Wb (&dst)[NT], int b) {
-        const uint8_t *p = w_src + (size_t)b * TB;
-#pragma unroll
-        for (int j = 0; j < NT; j++) dst[j].load(p, w_off[j], (uint32_t)r16, slot);
-    };
-    auto block = [&](int b, int bn, auto MORE) {
-        constexpr bool more = decltype(MORE)::value;
-        typename Fm::Consts cs[NT];
-#pragma unroll
-        for (int j = 0; j < NT; j++) cs[j] = Fm::consts(wcur[j].hdr(), g32, ws);
-        static_for<4>([&](auto KS) {
-            constexpr int ks = decltype(KS)::value, ahead = ks + RA - 1;
-            if constexpr (ahead < 4) load_a(b, std::integral_constant<int, ahead>{});
-            else if constexpr (more) load_a(bn, std::integral_constant<int, (ahead & 3)>{});
-            if constexpr (more && ks == 2) load_w(wnext, bn);
-            __builtin_amdgcn_sched_barrier(0);
-            static_for<4>([&](auto ST) {
-                constexpr int st = decltype(ST)::value;
-                half8v bop[NT];
-#pragma unroll
-                for (int j = 0; j < NT; j++) bop[j] = Fm::template operand<ks, st>(wcur[j].template stage<ks>(), cs[j]);
-#pragma unroll
-                for (int i = 0; i < MT; i++)
-#pragma unroll
-                    for (int j = 0; j < NT; j++) acc[i][j] = mfma32x32x16(ra[ks % RA].f[i][st], bop[j], acc[i][j]);
-            });
+                for (int st = 0; st < 4; st++) ra[ks % RA].f[i][st] = __builtin_bit_cast(half8v, ld16(p, lane16 + (uint32_t)(st * 1024)));
+            }
             if constexpr (SUMS && ks == 3) {
 #pragma unroll
-                for (int i = 0; i < MT; i++)
-#pragma unroll
-                    for (int j = 0; j < NT; j++) acc[i][j] = mfma32x32x16(sf[i], Fm::bmin(cs[j]), acc[i][j]);
+                for (int i = 0; i < MT; i++) sf[i] = __builtin_bit_cast(half8v, ld16(a_src[i] + ((size_t)(b * 17 + 16) << 10), lane16));
             }
-            __builtin_amdgcn_sched_barrier(0);
-        });
-        if constexpr (more) {
+        };
+        auto load_w = [&](Wb (&dst)[NT], int b) {
+            const uint8_t *p = w_src + (size_t)b * TB;
 #pragma unroll
-            for (int j = 0; j < NT; j++) wcur[j] = wnext[j];
+            for (int j = 0; j < NT; j++) {
+                dst[j].load_hdr(p, w_off[j], (uint32_t)r16, slot);
+                static_for<4>([&](auto KS) { dst[j].template load<decltype(KS)::value>(p, w_off[j], slot); });
+            }
+        };
+        auto block = [&](int b, int bn, auto MORE) {
+            constexpr bool more = decltype(MORE)::value;
+            typename Fm::Consts cs[NT];
+#pragma unroll
+            for (int j = 0; j < NT; j++) cs[j] = Fm::consts(wcur[j].hdr(), g32, ws);
+            static_for<4>([&](auto KS) {
+                constexpr int ks = decltype(KS)::value, ahead = ks + RA - 1;
+                if constexpr (ahead < 4) load_a(b, std::integral_constant<int, ahead>{});
+                else if constexpr (more) load_a(bn, std::integral_constant<int, (ahead & 3)>{});
+                if constexpr (more && ks == 2) load_w(wnext, bn);
+                __builtin_amdgcn_sched_barrier(0);
+                static_for<4>([&](auto ST) {
+                    constexpr int st = decltype(ST)::value;
+                    half8v bop[NT];
+#pragma unroll
+                    for (int j = 0; j < NT; j++) bop[j] = Fm::template operand<ks, st>(wcur[j].template stage<ks>(), cs[j]);
+#pragma unroll
+                    for (int i = 0; i < MT; i++)
+#pragma unroll
+                        for (int j = 0; j < NT; j++) acc[i][j] = mfma32x32x16(ra[ks % RA].f[i][st], bop[j], acc[i][j]);
+                });
+                if constexpr (SUMS && ks == 3) {
+#pragma unroll
+                    for (int i = 0; i < MT; i++)
+#pragma unroll
+                        for (int j = 0; j < NT; j++) acc[i][j] = mfma32x32x16(sf[i], Fm::bmin(cs[j]), acc[i][j]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            if constexpr (more) {
+#pragma unroll
+                for (int j = 0; j < NT; j++) wcur[j] = wnext[j];
+            }
+        };
+        if (b0 < b1) {
+            const int cnt = b1 - b0;
+            int b = b0;
+            load_w(wcur, b);
+            static_for<RA - 1>([&](auto KS) { load_a(b, KS); });
+            for (int i = 1; i < cnt; i++) {
+                asm volatile("" : "+v"(lane16));
+                const int bn = b + 1 == b1 ? b0 : b + 1;
+                block(b, bn, std::true_type{});
+                b = bn;
+            }
+            block(b, b, std::false_type{});
         }
-    };
-    if (b0 < b1) {
-        const int cnt = b1 - b0;
-        int b = b0;
-        load_w(wcur, b);
-        static_for<RA - 1>([&](auto KS) { load_a(b, KS); });
-        for (int i = 1; i < cnt; i++) {
-            asm volatile("" : "+v"(lane16));
-            const int bn = b + 1 == b1 ? b0 : b + 1;
-            block(b, bn, std::true_type{});
-            b = bn;
+    } else {
+        constexpr int D = 4;  // steps of fragments in registers
+        half8v ra[D][MT], sf[MT];
+        Wb wc[NT];
+        auto load_a = [&](int b, auto U) {  // step U of super-block b
+            constexpr int u = decltype(U)::value;
+#pragma unroll
+            for (int i = 0; i < MT; i++)
+                ra[u % D][i] = __builtin_bit_cast(half8v, ld16(a_src[i] + ((size_t)(b * 17 + (u & ~3)) << 10), lane16 + (uint32_t)((u & 3) * 1024)));
+        };
+        auto load_w = [&](int b, auto KS) {
+            const uint8_t *p = w_src + (size_t)b * TB;
+#pragma unroll
+            for (int j = 0; j < NT; j++) wc[j].template load<decltype(KS)::value>(p, w_off[j], slot);
+        };
+        auto load_h = [&](int b) {
+            const uint8_t *p = w_src + (size_t)b * TB;
+#pragma unroll
+            for (int j = 0; j < NT; j++) wc[j].load_hdr(p, w_off[j], (uint32_t)r16, slot);
+        };
+        auto block = [&](int b, auto MORE) {
+            constexpr bool more = decltype(MORE)::value;
+            typename Fm::Consts cs[NT];
+#pragma unroll
+            for (int j = 0; j < NT; j++) cs[j] = Fm::consts(wc[j].hdr(), g32, ws);
+            if constexpr (more) load_h(b + 1);
+            if constexpr (SUMS) {
+#pragma unroll
+                for (int i = 0; i < MT; i++) sf[i] = __builtin_bit_cast(half8v, ld16(a_src[i] + ((size_t)(b * 17 + 16) << 10), lane16));
+            }
+            static_for<4>([&](auto KS) {
+                constexpr int ks = decltype(KS)::value;
+                static_for<4>([&](auto ST) {
+                    constexpr int st = decltype(ST)::value, u = 4 * ks + st;
+                    half8v bop[NT];
+#pragma unroll
+                    for (int j = 0; j < NT; j++) bop[j] = Fm::template operand<ks, st>(wc[j].template stage<ks>(), cs[j]);
+#pragma unroll
+                    for (int i = 0; i < MT; i++)
+#pragma unroll
+                        for (int j = 0; j < NT; j++) acc[i][j] = mfma32x32x16(ra[u % D][i], bop[j], acc[i][j]);
+                    if constexpr (u + D < 16) load_a(b, std::integral_constant<int, u + D>{});
+                    else if constexpr (more) load_a(b + 1, std::integral_constant<int, (u + D) & 15>{});
+                });
+                if constexpr (SUMS && ks == 3) {
+#pragma unroll
+                    for (int i = 0; i < MT; i++)
+#pragma unroll
+                        for (int j = 0; j < NT; j++) acc[i][j] = mfma32x32x16(sf[i], Fm::bmin(cs[j]), acc[i][j]);
+                }
+                if constexpr (more) load_w(b + 1, KS);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        };
+        if (b0 < b1) {
+            load_h(b0);
+            // (in the order of the loop, whose waits the compiler counts for both ways into it)
+            static_for<4>([&](auto KS) {
+                if constexpr (decltype(KS)::value == 3) static_for<D>([&](auto U) { load_a(b0, U); });
+                load_w(b0, KS);
+            });
+            __builtin_amdgcn_sched_barrier(0);
+            int b = b0;
+            for (int i = b1 - b0; i > 1; i--) {
+                asm volatile("" : "+v"(lane16));
+                block(b, std::true_type{});
+                b++;
+            }
+            block(b, std::false_type{});
         }
-        block(b, b, std::false_type{});
     }
 
     // ---- the waves meet: thread t adds up, of every tile, the four columns 4 (t % 8) .. + 3 of row t / 8 ----
@@ -308,8 +383,9 @@ __device__ __forceinline__ void cols_body(const ColsGroup &grp, int wi, int nb, 
     turq_note_flush(bad);
 }
 
-template <int DTA, int DTB, int MT, int NT>
-__global__ void __launch_bounds__(64 * W) gemm_cols_kernel(ColsGroup grp, int64_t k, const uint8_t *__restrict__ frags, int64_t m, int yt,
+// MINB: workgroups that are to share a CU (2: the tight form of the 64 x 64 tile in 256 registers; otherwise what the tile leaves)
+template <int DTA, int DTB, int MT, int NT, bool TIGHT, int MINB>
+__global__ void __launch_bounds__(64 * W, MINB) gemm_cols_kernel(ColsGroup grp, int64_t k, const uint8_t *__restrict__ frags, int64_t m, int yt,
                                                            int nblocks_n, int nblocks_m, int vec_out) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     // consecutive logical ids run on one XCD (blockIdx % 8): the m-blocks of one n-block share its packed weights in that XCD's L2.  Also where
@@ -323,14 +399,14 @@ __global__ void __launch_bounds__(64 * W) gemm_cols_kernel(ColsGroup grp, int64_
     for (int i = 1; i < kMaxGroup; i++)
         if (i < grp.count && nb_all >= grp.first[i]) wi = i;
     const int nb = nb_all - grp.first[wi];
-    if (DTA == DTB || wi < grp.second) cols_body<DTA, MT, NT>(grp, wi, nb, mb, k, frags, m, yt, vec_out, lds);
-    else cols_body<DTB, MT, NT>(grp, wi, nb, mb, k, frags, m, yt, vec_out, lds);
+    if (DTA == DTB || wi < grp.second) cols_body<DTA, MT, NT, TIGHT>(grp, wi, nb, mb, k, frags, m, yt, vec_out, lds);
+    else cols_body<DTB, MT, NT, TIGHT>(grp, wi, nb, mb, k, frags, m, yt, vec_out, lds);
 }
 
-template <int DTA, int DTB, int MT, int NT>
+template <int DTA, int DTB, int MT, int NT, bool TIGHT = false, int MINB = 1>
 hipError_t launch_cols(const TurqGemmWeights &ws, int second, int64_t k, const void *frags, int64_t m, int yt, hipStream_t stream,
                        hipEvent_t ev_start, hipEvent_t ev_stop) {
-    const auto kernel = gemm_cols_kernel<DTA, DTB, MT, NT>;
+    const auto kernel = gemm_cols_kernel<DTA, DTB, MT, NT, TIGHT, MINB>;
     constexpr int LDS_BYTES = Meet<MT, NT>::LDS;
     static_assert(LDS_BYTES <= 64 * 1024, "no raised LDS limit");
     ColsGroup grp{};
@@ -358,19 +434,27 @@ hipError_t launch_cols(const TurqGemmWeights &ws, int second, int64_t k, const v
     return hipGetLastError();
 }
 
+int64_t cols_workgroups(int tile, int count, const int64_t *n, int64_t m) {
+    int64_t nbn = 0;
+    for (int i = 0; i < count; i++) nbn += (n[i] + 32 * (tile % 10) - 1) / (32 * (tile % 10));
+    return nbn * ((m + 32 * (tile / 10) - 1) / (32 * (tile / 10)));
+}
+
 template <int DTA, int DTB>
-hipError_t launch_tile(int tile, const TurqGemmWeights &ws, int second, int64_t k, const void *frags, int64_t m, int yt, hipStream_t stream,
-                       hipEvent_t ev_start, hipEvent_t ev_stop) {
+hipError_t launch_tile(int tile, const TurqGemmWeights &ws, int second, int64_t k, const void *frags, int64_t m, int yt, int64_t cus,
+                       hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop) {
     switch (tile) {
-#define TURQ_COLS(MT, NT) \
-    case 10 * MT + NT: return launch_cols<DTA, DTB, MT, NT>(ws, second, k, frags, m, yt, stream, ev_start, ev_stop)
-        TURQ_COLS(1, 1);
-        TURQ_COLS(2, 1);
-        TURQ_COLS(3, 1);
-        TURQ_COLS(2, 2);
-        TURQ_COLS(3, 2);
-        TURQ_COLS(2, 3);
-        TURQ_COLS(4, 2);
+#define TURQ_COLS(MT, NT, ...) launch_cols<DTA, DTB, MT, NT, ##__VA_ARGS__>(ws, second, k, frags, m, yt, stream, ev_start, ev_stop)
+    case 11: return TURQ_COLS(1, 1);
+    case 21: return TURQ_COLS(2, 1);
+    case 31: return TURQ_COLS(3, 1);
+    case 22:  // (more than one workgroup per CU: two of them at a time)
+        if (cols_workgroups(22, ws.count, ws.n, m) > cus) return TURQ_COLS(2, 2, true, 2);
+        return TURQ_COLS(2, 2);
+    case 32: return TURQ_COLS(3, 2);
+    case 23: return TURQ_COLS(2, 3);
+    case 42: return TURQ_COLS(4, 2);
+    case 33: return TURQ_COLS(3, 3, true);  // (the first form spills here)
 #undef TURQ_COLS
     default: return hipErrorInvalidValue;
     }
@@ -385,13 +469,32 @@ size_t row_tile_bytes(int dtype_a, int dtype_b, int64_t k) {
 
 bool turq_gemm_cols_mixed(int dtype_a, int dtype_b) { return (dtype_a == TURQ_Q4_K || dtype_a == TURQ_Q5_K) && dtype_b == TURQ_Q6_K; }
 
-// The tile (10 * MT + NT) with which `count` weights of n[i] rows and k columns go through this kernel in one launch, 0 where the launch
-// is gemm_kq_kernel's; *us: roughly what it takes.
-//
-// A launch of one round over the CUs takes about base + per_sb * super-blocks, one fit over launches of every format (graphs of launches over
-// more weights than the caches hold; Q4_K takes up to a quarter less, Q6_K of 32 x 32 tiles on full rounds up to a quarter more: 4096 x 12288 at 77
-// rows 35 us for 28), which serves to order the tiles and, for Q8_0, to choose between the kernels; a further round costs as much again without the launch itself, of the smallest tile, of which three workgroups
-// share a CU, three fifths of it.  So the smallest tile that makes the launch one round is the best of them.  Against gemm_kq_kernel:
+// What one launch of this kernel takes: one round over the CUs is `base` plus `per` for every super-block of 256 columns, the latter `fill`
+// longer on a chip that is full (L2 and clock); a further round costs `again` of that and `more` for the part of it that is there.  Fitted to
+// 628 launches (n 1024 .. 24576, k 1024 .. 18944, 40 .. 512 rows, weights from HBM), with an error of 6 % and of 25 % at most.
+struct ColsCost { int tile; double base, per[4], again, more, fill; };  // per: Q4_K, Q5_K, Q6_K, Q8_0
+static constexpr ColsCost kColsCost[] = {
+    {11, 2.58, {0.229, 0.270, 0.288, 0.277}, 0.51, 0.30, 0.33}, {21, 3.21, {0.375, 0.418, 0.433, 0.432}, 0.58, 0.31, 0.22},
+    {31, 3.58, {0.489, 0.528, 0.540, 0.547}, 0.60, 0.29, 0.29}, {22, 4.58, {0.498, 0.594, 0.652, 0.591}, 0.88, 0.25, 0.31},
+    {32, 5.48, {0.647, 0.748, 0.775, 0.721}, 0.79, 0.28, 0.43}, {23, 5.80, {0.674, 0.843, 0.929, 0.868}, 0.62, 0.41, 0.47},
+    {42, 6.95, {0.789, 0.893, 0.880, 0.880}, 0.74, 0.30, 0.54}, {33, 7.00, {0.919, 1.062, 1.116, 1.467}, 0.61, 0.39, 0.53},
+};
+static constexpr ColsCost kColsPair = {22, 3.84, {0.604, 0.707, 0.741, 0.715}, 0.42, 0.41, 0.25};  // two workgroups per CU
+
+static double cols_us(int tile, int dtype_a, int dtype_b, int count, const int64_t *n, int64_t k, int64_t m, int64_t cus) {
+    const auto fmt = [](int dt) { return dt == TURQ_Q4_K ? 0 : dt == TURQ_Q5_K ? 1 : dt == TURQ_Q6_K ? 2 : 3; };
+    const double x = (double)cols_workgroups(tile, count, n, m) / (double)cus;
+    const ColsCost *c = &kColsPair;
+    if (tile != 22 || x <= 1.0)
+        for (const ColsCost &t : kColsCost)
+            if (t.tile == tile) c = &t;
+    return turq_launch_model_us(c->base, std::max(c->per[fmt(dtype_a)], c->per[fmt(dtype_b)]) * (double)(k / 256), c->again, c->more, c->fill, x);
+}
+
+// The tile with which one weight goes through this kernel as far as single rounds over the CUs decide, 0: gemm_kq_kernel.
+// A launch of one round takes about base + per_sb * super-blocks, one line for every format; a further round costs as much again without the
+// launch itself, of the smallest tile, of which three workgroups share a CU, three fifths of it.  So the smallest tile that makes the launch one
+// round is the best of them.  Against gemm_kq_kernel:
 //   one or two MFMA tiles: Q4_K 1024 x 4096 at 40 / 300 / 512 rows 13.0 / 19.0 / 19.1 -> 6.6 / 9.3 / 10.7 us, 4096 x 4096 at 40 / 100 rows 19.2 /
 //   22.6 -> 8.7 / 11.3, Q6_K 4096 x 12288 33 / 43 -> 23 / 29, Q8_0 2048 x 2048 15 -> 5.4 / 5.5;
 //   three or four: K-quants from two super-blocks on (Q4_K 12288 x 256 at 48 rows 8.4 -> 9.4); Q8_0 2048 x 2048 at 300 / 512 rows 15.4 -> 8.5 / 10.2, Q4_K 4096 x 4096 at 256 24 -> 15;
@@ -399,8 +502,42 @@ bool turq_gemm_cols_mixed(int dtype_a, int dtype_b) { return (dtype_a == TURQ_Q4
 //   at 160 rows 11.1 -> 11.7);
 //   eight: from 40 super-blocks on, Q6_K from 24 (512 rows, 4096 x 12288: Q4_K 66 -> 64, Q5_K 76 -> 69, Q6_K 81 -> 66; 4096 x 4096: Q4_K 26.3 -> 27.5).
 // Q8_0, whose tile in gemm_kq_kernel is the narrow 128 x 64, takes whichever kernel has the smaller estimate, in any number of rounds
-// (4096 x 4096 at 512 / 700 rows 31 / 53 -> 29 / 41, 4096 x 12288 at 1024 / 2048 rows 160 / 300 -> 126 / 283); several weights, each
-// of which is this kernel's, go together where that is less than one after the other.
+// (4096 x 4096 at 512 / 700 rows 31 / 53 -> 29 / 41, 4096 x 12288 at 1024 / 2048 rows 160 / 300 -> 126 / 283).
+static int cols_tile_by_rounds(int dtype, int64_t n, int64_t k, int64_t m, int64_t cus, int compute_units) {
+    static constexpr struct { int mt, nt; double base, per_sb; } kTiles[] = {{1, 1, 3.2, 0.40}, {2, 1, 4.0, 0.52}, {3, 1, 4.6, 0.60}, {2, 2, 5.2, 0.68},
+                                                                             {3, 2, 6.2, 0.92}, {2, 3, 6.2, 0.92}, {4, 2, 7.0, 1.20}};
+    const bool eight = dtype == TURQ_Q8_0;
+    const int64_t ntc = k / 256;
+    double best_us = eight ? turq_gemm_launch_us(dtype, 1, &n, k, m, compute_units) : 1e30;
+    int best = 0;
+    for (const auto &c : kTiles) {
+        const int area = c.mt * c.nt;
+        const int64_t wgs = cols_workgroups(10 * c.mt + c.nt, 1, &n, m);
+        if (!eight) {
+            if (wgs > (area == 1 ? cus + cus / 2 : cus)) continue;
+            if (area == 4 && ntc < 2) continue;
+            if (area > 4 && ntc < (area == 6 ? 12 : dtype == TURQ_Q6_K ? 24 : 40)) continue;
+        }
+        const double x = (double)wgs / (double)cus;
+        const double rounds = x <= 1.0 ? 1.0 : area == 1 ? 1.0 + 0.6 * (x - 1.0) : (double)((wgs + cus - 1) / cus);
+        const double est = kTurqLaunchUs + (c.base + c.per_sb * (double)ntc - kTurqLaunchUs) * rounds;
+        if (est < best_us) {
+            best = 10 * c.mt + c.nt;
+            best_us = est;
+        }
+    }
+    return best;
+}
+
+// The tile (10 * MT + NT) with which `count` weights of n[i] rows and k columns go through this kernel in one launch, 0 where the launch
+// is gemm_kq_kernel's; *us: roughly what it takes.
+//
+// One weight: by the rounds, unless another tile's estimate over several rounds is a fifth (Q8_0: a quarter and a bit) below what that launch
+// takes: the estimates err by up to that much, and launches of more than one round are where the rounds alone misjudge (at 300 rows, 128 x 128 -> two
+// 64 x 64 workgroups per CU: Q4_K / Q5_K / Q6_K 6144 x 4096 36 / 42 / 40 -> 25 / 28 / 30 us, 6144 x 1024 13.3 / 15.0 / 14.6 -> 9.9 / 10.8 / 11.5; at 180
+// rows, 128 x 128 -> 96 x 96: Q5_K 12288 x 4096 45 -> 32).
+// Several weights, each of which is this kernel's alone: together, by the estimates, where that is less than one after the other (gate and up of
+// an 8B model at 77 rows, Q5_K 2 x 12288 x 4096: 45 -> 34).
 int turq_gemm_cols_tile(int dtype_a, int dtype_b, int count, const int64_t *n, int64_t k, int64_t m, int compute_units, double *us) {
     const TurqTuning &t = turq_tuning();
     const bool kq_forced = t.gemm_wide >= 0 || t.gemm_low >= 0 || t.gemm_split >= 0 || t.gemm_kgroups != 0 || t.gemm_grid_2x2 || t.gemm_merge >= 0;
@@ -412,37 +549,25 @@ int turq_gemm_cols_tile(int dtype_a, int dtype_b, int count, const int64_t *n, i
     // decide: columns that it refuses are not taken instead (six row tiles are the most of a workgroup here)
     if (row_tile_bytes(dtype_a, dtype_b, k) >= (1ull << 32) / (dtype_a == TURQ_Q8_0 ? 6 : 8)) return 0;
     if (t.gemm_cols > 0) return t.gemm_cols;
-    const int64_t cus = compute_units > 0 ? compute_units : 256, ntc = k / 256;
-    static constexpr struct { int mt, nt; double base, per_sb; } kTiles[] = {{1, 1, 3.2, 0.40}, {2, 1, 4.0, 0.52}, {3, 1, 4.6, 0.60}, {2, 2, 5.2, 0.68},
-                                                                             {3, 2, 6.2, 0.92}, {2, 3, 6.2, 0.92}, {4, 2, 7.0, 1.20}};
-    const bool eight = dtype_a == TURQ_Q8_0;
+    const int64_t cus = compute_units > 0 ? compute_units : 256;
     int best = 0;
-    double best_us = 1e30;
-    if (eight && count == 1) best_us = turq_gemm_launch_us(dtype_a, 1, n, k, m, compute_units);
-    if (eight && count > 1) {
-        best_us = 0.0;
+    double best_us = 0.0, least = 0.0;  // the launch to be beaten, and below what
+    if (count == 1) {
+        best = cols_tile_by_rounds(dtype_a, n[0], k, m, cus, compute_units);
+        best_us = best ? cols_us(best, dtype_a, dtype_a, 1, n, k, m, cus) : turq_gemm_kq_us(dtype_a, n[0], k, m, compute_units);
+        least = best_us / (dtype_a == TURQ_Q8_0 ? 1.27 : 1.2);
+    } else {
         for (int i = 0; i < count; i++) {
-            double alone = 0.0;
+            double alone = 0.0;  // (of a mixed launch as if of the first format: the estimate only has to order)
             if (!turq_gemm_cols_tile(dtype_a, dtype_a, 1, n + i, k, m, compute_units, &alone)) return 0;
-            best_us += alone;
+            least += alone;
         }
     }
-    for (const auto &c : kTiles) {
-        const int area = c.mt * c.nt;
-        int64_t nbn = 0;
-        for (int i = 0; i < count; i++) nbn += (n[i] + 32 * c.nt - 1) / (32 * c.nt);
-        const int64_t wgs = nbn * ((m + 32 * c.mt - 1) / (32 * c.mt));
-        if (!eight) {
-            if (wgs > (area == 1 ? cus + cus / 2 : cus)) continue;
-            if (area == 4 && ntc < 2) continue;
-            if (area > 4 && ntc < (area == 6 ? 12 : dtype_a == TURQ_Q6_K ? 24 : 40)) continue;
-        }
-        const double x = (double)wgs / (double)cus;
-        const double rounds = x <= 1.0 ? 1.0 : area == 1 ? 1.0 + 0.6 * (x - 1.0) : (double)((wgs + cus - 1) / cus);
-        const double est = kTurqLaunchUs + (c.base + c.per_sb * (double)ntc - kTurqLaunchUs) * rounds;
-        if (est < best_us) {
-            best = 10 * c.mt + c.nt;
-            best_us = est;
+    for (const ColsCost &c : kColsCost) {
+        const double est = cols_us(c.tile, dtype_a, dtype_b, count, n, k, m, cus);
+        if (est < least) {
+            best = c.tile;
+            best_us = least = est;
         }
     }
     if (us && best) *us = best_us;
@@ -451,7 +576,7 @@ int turq_gemm_cols_tile(int dtype_a, int dtype_b, int count, const int64_t *n, i
 
 // frags: as for turq_launch_gemm_mfma, in the order of the formats (Q8_0, or the K-quants); weights from `second` on are of dtype_b
 hipError_t turq_launch_gemm_cols(int dtype_a, int dtype_b, int second, int tile, const TurqGemmWeights &ws, int64_t k, const void *frags, int64_t m,
-                                 int y_dtype, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop) {
+                                 int y_dtype, int compute_units, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop) {
     if (ws.count < 1 || ws.count > kMaxGroup || k <= 0 || k % 256 != 0 || k / 256 > (1 << 20)) return hipErrorInvalidValue;
     int64_t n = 0;
     for (int i = 0; i < ws.count; i++) {
@@ -462,7 +587,7 @@ hipError_t turq_launch_gemm_cols(int dtype_a, int dtype_b, int second, int tile,
     if (m == 0) return hipSuccess;
     if (row_tile_bytes(dtype_a, second < ws.count ? dtype_b : dtype_a, k) * 2 * (size_t)(tile % 10) >= (1ull << 32)) return hipErrorInvalidValue;
     if ((n / 32 + ws.count) * ((m + 31) / 32) > 0x7FFFFFFF) return hipErrorInvalidValue;
-#define TURQ_COLS_TILE(A, B) return launch_tile<A, B>(tile, ws, second, k, frags, m, y_dtype, stream, ev_start, ev_stop)
+#define TURQ_COLS_TILE(A, B) return launch_tile<A, B>(tile, ws, second, k, frags, m, y_dtype, compute_units > 0 ? compute_units : 256, stream, ev_start, ev_stop)
     if (dtype_a != dtype_b && second < ws.count) {
         if (dtype_a == TURQ_Q4_K && dtype_b == TURQ_Q6_K) TURQ_COLS_TILE(TURQ_Q4_K, TURQ_Q6_K);
         if (dtype_a == TURQ_Q5_K && dtype_b == TURQ_Q6_K) TURQ_COLS_TILE(TURQ_Q5_K, TURQ_Q6_K);

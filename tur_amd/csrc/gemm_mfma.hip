@@ -852,9 +852,24 @@ double turq_gemm_fill(int dtype, int64_t n, int64_t k, int64_t m, int compute_un
     return rounds > 0 ? (double)wgs / (double)(rounds * cus) * gain : 0.0;
 }
 
-// Roughly what one launch of these weights takes, for choosing between this kernel and gemm_cols.hip where they are close: Q8_0 in any
-// number of rounds (4096 x 4096 at 40 .. 512 rows 25.5 .. 31.6 us, 1024 x 3072 20, 4096 x 1024 10); the K-quants where the launch is one round
-// of the low tile (Q4_K 4096 x 4096 23, 2048 x 2048 12.4, 6144 x 1024 9; Q6_K 4096 x 4096 27.5, 2048 x 6144 37.5), 0 elsewhere.
+// What one launch of n rows takes here, for choosing between this kernel and gemm_cols.hip: the same form of estimate as there, one line per
+// tile form (128 x 128; 2 x 2 waves; wide; low), fitted to the same 628 launches (error 1.4, 2.4, 1.9 and 4.5 %).
+double turq_gemm_kq_us(int dtype, int64_t n, int64_t k, int64_t m, int compute_units) {
+    struct Cost { double base, per[4], again, more, fill; };  // per: Q4_K, Q5_K, Q6_K, Q8_0
+    static constexpr Cost kCost[] = {{5.86, {1.73, 2.06, 2.00, 0.0}, 0.90, 0.1, 0.32}, {5.01, {2.58, 2.10, 2.10, 1.26}, 0.68, 0.34, 0.39},
+                                     {5.68, {2.71, 3.01, 3.34, 0.0}, 0.80, 0.1, 0.60}, {4.86, {0.99, 1.16, 1.33, 0.0}, 0.80, 0.1, 0.44}};
+    const int form = turq_gemm_form(dtype, n, k, m, compute_units);
+    if (form < 1 || form > 4) return 0.0;
+    const int64_t bm = form == 4 ? 64 : 128;
+    const int64_t bn = form == 3 ? 256 : form == 2 ? (dtype == TURQ_Q4_K ? 192 : dtype == TURQ_Q8_0 ? 64 : 128) : 128;
+    const double x = (double)(((n + bn - 1) / bn) * ((m + bm - 1) / bm)) / (double)(compute_units > 0 ? compute_units : 256);
+    const Cost &c = kCost[form - 1];
+    return turq_launch_model_us(c.base, c.per[dtype == TURQ_Q4_K ? 0 : dtype == TURQ_Q5_K ? 1 : dtype == TURQ_Q6_K ? 2 : 3] * (double)(k / 256), c.again, c.more,
+                                c.fill, x);
+}
+
+// Roughly what one launch of these weights takes where its sums do not depend on what else is in it (Q8_0; K-quants in one round of the low
+// tile), for deciding whether weights of several shapes go out together, 0 elsewhere.
 double turq_gemm_launch_us(int dtype, int count, const int64_t *n, int64_t k, int64_t m, int compute_units) {
     const int64_t cus = compute_units > 0 ? compute_units : 256, ntc = k / 256;
     int64_t total = 0, nbn = 0;

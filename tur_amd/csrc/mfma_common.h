@@ -342,9 +342,16 @@ hipError_t turq_launch_gemm_mfma_group(int dtype, const TurqGemmWeights &ws, int
 bool turq_gemm_cols_mixed(int dtype_a, int dtype_b);
 int turq_gemm_cols_tile(int dtype_a, int dtype_b, int count, const int64_t *n, int64_t k, int64_t m, int compute_units, double *us = nullptr);
 double turq_gemm_launch_us(int dtype, int count, const int64_t *n, int64_t k, int64_t m, int compute_units);
+double turq_gemm_kq_us(int dtype, int64_t n, int64_t k, int64_t m, int compute_units);  // an estimate of a launch of gemm_kq_kernel
 constexpr double kTurqLaunchUs = 2.5;  // the share of a launch's time that a further round over the CUs does not pay again
+// the estimate of a launch that both kernels' rules use: x workgroups per CU (gemm_cols.hip says what the other figures are)
+inline double turq_launch_model_us(double base, double loop, double again, double more, double fill, double x) {
+    const double full = x < 1.0 ? x : 1.0, rounds = x > 1.0 ? (double)(int64_t)(x + 0.999999) - 1.0 : 0.0;
+    const double one = base + loop * (1.0 + fill * full * full);
+    return kTurqLaunchUs + (one - kTurqLaunchUs) * (1.0 + again * rounds + (x > 1.0 ? more * (x - 1.0) : 0.0));
+}
 hipError_t turq_launch_gemm_cols(int dtype_a, int dtype_b, int second, int tile, const TurqGemmWeights &ws, int64_t k, const void *frags, int64_t m,
-                                 int y_dtype, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop);
+                                 int y_dtype, int compute_units, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop);
 // the workgroup tile the launch rules of gemm_kq_kernel pick (0: no kernel for the format)
 int turq_gemm_form(int dtype, int64_t n, int64_t k, int64_t m, int compute_units);
 // the launch the tile rules would make for these rows: its workgroups and the share of its CU rounds it keeps busy (x the wide

@@ -222,7 +222,7 @@ static TurqGemmWeights gemm_weights(int count, const turq_weight *const *w, void
 
 // the tile with which the first `count` weights go through gemm_cols.hip in one launch (one format, or Q4_K / Q5_K followed by
 // Q6_K), 0: not; *second: the first weight of the second format
-static int gemm_cols_tile(const turq_ctx *ctx, int count, const turq_weight *const *w, int64_t m, int *second) {
+static int gemm_cols_tile(const turq_ctx *ctx, int count, const turq_weight *const *w, int64_t m, int *second, double *us = nullptr) {
     int64_t n[4];
     int s = count;
     if (count < 1 || count > 4) return 0;
@@ -234,7 +234,7 @@ static int gemm_cols_tile(const turq_ctx *ctx, int count, const turq_weight *con
     if (second) *second = s;
     // (few tiles of very many columns: gemm_kq_kernel with the columns split over workgroups, where there is scratch for their meeting)
     if (count == 1 && !ctx->fixed_scratch && turq_gemm_split_scratch(w[0]->dtype, n[0], w[0]->k, m, ctx->compute_units, nullptr) != 0) return 0;
-    return turq_gemm_cols_tile(w[0]->dtype, w[s < count ? s : 0]->dtype, count, n, w[0]->k, m, ctx->compute_units);
+    return turq_gemm_cols_tile(w[0]->dtype, w[s < count ? s : 0]->dtype, count, n, w[0]->k, m, ctx->compute_units, us);
 }
 
 // the prefill GEMM of one weight on the fragments in ctx->act_prep, by either kernel
@@ -249,7 +249,7 @@ static int gemm_on_frags(turq_ctx *ctx, const turq_weight *w, int64_t m, void *y
     TURQ_HIP(ctx, turq_prof_next(ctx, &ev0, &ev1));
     if (cols)
         TURQ_HIP(ctx, turq_launch_gemm_cols(w->dtype, w->dtype, second, tile, gemm_weights(1, &w, &y, &ldy, &bias, &wscale), w->k, ctx->act_prep, m, yt,
-                                            ctx->stream, ev0, ev1));
+                                            ctx->compute_units, ctx->stream, ev0, ev1));
     else
         TURQ_HIP(ctx, turq_launch_gemm_mfma(w->dtype, w->dev, w->n, w->k, ctx->act_prep, m, y, yt, ldy, bias, wscale, ctx->compute_units,
                                             ctx->stream, ev0, ev1, sp.counters[0], sp.partials[0], sp.bytes[0]));
@@ -319,6 +319,16 @@ static bool gemm_run_pays(const turq_ctx *ctx, int run, const turq_weight *const
     return us > 0.0 && us < apart;
 }
 
+// whether `run` K-quant weights of one shape that gemm_cols.hip would take in one launch of `us` are less as one launch of gemm_kq_kernel
+// (Q4_K 2 x 12288 x 4096 at 256 rows: 73 against 61)
+static bool gemm_both_in_kq(const turq_ctx *ctx, int run, const turq_weight *const *w, int64_t m, double us) {
+    if (turq_tuning().gemm_cols > 0 || turq_tuning().gemm_merge >= 0 || run < 2 || us <= 0.0 || w[0]->dtype == TURQ_Q8_0 || w[0]->n % 256 != 0) return false;
+    for (int i = 1; i < run; i++)
+        if (w[i]->dtype != w[0]->dtype || w[i]->n != w[0]->n) return false;
+    const double kq = turq_gemm_kq_us(w[0]->dtype, w[0]->n * run, w[0]->k, m, ctx->compute_units);
+    return kq > 0.0 && kq < us;
+}
+
 int turq_qmatmul_multi_gemm(turq_ctx *ctx, int count, const turq_weight *const *w, const void *x, int xt, int64_t m, int64_t ldx,
                             void *const *y, int yt, const int64_t *ldy, const float *const *bias, bool *taken, const TurqNorm *norm) {
     *taken = false;
@@ -373,8 +383,14 @@ int turq_qmatmul_multi_gemm(turq_ctx *ctx, int count, const turq_weight *const *
             for (; run >= 2; run--) {
                 if ((w[i + run - 1]->dtype == TURQ_Q8_0) != (order == 2)) continue;
                 const int64_t n_cols = std::count(cols + i, cols + i + run, true);
-                if (n_cols == run) tile = gemm_cols_tile(ctx, run, w + i, m, &second);
+                double us = 0.0;
+                if (n_cols == run) tile = gemm_cols_tile(ctx, run, w + i, m, &second, &us);
                 if (n_cols == 0) kq = gemm_run_pays(ctx, run, w + i, m);
+                // (gate and up, each of which gemm_cols.hip takes alone: one launch of gemm_kq_kernel over the rows of both where that is less)
+                if (tile != 0 && gemm_both_in_kq(ctx, run, w + i, m, us)) {
+                    tile = 0;
+                    kq = true;
+                }
                 if (tile != 0 || kq) break;
             }
             // (one alone: unless it goes out together with its like below)
@@ -387,7 +403,7 @@ int turq_qmatmul_multi_gemm(turq_ctx *ctx, int count, const turq_weight *const *
                 if (e == hipSuccess)
                     e = kq ? turq_launch_gemm_mfma_group(w[i]->dtype, g, w[i]->k, ctx->act_prep, m, yt, ctx->compute_units, st, ev0, ev1)
                            : turq_launch_gemm_cols(w[i]->dtype, w[i + (second < run ? second : 0)]->dtype, second, tile, g, w[i]->k, ctx->act_prep, m,
-                                                   yt, st, ev0, ev1);
+                                                   yt, ctx->compute_units, st, ev0, ev1);
                 i += run - 1;
                 continue;
             }
