@@ -206,3 +206,29 @@ def test_prompt_chunks(gpu, dt_gu, dt_dn, m):
     assert np.array_equal(synth.to_bf16_bits(yb).reshape(m, n_out), synth.to_bf16_bits(y).reshape(m, n_out))
     for w in ws:
         gpu.release(w)
+
+
+@pytest.mark.parametrize("dt_gu,dt_dn,n_ff,k,m", [
+    (Q4_K, Q6_K, 2816, 512, 600), (Q4_K, Q5_K, 3328, 3072, 513), (Q4_K, Q8_0, 6400, 256, 545), (Q5_K, Q6_K, 2816, 512, 600),
+    (Q5_K, Q4_K, 6400, 256, 513), (Q6_K, Q6_K, 2816, 512, 600), (Q6_K, Q8_0, 6400, 256, 513), (Q8_0, Q8_0, 3328, 1024, 2017),
+    (Q8_0, Q4_K, 3328, 1024, 2017)])
+def test_prompt_pairs(gpu, dt_gu, dt_dn, n_ff, k, m):
+    """Gate and up in one launch that writes down_proj's fragments (128 x 128, 2 x 2 and wide tiles; blocks of n past the last row, rows
+    past m in the last 32; both fragment orders, with the sub-block sums of a Q4_K / Q5_K down_proj): bit-equal to the two calls.  The
+    scales of gate and up differ by 2^9, so that a column taken with the other's scale would show."""
+    n_out = 512
+    raws = [synth.random_weight(dt_gu, n_ff, k, seed=7), synth.random_weight(dt_gu, n_ff, k, seed=8), synth.random_weight(dt_dn, n_out, n_ff, seed=9)]
+    nb = synth.BLOCK_BYTES[dt_gu]
+    blocks = raws[1].reshape(-1, nb)
+    at = nb - 2 if dt_gu == Q6_K else 0
+    for o in (at, at + 2) if dt_gu in (Q4_K, Q5_K) else (at,):
+        d = blocks[:, o:o + 2].copy().view(np.float16)
+        blocks[:, o:o + 2] = (d * np.float16(2.0 ** -9)).view(np.uint8)
+    ws = [gpu.upload(dt, n, kk, raw, capi.LAYOUT_TILED) for dt, n, kk, raw in zip((dt_gu, dt_gu, dt_dn), (n_ff, n_ff, n_out), (k, k, n_ff), raws)]
+    rng = np.random.default_rng(m)
+    x = rng.standard_normal((m, k)).astype(np.float32) * XS
+    for bs in ((None, None, None), tuple(rng.standard_normal(n).astype(np.float32) * 0.1 for n in (n_ff, n_ff, n_out))):
+        y = gpu.mlp(*ws, x, n_ff, k, n_out, biases=bs)
+        assert np.array_equal(y, two_calls(gpu, ws, x, n_ff, k, n_out, biases=bs))
+    for w in ws:
+        gpu.release(w)

@@ -57,6 +57,26 @@ template <int OFF> __device__ inline void lds_read16(uint32_t &dst, uint32_t add
     asm volatile("ds_read_u16 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "n"(OFF));
 }
 
+// SiLU(g) * u in f16, the values of silu_mul_kernel and act_prep32_kernel<.., GU> (zeros where !live), and the sum of the rounded values in
+// order.  With one wave per SIMD the epilogue that calls this is bound by its vector instructions, so what is no finite number is looked
+// for without a compare per element: bad is set where a product is not (x * 0 stays 0 for finite x), and the rounded values are counted only
+// where their sum shows one that is not (no eight finite f16 values add up to an infinity).
+template <int N> __device__ inline float silu_mul_f16(const float (&g)[N], const float (&u)[N], bool live, _Float16 (&h)[N], uint32_t &bad) {
+    static_assert(N <= 8, "sums of finite values stay finite");
+    float v[N], fin = 0.0f, sum = 0.0f;
+#pragma unroll
+    for (int e = 0; e < N; e++) {
+        fin = __builtin_fmaf(g[e], 0.0f, fin);
+        fin = __builtin_fmaf(u[e], 0.0f, fin);
+        v[e] = live ? g[e] / (1.0f + expf(-g[e])) * u[e] : 0.0f;
+        h[e] = (_Float16)v[e];
+        sum += (float)h[e];
+    }
+    bad |= live && !(fin == 0.0f) ? 1u : 0u;
+    if (__builtin_expect(!(__builtin_fabsf(sum) < __builtin_inff()), 0)) turq_note_results<TURQ_ACT_F16>(v);
+    return sum;
+}
+
 template <int I> __device__ inline uint32_t word_of(uint4v v) { return I == 0 ? v.x : I == 1 ? v.y : I == 2 ? v.z : v.w; }
 
 

@@ -95,7 +95,9 @@ template <> struct GFmtWN<TURQ_Q8_0> { static constexpr int value = 1; };
 // activation bytes a launch pulls through the L2 per flop; to fit the LDS its rings are two deep (activation stages and
 // weight super-blocks alike) and the weights of a super-block are requested in two halves, at the last boundary of the
 // super-block before the previous one and at the first of the previous one.
-template <int DT, int WGM_> struct Geo {
+// PAIR: the n-block is made of 16-row tiles of two weights of one shape, gate and up in turn (see gemm_kq_kernel); the ring entry
+// holds the tiles of gate, padded to whole copies, and behind them those of up.
+template <int DT, int WGM_, bool PAIR = false> struct Geo {
     // WGM_ = 4 is the LOW form for launches that would leave CUs idle: 64 rows of m (two m-tiles) by 128 of n, four waves of
     // 64 x 32, i.e. twice the workgroups of the 128 x 128 tile; it uses the wide form's two-deep rings and copy schedule.
     static_assert(WGM_ >= 1 && WGM_ <= 4, "wave grid 2 x 2, 1 x 4, or 1 x 4 with the wide or the low tile");
@@ -111,7 +113,8 @@ template <int DT, int WGM_> struct Geo {
     static constexpr int NT16 = BN / 16;                           // 16-row weight tiles per workgroup
     static constexpr int TB = TiledFmt<DT>::kTileBytes;
     static constexpr int W_BYTES = NT16 * TB;
-    static constexpr int W_CHUNKS = (W_BYTES + 1023) / 1024;       // copies of 1 KiB; the last may be partial
+    static constexpr int P_CHUNKS = (W_BYTES / 2 + 1023) / 1024;   // (pair: of one weight)
+    static constexpr int W_CHUNKS = PAIR ? 2 * P_CHUNKS : (W_BYTES + 1023) / 1024;  // copies of 1 KiB; the last may be partial
     static constexpr int W_STRIDE = W_CHUNKS * 1024;               // ring stride: a partial last copy lands in padding
     static constexpr int CPW = 2 * ((W_CHUNKS + 7) / 8);           // wide form: weight copies per wave and super-block (even)
     static constexpr int A_OFF = 0, W_OFF = RA * GA_STAGE, S_OFF = W_OFF + RW * W_STRIDE;
@@ -180,14 +183,23 @@ __device__ inline uint32_t pack_f16x2(float a, float b) {
 // through rings of its own with the copy schedule, the waits and the barriers of the four-wave form (all eight waves pass the
 // same barriers, so the share must be an even number of super-blocks), which puts two waves on every SIMD; after the loop the
 // second group hands its accumulators to the first through the LDS.
-template <int DT, int WGM_, bool SK = false, int KG = 1>
+// PAIR: gate and up of an MLP against the same activations, and SiLU(gate) * up as down_proj's activation fragments for results.  The two
+// weights (grp.w[0], grp.w[1]; one shape) take turns by 16-row tiles, so the two halves of every 32-column MFMA tile are gate and up of the
+// same 16 columns and their products meet in the epilogue without leaving the workgroup.  y[0]: fragments as act_prep32_kernel<.., GU>
+// writes them (yt != 0: in the order of Q8_0) - the same bits, for the sums are those of the plain form in the same order.  What that saves
+// is the two f32 products' way to memory and back and a launch: 2048 rows of 2 x 12288 x 4096 write 201 MB, which the other kernel
+// reads again, in place of 50.  The epilogue (exponential and division, one wave per SIMD) costs about 2.5 us a round of that.  Whole MLPs with the
+// products through memory -> here: Q4_K 12288 x 4096 at 512 / 2048 rows 199 / 669 -> 187 / 636 us, Q5_K at 512 221 -> 210, Q4_K 3072 x 1024 at
+// 1024 51 -> 45.
+template <int DT, int WGM_, bool SK = false, int KG = 1, bool PAIR = false>
 __global__ void __launch_bounds__(256 * KG) gemm_kq_kernel(GemmGroup grp, int64_t k, const uint8_t *__restrict__ frags, int64_t m, int yt,
                                                            int nblocks_n, int nblocks_m, int vec_out, int split = 1,
                                                            uint8_t *__restrict__ partials = nullptr, uint32_t partial_bytes = 0,
                                                            uint32_t *__restrict__ counters = nullptr) {
     using Fm = GFmt<DT>;
-    using G = Geo<DT, WGM_>;
+    using G = Geo<DT, WGM_, PAIR>;
     constexpr int WGN = G::WGN, WM = G::WM, WN = G::WN, TB = G::TB;
+    static_assert(!PAIR || (!SK && KG == 1), "pairs: whole columns, one group of waves");
     constexpr bool SUMS = Fm::SUMS;
     // Workgroups of one XCD (blockIdx % 8) get consecutive logical ids and the m-blocks of one n-block are
     // consecutive in that order: the packed weights they share stay in that XCD's L2.
@@ -221,7 +233,7 @@ __global__ void __launch_bounds__(256 * KG) gemm_kq_kernel(GemmGroup grp, int64_
     int nb = nb_all;
 #pragma unroll
     for (int i = 1; i < kMaxGroup; i++)
-        if (i < grp.count && nb_all >= grp.first[i]) {
+        if (!PAIR && i < grp.count && nb_all >= grp.first[i]) {
             w = grp.w[i];
             y = grp.y[i];
             bias = grp.bias[i];
@@ -233,11 +245,12 @@ __global__ void __launch_bounds__(256 * KG) gemm_kq_kernel(GemmGroup grp, int64_
     // every block scale is multiplied by wscale (a power of two chosen per tensor so that the largest packed-f16 weight
     // lands near 2^15) and the results by its inverse: small scales keep their precision instead of dropping into the
     // f16 subnormals (d * sc / 16 of Q5_K does so from d around 1e-4)
-    const _Float16 ws = (_Float16)wscale;
-    const float inv_ws = 1.0f / wscale;  // (a power of two: exact)
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
+    if constexpr (PAIR) wscale = lane & 16 ? grp.wscale[1] : grp.wscale[0];
+    const _Float16 ws = (_Float16)wscale;
+    const float inv_ws = 1.0f / wscale;  // (a power of two: exact)
     static_assert(KG == 1 || (KG == 2 && G::LOW), "two groups of waves: the low tile only");
     const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int kg = KG > 1 ? wave_all >> 2 : 0;             // the wave's group and its place in it
@@ -269,20 +282,26 @@ __global__ void __launch_bounds__(256 * KG) gemm_kq_kernel(GemmGroup grp, int64_
     // weights: copy c of a super-block covers bytes [1024 c, 1024 c + 1024) of the concatenated tiles of the workgroup;
     // group g = 0..3 holds copies 4g + wave and 16 + 4g + wave (clamped to the last copy; lanes past the end of the
     // tiles re-read the last 16 bytes into the padding of the ring entry)
-    const int tile0 = nb * G::NT16;
+    // (pair: the copies of gate first, those of up from P_CHUNKS on, each over the tiles of its own weight)
+    const int tile0 = nb * (PAIR ? G::NT16 / 2 : G::NT16);
     const uint8_t *w_src = uniform_ptr(w + ((size_t)tile0 * ntc + kb0) * TB);  // + b * TB
+    const uint8_t *w_src2 = PAIR ? uniform_ptr(grp.w[1] + ((size_t)tile0 * ntc + kb0) * TB) : w_src;
     // (wide form: copies wave, wave + 4, ... of the super-block, CPW per wave, in two halves)
     constexpr int NG = G::WIDE ? G::CPW : 4, NI = G::WIDE ? 1 : 2;
+    auto copy_of = [&](int g, int i) {
+        const int c = G::WIDE ? 4 * g + wave : (i == 0 ? 4 * g + wave : 16 + 4 * g + wave);
+        return c < G::W_CHUNKS ? c : G::W_CHUNKS - 1;
+    };
     uint32_t w_voff[NG][NI];
     uint32_t w_dst[NG][NI];
 #pragma unroll
     for (int g = 0; g < NG; g++)
 #pragma unroll
         for (int i = 0; i < NI; i++) {
-            int c = G::WIDE ? 4 * g + wave : (i == 0 ? 4 * g + wave : 16 + 4 * g + wave);
-            c = c < G::W_CHUNKS ? c : G::W_CHUNKS - 1;
-            uint32_t o = (uint32_t)c * 1024u + lane_off;
-            o = o < (uint32_t)G::W_BYTES ? o : (uint32_t)G::W_BYTES - 16u;
+            const int c = copy_of(g, i);
+            constexpr uint32_t BYTES = PAIR ? G::W_BYTES / 2 : G::W_BYTES;
+            uint32_t o = (uint32_t)(PAIR && c >= G::P_CHUNKS ? c - G::P_CHUNKS : c) * 1024u + lane_off;
+            o = o < BYTES ? o : BYTES - 16u;
             const uint32_t t = o / (uint32_t)TB;
             const uint32_t within = o - t * (uint32_t)TB;
             int tg = tile0 + (int)t;
@@ -303,13 +322,17 @@ __global__ void __launch_bounds__(256 * KG) gemm_kq_kernel(GemmGroup grp, int64_
         }
     };
     auto issue_w = [&](int bb, int g, uint32_t ring) {  // group g of super-block bb
-        const uint8_t *src = w_src + (size_t)bb * (KG * TB);
+        const size_t at = (size_t)bb * (KG * TB);
+        auto src = [&](int g_, int i_) { return (PAIR && copy_of(g_, i_) >= G::P_CHUNKS ? w_src2 : w_src) + at; };
         if constexpr (G::WIDE) {  // half g of the wave's copies
 #pragma unroll
-            for (int i = 0; i < G::CPW / 2; i++) dma_set<0>(w_voff[g * (G::CPW / 2) + i][0], src, w_dst[g * (G::CPW / 2) + i][0] + ring);
+            for (int i = 0; i < G::CPW / 2; i++) {
+                const int c = g * (G::CPW / 2) + i;
+                dma_set<0>(w_voff[c][0], src(c, 0), w_dst[c][0] + ring);
+            }
         } else {
-            dma_set<0>(w_voff[g][0], src, w_dst[g][0] + ring);
-            dma_set<0>(w_voff[g][1], src, w_dst[g][1] + ring);
+            dma_set<0>(w_voff[g][0], src(g, 0), w_dst[g][0] + ring);
+            dma_set<0>(w_voff[g][1], src(g, 1), w_dst[g][1] + ring);
         }
     };
     auto issue_s = [&](int bb) {
@@ -321,7 +344,10 @@ __global__ void __launch_bounds__(256 * KG) gemm_kq_kernel(GemmGroup grp, int64_
     const uint32_t a_rd = lds_base + G::A_OFF + (uint32_t)wm * (WM * 4096u) + lane_off;
     const uint32_t s_rd = lds_base + G::S_OFF + (uint32_t)wm * (WM * 1024u) + lane_off;
     // weights: 32-row tile j of this wave = 16-row tiles 2 WN wn + 2 j + tsel of the ring entry
-    const typename Fm::Addr w_rd = Fm::addr(lds_base + G::W_OFF + (uint32_t)(2 * WN * wn + tsel) * TB, r16, g32);
+    // (pair: 16-row tile WN wn + j of gate or, from P_CHUNKS KiB on, of up)
+    constexpr int JS = PAIR ? TB : 2 * TB;
+    const typename Fm::Addr w_rd =
+        Fm::addr(lds_base + G::W_OFF + (PAIR ? (uint32_t)(WN * wn) * TB + (uint32_t)tsel * (G::P_CHUNKS * 1024u) : (uint32_t)(2 * WN * wn + tsel) * TB), r16, g32);
 
     float16v acc[WM][WN];
 #pragma unroll
@@ -362,8 +388,8 @@ __global__ void __launch_bounds__(256 * KG) gemm_kq_kernel(GemmGroup grp, int64_
     typename Fm::Consts cs[WN], cs_next[WN];
     static_for<WN>([&](auto J) {
         constexpr int j = decltype(J)::value;
-        Fm::template read_hdr<j * 2 * TB>(hd[j], w_rd, wr0);
-        Fm::template read_stage<0, j * 2 * TB>(wq[0][j], w_rd, wr0);
+        Fm::template read_hdr<j * JS>(hd[j], w_rd, wr0);
+        Fm::template read_stage<0, j * JS>(wq[0][j], w_rd, wr0);
     });
     static_for<WM>([&](auto I) { lds_read128<decltype(I)::value * 4096>(af[0][decltype(I)::value], a_rd); });
     wait_lds<0>();
@@ -440,12 +466,12 @@ __global__ void __launch_bounds__(256 * KG) gemm_kq_kernel(GemmGroup grp, int64_
                     const uint32_t ring_from = ks == 3 ? wr1 : wr0;
                     static_for<WN>([&](auto J) {
                         constexpr int j = decltype(J)::value;
-                        Fm::template read_stage<nks, j * 2 * TB>(wq[nxt][j], w_rd, ring_from);
+                        Fm::template read_stage<nks, j * JS>(wq[nxt][j], w_rd, ring_from);
                     });
                     if constexpr (ks == 2) {
                         static_for<WN>([&](auto J) {
                             constexpr int j = decltype(J)::value;
-                            Fm::template read_hdr<j * 2 * TB>(hd[j], w_rd, wr1);
+                            Fm::template read_hdr<j * JS>(hd[j], w_rd, wr1);
                         });
                     }
                     static_for<WM>([&](auto I) { lds_read128<(nks % G::RA) * G::GA_STAGE + decltype(I)::value * 4096>(af[0][decltype(I)::value], a_rd); });
@@ -603,6 +629,54 @@ __global__ void __launch_bounds__(256 * KG) gemm_kq_kernel(GemmGroup grp, int64_
     // ---- results ----
     // 32x32 result: lane (n32, g32), register e holds row 8 * (e / 4) + 4 * g32 + e % 4 of column n32
     constexpr int OUT_PITCH = G::OUT_PITCH;
+    if constexpr (PAIR) {
+        const int64_t wcol = (int64_t)nb * (G::BN / 2) + wn * (WN * 16) + r16;
+        const float *bs = tsel ? grp.bias[1] : grp.bias[0];
+        float *stage = (float *)lds + (size_t)wave * (WM * 32 * OUT_PITCH);
+#pragma unroll
+        for (int j = 0; j < WN; j++) {
+            const float bv = (bs && wcol + 16 * j < n) ? bs[wcol + 16 * j] : 0.0f;
+#pragma unroll
+            for (int i = 0; i < WM; i++)
+#pragma unroll
+                for (int e = 0; e < 16; e++)
+                    stage[(32 * i + 8 * (e >> 2) + 4 * g32 + (e & 3)) * OUT_PITCH + 32 * j + n32] = acc[i][j][e] * inv_ws + bv;
+        }
+        __syncthreads();
+        // A wave takes 16 rows of a sub-block of 32 columns at a time: lane (row l % 16, piece l / 16) makes one 16-byte chunk, 16 of which
+        // lie next to each other in a step of the fragments, and the four lanes that hold a row's sub-block add up its sums.
+        constexpr int SB = G::BN / 64;  // sub-blocks of the n-block
+        const int64_t hct = n / 256;    // (n a multiple of 256)
+        uint32_t bad = 0;
+        const int rl = lane & 15, piece = lane >> 4;
+#pragma unroll 2
+        for (int it = 0; it < SB * (G::GBM / 16) / 4; it++) {
+            const int u = it * 4 + wave;
+            const int sb = u % SB, row_l = u / SB * 16 + rl;
+            const int p = 4 * sb + piece, wnp = p / (2 * WN), pp = p - wnp * (2 * WN);  // the wave column that holds the piece
+            const float *from = (const float *)lds + ((size_t)((row_l / (WM * 32)) * WGN + wnp) * (WM * 32) + row_l % (WM * 32)) * OUT_PITCH +
+                                32 * (pp >> 1) + 8 * (pp & 1);
+            const int64_t row = (int64_t)mb * G::GBM + row_l, col0 = (int64_t)nb * (G::BN / 2) + 32 * sb;
+            if (col0 >= n || (row >> 5) >= mtiles) continue;  // (whole sub-blocks, whole halves of m-tiles: the same for every lane)
+            const float4v g0 = *(const float4v *)from, g1 = *(const float4v *)(from + 4), u0 = *(const float4v *)(from + 16), u1 = *(const float4v *)(from + 20);
+            const float g[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w}, up[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
+            _Float16 hv[8];
+            float sum = silu_mul_f16<8>(g, up, row < m, hv, bad);
+            const half8v h = {hv[0], hv[1], hv[2], hv[3], hv[4], hv[5], hv[6], hv[7]};
+            const int cc = (int)(col0 & 255) / 8 + piece;
+            const int fg = yt ? (cc >> 1) & 1 : cc >> 4, q = yt ? 2 * (cc >> 2) + (cc & 1) : cc & 15;
+            half8v *dst = (half8v *)y + ((row >> 5) * hct + (col0 >> 8)) * (17 * 64);
+            dst[q * 64 + (row & 31) + 32 * fg] = h;
+            sum += __shfl_xor(sum, 16, 64);
+            sum += __shfl_xor(sum, 32, 64);
+            if (!yt && piece == 0) {
+                const _Float16 hi = (_Float16)sum;
+                const _Float16 lo = (_Float16)(sum - (float)hi);
+                ((half2v *)&dst[16 * 64 + (row & 31) + 32 * fg])[(cc >> 2) & 3] = half2v{hi, lo};
+            }
+        }
+        turq_note_flush(bad);
+    } else {
     const bool accum = (yt & TURQ_OUT_ACCUMULATE) != 0;  // y += results: the residual stream
     const int ytb = yt & 0xFF;
     const int64_t row0 = (int64_t)mb * G::GBM + wm * (WM * 32);
@@ -704,16 +778,17 @@ __global__ void __launch_bounds__(256 * KG) gemm_kq_kernel(GemmGroup grp, int64_
         }
         turq_note_flush(badm != 0 ? 1u : 0u);
     }
+    }
 }
 
 // split > 1: the columns of every tile over `split` workgroups that meet in `partials`, counted on `counters`
 // (kSplitCounterBytes, zero between launches)
 constexpr size_t kSplitCounterBytes = TURQ_GEMM_SPLIT_COUNTER_BYTES;
-template <int DT, int WGM_, bool SK = false, int KG = 1>
+template <int DT, int WGM_, bool SK = false, int KG = 1, bool PAIR = false>
 hipError_t launch_gemm(const TurqGemmWeights &ws, int64_t k, const void *frags, int64_t m, int y_dtype, hipStream_t stream,
                        hipEvent_t ev_start, hipEvent_t ev_stop, int split = 1, void *counters = nullptr, void *partials = nullptr,
                        size_t partials_cap = 0) {
-    using G = Geo<DT, WGM_>;
+    using G = Geo<DT, WGM_, PAIR>;
     constexpr int RING_BYTES = KG * ((G::S_OFF + (GFmt<DT>::SUMS ? NS * S_BYTES : 0) + 1023) & ~1023);
     // (after the main loop: the staged results, behind them the sums that a second group of waves hands over)
     constexpr int STAGING_BYTES = 4 * G::WM * 32 * G::OUT_PITCH * 4 + (KG > 1 ? 4 * G::WM * G::WN * 4096 : 0);
@@ -723,7 +798,8 @@ hipError_t launch_gemm(const TurqGemmWeights &ws, int64_t k, const void *frags, 
     if ((uint64_t)G::NT16 * (uint64_t)(k / 256) * G::TB >= (1ull << 32)) return hipErrorInvalidValue;
     if ((k / 256 / (SK ? split : 1)) % KG != 0) return hipErrorInvalidValue;
     if (ws.count < 1 || ws.count > kMaxGroup) return hipErrorInvalidValue;
-    const hipError_t attr = turq_raise_lds_limit((const void *)gemm_kq_kernel<DT, WGM_, SK, KG>, LDS_BYTES);
+    if (PAIR && (ws.count != 2 || ws.n[0] != ws.n[1] || ws.n[0] % 256 != 0)) return hipErrorInvalidValue;
+    const hipError_t attr = turq_raise_lds_limit((const void *)gemm_kq_kernel<DT, WGM_, SK, KG, PAIR>, LDS_BYTES);
     if (attr != hipSuccess) return attr;
     GemmGroup grp{};
     grp.count = ws.count;
@@ -737,7 +813,8 @@ hipError_t launch_gemm(const TurqGemmWeights &ws, int64_t k, const void *frags, 
         grp.ldy[i] = ws.ldy[i];
         grp.wscale[i] = ws.wscale[i];
         grp.first[i] = nbn;
-        nbn += (int)((ws.n[i] + G::BN - 1) / G::BN);
+        if (PAIR) nbn = (int)((ws.n[i] + G::BN / 2 - 1) / (G::BN / 2));
+        else nbn += (int)((ws.n[i] + G::BN - 1) / G::BN);
         // rows of y can be written as aligned 16-byte pieces (every weight of the launch, or none)
         vec_out = vec_out && (uintptr_t)ws.y[i] % 16 == 0 && ((uint64_t)ws.ldy[i] * es) % 16 == 0 && ws.n[i] % 8 == 0;
     }
@@ -753,11 +830,11 @@ hipError_t launch_gemm(const TurqGemmWeights &ws, int64_t k, const void *frags, 
     }
     const dim3 grid((unsigned)(nbn * nbm * split)), block(256 * KG);
     if (ev_start) {
-        hipExtLaunchKernelGGL((gemm_kq_kernel<DT, WGM_, SK, KG>), grid, block, LDS_BYTES, stream, ev_start, ev_stop, 0, grp, k,
+        hipExtLaunchKernelGGL((gemm_kq_kernel<DT, WGM_, SK, KG, PAIR>), grid, block, LDS_BYTES, stream, ev_start, ev_stop, 0, grp, k,
                               (const uint8_t *)frags, m, y_dtype, nbn, nbm, vec_out, split, (uint8_t *)partials, (uint32_t)partial_bytes,
                               (uint32_t *)counters);
     } else {
-        gemm_kq_kernel<DT, WGM_, SK, KG><<<grid, block, LDS_BYTES, stream>>>(grp, k, (const uint8_t *)frags, m, y_dtype, nbn, nbm, vec_out, split,
+        gemm_kq_kernel<DT, WGM_, SK, KG, PAIR><<<grid, block, LDS_BYTES, stream>>>(grp, k, (const uint8_t *)frags, m, y_dtype, nbn, nbm, vec_out, split,
                                                                           (uint8_t *)partials, (uint32_t)partial_bytes, (uint32_t *)counters);
     }
     return hipGetLastError();
@@ -992,6 +1069,35 @@ hipError_t turq_launch_gemm_mfma_group(int dtype, const TurqGemmWeights &ws, int
     default: return hipErrorInvalidValue;
     }
 #undef TURQ_GEMM
+}
+
+// gate and up (ws.w[0], ws.w[1]; one shape, n a multiple of 256) in one launch that leaves down_proj's fragments, turq_act_prep32_bytes(m, n)
+// bytes at ws.y[0], in the order of down_dtype.  Which forms of the tile have it: those of more than one low tile per CU, without wave groups.
+bool turq_gemm_pair_takes(int dtype, int64_t n, int64_t k, int64_t m, int compute_units) {
+    if (n <= 0 || n % 256 != 0 || k <= 0 || k % 256 != 0) return false;
+    const int form = turq_gemm_form(dtype, 2 * n, k, m, compute_units);
+    return form == 3 || (form == 1 && dtype != TURQ_Q8_0) || (form == 2 && (dtype == TURQ_Q4_K || dtype == TURQ_Q8_0));
+}
+hipError_t turq_launch_gemm_mfma_pair(int dtype, int down_dtype, const TurqGemmWeights &ws, int64_t k, const void *frags, int64_t m,
+                                      int compute_units, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop) {
+    if (ws.count != 2 || ws.n[0] != ws.n[1] || !turq_gemm_pair_takes(dtype, ws.n[0], k, m, compute_units)) return hipErrorInvalidValue;
+    for (int i = 0; i < 2; i++)
+        if (!(ws.wscale[i] >= 6.103515625e-5f && ws.wscale[i] <= 32768.0f)) return hipErrorInvalidValue;
+    if (m == 0) return hipSuccess;
+    const int q8_order = down_dtype == TURQ_Q8_0 ? 1 : 0;
+#define TURQ_GEMM_PAIR(DT, F) return launch_gemm<DT, F, false, 1, true>(ws, k, frags, m, q8_order, stream, ev_start, ev_stop)
+    switch (dtype * 8 + turq_gemm_form(dtype, 2 * ws.n[0], k, m, compute_units)) {
+    case TURQ_Q4_K * 8 + 1: TURQ_GEMM_PAIR(TURQ_Q4_K, 1);
+    case TURQ_Q4_K * 8 + 2: TURQ_GEMM_PAIR(TURQ_Q4_K, 2);
+    case TURQ_Q4_K * 8 + 3: TURQ_GEMM_PAIR(TURQ_Q4_K, 3);
+    case TURQ_Q5_K * 8 + 1: TURQ_GEMM_PAIR(TURQ_Q5_K, 1);
+    case TURQ_Q5_K * 8 + 3: TURQ_GEMM_PAIR(TURQ_Q5_K, 3);
+    case TURQ_Q6_K * 8 + 1: TURQ_GEMM_PAIR(TURQ_Q6_K, 1);
+    case TURQ_Q6_K * 8 + 3: TURQ_GEMM_PAIR(TURQ_Q6_K, 3);
+    case TURQ_Q8_0 * 8 + 2: TURQ_GEMM_PAIR(TURQ_Q8_0, 2);
+    default: return hipErrorInvalidValue;
+    }
+#undef TURQ_GEMM_PAIR
 }
 
 TURQ_NONFINITE_READER(turq_nonfinite_gemm_mfma)

@@ -338,6 +338,10 @@ struct TurqGemmWeights {
 hipError_t turq_launch_gemm_mfma_group(int dtype, const TurqGemmWeights &ws, int64_t k, const void *frags, int64_t m, int y_dtype,
                                        int compute_units, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop,
                                        void *split_counters = nullptr, void *split_partials = nullptr, size_t split_partial_bytes = 0);
+// gate and up in one launch that leaves the fragments of SiLU(gate) * up at ws.y[0]; whether there is one for this shape
+bool turq_gemm_pair_takes(int dtype, int64_t n, int64_t k, int64_t m, int compute_units);
+hipError_t turq_launch_gemm_mfma_pair(int dtype, int down_dtype, const TurqGemmWeights &ws, int64_t k, const void *frags, int64_t m,
+                                      int compute_units, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop);
 // the kernel whose waves split the columns (gemm_cols.hip): its tile for a launch, 0 where gemm_kq_kernel takes it; the launch
 bool turq_gemm_cols_mixed(int dtype_a, int dtype_b);
 int turq_gemm_cols_tile(int dtype_a, int dtype_b, int count, const int64_t *n, int64_t k, int64_t m, int compute_units, double *us = nullptr);

@@ -237,8 +237,8 @@ static int gemm_cols_tile(const turq_ctx *ctx, int count, const turq_weight *con
     return turq_gemm_cols_tile(w[0]->dtype, w[s < count ? s : 0]->dtype, count, n, w[0]->k, m, ctx->compute_units, us);
 }
 
-// the prefill GEMM of one weight on the fragments in ctx->act_prep, by either kernel
-static int gemm_on_frags(turq_ctx *ctx, const turq_weight *w, int64_t m, void *y, int yt, int64_t ldy, const float *bias, float wscale) {
+// the prefill GEMM of one weight on prepared fragments, by either kernel
+static int gemm_on_frags(turq_ctx *ctx, const turq_weight *w, const void *frags, int64_t m, void *y, int yt, int64_t ldy, const float *bias, float wscale) {
     int second = 1;
     const int tile = gemm_cols_tile(ctx, 1, &w, m, &second);
     const bool cols = tile != 0;
@@ -248,10 +248,10 @@ static int gemm_on_frags(turq_ctx *ctx, const turq_weight *w, int64_t m, void *y
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     TURQ_HIP(ctx, turq_prof_next(ctx, &ev0, &ev1));
     if (cols)
-        TURQ_HIP(ctx, turq_launch_gemm_cols(w->dtype, w->dtype, second, tile, gemm_weights(1, &w, &y, &ldy, &bias, &wscale), w->k, ctx->act_prep, m, yt,
+        TURQ_HIP(ctx, turq_launch_gemm_cols(w->dtype, w->dtype, second, tile, gemm_weights(1, &w, &y, &ldy, &bias, &wscale), w->k, frags, m, yt,
                                             ctx->compute_units, ctx->stream, ev0, ev1));
     else
-        TURQ_HIP(ctx, turq_launch_gemm_mfma(w->dtype, w->dev, w->n, w->k, ctx->act_prep, m, y, yt, ldy, bias, wscale, ctx->compute_units,
+        TURQ_HIP(ctx, turq_launch_gemm_mfma(w->dtype, w->dev, w->n, w->k, frags, m, y, yt, ldy, bias, wscale, ctx->compute_units,
                                             ctx->stream, ev0, ev1, sp.counters[0], sp.partials[0], sp.bytes[0]));
     return TURQ_OK;
 }
@@ -329,6 +329,49 @@ static bool gemm_both_in_kq(const turq_ctx *ctx, int run, const turq_weight *con
     return kq > 0.0 && kq < us;
 }
 
+// The next launch of a call with `left` weights to go.  As many neighbouring weights as one launch takes in about one round over the CUs (q, k
+// and v; k and v; gate and up of a small model): a launch of few tiles is mostly its start and its end (Q8_0 2 x 3072 x 1024 at 256 rows 21.1 ->
+// 11.1 us), and a second format costs a launch of gemm_cols.hip nothing.  All by the kernel that each takes alone, whose sums do not depend on the
+// launch: in gemm_cols.hip they are the same for every tile, in the one-round launches of gemm_kq_kernel asked here the low
+// tile keeps its wave groups and Q8_0 has one tile.  tile != 0: gemm_cols.hip's, kq: one of gemm_kq_kernel; neither: gemm_run() says.
+// cols[i]: gemm_cols.hip takes weight i alone; may_split: there is scratch for the parts of the first one's columns to meet in.
+struct GemmNext { int run, tile, second; bool kq; };
+static GemmNext gemm_next(const turq_ctx *ctx, int left, const turq_weight *const *w, const bool *cols, int64_t m, bool may_split) {
+    GemmNext g{std::min(left, 4), 0, 0, false};
+    for (; g.run >= 2; g.run--) {
+        if ((w[g.run - 1]->dtype == TURQ_Q8_0) != (w[0]->dtype == TURQ_Q8_0)) continue;
+        const int64_t n_cols = std::count(cols, cols + g.run, true);
+        double us = 0.0;
+        if (n_cols == g.run) g.tile = gemm_cols_tile(ctx, g.run, w, m, &g.second, &us);
+        if (n_cols == 0) g.kq = gemm_run_pays(ctx, g.run, w, m);
+        // (gate and up, each of which gemm_cols.hip takes alone: one launch of gemm_kq_kernel over the rows of both where that is less)
+        if (g.tile != 0 && gemm_both_in_kq(ctx, g.run, w, m, us)) {
+            g.tile = 0;
+            g.kq = true;
+        }
+        if (g.tile != 0 || g.kq) return g;
+    }
+    // (one alone: unless it goes out together with its like, see gemm_run)
+    g.run = 1;
+    if (cols[0] && !gemm_run(ctx, left, w, m, may_split)) g.tile = gemm_cols_tile(ctx, 1, w, m, &g.second);
+    return g;
+}
+
+// Whether gate and up go out as one launch that leaves down_proj's fragments (turq_launch_gemm_mfma_pair): where the two products would come from
+// gemm_kq_kernel without wave groups or split columns, whose sums the pair has too (turq_mlp and the two calls agree to the bit).
+static bool gemm_pair(const turq_ctx *ctx, const turq_weight *const *gu, int64_t m) {
+    const TurqTuning &t = turq_tuning();
+    if (t.mlp_pair == 0 || gu[0]->dtype != gu[1]->dtype || gu[0]->n != gu[1]->n || gu[0]->k != gu[1]->k || gu[0]->n % 256 != 0) return false;
+    const int cus = ctx->compute_units, dt = gu[0]->dtype;
+    const int64_t n = gu[0]->n, k = gu[0]->k;
+    const bool both[2] = {gemm_cols_tile(ctx, 1, gu, m, nullptr) != 0, gemm_cols_tile(ctx, 1, gu + 1, m, nullptr) != 0};
+    const bool split = !both[0] && turq_gemm_split_scratch(dt, n, k, m, cus, nullptr) != 0;
+    const GemmNext g = gemm_next(ctx, 2, gu, both, m, split);
+    if (g.tile != 0 || !turq_gemm_pair_takes(dt, n, k, m, cus)) return false;
+    if (g.kq || gemm_run(ctx, 2, gu, m, split) == 2) return true;
+    return !split && !(turq_gemm_form(dt, n, k, m, cus) == 4 && turq_gemm_low_two_groups(n, k, m, 1, cus));
+}
+
 int turq_qmatmul_multi_gemm(turq_ctx *ctx, int count, const turq_weight *const *w, const void *x, int xt, int64_t m, int64_t ldx,
                             void *const *y, int yt, const int64_t *ldy, const float *const *bias, bool *taken, const TurqNorm *norm) {
     *taken = false;
@@ -372,29 +415,8 @@ int turq_qmatmul_multi_gemm(turq_ctx *ctx, int count, const turq_weight *const *
             prepared = order;
         }
         hipStream_t st = ctx->stream;
-        // As many neighbouring weights as one launch takes in about one round over the CUs (q, k and v; k and v; gate and up of a small
-        // model): a launch of few tiles is mostly its start and its end (Q8_0 2 x 3072 x 1024 at 256 rows 21.1 -> 11.1 us), and a
-        // second format costs a launch of gemm_cols.hip nothing.  All by the kernel that each takes alone, whose sums do not depend on the
-        // launch: in gemm_cols.hip they are the same for every tile, in the one-round launches of gemm_kq_kernel asked here the low
-        // tile keeps its wave groups and Q8_0 has one tile.
         {
-            int run = std::min(count - i, 4), tile = 0, second = 0;
-            bool kq = false;
-            for (; run >= 2; run--) {
-                if ((w[i + run - 1]->dtype == TURQ_Q8_0) != (order == 2)) continue;
-                const int64_t n_cols = std::count(cols + i, cols + i + run, true);
-                double us = 0.0;
-                if (n_cols == run) tile = gemm_cols_tile(ctx, run, w + i, m, &second, &us);
-                if (n_cols == 0) kq = gemm_run_pays(ctx, run, w + i, m);
-                // (gate and up, each of which gemm_cols.hip takes alone: one launch of gemm_kq_kernel over the rows of both where that is less)
-                if (tile != 0 && gemm_both_in_kq(ctx, run, w + i, m, us)) {
-                    tile = 0;
-                    kq = true;
-                }
-                if (tile != 0 || kq) break;
-            }
-            // (one alone: unless it goes out together with its like below)
-            if (run == 1 && cols[i] && !gemm_run(ctx, count - i, w + i, m, sp.counters[i] != nullptr)) tile = gemm_cols_tile(ctx, 1, w + i, m, &second);
+            const auto [run, tile, second, kq] = gemm_next(ctx, count - i, w + i, cols + i, m, sp.counters[i] != nullptr);
             if (tile != 0 || kq) {
                 group_n = 0;  // (closes a group of small ones)
                 const TurqGemmWeights g = gemm_weights(run, w + i, y + i, ldy + i, bias ? bias + i : nullptr, ws + i);
@@ -490,14 +512,34 @@ int turq_mlp_prefill(turq_ctx *ctx, const turq_weight *gate, const turq_weight *
     *taken = false;
     const bool off = turq_tuning().mlp_prefill_off;
     const turq_weight *gu[2] = {gate, up};
-    float ws_down = 1.0f, ws_tmp = 1.0f;
+    float ws_down = 1.0f, ws_gu[2] = {1.0f, 1.0f};
     if (off || m <= TURQ_GEMV_MAX_M || ctx->fixed_scratch) return TURQ_OK;
     for (const turq_weight *w : {gate, up, down})
-        if (w->device != ctx->device || w->layout != TURQ_LAYOUT_TILED || w->n <= 0 || w->k <= 0 || !gemm_takes(w, &ws_tmp)) return TURQ_OK;
-    if (!gemm_takes(down, &ws_down) || down->k != gate->n || gate->n != up->n || gate->k != up->k) return TURQ_OK;
+        if (w->device != ctx->device || w->layout != TURQ_LAYOUT_TILED || w->n <= 0 || w->k <= 0 ||
+            !gemm_takes(w, w == gate ? ws_gu : w == up ? ws_gu + 1 : &ws_down)) return TURQ_OK;
+    if (down->k != gate->n || gate->n != up->n || gate->k != up->k) return TURQ_OK;
     if (ldx < gate->k || ldy < down->n || !turq_act_bytes(xt) || !turq_act_bytes(yt)) return TURQ_OK;
     if (turq_rows_in_chunks(ctx, 2, gu, x, xt, ldx, m)) return TURQ_OK;  // gate / up through the kernels of up to 32 rows
     const int64_t n_ff = gate->n;
+    if (gemm_pair(ctx, gu, m) && (!norm || (gate->k % 256 == 0 && gate->k <= 16384))) {
+        int rc = turq_ctx_reserve(ctx, &ctx->gate_up, &ctx->gate_up_cap, turq_act_prep32_bytes(m, n_ff));
+        if (rc != TURQ_OK) return rc;
+        rc = turq_ctx_reserve(ctx, &ctx->act_prep, &ctx->act_prep_cap, turq_act_prep32_bytes(m, gate->k));
+        if (rc != TURQ_OK) return rc;
+        TURQ_HIP(ctx, norm ? turq_launch_rms_norm_prep32(gate->dtype, x, xt, m, gate->k, ldx, norm->w, norm->eps, ctx->act_prep, ctx->stream)
+                           : turq_launch_act_prep32(gate->dtype, x, xt, m, gate->k, ldx, ctx->act_prep, ctx->stream));
+        void *const ys[2] = {ctx->gate_up, nullptr};
+        const int64_t lds[2] = {n_ff, n_ff};
+        const float *const biases[2] = {bias_gate, bias_up};
+        hipEvent_t ev0 = nullptr, ev1 = nullptr;
+        TURQ_HIP(ctx, turq_prof_next(ctx, &ev0, &ev1));
+        TURQ_HIP(ctx, turq_launch_gemm_mfma_pair(gate->dtype, down->dtype, gemm_weights(2, gu, ys, lds, biases, ws_gu), gate->k, ctx->act_prep, m,
+                                                 ctx->compute_units, ctx->stream, ev0, ev1));
+        rc = gemm_on_frags(ctx, down, ctx->gate_up, m, y, yt, ldy, bias_down, ws_down);
+        if (rc != TURQ_OK) return rc;
+        *taken = true;
+        return TURQ_OK;
+    }
     const size_t half = (size_t)m * (size_t)n_ff;
     int rc = turq_ctx_reserve(ctx, &ctx->gate_up, &ctx->gate_up_cap, 2 * half * sizeof(float) + 16);
     if (rc != TURQ_OK) return rc;
@@ -511,7 +553,7 @@ int turq_mlp_prefill(turq_ctx *ctx, const turq_weight *gate, const turq_weight *
     rc = turq_qmatmul_multi_gemm(ctx, 2, gu, x, xt, m, ldx, ys, TURQ_ACT_F32, ldys, biases, &gu_taken, norm);
     if (rc != TURQ_OK || !gu_taken) return rc;
     TURQ_HIP(ctx, turq_launch_silu_mul_prep32(down->dtype, (const float *)ys[0], (const float *)ys[1], m, n_ff, ctx->act_prep, ctx->stream));
-    rc = gemm_on_frags(ctx, down, m, y, yt, ldy, bias_down, ws_down);
+    rc = gemm_on_frags(ctx, down, ctx->act_prep, m, y, yt, ldy, bias_down, ws_down);
     if (rc != TURQ_OK) return rc;
     *taken = true;
     return TURQ_OK;
@@ -535,7 +577,7 @@ int turq_qmatmul_mfma(turq_ctx *ctx, const turq_weight *w, const void *x, int xt
         if (rc != TURQ_OK) return rc;
         if (norm) TURQ_HIP(ctx, turq_launch_rms_norm_prep32(w->dtype, x, xt, m, w->k, ldx, norm->w, norm->eps, ctx->act_prep, ctx->stream));
         else TURQ_HIP(ctx, turq_launch_act_prep32(w->dtype, x, xt, m, w->k, ldx, ctx->act_prep, ctx->stream));
-        return gemm_on_frags(ctx, w, m, y, yt, ldy, bias, wscale);
+        return gemm_on_frags(ctx, w, ctx->act_prep, m, y, yt, ldy, bias, wscale);
     }
     const int nwaves = pick_waves(ctx, w->n, w->k);
     for (int64_t m0 = 0; m0 < m; m0 += TURQ_GEMV_MAX_M) {

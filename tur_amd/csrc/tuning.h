@@ -32,6 +32,7 @@
     X(gateup_no_frag, "TURQ_GATEUP_NO_FRAG", FLAG, 0, "turq_qmatmul_gate_up at 17 .. 32 rows: leave the prepared-fragment route out")       \
     X(rows_in_chunks_off, "TURQ_ROWS_IN_CHUNKS", OFF, 0, "33 .. 64 rows never go through the decode kernels in two chunks")                 \
     X(norm_fused_off, "TURQ_NORM_FUSED", OFF, 0, "turq_norm_*: always normalise into scratch first")                                        \
+    X(mlp_pair, "TURQ_MLP_PAIR", TRI, -1, "gate and up of a prompt chunk in one launch that leaves down_proj's fragments (0: never)")       \
     X(mlp_prefill_off, "TURQ_MLP_PREFILL", OFF, 0, "turq_mlp above 32 rows: separate calls instead of the fused middle kernel")             \
     X(gemm_no_side, "TURQ_GEMM_NO_SIDE", FLAG, 0, "turq_qmatmul_multi above 32 rows: every launch on the context's stream")                 \
     X(gemm_merge, "TURQ_GEMM_MERGE", INT, -1, "gate / up as one prefill launch: 0 never, 2 always (default: the rule)")                     \
