@@ -211,9 +211,12 @@ def test_prompt_chunks(gpu, dt_gu, dt_dn, m):
 @pytest.mark.parametrize("dt_gu,dt_dn,n_ff,k,m", [
     (Q4_K, Q6_K, 2816, 512, 600), (Q4_K, Q5_K, 3328, 3072, 513), (Q4_K, Q8_0, 6400, 256, 545), (Q5_K, Q6_K, 2816, 512, 600),
     (Q5_K, Q4_K, 6400, 256, 513), (Q6_K, Q6_K, 2816, 512, 600), (Q6_K, Q8_0, 6400, 256, 513), (Q8_0, Q8_0, 3328, 1024, 2017),
-    (Q8_0, Q4_K, 3328, 1024, 2017)])
+    (Q8_0, Q4_K, 3328, 1024, 2017),
+    # the kernel whose waves split the columns, by tiles: 32 x 32, 64 x 32, 64 x 64 alone and two per CU, 96 x 64, 128 x 64, 96 x 96
+    (Q4_K, Q6_K, 256, 256, 33), (Q4_K, Q6_K, 1280, 1024, 70), (Q5_K, Q6_K, 3328, 2048, 65), (Q8_0, Q8_0, 3072, 1024, 300),
+    (Q6_K, Q6_K, 5120, 4096, 77), (Q8_0, Q6_K, 5376, 3072, 100), (Q5_K, Q8_0, 12288, 4096, 77), (Q4_K, Q8_0, 4352, 4096, 190), (Q8_0, Q8_0, 2304, 1024, 47)])
 def test_prompt_pairs(gpu, dt_gu, dt_dn, n_ff, k, m):
-    """Gate and up in one launch that writes down_proj's fragments (128 x 128, 2 x 2 and wide tiles; blocks of n past the last row, rows
+    """Gate and up in one launch that writes down_proj's fragments (the LDS-tiled kernel first: 128 x 128, 2 x 2 and wide tiles; blocks of n past the last row, rows
     past m in the last 32; both fragment orders, with the sub-block sums of a Q4_K / Q5_K down_proj): bit-equal to the two calls.  The
     scales of gate and up differ by 2^9, so that a column taken with the other's scale would show."""
     n_out = 512

@@ -106,7 +106,13 @@ template <int MT, int NT> struct Meet {
     static constexpr int LDS = W * T * 32 * kPitch * 4;
 };
 
-template <int DT, int MT, int NT, bool TIGHT>
+// PAIR: gate and up of an MLP (weights 0 and 1, one shape), which take turns by 16-row tiles, and SiLU(gate) * up as down_proj's activation fragments
+// for results: see gemm_kq_kernel, whose pair does the same.  The halves of a 32-column MFMA tile are the two products of the same 16 columns, so a
+// lane's weights are those of one of the two, which takes a 64-bit address per 32-row tile.  Without the sub-block sums of the fragments, whose 32
+// columns may be two workgroups': for a down_proj of Q6_K or Q8_0, which read none.  These launches are 6 - 35 us, and what the pair saves is the
+// 5 us launch between it and down_proj: whole MLPs Q8_0 1024 x 3072 at 34 / 300 rows 19.3 / 30.3 -> 16.5 / 25.0 us, Q5_K / Q6_K
+// 4096 x 12288 at 77 rows 66.6 -> 62.2, at 180 rows 108 -> 96; nowhere slower (4096 x 12288 .. 5120 x 15360, 34 - 600 rows, every format).
+template <int DT, int MT, int NT, bool TIGHT, bool PAIR>
 __device__ __forceinline__ void cols_body(const ColsGroup &grp, int wi, int nb, int mb, int64_t k, const uint8_t *__restrict__ frags, int64_t m,
                                           int yt, int vec_out, uint8_t *lds) {
     using Fm = GFmt<DT>;
@@ -131,18 +137,21 @@ __device__ __forceinline__ void cols_body(const ColsGroup &grp, int wi, int nb, 
         const uint64_t off = ((uint64_t)((mt < mtiles ? mt : mtiles - 1) * ntc * 17)) << 10;  // (wave-uniform: kept in scalar registers)
         a_src[i] = frags + (((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(off >> 32)) << 32) | __builtin_amdgcn_readfirstlane((uint32_t)off));
     }
-    const int tile0 = nb * NT * 2;
+    const int tile0 = nb * NT * (PAIR ? 1 : 2);
     const uint8_t *w_src = w + (size_t)tile0 * ntc * TB;
     uint32_t w_off[NT];  // the lane's 16-row tile of every 32-row tile
+    const uint8_t *w_lane[NT];  // (pair: its address)
 #pragma unroll
     for (int j = 0; j < NT; j++) {
-        int t = tile0 + 2 * j + tsel;
+        int t = PAIR ? tile0 + j : tile0 + 2 * j + tsel;
         t = t < nrt ? t : nrt - 1;  // (row tiles past the end: the last one again, never stored)
-        w_off[j] = (uint32_t)(t - tile0) * (uint32_t)ntc * (uint32_t)TB;
+        w_off[j] = PAIR ? 0u : (uint32_t)(t - tile0) * (uint32_t)ntc * (uint32_t)TB;
+        w_lane[j] = PAIR ? (tsel ? grp.w[1] : grp.w[0]) + (size_t)t * ntc * TB : nullptr;
     }
+    auto w_at = [&](int b, int j) { return (PAIR ? w_lane[j] : w_src) + (size_t)b * TB; };
     uint32_t lane16 = 16u * (uint32_t)lane;
     const uint32_t slot = (uint32_t)(r16 + 32 * g32);
-    const _Float16 ws = (_Float16)grp.wscale[wi];
+    const _Float16 ws = (_Float16)(PAIR ? (tsel ? grp.wscale[1] : grp.wscale[0]) : grp.wscale[wi]);
 
     float16v acc[MT][NT];
 #pragma unroll
@@ -170,9 +179,9 @@ __device__ __forceinline__ void cols_body(const ColsGroup &grp, int wi, int nb, 
             }
         };
         auto load_w = [&](Wb (&dst)[NT], int b) {
-            const uint8_t *p = w_src + (size_t)b * TB;
 #pragma unroll
             for (int j = 0; j < NT; j++) {
+                const uint8_t *p = w_at(b, j);
                 dst[j].load_hdr(p, w_off[j], (uint32_t)r16, slot);
                 static_for<4>([&](auto KS) { dst[j].template load<decltype(KS)::value>(p, w_off[j], slot); });
             }
@@ -235,14 +244,12 @@ __device__ __forceinline__ void cols_body(const ColsGroup &grp, int wi, int nb, 
                 ra[u % D][i] = __builtin_bit_cast(half8v, ld16(a_src[i] + ((size_t)(b * 17 + (u & ~3)) << 10), lane16 + (uint32_t)((u & 3) * 1024)));
         };
         auto load_w = [&](int b, auto KS) {
-            const uint8_t *p = w_src + (size_t)b * TB;
 #pragma unroll
-            for (int j = 0; j < NT; j++) wc[j].template load<decltype(KS)::value>(p, w_off[j], slot);
+            for (int j = 0; j < NT; j++) wc[j].template load<decltype(KS)::value>(w_at(b, j), w_off[j], slot);
         };
         auto load_h = [&](int b) {
-            const uint8_t *p = w_src + (size_t)b * TB;
 #pragma unroll
-            for (int j = 0; j < NT; j++) wc[j].load_hdr(p, w_off[j], (uint32_t)r16, slot);
+            for (int j = 0; j < NT; j++) wc[j].load_hdr(w_at(b, j), w_off[j], (uint32_t)r16, slot);
         };
         auto block = [&](int b, auto MORE) {
             constexpr bool more = decltype(MORE)::value;
@@ -300,6 +307,52 @@ __device__ __forceinline__ void cols_body(const ColsGroup &grp, int wi, int nb, 
     // (stored as they lie: 16 or 8 bytes per lane.  With a lane's four values in one column, as the MFMA leaves them, the stores were 4 us of a
     // launch of eight tiles per workgroup and 3 us of one of four)
     using M = Meet<MT, NT>;
+    if constexpr (PAIR) {
+        // thread: half a 16-byte chunk, 32 rows of which lie next to each other in a step of the fragments
+        const float inv_g = 1.0f / grp.wscale[0], inv_u = 1.0f / grp.wscale[1];
+        const float *bg = grp.bias[0], *bu = grp.bias[1];
+        float *red = (float *)lds;
+        const int half = tid & 1, row_l = (tid >> 1) & 31, chunk = (tid >> 6) & 1;
+        uint32_t bad = 0;
+#pragma unroll
+        for (int r = 0; r < M::ROUNDS; r++) {
+            if (r) __syncthreads();
+#pragma unroll
+            for (int t = 0; t < M::T; t++) {
+                if (r * M::T + t >= MT * NT) continue;
+                const int i = (r * M::T + t) / NT, j = (r * M::T + t) % NT;
+#pragma unroll
+                for (int e = 0; e < 16; e++) red[((wave * M::T + t) * 32 + 8 * (e >> 2) + 4 * g32 + (e & 3)) * kPitch + n32] = acc[i][j][e];
+            }
+            __syncthreads();
+            for (int t = tid >> 7; t < M::T; t += 2) {
+                const int tile = r * M::T + t;
+                const int64_t mt = (int64_t)mb * MT + tile / NT, col = ((int64_t)nb * NT + tile % NT) * 16 + 8 * chunk + 4 * half;
+                if (tile >= MT * NT || mt >= mtiles || col >= n) continue;
+                const int at_lds = (t * 32 + row_l) * kPitch + 8 * chunk + 4 * half;
+                float4v sg = *(const float4v *)(red + at_lds), su = *(const float4v *)(red + at_lds + 16);
+#pragma unroll
+                for (int v = 1; v < W; v++) {
+                    sg += *(const float4v *)(red + v * (M::T * 32 * kPitch) + at_lds);
+                    su += *(const float4v *)(red + v * (M::T * 32 * kPitch) + at_lds + 16);
+                }
+                float g[4], u[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    g[e] = (sg[e] * inv_g + (bg ? bg[col + e] : 0.0f)) + 0.0f;
+                    u[e] = (su[e] * inv_u + (bu ? bu[col + e] : 0.0f)) + 0.0f;
+                }
+                _Float16 h[4];
+                silu_mul_f16<4>(g, u, mt * 32 + row_l < m, h, bad);
+                const int cc = (int)(col & 255) >> 3;
+                const int fg = yt ? (cc >> 1) & 1 : cc >> 4, q = yt ? 2 * (cc >> 2) + (cc & 1) : cc & 15;
+                uint8_t *dst = (uint8_t *)grp.y[0] + ((size_t)((mt * (n >> 8) + (col >> 8)) * 17 + q) << 10);
+                *(uint2v *)(dst + 16 * (row_l + 32 * fg) + 8 * half) = uint2v{as_u32(half2v{h[0], h[1]}), as_u32(half2v{h[2], h[3]})};
+            }
+        }
+        turq_note_flush(bad);
+        return;
+    }
     const float inv_ws = 1.0f / grp.wscale[wi];  // (a power of two: exact)
     const float *bias = grp.bias[wi];
     void *y = grp.y[wi];
@@ -384,7 +437,7 @@ __device__ __forceinline__ void cols_body(const ColsGroup &grp, int wi, int nb, 
 }
 
 // MINB: workgroups that are to share a CU (2: the tight form of the 64 x 64 tile in 256 registers; otherwise what the tile leaves)
-template <int DTA, int DTB, int MT, int NT, bool TIGHT, int MINB>
+template <int DTA, int DTB, int MT, int NT, bool TIGHT, int MINB, bool PAIR>
 __global__ void __launch_bounds__(64 * W, MINB) gemm_cols_kernel(ColsGroup grp, int64_t k, const uint8_t *__restrict__ frags, int64_t m, int yt,
                                                            int nblocks_n, int nblocks_m, int vec_out) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -397,16 +450,16 @@ __global__ void __launch_bounds__(64 * W, MINB) gemm_cols_kernel(ColsGroup grp, 
     int wi = 0;
 #pragma unroll
     for (int i = 1; i < kMaxGroup; i++)
-        if (i < grp.count && nb_all >= grp.first[i]) wi = i;
+        if (!PAIR && i < grp.count && nb_all >= grp.first[i]) wi = i;
     const int nb = nb_all - grp.first[wi];
-    if (DTA == DTB || wi < grp.second) cols_body<DTA, MT, NT, TIGHT>(grp, wi, nb, mb, k, frags, m, yt, vec_out, lds);
-    else cols_body<DTB, MT, NT, TIGHT>(grp, wi, nb, mb, k, frags, m, yt, vec_out, lds);
+    if (DTA == DTB || wi < grp.second) cols_body<DTA, MT, NT, TIGHT, PAIR>(grp, wi, nb, mb, k, frags, m, yt, vec_out, lds);
+    else cols_body<DTB, MT, NT, TIGHT, PAIR>(grp, wi, nb, mb, k, frags, m, yt, vec_out, lds);
 }
 
-template <int DTA, int DTB, int MT, int NT, bool TIGHT = false, int MINB = 1>
+template <int DTA, int DTB, int MT, int NT, bool TIGHT = false, int MINB = 1, bool PAIR = false>
 hipError_t launch_cols(const TurqGemmWeights &ws, int second, int64_t k, const void *frags, int64_t m, int yt, hipStream_t stream,
                        hipEvent_t ev_start, hipEvent_t ev_stop) {
-    const auto kernel = gemm_cols_kernel<DTA, DTB, MT, NT, TIGHT, MINB>;
+    const auto kernel = gemm_cols_kernel<DTA, DTB, MT, NT, TIGHT, MINB, PAIR>;
     constexpr int LDS_BYTES = Meet<MT, NT>::LDS;
     static_assert(LDS_BYTES <= 64 * 1024, "no raised LDS limit");
     ColsGroup grp{};
@@ -423,7 +476,8 @@ hipError_t launch_cols(const TurqGemmWeights &ws, int second, int64_t k, const v
         grp.ldy[i] = ws.ldy[i];
         grp.wscale[i] = ws.wscale[i];
         grp.first[i] = nbn;
-        nbn += (int)((ws.n[i] + 32 * NT - 1) / (32 * NT));
+        if (PAIR) nbn = (int)((ws.n[i] + 16 * NT - 1) / (16 * NT));
+        else nbn += (int)((ws.n[i] + 32 * NT - 1) / (32 * NT));
     }
     const int nbm = (int)((m + 32 * MT - 1) / (32 * MT));
     const dim3 grid((unsigned)(nbn * nbm)), block(64 * W);
@@ -458,6 +512,27 @@ hipError_t launch_tile(int tile, const TurqGemmWeights &ws, int second, int64_t 
 #undef TURQ_COLS
     default: return hipErrorInvalidValue;
     }
+}
+
+// the pair's tiles: of those above, without two that the estimates hardly ever pick for two weights
+constexpr int kPairTiles[] = {11, 21, 22, 32, 42, 33};
+template <int DT>
+hipError_t launch_pair(int tile, const TurqGemmWeights &ws, int64_t k, const void *frags, int64_t m, int yt, int64_t cus, hipStream_t stream,
+                       hipEvent_t ev_start, hipEvent_t ev_stop) {
+    const int64_t n2 = 2 * ws.n[0];
+#define TURQ_COLS(MT, NT, TIGHT, MINB) launch_cols<DT, DT, MT, NT, TIGHT, MINB, true>(ws, 2, k, frags, m, yt, stream, ev_start, ev_stop)
+    switch (tile) {
+    case 11: return TURQ_COLS(1, 1, false, 1);
+    case 21: return TURQ_COLS(2, 1, false, 1);
+    case 22:
+        if (cols_workgroups(22, 1, &n2, m) > cus) return TURQ_COLS(2, 2, true, 2);
+        return TURQ_COLS(2, 2, false, 1);
+    case 32: return TURQ_COLS(3, 2, false, 1);
+    case 42: return TURQ_COLS(4, 2, false, 1);
+    case 33: return TURQ_COLS(3, 3, true, 1);
+    default: return hipErrorInvalidValue;
+    }
+#undef TURQ_COLS
 }
 
 // bytes of one row tile's super-blocks, the larger of the two formats'
@@ -601,6 +676,43 @@ hipError_t turq_launch_gemm_cols(int dtype_a, int dtype_b, int second, int tile,
     default: return hipErrorInvalidValue;
     }
 #undef TURQ_COLS_TILE
+}
+
+// The tile with which gate and up of n rows each go through this kernel as a pair, by the estimates; *us: what that takes.  0: there is none.
+int turq_gemm_cols_pair_tile(int dtype, int down_dtype, int64_t n, int64_t k, int64_t m, int compute_units, double *us) {
+    *us = 0.0;
+    if (!turq_dt_is_quant(dtype) || (down_dtype != TURQ_Q6_K && down_dtype != TURQ_Q8_0)) return 0;
+    if (n <= 0 || n % 256 != 0 || k <= 0 || k % 256 != 0 || m <= 0) return 0;
+    const int64_t n2 = 2 * n;
+    int best = 0;
+    for (const int tile : kPairTiles) {
+        const double est = cols_us(tile, dtype, dtype, 1, &n2, k, m, compute_units > 0 ? compute_units : 256);
+        if (!best || est < *us) {
+            best = tile;
+            *us = est;
+        }
+    }
+    return best;
+}
+
+// gate and up (ws.w[0], ws.w[1]; one shape, n a multiple of 256) as a pair: down_proj's fragments, turq_act_prep32_bytes(m, n) bytes at ws.y[0]
+hipError_t turq_launch_gemm_cols_pair(int dtype, int down_dtype, int tile, const TurqGemmWeights &ws, int64_t k, const void *frags, int64_t m,
+                                      int compute_units, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop) {
+    if (ws.count != 2 || ws.n[0] != ws.n[1] || ws.n[0] <= 0 || ws.n[0] % 256 != 0 || k <= 0 || k % 256 != 0 || k / 256 > (1 << 20)) return hipErrorInvalidValue;
+    if (down_dtype != TURQ_Q6_K && down_dtype != TURQ_Q8_0) return hipErrorInvalidValue;
+    for (int i = 0; i < 2; i++)
+        if (!(ws.wscale[i] >= 6.103515625e-5f && ws.wscale[i] <= 32768.0f)) return hipErrorInvalidValue;
+    if (m == 0) return hipSuccess;
+    if ((ws.n[0] / 16 + 1) * ((m + 31) / 32) > 0x7FFFFFFF) return hipErrorInvalidValue;
+    const int64_t cus = compute_units > 0 ? compute_units : 256;
+    const int q8_order = down_dtype == TURQ_Q8_0 ? 1 : 0;
+    switch (dtype) {
+    case TURQ_Q4_K: return launch_pair<TURQ_Q4_K>(tile, ws, k, frags, m, q8_order, cus, stream, ev_start, ev_stop);
+    case TURQ_Q5_K: return launch_pair<TURQ_Q5_K>(tile, ws, k, frags, m, q8_order, cus, stream, ev_start, ev_stop);
+    case TURQ_Q6_K: return launch_pair<TURQ_Q6_K>(tile, ws, k, frags, m, q8_order, cus, stream, ev_start, ev_stop);
+    case TURQ_Q8_0: return launch_pair<TURQ_Q8_0>(tile, ws, k, frags, m, q8_order, cus, stream, ev_start, ev_stop);
+    default: return hipErrorInvalidValue;
+    }
 }
 
 TURQ_NONFINITE_READER(turq_nonfinite_gemm_cols)

@@ -345,6 +345,9 @@ hipError_t turq_launch_gemm_mfma_pair(int dtype, int down_dtype, const TurqGemmW
 // the kernel whose waves split the columns (gemm_cols.hip): its tile for a launch, 0 where gemm_kq_kernel takes it; the launch
 bool turq_gemm_cols_mixed(int dtype_a, int dtype_b);
 int turq_gemm_cols_tile(int dtype_a, int dtype_b, int count, const int64_t *n, int64_t k, int64_t m, int compute_units, double *us = nullptr);
+int turq_gemm_cols_pair_tile(int dtype, int down_dtype, int64_t n, int64_t k, int64_t m, int compute_units, double *us);
+hipError_t turq_launch_gemm_cols_pair(int dtype, int down_dtype, int tile, const TurqGemmWeights &ws, int64_t k, const void *frags, int64_t m,
+                                      int compute_units, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop);
 double turq_gemm_launch_us(int dtype, int count, const int64_t *n, int64_t k, int64_t m, int compute_units);
 double turq_gemm_kq_us(int dtype, int64_t n, int64_t k, int64_t m, int compute_units);  // an estimate of a launch of gemm_kq_kernel
 constexpr double kTurqLaunchUs = 2.5;  // the share of a launch's time that a further round over the CUs does not pay again

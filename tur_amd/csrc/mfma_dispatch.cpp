@@ -335,17 +335,17 @@ static bool gemm_both_in_kq(const turq_ctx *ctx, int run, const turq_weight *con
 // launch: in gemm_cols.hip they are the same for every tile, in the one-round launches of gemm_kq_kernel asked here the low
 // tile keeps its wave groups and Q8_0 has one tile.  tile != 0: gemm_cols.hip's, kq: one of gemm_kq_kernel; neither: gemm_run() says.
 // cols[i]: gemm_cols.hip takes weight i alone; may_split: there is scratch for the parts of the first one's columns to meet in.
-struct GemmNext { int run, tile, second; bool kq; };
+// us: what gemm_cols.hip's launch takes, roughly.
+struct GemmNext { int run, tile, second; bool kq; double us; };
 static GemmNext gemm_next(const turq_ctx *ctx, int left, const turq_weight *const *w, const bool *cols, int64_t m, bool may_split) {
-    GemmNext g{std::min(left, 4), 0, 0, false};
+    GemmNext g{std::min(left, 4), 0, 0, false, 0.0};
     for (; g.run >= 2; g.run--) {
         if ((w[g.run - 1]->dtype == TURQ_Q8_0) != (w[0]->dtype == TURQ_Q8_0)) continue;
         const int64_t n_cols = std::count(cols, cols + g.run, true);
-        double us = 0.0;
-        if (n_cols == g.run) g.tile = gemm_cols_tile(ctx, g.run, w, m, &g.second, &us);
+        if (n_cols == g.run) g.tile = gemm_cols_tile(ctx, g.run, w, m, &g.second, &g.us);
         if (n_cols == 0) g.kq = gemm_run_pays(ctx, g.run, w, m);
         // (gate and up, each of which gemm_cols.hip takes alone: one launch of gemm_kq_kernel over the rows of both where that is less)
-        if (g.tile != 0 && gemm_both_in_kq(ctx, g.run, w, m, us)) {
+        if (g.tile != 0 && gemm_both_in_kq(ctx, g.run, w, m, g.us)) {
             g.tile = 0;
             g.kq = true;
         }
@@ -353,23 +353,31 @@ static GemmNext gemm_next(const turq_ctx *ctx, int left, const turq_weight *cons
     }
     // (one alone: unless it goes out together with its like, see gemm_run)
     g.run = 1;
-    if (cols[0] && !gemm_run(ctx, left, w, m, may_split)) g.tile = gemm_cols_tile(ctx, 1, w, m, &g.second);
+    if (cols[0] && !gemm_run(ctx, left, w, m, may_split)) g.tile = gemm_cols_tile(ctx, 1, w, m, &g.second, &g.us);
     return g;
 }
 
-// Whether gate and up go out as one launch that leaves down_proj's fragments (turq_launch_gemm_mfma_pair): where the two products would come from
-// gemm_kq_kernel without wave groups or split columns, whose sums the pair has too (turq_mlp and the two calls agree to the bit).
-static bool gemm_pair(const turq_ctx *ctx, const turq_weight *const *gu, int64_t m) {
+// Whether gate and up go out as one launch that leaves down_proj's fragments: kGemmPairKq (turq_launch_gemm_mfma_pair) where the two products
+// would come from gemm_kq_kernel without wave groups or split columns, a tile (turq_launch_gemm_cols_pair) where they would come from
+// gemm_cols.hip, 0: neither.  The pairs have those kernels' sums (turq_mlp and the two calls agree to the bit).  From gemm_cols.hip: unless
+// the launch over both is slower than the products' launches by more than the one it saves, which reads them again (4 us and more).
+constexpr int kGemmPairKq = -1;
+static int gemm_pair(const turq_ctx *ctx, const turq_weight *const *gu, int down_dtype, int64_t m) {
     const TurqTuning &t = turq_tuning();
-    if (t.mlp_pair == 0 || gu[0]->dtype != gu[1]->dtype || gu[0]->n != gu[1]->n || gu[0]->k != gu[1]->k || gu[0]->n % 256 != 0) return false;
+    if (t.mlp_pair == 0 || gu[0]->dtype != gu[1]->dtype || gu[0]->n != gu[1]->n || gu[0]->k != gu[1]->k || gu[0]->n % 256 != 0) return 0;
     const int cus = ctx->compute_units, dt = gu[0]->dtype;
     const int64_t n = gu[0]->n, k = gu[0]->k;
     const bool both[2] = {gemm_cols_tile(ctx, 1, gu, m, nullptr) != 0, gemm_cols_tile(ctx, 1, gu + 1, m, nullptr) != 0};
     const bool split = !both[0] && turq_gemm_split_scratch(dt, n, k, m, cus, nullptr) != 0;
     const GemmNext g = gemm_next(ctx, 2, gu, both, m, split);
-    if (g.tile != 0 || !turq_gemm_pair_takes(dt, n, k, m, cus)) return false;
-    if (g.kq || gemm_run(ctx, 2, gu, m, split) == 2) return true;
-    return !split && !(turq_gemm_form(dt, n, k, m, cus) == 4 && turq_gemm_low_two_groups(n, k, m, 1, cus));
+    if (g.tile != 0) {
+        double us = 0.0;
+        const int tile = turq_gemm_cols_pair_tile(dt, down_dtype, n, k, m, cus, &us);
+        return tile != 0 && us < (g.run == 2 ? g.us : 2.0 * g.us) + 4.0 ? tile : 0;
+    }
+    if (!turq_gemm_pair_takes(dt, n, k, m, cus)) return 0;
+    const bool plain = g.kq || gemm_run(ctx, 2, gu, m, split) == 2 || (!split && !(turq_gemm_form(dt, n, k, m, cus) == 4 && turq_gemm_low_two_groups(n, k, m, 1, cus)));
+    return plain ? kGemmPairKq : 0;
 }
 
 int turq_qmatmul_multi_gemm(turq_ctx *ctx, int count, const turq_weight *const *w, const void *x, int xt, int64_t m, int64_t ldx,
@@ -416,7 +424,7 @@ int turq_qmatmul_multi_gemm(turq_ctx *ctx, int count, const turq_weight *const *
         }
         hipStream_t st = ctx->stream;
         {
-            const auto [run, tile, second, kq] = gemm_next(ctx, count - i, w + i, cols + i, m, sp.counters[i] != nullptr);
+            const auto [run, tile, second, kq, us] = gemm_next(ctx, count - i, w + i, cols + i, m, sp.counters[i] != nullptr);
             if (tile != 0 || kq) {
                 group_n = 0;  // (closes a group of small ones)
                 const TurqGemmWeights g = gemm_weights(run, w + i, y + i, ldy + i, bias ? bias + i : nullptr, ws + i);
@@ -521,7 +529,7 @@ int turq_mlp_prefill(turq_ctx *ctx, const turq_weight *gate, const turq_weight *
     if (ldx < gate->k || ldy < down->n || !turq_act_bytes(xt) || !turq_act_bytes(yt)) return TURQ_OK;
     if (turq_rows_in_chunks(ctx, 2, gu, x, xt, ldx, m)) return TURQ_OK;  // gate / up through the kernels of up to 32 rows
     const int64_t n_ff = gate->n;
-    if (gemm_pair(ctx, gu, m) && (!norm || (gate->k % 256 == 0 && gate->k <= 16384))) {
+    if (const int pair = !norm || gate->k <= 16384 ? gemm_pair(ctx, gu, down->dtype, m) : 0) {
         int rc = turq_ctx_reserve(ctx, &ctx->gate_up, &ctx->gate_up_cap, turq_act_prep32_bytes(m, n_ff));
         if (rc != TURQ_OK) return rc;
         rc = turq_ctx_reserve(ctx, &ctx->act_prep, &ctx->act_prep_cap, turq_act_prep32_bytes(m, gate->k));
@@ -533,8 +541,11 @@ int turq_mlp_prefill(turq_ctx *ctx, const turq_weight *gate, const turq_weight *
         const float *const biases[2] = {bias_gate, bias_up};
         hipEvent_t ev0 = nullptr, ev1 = nullptr;
         TURQ_HIP(ctx, turq_prof_next(ctx, &ev0, &ev1));
-        TURQ_HIP(ctx, turq_launch_gemm_mfma_pair(gate->dtype, down->dtype, gemm_weights(2, gu, ys, lds, biases, ws_gu), gate->k, ctx->act_prep, m,
-                                                 ctx->compute_units, ctx->stream, ev0, ev1));
+        const TurqGemmWeights g = gemm_weights(2, gu, ys, lds, biases, ws_gu);
+        TURQ_HIP(ctx, pair == kGemmPairKq ? turq_launch_gemm_mfma_pair(gate->dtype, down->dtype, g, gate->k, ctx->act_prep, m, ctx->compute_units,
+                                                                       ctx->stream, ev0, ev1)
+                                          : turq_launch_gemm_cols_pair(gate->dtype, down->dtype, pair, g, gate->k, ctx->act_prep, m,
+                                                                       ctx->compute_units, ctx->stream, ev0, ev1));
         rc = gemm_on_frags(ctx, down, ctx->gate_up, m, y, yt, ldy, bias_down, ws_down);
         if (rc != TURQ_OK) return rc;
         *taken = true;
