@@ -843,7 +843,7 @@ def test_prefill_column_split_edges(gpu, dt, n, k, m):
     gpu.release(w)
 
 
-def test_prefill_column_split_largest_tile():
+def test_columns_over_waves_largest_tile():
     # 96 x 96, the tile of gate and up together at 65 - 96 rows, on the edges of the test above
     import os
     import subprocess
@@ -858,7 +858,7 @@ def test_prefill_column_split_largest_tile():
 
 @pytest.mark.parametrize("dt", [Q4_K, Q5_K, Q6_K, Q8_0])
 @pytest.mark.parametrize("k", [1024, 1280])
-def test_prefill_column_split_two_workgroups_per_cu(gpu, dt, k):
+def test_columns_over_waves_two_workgroups_per_cu(gpu, dt, k):
     # 485 workgroups of the 64 x 64 tile, two of which share a CU in a form of the loop of its own: one super-block per wave, and two for one of
     # the four; the bound of the prefill kernels, and the same bits as fewer rows give in another tile and form
     import ctypes
