@@ -48,6 +48,58 @@ template <int XT> __device__ inline void ld_piece(const void *x, int64_t row_off
     }
 }
 
+// The pieces tid, tid + 256, ... of a row (+0 past k, and everywhere where !live) and, up to WPER of them, of its weight.  Where rows, weight and
+// k allow 16-byte loads all of them are requested before the first is looked at: a weight that is first asked for behind the sum, as the
+// store needs it, waits for HBM a second time, and pieces that are converted one by one a time each (three layers at 77 bf16 rows of 4096 columns,
+// six such launches in 338 us: 5 us less; 1024 columns, one piece per thread: no difference).
+template <int XT, int PER, int WPER>
+__device__ inline void ld_pieces(const void *x, int64_t row_off, int64_t k, bool live, bool vec_x, const float *w, bool vec_w, int tid, float (&v)[PER][8],
+                                 float (&wv)[WPER][8]) {
+    static_assert(WPER <= PER);
+    if (vec_x && vec_w && (k & 7) == 0) {
+        constexpr int ES = XT == TURQ_ACT_F32 ? 4 : 2;
+        uint4v raw[PER][ES / 2];
+        float4v rw[WPER][2];
+        const uint8_t *px = (const uint8_t *)x + (live ? row_off : 0) * ES;  // (the first row exists)
+#pragma unroll
+        for (int j = 0; j < PER; j++) {
+            const int64_t col0 = ((int64_t)j * 256 + tid) * 8, at = col0 < k ? col0 : 0;
+#pragma unroll
+            for (int h = 0; h < ES / 2; h++) raw[j][h] = ((const uint4v *)(px + at * ES))[h];
+        }
+#pragma unroll
+        for (int j = 0; j < WPER; j++) {
+            const int64_t col0 = ((int64_t)j * 256 + tid) * 8, at = col0 < k ? col0 : 0;
+            rw[j][0] = ((const float4v *)(w + at))[0], rw[j][1] = ((const float4v *)(w + at))[1];
+        }
+#pragma unroll
+        for (int j = 0; j < PER; j++) {
+            const bool on = live && ((int64_t)j * 256 + tid) * 8 < k;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                if constexpr (XT == TURQ_ACT_F32) {
+                    v[j][e] = on ? __uint_as_float(raw[j][e >> 2][e & 3]) : 0.0f;
+                } else if constexpr (XT == TURQ_ACT_BF16) {
+                    const uint32_t u = raw[j][0][e >> 1];
+                    v[j][e] = on ? __uint_as_float(e & 1 ? u & 0xFFFF0000u : u << 16) : 0.0f;
+                } else {
+                    const half2v hh = as_half2(raw[j][0][e >> 1]);
+                    v[j][e] = on ? (float)(e & 1 ? hh.y : hh.x) : 0.0f;
+                }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < WPER; j++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) wv[j][e] = rw[j][e >> 2][e & 3];
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < PER; j++) ld_piece<XT>(x, row_off, ((int64_t)j * 256 + tid) * 8, live ? k : 0, vec_x, v[j]);
+#pragma unroll
+    for (int j = 0; j < WPER; j++) ld_piece<TURQ_ACT_F32>(w, 0, ((int64_t)j * 256 + tid) * 8, k, vec_w, wv[j]);
+}
+
 __device__ inline bool vec_row(const void *p, int64_t ld, int elem_bytes) {
     return ((uintptr_t)p & 15) == 0 && ((ld * elem_bytes) & 15) == 0;
 }
@@ -130,13 +182,9 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(const void *__restrict__ 
     const int64_t xo = row * ldx, yo = row * ldy;
     const bool vx = vec_row(x, ldx, XT == TURQ_ACT_F32 ? 4 : 2), vy = vec_row(y, ldy, YT == TURQ_ACT_F32 ? 4 : 2);
     const bool vw = ((uintptr_t)w & 15) == 0;
-    float v[PER][8];
+    float v[PER][8], wv[PER][8];
     float s = 0.0f;
-#pragma unroll
-    for (int j = 0; j < PER; j++) {
-        const int64_t col0 = ((int64_t)j * 256 + tid) * 8;
-        ld_piece<XT>(x, xo, col0, k, vx, v[j]);
-    }
+    ld_pieces<XT, PER, PER>(x, xo, k, true, vx, w, vw, tid, v, wv);
 #pragma unroll
     for (int j = 0; j < PER; j++)
 #pragma unroll
@@ -148,13 +196,12 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(const void *__restrict__ 
         for (int e = 0; e < 8; e++) s = __builtin_fmaf(t[e], t[e], s);
     }
     const RowDiv div(rms_of(s, k, eps, part));
-    auto store = [&](int64_t col0, const float (&t)[8]) {
+    auto store = [&](int64_t col0, const float (&t)[8], const float (&tw)[8]) {
         if (col0 >= k) return;
-        float wv[8], o[8];
-        ld_piece<TURQ_ACT_F32>(w, 0, col0, k, vw, wv);
+        float o[8];
         div(t, o);
 #pragma unroll
-        for (int e = 0; e < 8; e++) o[e] *= wv[e];
+        for (int e = 0; e < 8; e++) o[e] *= tw[e];
         if (vy && col0 + 8 <= k) {
             turq_note_results<YT>(o);
             uint8_t *p = (uint8_t *)y + (yo + col0) * (YT == TURQ_ACT_F32 ? 4 : 2);
@@ -176,11 +223,12 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(const void *__restrict__ 
         }
     };
 #pragma unroll
-    for (int j = 0; j < PER; j++) store(((int64_t)j * 256 + tid) * 8, v[j]);
+    for (int j = 0; j < PER; j++) store(((int64_t)j * 256 + tid) * 8, v[j], wv[j]);
     for (int64_t col0 = ((int64_t)PER * 256 + tid) * 8; PER == 3 && col0 < k; col0 += 2048) {
-        float t[8];
+        float t[8], tw[8];
         ld_piece<XT>(x, xo, col0, k, vx, t);
-        store(col0, t);
+        ld_piece<TURQ_ACT_F32>(w, 0, col0, k, vw, tw);
+        store(col0, t, tw);
     }
 }
 
@@ -207,13 +255,10 @@ __global__ void __launch_bounds__(256 * kPrepRows) rms_norm_prep32_kernel(const 
     const bool live = row < m;
     const int64_t xo = row * ldx;
     const bool vx = vec_row(x, ldx, XT == TURQ_ACT_F32 ? 4 : 2), vw = ((uintptr_t)w & 15) == 0;
-    float v[PER][8];
+    constexpr int WPER = PER <= 2 ? PER : 1;  // (longer rows: two workgroups share a CU up to 64 registers)
+    float v[PER][8], wv[WPER][8];
     float s = 0.0f;
-#pragma unroll
-    for (int j = 0; j < PER; j++) {
-        const int64_t col0 = ((int64_t)j * 256 + tid) * 8;
-        ld_piece<XT>(x, xo, col0, live ? k : 0, vx, v[j]);
-    }
+    ld_pieces<XT, PER, WPER>(x, xo, k, live, vx, w, vw, tid, v, wv);
     if (PER == 1 && k <= kShort) {  // (the order of rms_norm_short_kernel)
         float sq[2];
         s = short_square_sum<XT>(x, xo, live ? k : 0, tid, sq);
@@ -228,14 +273,14 @@ __global__ void __launch_bounds__(256 * kPrepRows) rms_norm_prep32_kernel(const 
     for (int j = 0; j < PER; j++) {
         const int64_t piece = (int64_t)j * 256 + tid, col0 = piece * 8;
         if (col0 >= k) continue;  // (k is a multiple of 256: whole pieces, and whole groups of four lanes)
-        float wv[8];
-        ld_piece<TURQ_ACT_F32>(w, 0, col0, k, vw, wv);
+        if (j >= WPER) ld_piece<TURQ_ACT_F32>(w, 0, col0, k, vw, wv[0]);
+        const float (&wj)[8] = wv[j < WPER ? j : 0];
         half8v h;
         float sum = 0.0f, f[8];
         div(v[j], f);
 #pragma unroll
         for (int e = 0; e < 8; e++) {
-            f[e] = live ? f[e] * wv[e] : 0.0f;
+            f[e] = live ? f[e] * wj[e] : 0.0f;
             h[e] = (_Float16)f[e];
             sum += (float)h[e];
         }
