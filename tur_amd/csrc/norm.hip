@@ -234,28 +234,25 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(const void *__restrict__ 
 
 // The same rows written straight into the fragments of the prefill GEMM (the order act_prep32_kernel writes, see there): what
 // rms_norm_kernel with an f32 output followed by that kernel would leave - the same sums in the same order, the same one rounding
-// to f16 - without the launch and the round trip in between.  A workgroup takes kPrepRows neighbouring rows of a 32-row m-tile
-// (rows past m: zeros), 256 threads each: a fragment block holds 16 bytes of each row next to each other, and rows that are
-// written by one workgroup meet in one cache line of one L2 (with a row per workgroup every 128-byte line was written in eight pieces
-// from eight XCDs; 4096 bf16 columns: 2048 rows 34.7 -> 12.5 us, 512 rows 15 -> 7, 77 rows 10.4 -> 5.6).  A thread keeps its PER pieces of 8 columns in registers between the two passes (k <= 2048 * PER); the
-// sub-block sums of the fragments (32 columns) are added up between the four neighbouring lanes that hold a sub-block.
-constexpr int kPrepRows = 4;
+// to f16 - without the launch and the round trip in between.  One workgroup per row (rows past m, to the end of a 32-row m-tile: zeros); a fragment
+// block holds 16 bytes of each row next to each other, so neighbouring rows, which meet in a cache line, run on one XCD and meet in its L2.  Four rows per
+// workgroup, which wrote 64 bytes together, kept 24 of 256 CUs at 77 rows: the layers of 4096 columns at 77 / 512 rows took 342 / 557 us with them
+// and 329 / 552 now, those of 1024 columns at 300 rows 846 and 810, 4096 columns at 2048 rows the same.  A thread keeps its PER pieces of 8 columns in registers
+// between the two passes (k <= 2048 * PER); the sub-block sums of the fragments (32 columns) are added up between the four neighbouring lanes that hold
+// a sub-block.
 template <int XT, bool Q8, int PER>
-__global__ void __launch_bounds__(256 * kPrepRows) rms_norm_prep32_kernel(const void *__restrict__ x, int64_t m, int64_t k, int64_t ldx,
-                                                                          const float *__restrict__ w, float eps, int64_t ntc,
-                                                                          half8v *__restrict__ frags) {
-    __shared__ float part[kPrepRows][4];
-    const int tid = threadIdx.x & 255, sub = threadIdx.x >> 8;
-    // workgroups of one XCD (blockIdx % 8) take neighbouring rows
-    const int nwg = (int)gridDim.x;
-    const int lid = (nwg & 7) == 0 ? ((int)blockIdx.x & 7) * (nwg >> 3) + ((int)blockIdx.x >> 3) : (int)blockIdx.x;
-    const int64_t row = (int64_t)lid * kPrepRows + sub;
+__global__ void __launch_bounds__(256) rms_norm_prep32_kernel(const void *__restrict__ x, int64_t m, int64_t k, int64_t ldx, const float *__restrict__ w,
+                                                              float eps, int64_t ntc, half8v *__restrict__ frags) {
+    __shared__ float part[4];
+    const int tid = threadIdx.x;
+    // workgroups of one XCD (blockIdx % 8) take neighbouring rows (the grid: a multiple of 32)
+    const int64_t row = (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
     const int64_t mt = row >> 5;
     const int r = (int)(row & 31);
     const bool live = row < m;
     const int64_t xo = row * ldx;
     const bool vx = vec_row(x, ldx, XT == TURQ_ACT_F32 ? 4 : 2), vw = ((uintptr_t)w & 15) == 0;
-    constexpr int WPER = PER <= 2 ? PER : 1;  // (longer rows: two workgroups share a CU up to 64 registers)
+    constexpr int WPER = PER <= 2 ? PER : 1;  // (longer rows: eight waves share a SIMD up to 64 registers)
     float v[PER][8], wv[WPER][8];
     float s = 0.0f;
     ld_pieces<XT, PER, WPER>(x, xo, k, live, vx, w, vw, tid, v, wv);
@@ -268,7 +265,7 @@ __global__ void __launch_bounds__(256 * kPrepRows) rms_norm_prep32_kernel(const 
 #pragma unroll
             for (int e = 0; e < 8; e++) s = __builtin_fmaf(v[j][e], v[j][e], s);
     }
-    const RowDiv div(rms_of(s, k, eps, part[sub]));
+    const RowDiv div(rms_of(s, k, eps, part));
 #pragma unroll
     for (int j = 0; j < PER; j++) {
         const int64_t piece = (int64_t)j * 256 + tid, col0 = piece * 8;
@@ -342,11 +339,11 @@ hipError_t turq_launch_rms_norm_prep32(int dtype, const void *x, int x_dtype, in
     if (m == 0 || k == 0) return hipSuccess;
     if (k % 256 != 0 || k > 16384 || m > (1 << 26)) return hipErrorInvalidValue;
     const int64_t ntc = k / 256;
-    const unsigned grid = (unsigned)(((m + 31) / 32) * (32 / kPrepRows));
+    const unsigned grid = (unsigned)((m + 31) / 32 * 32);
     const bool q8 = dtype == TURQ_Q8_0;
 #define TURQ_NP32(XT, PER)                                                                                                           \
-    if (q8) rms_norm_prep32_kernel<XT, true, PER><<<grid, 256 * kPrepRows, 0, stream>>>(x, m, k, ldx, weight, eps, ntc, (half8v *)frags);       \
-    else rms_norm_prep32_kernel<XT, false, PER><<<grid, 256 * kPrepRows, 0, stream>>>(x, m, k, ldx, weight, eps, ntc, (half8v *)frags)
+    if (q8) rms_norm_prep32_kernel<XT, true, PER><<<grid, 256, 0, stream>>>(x, m, k, ldx, weight, eps, ntc, (half8v *)frags);       \
+    else rms_norm_prep32_kernel<XT, false, PER><<<grid, 256, 0, stream>>>(x, m, k, ldx, weight, eps, ntc, (half8v *)frags)
 #define TURQ_NP32_X(XT)                                  \
     if (k <= 2048) { TURQ_NP32(XT, 1); }                 \
     else if (k <= 2048 * 2) { TURQ_NP32(XT, 2); }        \
