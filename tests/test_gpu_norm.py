@@ -111,6 +111,36 @@ def test_rms_norm_pieces_of_every_type(gpu, k, xt, yt):
         assert rel_l2(call(gpu, x, w, 1e-6, x_dtype=xt, y_dtype=yt, ldx=ld, ldy=ld, mem=capi.MEM_DEVICE), want_norm(x, w, 1e-6)) <= bar, ld
 
 
+@pytest.mark.parametrize("xt", [capi.ACT_F32, capi.ACT_BF16, capi.ACT_F16])
+@pytest.mark.parametrize("k", [520, 2048, 2304, 6144, 12288, 14336])
+def test_weights_at_any_address_give_the_same_bits(gpu, k, xt):
+    # a row and its weight are requested together where both allow 16-byte loads; a weight at another address is loaded by element, when it is
+    # needed: to rows, and (33 rows and more, whole super-blocks) to the fragments of the prefill GEMM, one row past the last 32
+    m, n = 33, 32
+    x = synth.random_activation(m, k, seed=k, bf16=True)
+    send = synth.to_bf16_bits(x).reshape(m, k) if xt == capi.ACT_BF16 else x.astype(np.float16) if xt == capi.ACT_F16 else x
+    w = np.random.default_rng(k).standard_normal(k).astype(np.float32)
+    xd, at = gpu.dev_buffer(send), [gpu.dev_buffer(w), gpu.dev_buffer(np.concatenate([np.zeros(1, np.float32), w]))]
+    weights = [ctypes.c_void_p(at[0].value), ctypes.c_void_p(at[1].value + 4)]
+    yd = [gpu.dev_buffer(np.zeros((m, k), np.float32)) for _ in weights]
+    for wd, y in zip(weights, yd):
+        capi.check(gpu.L.turq_rms_norm(gpu.ctx, xd, xt, m, k, k, wd, 1e-6, y, capi.ACT_F32, k, capi.MEM_DEVICE), gpu.ctx)
+    rows = [gpu.read_back(y, (m, k), np.float32) for y in yd]
+    assert np.array_equal(rows[0].view(np.uint32), rows[1].view(np.uint32))
+    assert rel_l2(rows[0], want_norm(x if xt != capi.ACT_F16 else send.astype(np.float32), w, 1e-6)) <= 1e-6
+    if k % 256 == 0:
+        q = gpu.upload(capi.Q4_K, n, k, synth.random_weight(capi.Q4_K, n, k, seed=1), capi.LAYOUT_TILED)
+        out = []
+        for wd, y in zip(weights, yd):
+            capi.check(gpu.L.turq_norm_qmatmul_multi(gpu.ctx, 1, (ctypes.c_void_p * 1)(q.value), xd, xt, m, k, wd, 1e-6, (ctypes.c_void_p * 1)(y.value),
+                                                     capi.ACT_F32, (ctypes.c_int64 * 1)(n), None, capi.MEM_DEVICE), gpu.ctx)
+            out.append(gpu.read_back(y, (m, n), np.float32))
+        assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
+        gpu.release(q)
+    for p in (xd, *at, *yd):
+        gpu.dev_free(p)
+
+
 def test_rms_norm_small_elements_and_signed_zeros(gpu):
     # the squares of all but four elements vanish in the sum, which makes the root exactly 3: every other element is v / 3 to the last
     # bit, whatever its size (quotients and remainders below the f32 range among them), and a zero keeps its sign
