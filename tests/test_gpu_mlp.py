@@ -235,3 +235,32 @@ def test_prompt_pairs(gpu, dt_gu, dt_dn, n_ff, k, m):
         assert np.array_equal(y, two_calls(gpu, ws, x, n_ff, k, n_out, biases=bs))
     for w in ws:
         gpu.release(w)
+
+
+@pytest.mark.parametrize("dt_gu,dt_dn,n_ff,k,m,places", [
+    (Q5_K, Q6_K, 512, 512, 48, "aab"), (Q5_K, Q6_K, 2816, 512, 600, "aab"),
+    (Q6_K, Q6_K, 512, 512, 48, "aba"), (Q8_0, Q8_0, 512, 512, 40, "abb"), (Q4_K, Q4_K, 512, 512, 64, "aba"), (Q6_K, Q6_K, 512, 512, 48, "aaa")])
+def test_one_weight_in_several_places(gpu, dt_gu, dt_dn, n_ff, k, m, places):
+    """A prompt chunk's MLP whose gate, up or (square matrices) down is one handle, with block scales of about 2e-5: without the power of two that
+    every place's launch multiplies them by, they would lose bits in the f16 subnormals.  Bit-equal to the two calls, each of which looks at
+    one place, and near the oracle: 1e-3 of the f16 operands, three times over (gate, up, down)."""
+    n_out = k if "a" in places[2] or places[1:] == "bb" else 256
+    shapes = [(dt_gu, n_ff, k), (dt_gu, n_ff, k), (dt_dn, n_out, n_ff)]
+    made = {}
+    for c, (dt, n, kk) in zip(places, shapes):
+        if c in made:
+            continue
+        raw = synth.random_weight(dt, n, kk, seed=ord(c))
+        nb = synth.BLOCK_BYTES[dt]
+        blocks = raw.reshape(-1, nb)
+        at = nb - 2 if dt == Q6_K else 0
+        for o in (at, at + 2) if dt in (Q4_K, Q5_K) else (at,):
+            blocks[:, o:o + 2] = (blocks[:, o:o + 2].copy().view(np.float16) * np.float16(2.0 ** -9)).view(np.uint8)
+        made[c] = (raw, gpu.upload(dt, n, kk, raw, capi.LAYOUT_TILED))
+    raws, ws = [made[c][0] for c in places], [made[c][1] for c in places]
+    x = synth.random_activation(m, k, seed=m)
+    y = gpu.mlp(*ws, x, n_ff, k, n_out)
+    assert np.array_equal(y, two_calls(gpu, ws, x, n_ff, k, n_out))
+    assert rel_l2(y, expected(dt_gu, dt_dn, f16_round(x), *raws, n_ff, k, n_out)) <= 3e-3
+    for raw, w in made.values():
+        gpu.release(w)

@@ -523,8 +523,9 @@ int turq_mlp_prefill(turq_ctx *ctx, const turq_weight *gate, const turq_weight *
     float ws_down = 1.0f, ws_gu[2] = {1.0f, 1.0f};
     if (off || m <= TURQ_GEMV_MAX_M || ctx->fixed_scratch) return TURQ_OK;
     for (const turq_weight *w : {gate, up, down})
-        if (w->device != ctx->device || w->layout != TURQ_LAYOUT_TILED || w->n <= 0 || w->k <= 0 ||
-            !gemm_takes(w, w == gate ? ws_gu : w == up ? ws_gu + 1 : &ws_down)) return TURQ_OK;
+        if (w->device != ctx->device || w->layout != TURQ_LAYOUT_TILED || w->n <= 0 || w->k <= 0) return TURQ_OK;
+    // (by place: one weight may stand in several)
+    if (!gemm_takes(gate, &ws_gu[0]) || !gemm_takes(up, &ws_gu[1]) || !gemm_takes(down, &ws_down)) return TURQ_OK;
     if (down->k != gate->n || gate->n != up->n || gate->k != up->k) return TURQ_OK;
     if (ldx < gate->k || ldy < down->n || !turq_act_bytes(xt) || !turq_act_bytes(yt)) return TURQ_OK;
     if (turq_rows_in_chunks(ctx, 2, gu, x, xt, ldx, m)) return TURQ_OK;  // gate / up through the kernels of up to 32 rows
