@@ -237,9 +237,9 @@ int turq_qmatmul_noalloc(turq_ctx *ctx, const turq_weight *w, const void *x, int
  * calls, bit for bit; neighbouring weights that make few workgroup tiles each - q, k and v of a prompt chunk - go out as one launch of
  * the kernel that each takes alone; launches of the other kernel that still leave half of the GPU free run next to each other,
  * up to three at a time, on further streams of the context that are joined to the first before the call returns, so the
- * caller still sees one stream; neighbouring large weights of one K-quant format and shape - gate_proj and up_proj - go out as ONE
- * GEMM launch over the rows of all of them where that fills the GPU better, with the tile and the kernel chosen for all the rows: the
- * same products, in another order of the f32 sums, within 2e-6 relative L2 of the single calls); every other case is exactly the
+ * caller still sees one stream; neighbouring large weights of one K-quant format and shape - gate_proj and up_proj, each of which alone takes more
+ * than half of the GPU's compute units - go out as ONE GEMM launch over the rows of all of them where that fills the GPU better, with the tile and the
+ * kernel chosen for all the rows: the same products, in another order of the f32 sums, within 2e-6 relative L2 of the single calls); every other case is exactly the
  * turq_qmatmul calls one after the other (including their errors).  `biases` may be NULL, and so may its entries.
  * Replaces: the back-to-back `forward` calls on one input in the reference's decoder layer - q_proj / k_proj /
  * v_proj (src/models/qwen3.rs:272-274) and gate_proj / up_proj (src/models/qwen3.rs:161-167). */

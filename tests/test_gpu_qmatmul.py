@@ -552,6 +552,23 @@ def test_multi_weight_prefill_keeps_the_bits_of_the_single_calls(gpu, dts, ns, k
         gpu.release(w)
 
 
+@pytest.mark.parametrize("dt,count,n,k,m", [(Q4_K, 3, 1024, 1024, 1000), (Q6_K, 3, 1024, 5120, 1021), (Q6_K, 2, 1280, 3328, 1378),
+                                             (Q4_K, 4, 512, 1024, 1800), (Q6_K, 2, 3584, 1280, 324)])
+def test_small_weights_of_one_shape_keep_the_bits_of_the_single_calls(gpu, dt, count, n, k, m):
+    # several K-quant weights of one shape, each of which fills no more than half of the GPU: together they would be less in the other kernel, whose
+    # sums are in another order
+    raws = [synth.random_weight(dt, n, k, seed=i) for i in range(count)]
+    ws = [gpu.upload(dt, n, k, raw, capi.LAYOUT_TILED) for raw in raws]
+    x = synth.random_activation(m, k, seed=m, bf16=True)
+    ys = gpu.qmatmul_multi(ws, x, [n] * count, k, x_dtype=capi.ACT_BF16)
+    for raw, w, y in zip(raws, ws, ys):
+        assert np.array_equal(y, gpu.qmatmul_device(w, x, n, k, x_dtype=capi.ACT_BF16))
+        rows = np.arange(0, n, 32)
+        assert rel_l2(y[:, rows], orc.matmul_dequant(dt, x, raw.reshape(n, -1)[rows].reshape(-1), len(rows), k)) <= 1e-3
+    for w in ws:
+        gpu.release(w)
+
+
 def test_multi_weight_prefill_runs_of_one_format(gpu):
     # neighbouring weights of one K-quant format and shape (rows a multiple of 256) may go out as ONE launch of the prefill GEMM
     # whose n-blocks are dealt out to the weights; the rule only does that for weights that fill half the machine, so this test

@@ -319,21 +319,23 @@ static bool gemm_run_pays(const turq_ctx *ctx, int run, const turq_weight *const
     return us > 0.0 && us < apart;
 }
 
-// whether `run` K-quant weights of one shape that gemm_cols.hip would take in one launch of `us` are less as one launch of gemm_kq_kernel
-// (Q4_K 2 x 12288 x 4096 at 256 rows: 73 against 61)
+// Whether `run` weights, each of which gemm_cols.hip takes alone and which it would take in one launch of `us`, go out as one launch of
+// gemm_kq_kernel after all, whose sums are in another order.  Only the large ones of gemm_run, which the contract of turq_qmatmul_multi excepts from the
+// bits of the single calls, and unless gemm_cols.hip's estimate is a twelfth below: of 57 such launches gemm_cols.hip took 0.96 - 1.22 of the other
+// kernel's time (on average 1.05; Q5_K 2 x 7168 x 6144 at 1190 rows 334 us for 275) where its estimate was between that and gemm_kq_kernel's, 0.73 - 1.01
+// (0.88; Q5_K 2 x 12288 x 4096 at 77 rows 34 for 45) where it was below.
 static bool gemm_both_in_kq(const turq_ctx *ctx, int run, const turq_weight *const *w, int64_t m, double us) {
-    if (turq_tuning().gemm_cols > 0 || turq_tuning().gemm_merge >= 0 || run < 2 || us <= 0.0 || w[0]->dtype == TURQ_Q8_0 || w[0]->n % 256 != 0) return false;
-    for (int i = 1; i < run; i++)
-        if (w[i]->dtype != w[0]->dtype || w[i]->n != w[0]->n) return false;
+    if (turq_tuning().gemm_cols > 0 || turq_tuning().gemm_merge >= 0 || run < 2 || us <= 0.0 || w[0]->dtype == TURQ_Q8_0) return false;
+    if (gemm_run(ctx, run, w, m, false) != run) return false;
     const double kq = turq_gemm_kq_us(w[0]->dtype, w[0]->n * run, w[0]->k, m, ctx->compute_units);
-    return kq > 0.0 && kq < us;
+    return kq > 0.0 && kq < 1.09 * us;
 }
 
 // The next launch of a call with `left` weights to go.  As many neighbouring weights as one launch takes in about one round over the CUs (q, k
 // and v; k and v; gate and up of a small model): a launch of few tiles is mostly its start and its end (Q8_0 2 x 3072 x 1024 at 256 rows 21.1 ->
 // 11.1 us), and a second format costs a launch of gemm_cols.hip nothing.  All by the kernel that each takes alone, whose sums do not depend on the
 // launch: in gemm_cols.hip they are the same for every tile, in the one-round launches of gemm_kq_kernel asked here the low
-// tile keeps its wave groups and Q8_0 has one tile.  tile != 0: gemm_cols.hip's, kq: one of gemm_kq_kernel; neither: gemm_run() says.
+// tile keeps its wave groups and Q8_0 has one tile; except large weights of one shape (gemm_both_in_kq, gemm_run).  tile != 0: gemm_cols.hip's, kq: one of gemm_kq_kernel; neither: gemm_run() says.
 // cols[i]: gemm_cols.hip takes weight i alone; may_split: there is scratch for the parts of the first one's columns to meet in.
 // us: what gemm_cols.hip's launch takes, roughly.
 struct GemmNext { int run, tile, second; bool kq; double us; };
@@ -344,7 +346,7 @@ static GemmNext gemm_next(const turq_ctx *ctx, int left, const turq_weight *cons
         const int64_t n_cols = std::count(cols, cols + g.run, true);
         if (n_cols == g.run) g.tile = gemm_cols_tile(ctx, g.run, w, m, &g.second, &g.us);
         if (n_cols == 0) g.kq = gemm_run_pays(ctx, g.run, w, m);
-        // (gate and up, each of which gemm_cols.hip takes alone: one launch of gemm_kq_kernel over the rows of both where that is less)
+        // (large gate and up, each of which gemm_cols.hip takes alone)
         if (g.tile != 0 && gemm_both_in_kq(ctx, g.run, w, m, g.us)) {
             g.tile = 0;
             g.kq = true;
