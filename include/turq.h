@@ -367,16 +367,16 @@ int turq_profile_end(turq_ctx *ctx, int64_t *launches, double *total_ms);
 int turq_read_yardstick(turq_ctx *ctx, const void *dev_ptr, size_t nbytes);
 /* Which launch the rules for prompt chunks (more than 32 rows, K-quant or Q8_0 weights in the tiled layout) make for a weight of
  * n rows and k columns on a device with `compute_units` CUs; no GPU is needed and nothing is launched.  tile: 1 = 128 x 128,
- * 2 = 128 x 192 (Q8_0: 128 x 64), 3 = 128 x 256, 4 = 64 x 128 of the LDS-staged GEMM; 11, 21, 31, 22, 32, 23, 42: 10 r + c = 32 r x 32 c of
+ * 2 = 128 x 192 (Q8_0: 128 x 64), 3 = 128 x 256, 4 = 64 x 128 of the LDS-staged GEMM; 11, 21, 31, 22, 32, 23, 42, 33: 10 r + c = 32 r x 32 c of
  * the kernel whose waves split the columns, which launches of few tiles go through; split: workgroups that share the columns of
  * every tile (1: none); wave_groups: 2 where the 64 x 128 tile runs eight waves as two groups on alternate super-blocks.  Not part of the
  * path, no counterpart in the reference: for tests of the rules and for tuning them on another device. */
 int turq_prefill_plan(int dtype, int64_t n, int64_t k, int64_t m, int compute_units, int *tile, int *split, int *wave_groups);
 /* ... and whether turq_qmatmul_multi sends `count` (1 .. 4) neighbouring weights of that format and shape - gate_proj and up_proj -
  * out as ONE launch over the rows of all of them, with the tile and the kernel chosen for all the rows (merged = 1), or not (0: a launch each,
- * or, where each makes few tiles and for Q8_0, one launch of the kernel that each takes alone).  The rule compares how well the two
- * choices fill their rounds over the device's CUs, so the answer depends on compute_units; the kernels give the same products
- * either way (another order of the f32 sums where a tile's waves split k: within 2e-6). */
+ * or, where each makes few tiles and for Q8_0, one launch of the kernel that each takes alone).  Asked of the call's own rules, which compare
+ * how well the choices fill their rounds over the device's CUs and what they take, so the answer depends on compute_units; the kernels give the same products
+ * either way (another order of the f32 sums: within 2e-6). */
 int turq_prefill_plan_multi(int dtype, int64_t n, int64_t k, int64_t m, int count, int compute_units, int *merged);
 /* The environment switches that override the library's kernel-selection rules (names TURQ_*; for A/B timing and tests, none
  * is needed in production), as this process runs with them: one line per switch, "NAME=value  (default | set)  what it

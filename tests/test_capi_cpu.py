@@ -288,6 +288,18 @@ def test_prefill_launch_rules_on_a_256_cu_device():
     assert L.turq_prefill_plan(capi.F32, 4096, 4096, 64, 256, ctypes.byref(t), None, None) == capi.ERR_DTYPE
 
 
+@pytest.mark.parametrize("dt,n,k,m,count,merged", [
+    # gate and up at rows where the kernel whose waves split the columns takes both in one launch, and nearby where it does not
+    (capi.Q4_K, 12288, 4096, 77, 2, 0), (capi.Q5_K, 12288, 4096, 96, 2, 0), (capi.Q4_K, 12288, 4096, 180, 2, 0), (capi.Q4_K, 12544, 1536, 135, 2, 1),
+    (capi.Q5_K, 7168, 6144, 1190, 2, 1), (capi.Q6_K, 2560, 2048, 476, 2, 1),
+    # small weights: never in another kernel than alone
+    (capi.Q4_K, 1024, 1024, 1000, 3, 0), (capi.Q6_K, 1280, 3328, 1378, 2, 0)])
+def test_prefill_plan_of_several_weights_is_what_the_call_does(dt, n, k, m, count, merged):
+    g = ctypes.c_int(-1)
+    capi.check(capi.lib().turq_prefill_plan_multi(dt, n, k, m, count, 256, ctypes.byref(g)))
+    assert g.value == merged
+
+
 @pytest.mark.parametrize("dt,row_tiles", [(capi.Q4_K, 8), (capi.Q5_K, 8), (capi.Q6_K, 8), (capi.Q8_0, 6)])
 def test_prefill_columns_beyond_32_bit_offsets(dt, row_tiles):
     # a lane's offset to the last row tile of its workgroup has 32 bits: from the column count on where it would wrap the launch belongs to the

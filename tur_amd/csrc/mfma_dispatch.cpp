@@ -905,16 +905,27 @@ int turq_qmatmul_multi_mfma(turq_ctx *ctx, int count, const turq_weight *const *
     return TURQ_OK;
 }
 
-// whether turq_qmatmul_multi sends `count` neighbouring weights of this format and shape out as one prefill launch whose tile is chosen for
-// all the rows (no GPU needed; Q8_0 weights only go together in the kernel and the tile order that each takes alone)
+// whether turq_qmatmul_multi sends `count` neighbouring weights of this format and shape out as one prefill launch whose kernel and tile are
+// chosen for all the rows: its own rules, asked for a context of that many CUs (no GPU needed; Q8_0 weights, and launches of the kernel that
+// each takes alone, keep the sums of the single calls and are not meant)
 extern "C" int turq_prefill_plan_multi(int dtype, int64_t n, int64_t k, int64_t m, int count, int compute_units, int *merged) {
     if (merged) *merged = 0;
     if (!turq_dt_is_quant(dtype)) return turq_fail(nullptr, TURQ_ERR_DTYPE, "turq_prefill_plan_multi: dtype %d has no prefill kernel", dtype);
     if (n <= 0 || k <= 0 || k % 256 != 0 || m <= TURQ_GEMV_MAX_M || compute_units <= 0 || count < 1 || count > 4)
         return turq_fail(nullptr, TURQ_ERR_SHAPE, "turq_prefill_plan_multi: n=%lld k=%lld m=%lld count=%d on %d compute units", (long long)n,
                          (long long)k, (long long)m, count, compute_units);
-    const int64_t alone = gemm_cus_taken_shape(compute_units, dtype, n, k, m, true);
-    if (merged) *merged = dtype != TURQ_Q8_0 && gemm_merge_rule(dtype, n, k, m, count, compute_units, alone) ? 1 : 0;
+    turq_ctx ctx;
+    ctx.compute_units = compute_units;
+    turq_weight one;
+    one.dtype = dtype;
+    one.n = n;
+    one.k = k;
+    const turq_weight *const w[4] = {&one, &one, &one, &one};
+    const bool alone = gemm_cols_tile(&ctx, 1, w, m, nullptr) != 0, cols[4] = {alone, alone, alone, alone};
+    const bool split = !alone && turq_gemm_split_scratch(dtype, n, k, m, compute_units, nullptr) != 0;
+    const GemmNext next = gemm_next(&ctx, count, w, cols, m, split);
+    const bool all = next.kq ? alone && next.run == count : next.tile == 0 && gemm_run(&ctx, count, w, m, split) == count;
+    if (merged) *merged = dtype != TURQ_Q8_0 && count >= 2 && all ? 1 : 0;
     return TURQ_OK;
 }
 
