@@ -300,6 +300,19 @@ def test_prefill_plan_of_several_weights_is_what_the_call_does(dt, n, k, m, coun
     assert g.value == merged
 
 
+@pytest.mark.parametrize("dt,n,k,m,tile", [
+    # 1000 rows and more against many columns: fragments that no L2 holds, which the smaller tiles read too often
+    (capi.Q4_K, 5128, 12800, 1577, 2), (capi.Q4_K, 5121, 7424, 1577, 2), (capi.Q5_K, 4779, 5632, 1783, 1), (capi.Q5_K, 4670, 7424, 1855, 1),
+    # ... which the larger ones do not, and launches of one round share
+    (capi.Q5_K, 4647, 9216, 1770, 42), (capi.Q6_K, 1365, 9216, 1455, 33), (capi.Q4_K, 1573, 2560, 1162, 22),
+    # one super-block
+    (capi.Q5_K, 14336, 256, 645, 1), (capi.Q5_K, 3072, 256, 954, 1), (capi.Q8_0, 18432, 256, 499, 2)])
+def test_prefill_tiles_beyond_the_fitted_sizes(dt, n, k, m, tile):
+    t = ctypes.c_int()
+    capi.check(capi.lib().turq_prefill_plan(dt, n, k, m, 256, ctypes.byref(t), None, None))
+    assert t.value == tile
+
+
 @pytest.mark.parametrize("dt,row_tiles", [(capi.Q4_K, 8), (capi.Q5_K, 8), (capi.Q6_K, 8), (capi.Q8_0, 6)])
 def test_prefill_columns_beyond_32_bit_offsets(dt, row_tiles):
     # a lane's offset to the last row tile of its workgroup has 32 bits: from the column count on where it would wrap the launch belongs to the

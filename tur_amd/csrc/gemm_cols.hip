@@ -556,14 +556,28 @@ static constexpr ColsCost kColsCost[] = {
 };
 static constexpr ColsCost kColsPair = {22, 3.84, {0.604, 0.707, 0.741, 0.715}, 0.42, 0.41, 0.25};  // two workgroups per CU
 
+// ... unless the activations are what takes the time: fragments larger than an XCD's 4 MB of L2 come from the memory side again for every 32 NT
+// rows of weights, and only the n-blocks that an XCD works on at a time share them.  In launches of several rounds of the smaller tiles that goes at
+// 2 (64 x 64: 2.4) TB/s for each such n-block and 6.8 at least (120 shapes of 40 .. 2040 rows in every tile: 32 x 32 took up to 2.5 times the line above
+// at 8 MB of fragments and more, 64 x 64 up to 1.5; from 96 x 64 on the line holds).  Q8_0 2 x 2560 x 5376 at 1953 rows: 64 x 64 241 us, 128 x 64 183.
+static double cols_frag_us(int tile, int64_t n_blocks, int64_t k, int64_t m, int64_t cus, double x) {
+    const double frag_mb = 2e-6 * (double)m * (double)k;
+    if (x <= 1.0 || frag_mb <= 4.2 || (tile / 10) * (tile % 10) > 4) return 0.0;
+    const int per_cu = tile == 22 ? 2 : 3;
+    const double at_once = (double)(cus / 8 * per_cu) / (double)((m + 32 * (tile / 10) - 1) / (32 * (tile / 10)));
+    return (double)n_blocks * frag_mb / std::max(6.8, (tile == 22 ? 2.4 : 2.0) * at_once);
+}
+
 static double cols_us(int tile, int dtype_a, int dtype_b, int count, const int64_t *n, int64_t k, int64_t m, int64_t cus) {
     const auto fmt = [](int dt) { return dt == TURQ_Q4_K ? 0 : dt == TURQ_Q5_K ? 1 : dt == TURQ_Q6_K ? 2 : 3; };
-    const double x = (double)cols_workgroups(tile, count, n, m) / (double)cus;
+    const int64_t wgs = cols_workgroups(tile, count, n, m);
+    const double x = (double)wgs / (double)cus;
     const ColsCost *c = &kColsPair;
     if (tile != 22 || x <= 1.0)
         for (const ColsCost &t : kColsCost)
             if (t.tile == tile) c = &t;
-    return turq_launch_model_us(c->base, std::max(c->per[fmt(dtype_a)], c->per[fmt(dtype_b)]) * (double)(k / 256), c->again, c->more, c->fill, x);
+    return std::max(turq_launch_model_us(c->base, std::max(c->per[fmt(dtype_a)], c->per[fmt(dtype_b)]) * (double)(k / 256), c->again, c->more, c->fill, x),
+                    cols_frag_us(tile, wgs / ((m + 32 * (tile / 10) - 1) / (32 * (tile / 10))), k, m, cus, x));
 }
 
 // The tile with which one weight goes through this kernel as far as single rounds over the CUs decide, 0: gemm_kq_kernel.
@@ -610,9 +624,12 @@ static int cols_tile_by_rounds(int dtype, int64_t n, int64_t k, int64_t m, int64
 // One weight: by the rounds, unless another tile's estimate over several rounds is a fifth (Q8_0: a quarter and a bit) below what that launch
 // takes: the estimates err by up to that much, and launches of more than one round are where the rounds alone misjudge (at 300 rows, 128 x 128 -> two
 // 64 x 64 workgroups per CU: Q4_K / Q5_K / Q6_K 6144 x 4096 36 / 42 / 40 -> 25 / 28 / 30 us, 6144 x 1024 13.3 / 15.0 / 14.6 -> 9.9 / 10.8 / 11.5; at 180
-// rows, 128 x 128 -> 96 x 96: Q5_K 12288 x 4096 45 -> 32).
+// rows, 128 x 128 -> 96 x 96: Q5_K 12288 x 4096 45 -> 32).  Not of one super-block, which is mostly epilogue and which the estimates were not
+// fitted to (Q5_K 14336 x 256 at 645 rows 26 us by the rounds, 35 by the estimates; Q8_0 4096 x 256 twice at 1001 rows 25 and 30; from two super-blocks
+// on the estimates are ahead in 9 of 10).
 // Several weights, each of which is this kernel's alone: together, by the estimates, where that is less than one after the other (gate and up of
-// an 8B model at 77 rows, Q5_K 2 x 12288 x 4096: 45 -> 34).
+// an 8B model at 77 rows, Q5_K 2 x 12288 x 4096: 45 -> 34), of Q8_0 also where they are up to 5 % above it (41 pairs of 1 - 2 rounds that the estimates
+// had up to 7 % above took 0.94 - 1.07 of that, on average 0.99).
 int turq_gemm_cols_tile(int dtype_a, int dtype_b, int count, const int64_t *n, int64_t k, int64_t m, int compute_units, double *us) {
     const TurqTuning &t = turq_tuning();
     const bool kq_forced = t.gemm_wide >= 0 || t.gemm_low >= 0 || t.gemm_split >= 0 || t.gemm_kgroups != 0 || t.gemm_grid_2x2 || t.gemm_merge >= 0;
@@ -630,13 +647,14 @@ int turq_gemm_cols_tile(int dtype_a, int dtype_b, int count, const int64_t *n, i
     if (count == 1) {
         best = cols_tile_by_rounds(dtype_a, n[0], k, m, cus, compute_units);
         best_us = best ? cols_us(best, dtype_a, dtype_a, 1, n, k, m, cus) : turq_gemm_kq_us(dtype_a, n[0], k, m, compute_units);
-        least = best_us / (dtype_a == TURQ_Q8_0 ? 1.27 : 1.2);
+        least = k < 512 ? 0.0 : best_us / (dtype_a == TURQ_Q8_0 ? 1.27 : 1.2);
     } else {
         for (int i = 0; i < count; i++) {
             double alone = 0.0;  // (of a mixed launch as if of the first format: the estimate only has to order)
             if (!turq_gemm_cols_tile(dtype_a, dtype_a, 1, n + i, k, m, compute_units, &alone)) return 0;
             least += alone;
         }
+        if (dtype_a == TURQ_Q8_0) least *= 1.05;
     }
     for (const ColsCost &c : kColsCost) {
         const double est = cols_us(c.tile, dtype_a, dtype_b, count, n, k, m, cus);

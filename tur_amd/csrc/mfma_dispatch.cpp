@@ -321,14 +321,14 @@ static bool gemm_run_pays(const turq_ctx *ctx, int run, const turq_weight *const
 
 // Whether `run` weights, each of which gemm_cols.hip takes alone and which it would take in one launch of `us`, go out as one launch of
 // gemm_kq_kernel after all, whose sums are in another order.  Only the large ones of gemm_run, which the contract of turq_qmatmul_multi excepts from the
-// bits of the single calls, and unless gemm_cols.hip's estimate is a twelfth below: of 57 such launches gemm_cols.hip took 0.96 - 1.22 of the other
-// kernel's time (on average 1.05; Q5_K 2 x 7168 x 6144 at 1190 rows 334 us for 275) where its estimate was between that and gemm_kq_kernel's, 0.73 - 1.01
-// (0.88; Q5_K 2 x 12288 x 4096 at 77 rows 34 for 45) where it was below.
+// bits of the single calls, and unless gemm_cols.hip's estimate is 4 % below: of 57 such launches gemm_cols.hip took 0.98 - 1.22 of the other kernel's
+// time (on average 1.06; Q5_K 2 x 7168 x 6144 at 1190 rows 334 us for 275) where its estimate was between that and gemm_kq_kernel's, 0.73 - 1.09
+// (0.91; Q5_K 2 x 12288 x 4096 at 77 rows 34 for 45) where it was below.
 static bool gemm_both_in_kq(const turq_ctx *ctx, int run, const turq_weight *const *w, int64_t m, double us) {
     if (turq_tuning().gemm_cols > 0 || turq_tuning().gemm_merge >= 0 || run < 2 || us <= 0.0 || w[0]->dtype == TURQ_Q8_0) return false;
     if (gemm_run(ctx, run, w, m, false) != run) return false;
     const double kq = turq_gemm_kq_us(w[0]->dtype, w[0]->n * run, w[0]->k, m, ctx->compute_units);
-    return kq > 0.0 && kq < 1.09 * us;
+    return kq > 0.0 && kq < 1.04 * us;
 }
 
 // The next launch of a call with `left` weights to go.  As many neighbouring weights as one launch takes in about one round over the CUs (q, k
