@@ -208,17 +208,36 @@ def test_prompt_chunks(gpu, dt_gu, dt_dn, m):
         gpu.release(w)
 
 
-@pytest.mark.parametrize("dt_gu,dt_dn,n_ff,k,m", [
-    (Q4_K, Q6_K, 2816, 512, 600), (Q4_K, Q5_K, 3328, 3072, 513), (Q4_K, Q8_0, 6400, 256, 545), (Q5_K, Q6_K, 2816, 512, 600),
-    (Q5_K, Q4_K, 6400, 256, 513), (Q6_K, Q6_K, 2816, 512, 600), (Q6_K, Q8_0, 6400, 256, 513), (Q8_0, Q8_0, 3328, 1024, 2017),
-    (Q8_0, Q4_K, 3328, 1024, 2017),
-    # the kernel whose waves split the columns, by tiles: 32 x 32, 64 x 32, 64 x 64 alone and two per CU, 96 x 64, 128 x 64, 96 x 96
-    (Q4_K, Q6_K, 256, 256, 33), (Q4_K, Q6_K, 1280, 1024, 70), (Q5_K, Q6_K, 3328, 2048, 65), (Q8_0, Q8_0, 3072, 1024, 300),
-    (Q6_K, Q6_K, 5120, 4096, 77), (Q8_0, Q6_K, 5376, 3072, 100), (Q5_K, Q8_0, 12288, 4096, 77), (Q4_K, Q8_0, 4352, 4096, 190), (Q8_0, Q8_0, 2304, 1024, 47)])
-def test_prompt_pairs(gpu, dt_gu, dt_dn, n_ff, k, m):
-    """Gate and up in one launch that writes down_proj's fragments (the LDS-tiled kernel first: 128 x 128, 2 x 2 and wide tiles; blocks of n past the last row, rows
-    past m in the last 32; both fragment orders, with the sub-block sums of a Q4_K / Q5_K down_proj): bit-equal to the two calls.  The
-    scales of gate and up differ by 2^9, so that a column taken with the other's scale would show."""
+def launched_as_a_pair(gpu, n_ff, k, m):
+    """the fragments of down_proj go to memory of their own only from gate and up in one launch: the context's other buffer then holds those of x, for
+    which a new context took a quarter more than it needs"""
+    n = ctypes.c_size_t()
+    capi.check(gpu.L.turq_ctx_scratch_info(gpu.ctx, None, None, ctypes.byref(n)), gpu.ctx)
+    assert n_ff > k
+    return n.value < 68 * n_ff * ((m + 31) // 32) * 5 // 4
+
+
+# form: the tile of the LDS-tiled kernel (1: 128 x 128, 2: 2 x 2 waves, 3: wide); 0: the kernel whose waves split the columns
+@pytest.mark.parametrize("dt_gu,dt_dn,n_ff,k,m,form", [
+    (Q4_K, Q6_K, 2816, 512, 600, 1), (Q5_K, Q6_K, 2816, 512, 600, 1), (Q6_K, Q6_K, 2816, 512, 600, 1),
+    (Q4_K, Q5_K, 3840, 512, 513, 2), (Q4_K, Q6_K, 3840, 512, 513, 2), (Q4_K, Q4_K, 2816, 512, 700, 2), (Q4_K, Q8_0, 2816, 512, 700, 2),
+    (Q8_0, Q8_0, 3328, 1024, 2017, 2), (Q8_0, Q4_K, 3328, 1024, 2017, 2),
+    (Q4_K, Q8_0, 6400, 256, 545, 3), (Q5_K, Q4_K, 6400, 256, 513, 3), (Q6_K, Q8_0, 6400, 256, 513, 3),
+    # by tiles: 32 x 32, 64 x 32, 64 x 64 alone and two per CU, 96 x 64, 128 x 64, 96 x 96
+    (Q4_K, Q6_K, 512, 256, 33, 0), (Q4_K, Q6_K, 1280, 1024, 70, 0), (Q8_0, Q8_0, 2304, 1024, 47, 0), (Q6_K, Q6_K, 3072, 1024, 33, 0),
+    (Q8_0, Q8_0, 2304, 1024, 174, 0), (Q8_0, Q8_0, 3072, 1024, 300, 0), (Q4_K, Q8_0, 4352, 4096, 190, 0), (Q6_K, Q6_K, 5120, 4096, 77, 0),
+    (Q8_0, Q6_K, 5376, 3072, 100, 0), (Q5_K, Q8_0, 12288, 4096, 77, 0)])
+def test_prompt_pairs(dt_gu, dt_dn, n_ff, k, m, form):
+    """Gate and up in one launch that writes down_proj's fragments (blocks of n past the last row, rows past m in the last 32; both fragment orders,
+    with the sub-block sums of a Q4_K / Q5_K down_proj): bit-equal to the two calls.  The scales of gate and up differ by 2^9, so that a
+    column taken with the other's scale would show."""
+    both, alone, merged = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    L = capi.lib()
+    capi.check(L.turq_prefill_plan(dt_gu, 2 * n_ff, k, m, 256, ctypes.byref(both), None, None))
+    capi.check(L.turq_prefill_plan(dt_gu, n_ff, k, m, 256, ctypes.byref(alone), None, None))
+    capi.check(L.turq_prefill_plan_multi(dt_gu, n_ff, k, m, 2, 256, ctypes.byref(merged)))
+    assert (merged.value == 1 or alone.value <= 4) == (form != 0) and (form == 0 or both.value == form)
+    gpu = Gpu()
     n_out = 512
     raws = [synth.random_weight(dt_gu, n_ff, k, seed=7), synth.random_weight(dt_gu, n_ff, k, seed=8), synth.random_weight(dt_dn, n_out, n_ff, seed=9)]
     nb = synth.BLOCK_BYTES[dt_gu]
@@ -232,9 +251,73 @@ def test_prompt_pairs(gpu, dt_gu, dt_dn, n_ff, k, m):
     x = rng.standard_normal((m, k)).astype(np.float32) * XS
     for bs in ((None, None, None), tuple(rng.standard_normal(n).astype(np.float32) * 0.1 for n in (n_ff, n_ff, n_out))):
         y = gpu.mlp(*ws, x, n_ff, k, n_out, biases=bs)
+        assert bs[0] is not None or launched_as_a_pair(gpu, n_ff, k, m)
         assert np.array_equal(y, two_calls(gpu, ws, x, n_ff, k, n_out, biases=bs))
     for w in ws:
         gpu.release(w)
+    gpu.close()
+
+
+# the second kernel's pair at the edges of its tiles: columns of one and of several blocks, super-blocks fewer than waves and not a multiple of them, rows
+# at and past every tile's height; and with each of its tiles forced
+@pytest.mark.parametrize("dt", [Q4_K, Q5_K, Q6_K, Q8_0])
+@pytest.mark.parametrize("n_ff,k,m", [(512, 256, 33), (768, 512, 96), (1536, 1280, 65), (512, 256, 129)])
+def test_column_pair_edges(dt, n_ff, k, m):
+    gpu = Gpu()
+    raws, ws = weights(gpu, dt, Q6_K if dt != Q6_K else Q8_0, n_ff, k, 256, seed=31)
+    x = synth.random_activation(m, k, seed=m) * XS
+    y = gpu.mlp(*ws, x, n_ff, k, 256)
+    assert launched_as_a_pair(gpu, n_ff, k, m)
+    assert np.array_equal(y, two_calls(gpu, ws, x, n_ff, k, 256))
+    assert rel_l2(y, expected(dt, Q6_K if dt != Q6_K else Q8_0, f16_round(x), *raws, n_ff, k, 256)) <= 1e-3
+    for w in ws:
+        gpu.release(w)
+    gpu.close()
+
+
+@pytest.mark.parametrize("tile", ["21", "22", "32", "42", "33"])
+def test_column_pair_tiles(tile):
+    import os
+    import subprocess
+    import sys
+
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    out = subprocess.run([sys.executable, "-m", "pytest", "-q", "-x", "-m", "gpu", "-k", "test_column_pair_edges", "-p", "no:cacheprovider",
+                          os.path.join(root, "tests", "test_gpu_mlp.py")],
+                         cwd=root, env=dict(os.environ, TURQ_GEMM_COLS=tile), capture_output=True, text=True, timeout=280)
+    assert out.returncode == 0, out.stdout[-3000:] + out.stderr[-1000:]
+
+
+@pytest.mark.parametrize("dt_gu,dt_dn,n_ff,k,m", [(Q4_K, Q6_K, 2816, 512, 600), (Q5_K, Q4_K, 6400, 256, 513), (Q8_0, Q8_0, 3328, 1024, 2017), (Q4_K, Q6_K, 1280, 1024, 70)])
+def test_overflow_inside_a_pair_is_counted(dt_gu, dt_dn, n_ff, k, m):
+    """Rows whose gate or up product, or whose SiLU(gate) * up as f16, is no finite number: the same infinities and NaNs as from the two calls in the same
+    rows, the other rows as if they were alone, and the count sees each kind by itself."""
+    gpu = Gpu()
+
+    def counted():
+        n = ctypes.c_uint64()
+        capi.check(gpu.L.turq_ctx_nonfinite_count(gpu.ctx, ctypes.byref(n), 1), gpu.ctx)
+        return n.value
+
+    _, ws = weights(gpu, dt_gu, dt_dn, n_ff, k, 256, seed=41)
+    ok = synth.random_activation(m, k, seed=m) * XS
+    counted()
+    y_ok = gpu.mlp(*ws, ok, n_ff, k, 256)
+    assert launched_as_a_pair(gpu, n_ff, k, m) and np.isfinite(y_ok).all() and counted() == 0
+    for row, scale in ((m - 1, 3e3), (5, np.inf), (m // 2, np.nan)):  # finite products too large for f16 together; and none
+        x = ok.copy()
+        x[row, 3 if not np.isfinite(scale) else slice(None)] = scale if not np.isfinite(scale) else ok[row] * scale
+        y = gpu.mlp(*ws, x, n_ff, k, 256)
+        assert counted() > 0, scale
+        assert not np.isfinite(y[row]).any()
+        others = np.arange(m) != row
+        assert np.array_equal(y[others], y_ok[others])
+        two = two_calls(gpu, ws, x, n_ff, k, 256)
+        assert np.array_equal(np.isnan(y[row]), np.isnan(two[row])) and np.array_equal(y[row][~np.isnan(y[row])], two[row][~np.isnan(two[row])])
+        counted()
+    for w in ws:
+        gpu.release(w)
+    gpu.close()
 
 
 @pytest.mark.parametrize("dt_gu,dt_dn,n_ff,k,m,places", [

@@ -702,8 +702,10 @@ int turq_gemm_cols_pair_tile(int dtype, int down_dtype, int64_t n, int64_t k, in
     if (!turq_dt_is_quant(dtype) || (down_dtype != TURQ_Q6_K && down_dtype != TURQ_Q8_0)) return 0;
     if (n <= 0 || n % 256 != 0 || k <= 0 || k % 256 != 0 || m <= 0) return 0;
     const int64_t n2 = 2 * n;
+    const int forced = turq_tuning().gemm_cols;
     int best = 0;
     for (const int tile : kPairTiles) {
+        if (forced > 0 && tile != forced) continue;
         const double est = cols_us(tile, dtype, dtype, 1, &n2, k, m, compute_units > 0 ? compute_units : 256);
         if (!best || est < *us) {
             best = tile;

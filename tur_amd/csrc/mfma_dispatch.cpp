@@ -375,7 +375,7 @@ static int gemm_pair(const turq_ctx *ctx, const turq_weight *const *gu, int down
     if (g.tile != 0) {
         double us = 0.0;
         const int tile = turq_gemm_cols_pair_tile(dt, down_dtype, n, k, m, cus, &us);
-        return tile != 0 && us < (g.run == 2 ? g.us : 2.0 * g.us) + 4.0 ? tile : 0;
+        return tile != 0 && (t.gemm_cols > 0 || us < (g.run == 2 ? g.us : 2.0 * g.us) + 4.0) ? tile : 0;
     }
     if (!turq_gemm_pair_takes(dt, n, k, m, cus)) return 0;
     const bool plain = g.kq || gemm_run(ctx, 2, gu, m, split) == 2 || (!split && !(turq_gemm_form(dt, n, k, m, cus) == 4 && turq_gemm_low_two_groups(n, k, m, 1, cus)));

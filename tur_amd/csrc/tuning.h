@@ -41,7 +41,7 @@
     X(gemm_low, "TURQ_GEMM_LOW", TRI, -1, "prefill: the low tile 64 x 128 always (1) or never (0)")                                         \
     X(gemm_split, "TURQ_GEMM_SPLIT", INT, -1, "prefill: workgroups per tile that share its columns (0 / 1: never split)")                   \
     X(gemm_kgroups, "TURQ_GEMM_KGROUPS", INT, 0, "prefill low tile: 1 four waves, 2 eight waves as two groups")                             \
-    X(gemm_cols, "TURQ_GEMM_COLS", INT, -1, "prefill kernel whose waves split the columns: 0 never, 11 21 31 22 32 23 42 always in that tile")  \
+    X(gemm_cols, "TURQ_GEMM_COLS", INT, -1, "prefill kernel whose waves split the columns: 0 never, 11 21 31 22 32 23 42 33 always in that tile")  \
     X(prefetch_wgs, "TURQ_PREFETCH_WGS", INT, 0, "workgroups of turq_weight_prefetch (1 .. 4096)")                                          \
     X(prefetch_depth, "TURQ_PREFETCH_DEPTH", INT, 0, "4 KiB chunks in flight per wave of turq_weight_prefetch (1 .. 4)")
 
