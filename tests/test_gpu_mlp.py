@@ -208,36 +208,27 @@ def test_prompt_chunks(gpu, dt_gu, dt_dn, m):
         gpu.release(w)
 
 
-def launched_as_a_pair(gpu, n_ff, k, m):
-    """the fragments of down_proj go to memory of their own only from gate and up in one launch: the context's other buffer then holds those of x, for
-    which a new context took a quarter more than it needs"""
-    n = ctypes.c_size_t()
-    capi.check(gpu.L.turq_ctx_scratch_info(gpu.ctx, None, None, ctypes.byref(n)), gpu.ctx)
-    assert n_ff > k
-    return n.value < 68 * n_ff * ((m + 31) // 32) * 5 // 4
+def pair_plan(dt_gu, dt_dn, n_ff, k, m):
+    """the pair that the call's rules make of gate and up: a tile of the kernel whose waves split the columns, minus the tile form of the other, 0: none"""
+    f = capi.lib().turq_mlp_pair_plan
+    f.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int]
+    return f(dt_gu, dt_dn, n_ff, k, m, 256)
 
 
-# form: the tile of the LDS-tiled kernel (1: 128 x 128, 2: 2 x 2 waves, 3: wide); 0: the kernel whose waves split the columns
-@pytest.mark.parametrize("dt_gu,dt_dn,n_ff,k,m,form", [
-    (Q4_K, Q6_K, 2816, 512, 600, 1), (Q5_K, Q6_K, 2816, 512, 600, 1), (Q6_K, Q6_K, 2816, 512, 600, 1),
-    (Q4_K, Q5_K, 3840, 512, 513, 2), (Q4_K, Q6_K, 3840, 512, 513, 2), (Q4_K, Q4_K, 2816, 512, 700, 2), (Q4_K, Q8_0, 2816, 512, 700, 2),
-    (Q8_0, Q8_0, 3328, 1024, 2017, 2), (Q8_0, Q4_K, 3328, 1024, 2017, 2),
-    (Q4_K, Q8_0, 6400, 256, 545, 3), (Q5_K, Q4_K, 6400, 256, 513, 3), (Q6_K, Q8_0, 6400, 256, 513, 3),
-    # by tiles: 32 x 32, 64 x 32, 64 x 64 alone and two per CU, 96 x 64, 128 x 64, 96 x 96
-    (Q4_K, Q6_K, 512, 256, 33, 0), (Q4_K, Q6_K, 1280, 1024, 70, 0), (Q8_0, Q8_0, 2304, 1024, 47, 0), (Q6_K, Q6_K, 3072, 1024, 33, 0),
-    (Q8_0, Q8_0, 2304, 1024, 174, 0), (Q8_0, Q8_0, 3072, 1024, 300, 0), (Q4_K, Q8_0, 4352, 4096, 190, 0), (Q6_K, Q6_K, 5120, 4096, 77, 0),
-    (Q8_0, Q6_K, 5376, 3072, 100, 0), (Q5_K, Q8_0, 12288, 4096, 77, 0)])
-def test_prompt_pairs(dt_gu, dt_dn, n_ff, k, m, form):
+# pair: minus the tile form of the LDS-tiled kernel (1: 128 x 128, 2: 2 x 2 waves, 3: wide), or 10 r + c: 32 r x 32 c of the other (22 alone and two per CU)
+@pytest.mark.parametrize("dt_gu,dt_dn,n_ff,k,m,pair", [
+    (Q4_K, Q6_K, 2816, 512, 600, -1), (Q5_K, Q6_K, 2816, 512, 600, -1), (Q6_K, Q6_K, 2816, 512, 600, -1),
+    (Q4_K, Q5_K, 3840, 512, 513, -2), (Q4_K, Q6_K, 3840, 512, 513, -2), (Q4_K, Q4_K, 2816, 512, 700, -2), (Q4_K, Q8_0, 2816, 512, 700, -2),
+    (Q8_0, Q8_0, 3328, 1024, 2017, -2), (Q8_0, Q4_K, 3328, 1024, 2017, -2),
+    (Q4_K, Q8_0, 6400, 256, 545, -3), (Q5_K, Q4_K, 6400, 256, 513, -3), (Q6_K, Q8_0, 6400, 256, 513, -3),
+    (Q4_K, Q6_K, 256, 256, 33, 11), (Q4_K, Q6_K, 1280, 1024, 70, 11), (Q8_0, Q8_0, 2304, 1024, 47, 11), (Q6_K, Q6_K, 3072, 1024, 33, 21),
+    (Q8_0, Q8_0, 2304, 1024, 174, 22), (Q8_0, Q8_0, 3072, 1024, 300, 22), (Q4_K, Q8_0, 4352, 4096, 190, 22), (Q6_K, Q6_K, 5120, 4096, 77, 32),
+    (Q8_0, Q6_K, 5376, 3072, 100, 42), (Q5_K, Q8_0, 12288, 4096, 77, 33)])
+def test_prompt_pairs(gpu, dt_gu, dt_dn, n_ff, k, m, pair):
     """Gate and up in one launch that writes down_proj's fragments (blocks of n past the last row, rows past m in the last 32; both fragment orders,
     with the sub-block sums of a Q4_K / Q5_K down_proj): bit-equal to the two calls.  The scales of gate and up differ by 2^9, so that a
     column taken with the other's scale would show."""
-    both, alone, merged = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
-    L = capi.lib()
-    capi.check(L.turq_prefill_plan(dt_gu, 2 * n_ff, k, m, 256, ctypes.byref(both), None, None))
-    capi.check(L.turq_prefill_plan(dt_gu, n_ff, k, m, 256, ctypes.byref(alone), None, None))
-    capi.check(L.turq_prefill_plan_multi(dt_gu, n_ff, k, m, 2, 256, ctypes.byref(merged)))
-    assert (merged.value == 1 or alone.value <= 4) == (form != 0) and (form == 0 or both.value == form)
-    gpu = Gpu()
+    assert pair_plan(dt_gu, dt_dn, n_ff, k, m) == pair
     n_out = 512
     raws = [synth.random_weight(dt_gu, n_ff, k, seed=7), synth.random_weight(dt_gu, n_ff, k, seed=8), synth.random_weight(dt_dn, n_out, n_ff, seed=9)]
     nb = synth.BLOCK_BYTES[dt_gu]
@@ -251,28 +242,28 @@ def test_prompt_pairs(dt_gu, dt_dn, n_ff, k, m, form):
     x = rng.standard_normal((m, k)).astype(np.float32) * XS
     for bs in ((None, None, None), tuple(rng.standard_normal(n).astype(np.float32) * 0.1 for n in (n_ff, n_ff, n_out))):
         y = gpu.mlp(*ws, x, n_ff, k, n_out, biases=bs)
-        assert bs[0] is not None or launched_as_a_pair(gpu, n_ff, k, m)
         assert np.array_equal(y, two_calls(gpu, ws, x, n_ff, k, n_out, biases=bs))
     for w in ws:
         gpu.release(w)
-    gpu.close()
 
 
 # the second kernel's pair at the edges of its tiles: columns of one and of several blocks, super-blocks fewer than waves and not a multiple of them, rows
 # at and past every tile's height; and with each of its tiles forced
 @pytest.mark.parametrize("dt", [Q4_K, Q5_K, Q6_K, Q8_0])
 @pytest.mark.parametrize("n_ff,k,m", [(512, 256, 33), (768, 512, 96), (1536, 1280, 65), (512, 256, 129)])
-def test_column_pair_edges(dt, n_ff, k, m):
-    gpu = Gpu()
+def test_column_pair_edges(gpu, dt, n_ff, k, m):
+    import os
+
+    forced = int(os.environ.get("TURQ_GEMM_COLS", "0"))
+    pair = pair_plan(dt, Q6_K if dt != Q6_K else Q8_0, n_ff, k, m)
+    assert pair == forced if forced else pair > 0
     raws, ws = weights(gpu, dt, Q6_K if dt != Q6_K else Q8_0, n_ff, k, 256, seed=31)
     x = synth.random_activation(m, k, seed=m) * XS
     y = gpu.mlp(*ws, x, n_ff, k, 256)
-    assert launched_as_a_pair(gpu, n_ff, k, m)
     assert np.array_equal(y, two_calls(gpu, ws, x, n_ff, k, 256))
     assert rel_l2(y, expected(dt, Q6_K if dt != Q6_K else Q8_0, f16_round(x), *raws, n_ff, k, 256)) <= 1e-3
     for w in ws:
         gpu.release(w)
-    gpu.close()
 
 
 @pytest.mark.parametrize("tile", ["21", "22", "32", "42", "33"])
@@ -289,10 +280,10 @@ def test_column_pair_tiles(tile):
 
 
 @pytest.mark.parametrize("dt_gu,dt_dn,n_ff,k,m", [(Q4_K, Q6_K, 2816, 512, 600), (Q5_K, Q4_K, 6400, 256, 513), (Q8_0, Q8_0, 3328, 1024, 2017), (Q4_K, Q6_K, 1280, 1024, 70)])
-def test_overflow_inside_a_pair_is_counted(dt_gu, dt_dn, n_ff, k, m):
+def test_overflow_inside_a_pair_is_counted(gpu, dt_gu, dt_dn, n_ff, k, m):
     """Rows whose gate or up product, or whose SiLU(gate) * up as f16, is no finite number: the same infinities and NaNs as from the two calls in the same
     rows, the other rows as if they were alone, and the count sees each kind by itself."""
-    gpu = Gpu()
+    assert pair_plan(dt_gu, dt_dn, n_ff, k, m) != 0
 
     def counted():
         n = ctypes.c_uint64()
@@ -303,7 +294,7 @@ def test_overflow_inside_a_pair_is_counted(dt_gu, dt_dn, n_ff, k, m):
     ok = synth.random_activation(m, k, seed=m) * XS
     counted()
     y_ok = gpu.mlp(*ws, ok, n_ff, k, 256)
-    assert launched_as_a_pair(gpu, n_ff, k, m) and np.isfinite(y_ok).all() and counted() == 0
+    assert np.isfinite(y_ok).all() and counted() == 0
     for row, scale in ((m - 1, 3e3), (5, np.inf), (m // 2, np.nan)):  # finite products too large for f16 together; and none
         x = ok.copy()
         x[row, 3 if not np.isfinite(scale) else slice(None)] = scale if not np.isfinite(scale) else ok[row] * scale
@@ -317,7 +308,6 @@ def test_overflow_inside_a_pair_is_counted(dt_gu, dt_dn, n_ff, k, m):
         counted()
     for w in ws:
         gpu.release(w)
-    gpu.close()
 
 
 @pytest.mark.parametrize("dt_gu,dt_dn,n_ff,k,m,places", [
@@ -347,3 +337,38 @@ def test_one_weight_in_several_places(gpu, dt_gu, dt_dn, n_ff, k, m, places):
     assert rel_l2(y, expected(dt_gu, dt_dn, f16_round(x), *raws, n_ff, k, n_out)) <= 3e-3
     for raw, w in made.values():
         gpu.release(w)
+
+
+def test_scratch_of_more_rows_serves_a_capture_of_fewer():
+    """540 rows take gate and up as a pair, 500 take the two products through memory: what the first call left behind is enough for a capture of the
+    second, in which nothing may be allocated"""
+    gpu = Gpu()
+    n_ff, k, n_out, big, small = 4096, 1024, 256, 540, 500
+    assert pair_plan(Q4_K, Q4_K, n_ff, k, big) != 0 and pair_plan(Q4_K, Q4_K, n_ff, k, small) == 0
+    _, ws = weights(gpu, Q4_K, Q4_K, n_ff, k, n_out, seed=43)
+    L, ctx = gpu.L, gpu.ctx
+    x, y = gpu.dev_buffer(synth.random_activation(big, k, seed=2) * XS), gpu.dev_buffer(np.zeros((big, n_out), np.float32))
+
+    def call(m):
+        capi.check(L.turq_mlp(ctx, *ws, x, capi.ACT_F32, m, k, y, capi.ACT_F32, n_out, None, None, None, 0, capi.MEM_DEVICE), ctx)
+
+    call(big)
+    capi.check(L.turq_sync(ctx), ctx)
+    capi.check(L.turq_graph_begin(ctx), ctx)
+    call(small)
+    g = ctypes.c_void_p()
+    capi.check(L.turq_graph_end(ctx, ctypes.byref(g)), ctx)
+    call(small)
+    want = gpu.read_back(y, (small, n_out), np.float32)
+    for _ in range(3):
+        call(big)
+        capi.check(L.turq_memcpy_h2d(ctx, y, capi.ptr(np.zeros((small, n_out), np.float32)), 4 * small * n_out), ctx)
+        capi.check(L.turq_graph_launch(ctx, g), ctx)
+        capi.check(L.turq_sync(ctx), ctx)
+        assert np.array_equal(gpu.read_back(y, (small, n_out), np.float32), want)
+    L.turq_graph_destroy(g)
+    for p in (x, y):
+        gpu.dev_free(p)
+    for w in ws:
+        gpu.release(w)
+    gpu.close()

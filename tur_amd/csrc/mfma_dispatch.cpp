@@ -532,11 +532,15 @@ int turq_mlp_prefill(turq_ctx *ctx, const turq_weight *gate, const turq_weight *
     if (ldx < gate->k || ldy < down->n || !turq_act_bytes(xt) || !turq_act_bytes(yt)) return TURQ_OK;
     if (turq_rows_in_chunks(ctx, 2, gu, x, xt, ldx, m)) return TURQ_OK;  // gate / up through the kernels of up to 32 rows
     const int64_t n_ff = gate->n;
+    // One fragment buffer serves both preparations, sized for the larger before anything is queued.  Sized alike for every route below (the pair's
+    // fragments take less than the two products, and x's less than the intermediate's): a call of fewer rows, whatever its route, then finds the
+    // scratch of one of more rows enough, which matters where nothing may be allocated - in a capture.
+    const size_t half = (size_t)m * (size_t)n_ff;
+    int rc = turq_ctx_reserve(ctx, &ctx->gate_up, &ctx->gate_up_cap, std::max(2 * half * sizeof(float) + 16, turq_act_prep32_bytes(m, n_ff)));
+    if (rc != TURQ_OK) return rc;
+    rc = turq_ctx_reserve(ctx, &ctx->act_prep, &ctx->act_prep_cap, std::max(turq_act_prep32_bytes(m, gate->k), turq_act_prep32_bytes(m, n_ff)));
+    if (rc != TURQ_OK) return rc;
     if (const int pair = !norm || gate->k <= 16384 ? gemm_pair(ctx, gu, down->dtype, m) : 0) {
-        int rc = turq_ctx_reserve(ctx, &ctx->gate_up, &ctx->gate_up_cap, turq_act_prep32_bytes(m, n_ff));
-        if (rc != TURQ_OK) return rc;
-        rc = turq_ctx_reserve(ctx, &ctx->act_prep, &ctx->act_prep_cap, turq_act_prep32_bytes(m, gate->k));
-        if (rc != TURQ_OK) return rc;
         TURQ_HIP(ctx, norm ? turq_launch_rms_norm_prep32(gate->dtype, x, xt, m, gate->k, ldx, norm->w, norm->eps, ctx->act_prep, ctx->stream)
                            : turq_launch_act_prep32(gate->dtype, x, xt, m, gate->k, ldx, ctx->act_prep, ctx->stream));
         void *const ys[2] = {ctx->gate_up, nullptr};
@@ -554,12 +558,6 @@ int turq_mlp_prefill(turq_ctx *ctx, const turq_weight *gate, const turq_weight *
         *taken = true;
         return TURQ_OK;
     }
-    const size_t half = (size_t)m * (size_t)n_ff;
-    int rc = turq_ctx_reserve(ctx, &ctx->gate_up, &ctx->gate_up_cap, 2 * half * sizeof(float) + 16);
-    if (rc != TURQ_OK) return rc;
-    // one fragment buffer serves both preparations: sized for the larger before anything is queued
-    rc = turq_ctx_reserve(ctx, &ctx->act_prep, &ctx->act_prep_cap, std::max(turq_act_prep32_bytes(m, gate->k), turq_act_prep32_bytes(m, n_ff)));
-    if (rc != TURQ_OK) return rc;
     void *ys[2] = {ctx->gate_up, (float *)ctx->gate_up + half};
     const int64_t ldys[2] = {n_ff, n_ff};
     const float *biases[2] = {bias_gate, bias_up};
@@ -927,6 +925,21 @@ extern "C" int turq_prefill_plan_multi(int dtype, int64_t n, int64_t k, int64_t 
     const bool all = next.kq ? alone && next.run == count : next.tile == 0 && gemm_run(&ctx, count, w, m, split) == count;
     if (merged) *merged = dtype != TURQ_Q8_0 && count >= 2 && all ? 1 : 0;
     return TURQ_OK;
+}
+
+// For tests of the rules (not part of the C ABI): the pair that turq_mlp makes of gate and up on a device of that many CUs: the tile of
+// gemm_cols.hip, minus the tile form of gemm_kq_kernel, 0: none
+extern "C" int turq_mlp_pair_plan(int dtype, int down_dtype, int64_t n_ff, int64_t k, int64_t m, int compute_units) {
+    if (!turq_dt_is_quant(dtype) || n_ff <= 0 || k <= 0 || k % 256 != 0 || m <= TURQ_GEMV_MAX_M || compute_units <= 0) return 0;
+    turq_ctx ctx;
+    ctx.compute_units = compute_units;
+    turq_weight one;
+    one.dtype = dtype;
+    one.n = n_ff;
+    one.k = k;
+    const turq_weight *const gu[2] = {&one, &one};
+    const int pair = gemm_pair(&ctx, gu, down_dtype, m);
+    return pair == kGemmPairKq ? -turq_gemm_form(dtype, 2 * n_ff, k, m, compute_units) : pair;
 }
 
 // which launch the rules above, in gemm_cols.hip and in gemm_mfma.hip make for a prompt chunk (no GPU needed)
