@@ -95,7 +95,7 @@ template <> struct WBlk<TURQ_Q8_0> {
 template <int MT> struct AStage { half8v f[MT][4]; };
 
 // Four waves in every tile shape and form, and (first form) one stage of fragments in flight besides the one being used.  The sums of a result are then the
-// same numbers in the same order whatever the tile (a weight alone and in a launch with others agree to the bit).  Eight waves were up
+// same numbers in the same order whatever the tile (a weight alone and in a launch of this kernel with others agree to the bit).  Eight waves were up
 // to 7 % faster on the 64-row tile and spill on the larger ones; three stages in flight measured 1 - 8 % slower than one (registers).
 constexpr int W = 4, RA = 2;
 // The waves meet in rounds of T tiles, rows of kPitch floats (rows r and r + 4, which a store of a wave writes, lie 16 banks apart).
@@ -109,7 +109,8 @@ template <int MT, int NT> struct Meet {
 // PAIR: gate and up of an MLP (weights 0 and 1, one shape), which take turns by 16-row tiles, and SiLU(gate) * up as down_proj's activation fragments
 // for results: see gemm_kq_kernel, whose pair does the same.  The halves of a 32-column MFMA tile are the two products of the same 16 columns, so a
 // lane's weights are those of one of the two, which takes a 64-bit address per 32-row tile.  Without the sub-block sums of the fragments, whose 32
-// columns may be two workgroups': for a down_proj of Q6_K or Q8_0, which read none.  These launches are 6 - 35 us, and what the pair saves is the
+// columns are two workgroups' in tiles of 32 and 96 rows of weights: for a down_proj of Q6_K or Q8_0, which read none (with Q4_K and Q5_K the products go
+// through memory, also where a tile of 64 would hold whole sub-blocks).  These launches are 6 - 35 us, and what the pair saves is the
 // 5 us launch between it and down_proj: whole MLPs Q8_0 1024 x 3072 at 34 / 300 rows 19.3 / 30.3 -> 16.5 / 25.0 us, Q5_K / Q6_K
 // 4096 x 12288 at 77 rows 66.6 -> 62.2, at 180 rows 108 -> 96; nowhere slower (4096 x 12288 .. 5120 x 15360, 34 - 600 rows, every format).
 template <int DT, int MT, int NT, bool TIGHT, bool PAIR>
@@ -583,7 +584,8 @@ static double cols_us(int tile, int dtype_a, int dtype_b, int count, const int64
 // The tile with which one weight goes through this kernel as far as single rounds over the CUs decide, 0: gemm_kq_kernel.
 // A launch of one round takes about base + per_sb * super-blocks, one line for every format; a further round costs as much again without the
 // launch itself, of the smallest tile, of which three workgroups share a CU, three fifths of it.  So the smallest tile that makes the launch one
-// round is the best of them.  Against gemm_kq_kernel:
+// round is taken, and the smallest of all up to one and a half (which at 1.5 is behind the one-round tile: Q6_K 4096 x 12288 at 65 - 96 rows 34.6 us against 27.5 of
+// 64 x 32, Q5_K 4096 x 4096 14.1 against 12.9).  Against gemm_kq_kernel:
 //   one or two MFMA tiles: Q4_K 1024 x 4096 at 40 / 300 / 512 rows 13.0 / 19.0 / 19.1 -> 6.6 / 9.3 / 10.7 us, 4096 x 4096 at 40 / 100 rows 19.2 /
 //   22.6 -> 8.7 / 11.3, Q6_K 4096 x 12288 33 / 43 -> 23 / 29, Q8_0 2048 x 2048 15 -> 5.4 / 5.5;
 //   three or four: K-quants from two super-blocks on (Q4_K 12288 x 256 at 48 rows 8.4 -> 9.4); Q8_0 2048 x 2048 at 300 / 512 rows 15.4 -> 8.5 / 10.2, Q4_K 4096 x 4096 at 256 24 -> 15;
