@@ -270,7 +270,7 @@ int turq_qmatmul_gate_up(turq_ctx *ctx, const turq_weight *gate, const turq_weig
 /* The reference's whole MLP in one call: y[m, n_out] = (act(x * gate^T + bias_gate) * (x * up^T + bias_up)) * down^T + bias_down.
  * gate and up are two weights of one shape [n_ff, k], down is [n_out, n_ff]; the intermediate lives in scratch memory of the
  * context (m * n_ff values; above 32 rows 8 bytes for each, enough for the two products, and the fragments of the wider of x and the intermediate;
- * it grows on demand, never inside a graph capture, and what a call of more rows left is enough for one of fewer).  The results are those of
+ * it grows on demand, never inside a graph capture).  The results are those of
  * turq_qmatmul_gate_up into an f32 buffer followed by turq_qmatmul on it, bit for bit, and so are the errors and the meaning of
  * x, y, the strides, the biases (NULL: none), `act` and `mem`.  (Where down_proj runs on the matrix cores - a tiled
  * quantized weight, wide activations off - its kernels round the activations to f16 first thing, so the intermediate is

@@ -533,8 +533,8 @@ int turq_mlp_prefill(turq_ctx *ctx, const turq_weight *gate, const turq_weight *
     if (turq_rows_in_chunks(ctx, 2, gu, x, xt, ldx, m)) return TURQ_OK;  // gate / up through the kernels of up to 32 rows
     const int64_t n_ff = gate->n;
     // One fragment buffer serves both preparations, sized for the larger before anything is queued.  Sized alike for every route below (the pair's
-    // fragments take less than the two products, and x's less than the intermediate's): a call of fewer rows, whatever its route, then finds the
-    // scratch of one of more rows enough, which matters where nothing may be allocated - in a capture.
+    // fragments take less than the two products, and x's less than the intermediate's): a call of fewer rows that takes another of them then finds
+    // the scratch of one of more rows enough, which matters where nothing may be allocated - in a capture.
     const size_t half = (size_t)m * (size_t)n_ff;
     int rc = turq_ctx_reserve(ctx, &ctx->gate_up, &ctx->gate_up_cap, std::max(2 * half * sizeof(float) + 16, turq_act_prep32_bytes(m, n_ff)));
     if (rc != TURQ_OK) return rc;
