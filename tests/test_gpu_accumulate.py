@@ -199,3 +199,24 @@ def test_the_flag_belongs_to_qmatmul_and_mlp(gpu):
     assert L.turq_qmatmul(ctx, w, capi.ptr(x), capi.ACT_F32, 1, 256, capi.ptr(y), capi.ACT_F32 | 0x200, 64, None, capi.MEM_HOST, capi.ALGO_AUTO) == capi.ERR_DTYPE
     assert L.turq_qmatmul(ctx, w, capi.ptr(x), capi.ACT_F32, 1, 256, capi.ptr(y), capi.ACT_F32 | ACC, 64, None, capi.MEM_HOST, capi.ALGO_AUTO) == capi.OK
     gpu.release(w)
+
+
+# The one-row kernels request the bias and the bits of the element they add to ahead of the sums, for the first result of a wave, and sum up
+# eight waves at a time: one wave (one column tile) with one result and with as many as there are activation rows or row tiles, nine waves of two
+# turns, eleven of three, rows that end inside a column tile, weight rows that end inside a row tile and (65544, two row tiles per
+# workgroup) inside a workgroup.  Products of f16-exact rows to 2e-5, as in test_one_row; the sum with y exact.
+@pytest.mark.parametrize("dt,n,k,m", [(Q8_0, 8, 256, 1), (Q4_K, 53, 4352, 1), (Q6_K, 48, 8448, 1), (Q8_0, 40, 8224, 1), (Q5_K, 65544, 256, 1),
+                                      (Q4_K, 65528, 256, 4), (Q5_K, 65528, 256, 3), (Q6_K, 65528, 256, 2)])
+def test_one_row_first_results(gpu, dt, n, k, m):
+    raw = synth.random_weight(dt, n, k, seed=n + k)
+    w = gpu.upload(dt, n, k, raw, capi.LAYOUT_TILED)
+    rng = np.random.default_rng(n + k + m)
+    x = synth.random_activation(m, k, seed=m + 5).astype(np.float16).astype(np.float32)
+    bias = rng.standard_normal(n).astype(np.float32)
+    plain = run(gpu, w, x, n, k, np.zeros((m, n), np.float32), capi.ACT_F32, 0, bias)
+    prod = orc.matmul_dequant(dt, x, raw, n, k)
+    assert np.linalg.norm(plain - bias - prod) <= 2e-5 * np.linalg.norm(prod) + 1e-7 * np.linalg.norm(bias)
+    for yt in (capi.ACT_F32, capi.ACT_BF16, capi.ACT_F16):
+        y0 = to_type(rng.standard_normal((m, n)), yt)
+        assert np.array_equal(run(gpu, w, x, n, k, y0, yt, ACC, bias), to_type(plain + y0, yt))
+    gpu.release(w)

@@ -30,6 +30,8 @@
 #include <cstdlib>
 
 #include <algorithm>
+#include <climits>
+#include <initializer_list>
 
 #include "layout.h"
 #include "mfma_common.h"
@@ -69,25 +71,27 @@ __device__ inline float dot2(half2v a, _Float16 b0, float c) { return __builtin_
 // raw activations of one tile: 4 consecutive columns per lane
 template <int XT> struct X1Regs { uint32_t r[XT == TURQ_ACT_F32 ? 4 : 2]; };
 
-// RAGGED: k may end inside the tile (Q8_0: a multiple of 32, four columns are in or out together); the K-quants' k is a
-// multiple of 256 and needs no test
-template <int XT, bool RAGGED>
-__device__ inline X1Regs<XT> load_x1(const void *__restrict__ x, int64_t k, int64_t b, int lane, const GOff &o) {
-    // x: the activation row (wave-uniform pointer)
+// The four columns of lane `lane` in column tile b of the activation row x (wave-uniform pointers).  RAGGED: k may end inside the tile (Q8_0: a
+// multiple of 32, four columns are in or out together); columns past k load the tile's first ones, stage as zeros
+// (in_tile).  The K-quants' k is a multiple of 256 and needs no test.
+template <int XT> __device__ inline X1Regs<XT> load_x1(const uint8_t *__restrict__ x, uint32_t b, const GOff &o, bool ok) {
     X1Regs<XT> v;
     constexpr int ES = XT == TURQ_ACT_F32 ? 4 : 2;
-    const bool ok = !RAGGED || b * 256 + 4 * lane < k;
     const uint32_t off = XT == TURQ_ACT_F32 ? o.o16 : o.o8;
-    const uint8_t *src = (const uint8_t *)x + b * (256 * ES) + (ok ? off : 0u);
-    if (RAGGED && !ok) src = (const uint8_t *)x;
+    const uint8_t *src = x + (uint64_t)b * (256 * ES) + (ok ? off : 0u);
     if constexpr (XT == TURQ_ACT_F32) {
         const uint4v t = *(const uint4v *)src;
-        v.r[0] = ok ? t.x : 0u; v.r[1] = ok ? t.y : 0u; v.r[2] = ok ? t.z : 0u; v.r[3] = ok ? t.w : 0u;
+        v.r[0] = t.x; v.r[1] = t.y; v.r[2] = t.z; v.r[3] = t.w;
     } else {
         const uint2v t = *(const uint2v *)src;
-        v.r[0] = ok ? t.x : 0u; v.r[1] = ok ? t.y : 0u;
+        v.r[0] = t.x; v.r[1] = t.y;
     }
     return v;
+}
+template <bool RAGGED> __device__ inline bool in_tile(int64_t k, uint32_t b, int lane) { return !RAGGED || 4 * lane < (int)(k - (int64_t)b * 256); }
+template <int XT> __device__ inline void drop_outside(X1Regs<XT> &v, bool ok) {
+#pragma unroll
+    for (uint32_t &r : v.r) r = ok ? r : 0u;
 }
 
 template <int XT>
@@ -108,7 +112,7 @@ __device__ inline void to_half4(const X1Regs<XT> &v, half2v &h01, half2v &h23) {
 //   Lane:   per-lane constants (LDS offsets of the A operand, header addressing)
 //   W:      what a lane loads from HBM for one tile
 //   sums(): what the accumulator starts from, from a lane's four staged columns (h01, h23), written to region + kInit
-//   chain(): the eight MFMA steps of a tile;  scales(): the tile's scale factors;
+//   step(), a_off(): the B operand of one of a tile's eight MFMA steps, and where its A operand lies;  scales(): the tile's scale factors;
 //   finish(): the scales on the result of the chain = the lane's contribution to its partial y
 template <int DT> struct Row1Fmt;
 
@@ -163,21 +167,8 @@ template <int DT> struct Row1K45 {
         }
         return make_half8(as_half2(t0), as_half2(t1), as_half2(t2), as_half2(t3));
     }
-    // M activation rows: their regions follow each other; every operand is unpacked once and used for all of them
-    template <int M> __device__ static void chain(const W &w, const uint8_t *reg, const Lane &l, int g, float4v *c) {
-#pragma unroll
-        for (int mm = 0; mm < M; mm++) c[mm] = *(const float4v *)(reg + mm * kRegion + kInit + 16 * g);
-        const uint32_t wq[8] = {w.qa.x, w.qa.y, w.qa.z, w.qa.w, w.qb.x, w.qb.y, w.qb.z, w.qb.w};
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const half8v bop = operand(wq[i], w.hh.x, w.hh.y, 2 * i);
-#pragma unroll
-            for (int mm = 0; mm < M; mm++) {
-                const half8v av = *(const half8v *)(reg + mm * kRegion + (i < 4 ? l.offA : l.offB) + 16 * (i & 3));
-                c[mm] = mfma16x16x32(av, bop, c[mm]);
-            }
-        }
-    }
+    __device__ static int a_off(const Lane &l, int i) { return (i < 4 ? l.offA : l.offB) + 16 * (i & 3); }
+    __device__ static half8v step(const W &w, int i) { return operand(i < 4 ? w.qa[i] : w.qb[i - 4], w.hh.x, w.hh.y, 2 * i); }
     // ---- packed form: two activation rows per chain.  A row R = 4 g' + 2 s + a carries sub-block 2 g' + s of activation row
     // a of the pair, so lane (n, g) of the result finds (sub-block 2g, row 0), (2g, row 1), (2g + 1, row 0), (2g + 1, row 1) in
     // its four registers; no row is left for sum(x), which the staging keeps in the LDS instead (kPSum, same index).
@@ -264,30 +255,20 @@ template <> struct Row1Fmt<TURQ_Q6_K> {
         const float nb = sum4(dot2(h23, (_Float16)-288.0f, dot2(h01, (_Float16)-288.0f, 0.0f)));
         if ((lane & 3) == 0) *(float *)(region + kInit + lane) = nb;
     }
-    template <int M> __device__ static void chain(const W &w, const uint8_t *reg, const Lane &l, int g, float4v *c) {
+    __device__ static int a_off(const Lane &l, int i) { return l.off[i >> 1] + 16 * (i & 1); }
+    __device__ static half8v step(const W &w, int i) {
+        const uint32_t wl = i < 4 ? w.qla[i] : w.qlb[i - 4], wh = w.qh[i >> 1];
+        // pair t of the step: the nibbles sit 4 t bits above mantissa bits 2..5, the two high bits 2 t + 8 (i % 2)
+        // bits above mantissa bits 6..7; together the 6-bit quant in the mantissa of 256.0 (ulp 1/4)
+        uint32_t v[4];
 #pragma unroll
-        for (int mm = 0; mm < M; mm++) c[mm] = *(const float4v *)(reg + mm * kRegion + kInit + 16 * g);
-        const uint32_t wl[8] = {w.qla.x, w.qla.y, w.qla.z, w.qla.w, w.qlb.x, w.qlb.y, w.qlb.z, w.qlb.w};
-        const uint32_t wh[4] = {w.qh.x, w.qh.y, w.qh.z, w.qh.w};
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            // pair t of the step: the nibbles sit 4 t bits above mantissa bits 2..5, the two high bits 2 t + 8 (i % 2)
-            // bits above mantissa bits 6..7; together the 6-bit quant in the mantissa of 256.0 (ulp 1/4)
-            uint32_t v[4];
-#pragma unroll
-            for (int t = 0; t < 4; t++) {
-                const uint32_t lo = t ? rotr32(wl[i], 4u * t) : wl[i];
-                const uint32_t rh = 2u * t + 8u * (i & 1);
-                const uint32_t hi = rh ? rotr32(wh[i >> 1], rh) : wh[i >> 1];
-                v[t] = and_or_u32(hi, 0x00C000C0u, and_or_u32(lo, 0x003C003Cu, kMagic256));
-            }
-            const half8v bop = make_half8(as_half2(v[0]), as_half2(v[1]), as_half2(v[2]), as_half2(v[3]));
-#pragma unroll
-            for (int mm = 0; mm < M; mm++) {
-                const half8v av = *(const half8v *)(reg + mm * kRegion + l.off[i >> 1] + 16 * (i & 1));
-                c[mm] = mfma16x16x32(av, bop, c[mm]);
-            }
+        for (int t = 0; t < 4; t++) {
+            const uint32_t lo = t ? rotr32(wl, 4u * t) : wl;
+            const uint32_t rh = 2u * t + 8u * (i & 1);
+            const uint32_t hi = rh ? rotr32(wh, rh) : wh;
+            v[t] = and_or_u32(hi, 0x00C000C0u, and_or_u32(lo, 0x003C003Cu, kMagic256));
         }
+        return make_half8(as_half2(v[0]), as_half2(v[1]), as_half2(v[2]), as_half2(v[3]));
     }
     struct Sc { float s[4]; float d; };
     __device__ static Sc scales(const W &w, const Lane &) {
@@ -331,21 +312,12 @@ template <> struct Row1Fmt<TURQ_Q8_0> {
         const float nb = sum8(dot2(h23, (_Float16)-1152.0f, dot2(h01, (_Float16)-1152.0f, 0.0f)));
         if ((lane & 7) == 0) *(float *)(region + kInit + (lane >> 1)) = nb;
     }
-    template <int M> __device__ static void chain(const W &w, const uint8_t *reg, const Lane &l, int g, float4v *c) {
-#pragma unroll
-        for (int mm = 0; mm < M; mm++) c[mm] = *(const float4v *)(reg + mm * kRegion + kInit + 16 * g);
-#pragma unroll
-        for (int q = 0; q < 8; q++) {
-            const uint32_t w0 = (q & 1) ? w.p[q >> 1].z : w.p[q >> 1].x;
-            const uint32_t w1 = (q & 1) ? w.p[q >> 1].w : w.p[q >> 1].y;
-            const half8v bop = make_half8(as_half2(and_or_u32(w0, 0x00FF00FFu, kMagic1024)), as_half2(and_or_u32(w0 >> 8, 0x00FF00FFu, kMagic1024)),
-                                          as_half2(and_or_u32(w1, 0x00FF00FFu, kMagic1024)), as_half2(and_or_u32(w1 >> 8, 0x00FF00FFu, kMagic1024)));
-#pragma unroll
-            for (int mm = 0; mm < M; mm++) {
-                const half8v av = *(const half8v *)(reg + mm * kRegion + l.off[q]);
-                c[mm] = mfma16x16x32(av, bop, c[mm]);
-            }
-        }
+    __device__ static int a_off(const Lane &l, int i) { return l.off[i]; }
+    __device__ static half8v step(const W &w, int i) {
+        const uint32_t w0 = (i & 1) ? w.p[i >> 1].z : w.p[i >> 1].x;
+        const uint32_t w1 = (i & 1) ? w.p[i >> 1].w : w.p[i >> 1].y;
+        return make_half8(as_half2(and_or_u32(w0, 0x00FF00FFu, kMagic1024)), as_half2(and_or_u32(w0 >> 8, 0x00FF00FFu, kMagic1024)),
+                          as_half2(and_or_u32(w1, 0x00FF00FFu, kMagic1024)), as_half2(and_or_u32(w1 >> 8, 0x00FF00FFu, kMagic1024)));
     }
     struct Sc { half2v d01, d23; };
     __device__ static Sc scales(const W &w, const Lane &) { return Sc{as_half2(w.dd.x), as_half2(w.dd.y)}; }
@@ -363,14 +335,43 @@ __device__ inline void stage_x1(const X1Regs<XT> &v, uint8_t *region, int lane) 
     Row1Fmt<DT>::sums(h01, h23, region, lane);
 }
 
+// the sum over the 64 lanes, in every lane
+__device__ inline float sum64(float v) {
+    float r = dpp_add<0x140>(sum8(v));  // row_mirror: lane i <- lane 15 - i of its row
+    asm volatile("" : "+v"(r));
+    auto row = [&](int i) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r), 16 * i)); };
+    return (row(0) + row(1)) + (row(2) + row(3));
+}
+// The sums over the waves of what each has left 64 floats apart from the next, in wave order, for N such runs together.  Eight reads of each at a
+// time, those past the last wave dropped: a wait per read, as a loop over the waves makes it, was half of what the end of a small launch took.
+template <int N> __device__ inline void sum_waves(const float *const (&p)[N], int nwaves, float (&s)[N]) {
+#pragma unroll
+    for (int j = 0; j < N; j++) s[j] = 0.0f;
+    for (int wv = 0; wv < nwaves; wv += 8) {
+        float v[N][8];
+#pragma unroll
+        for (int j = 0; j < N; j++)
+#pragma unroll
+            for (int i = 0; i < 8; i++) v[j][i] = p[j][(wv + i) * 64];
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+#pragma unroll
+            for (int j = 0; j < N; j++) s[j] += wv + i < nwaves ? v[j][i] : 0.0f;
+    }
+}
+constexpr int kSumPad = 7 * 64 * 4;  // bytes of LDS that sum_waves may read past the last wave's floats
+// an element of y as it lies in memory
+__device__ inline float out_value(uint32_t bits, int yt) {
+    return yt == TURQ_ACT_F32 ? __uint_as_float(bits) : yt == TURQ_ACT_BF16 ? __uint_as_float(bits << 16) : (float)as_half2(bits).x;
+}
+
 constexpr int kMaxRow1 = 4;
 struct Row1Args {
     const uint8_t *w[kMaxRow1];
     void *y[kMaxRow1];
     const float *bias[kMaxRow1];
     int64_t n[kMaxRow1], ldy[kMaxRow1];
-    int first[kMaxRow1];
-    int count;
+    int first[kMaxRow1];  // first workgroup of the weight (INT_MAX: there is none)
     int second;  // two-format launches: weights [0, second) are of the first format, [second, count) of the second
 };
 
@@ -385,7 +386,7 @@ struct Row1Args {
 // the round trip of its output go away.
 template <int DT, int XT, int P, int R, int M, bool GU = false, bool NORM = false, bool ACC = false>
 __device__ __forceinline__ void row1_body(const uint8_t *__restrict__ w, void *__restrict__ y, int64_t ldy, const float *__restrict__ bias,
-                                          int64_t n, int64_t rtb, int64_t k, const void *__restrict__ x, int64_t ldx, int m, int yt,
+                                          int64_t n, int64_t rtb, int64_t k, const void *__restrict__ x, int64_t ldx, int m, int yt, int nwaves,
                                           const uint8_t *__restrict__ w2 = nullptr, const float *__restrict__ bias2 = nullptr,
                                           const float *__restrict__ gw = nullptr, float eps = 0.0f) {
     static_assert(!GU || R == 2, "gate and up take the places of two row tiles");
@@ -394,13 +395,66 @@ __device__ __forceinline__ void row1_body(const uint8_t *__restrict__ w, void *_
     using Fmt = Row1Fmt<DT>;
     constexpr int TB = TiledFmt<DT>::kTileBytes;
     constexpr int ES = XT == TURQ_ACT_F32 ? 4 : 2;
-    const int64_t rt0 = GU ? rtb : rtb * R, nrt = turq_tile_rows(n);
-
+    constexpr bool RAGGED = DT == TURQ_Q8_0;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int nwaves = blockDim.x >> 6;
     const int g = lane >> 4;
-    const int64_t ntc = turq_tile_cols(k);
+    const uint32_t ntc = (uint32_t)turq_tile_cols(k), nrt = (uint32_t)turq_tile_rows(n), rt0 = (uint32_t)(GU ? rtb : rtb * R);
+
+    // The first loads go out before anything else is done: what a small launch takes is its longest chain of dependent steps, and at a wave or
+    // two per SIMD every instruction ahead of the loads is on it (about 170 were: 0.3 us of a launch of 4).  By the wall clock, entry to first
+    // load 0.4 us, x there after another 0.3, the weights after 0.7, sums 0.3, barrier to store 0.4, and 1.2 from there to the next
+    // launch's entry: a decode step of 112 launches of 2 - 7 MB at 493 us went to 461 with the arguments read together, 427 with this order, 407
+    // with one column tile per wave.
+    GOff go{16u * (uint32_t)lane, 8u * (uint32_t)lane, 4u * (uint32_t)lane, 16u * (uint32_t)(lane & 15), Fmt::aux_off(lane & 15, g), 0u};
+    const uint8_t *wrow[R];  // row tiles past the weight's last one re-read it; their results are not stored
+    const uint8_t *xrow[M];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        if constexpr (GU) wrow[r] = (r == 0 ? w : w2) + (uint64_t)(rt0 * ntc) * TB;
+        else wrow[r] = w + (uint64_t)((R == 1 || rt0 + r < nrt ? rt0 + r : nrt - 1) * ntc) * TB;
+    }
+#pragma unroll
+    for (int mm = 0; mm < M; mm++) xrow[mm] = (const uint8_t *)x + (mm < m ? mm : 0) * ldx * ES;
+    X1Regs<XT> xr[P][M];
+    float4v gv[NORM ? P : 1];
+    typename Fmt::W wr[P][R];
+    auto request = [&](uint32_t b0) {
+        go.touch();
+#pragma unroll
+        for (int p = 0; p < P; p++) {
+            const uint32_t b = b0 + (uint32_t)(p * nwaves), bb = b < ntc ? b : b0;
+            const bool ok = in_tile<RAGGED>(k, bb, lane);
+#pragma unroll
+            for (int mm = 0; mm < M; mm++) xr[p][mm] = load_x1<XT>(xrow[mm], bb, go, ok);
+            if constexpr (NORM) gv[p] = *(const float4v *)((const uint8_t *)gw + (uint64_t)bb * 1024 + (ok ? go.o16 : 0u));
+        }
+#pragma unroll
+        for (int p = 0; p < P; p++) {
+            const uint32_t b = b0 + (uint32_t)(p * nwaves);
+#pragma unroll
+            for (int r = 0; r < R; r++) wr[p][r] = Fmt::load(wrow[r] + (uint64_t)(b < ntc ? b : b0) * TB, go);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    uint32_t b0 = (uint32_t)wave;
+    if (b0 < ntc) request(b0);
+    // What the first result of this lane will need besides the sums, requested now so that it has long arrived when they are done (a load at
+    // the end of the kernel is a whole memory round trip on the critical path): its bias and, for ACC (TURQ_OUT_ACCUMULATE in yt; an
+    // instantiation of its own, since even the untaken branch cost the plain launches 2 %), the bits of the element it is added to - as
+    // they lie in memory: converted here they would be waited for here.  Waves without a result load the first one's.
+    const uint32_t r1 = !GU && wave < R * M ? (uint32_t)wave / M : 0u, mm1 = (GU ? wave < M : wave < R * M) ? (uint32_t)wave - r1 * M : 0u;
+    const int64_t col_first = (int64_t)(rt0 + (rt0 + r1 < nrt ? r1 : 0u)) * 16 + (lane >> 2), colc = col_first < n ? col_first : n - 1;
+    uint32_t old_bits = 0;
+    float bias_first = 0.0f, bias2_first = 0.0f;
+    if constexpr (ACC && !GU) {
+        const int64_t at = (int64_t)((int)mm1 < m ? mm1 : 0u) * ldy + colc;
+        if ((yt & 0xFF) == TURQ_ACT_F32) old_bits = ((const uint32_t *)y)[at];
+        else old_bits = ((const uint16_t *)y)[at];
+    }
+    if (bias) bias_first = bias[colc];
+    if (GU && bias2) bias2_first = bias2[colc];
+
     // several rows of a format that has the packed form: two rows per MFMA chain, regions per pair of rows
     constexpr bool PK = Fmt::kPacked && M > 1;
     constexpr int NP = M / 2;
@@ -408,7 +462,7 @@ __device__ __forceinline__ void row1_body(const uint8_t *__restrict__ w, void *_
     static_assert(!PK || M % 2 == 0, "packed pairs");
     uint8_t *region = smem + (size_t)wave * (P * PSTRIDE);  // [p][activation row] or [p][pair]
     float *red = (float *)(smem + (size_t)nwaves * (P * PSTRIDE));
-    float *red_ss = red + (size_t)nwaves * (R * M * 64);  // NORM: a sum of squares per wave
+    float *red_ss = red + (size_t)nwaves * (R * M * 64);  // NORM: the lanes' sums of squares
     float ss = 0.0f;
 
     // the zeros that the idle A rows read, and start values that no format overwrites
@@ -422,56 +476,19 @@ __device__ __forceinline__ void row1_body(const uint8_t *__restrict__ w, void *_
             for (int p = 0; p < P * M; p++) *(float *)(region + p * kRegion + kInit + 4 * lane) = 0.0f;  // float like the later writes
     }
     const typename Fmt::Lane lc = Fmt::lane_init(lane & 15, g);
-    GOff go{16u * (uint32_t)lane, 8u * (uint32_t)lane, 4u * (uint32_t)lane, 16u * (uint32_t)(lane & 15), Fmt::aux_off(lane & 15, g), 0u};
-
     float acc[R][M];
-    const uint8_t *wrow[R];  // row tiles past the weight's last one re-read it; their results are not stored
-    const uint8_t *xrow[M];
 #pragma unroll
-    for (int r = 0; r < R; r++) {
+    for (int r = 0; r < R; r++)
 #pragma unroll
         for (int mm = 0; mm < M; mm++) acc[r][mm] = 0.0f;
-        if constexpr (GU) wrow[r] = (r == 0 ? w : w2) + rt0 * ntc * TB;
-        else wrow[r] = w + (rt0 + r < nrt ? rt0 + r : nrt - 1) * ntc * TB;
-    }
+    while (b0 < ntc) {
+        if constexpr (RAGGED) {
 #pragma unroll
-    for (int mm = 0; mm < M; mm++) xrow[mm] = (const uint8_t *)x + (mm < m ? mm : 0) * ldx * ES;
-    // ACC (TURQ_OUT_ACCUMULATE in yt; an instantiation of its own, since even the untaken branch cost the plain launches 2 %):
-    // the element this lane will add its first result to, requested now so that it has long arrived when the sums are done (a
-    // load at the end of the kernel is a whole memory round trip on the critical path)
-    float old_first = 0.0f;
-    if constexpr (ACC && !GU) {
-        if (wave < R * M) {
-            const int r = wave / M, mm = wave - r * M;
-            const int64_t col = (rt0 + r) * 16 + (lane >> 2);
-            if ((lane & 3) == 0 && rt0 + r < nrt && col < n && mm < m) {
-                const int64_t at = (int64_t)mm * ldy + col;
-                const int base = yt & 0xFF;
-                old_first = base == TURQ_ACT_F32 ? turq_load_out<TURQ_ACT_F32>(y, at) : base == TURQ_ACT_BF16 ? turq_load_out<TURQ_ACT_BF16>(y, at) : turq_load_out<TURQ_ACT_F16>(y, at);
+            for (int p = 0; p < P; p++) {
+                const uint32_t b = b0 + (uint32_t)(p * nwaves);
+#pragma unroll
+                for (int mm = 0; mm < M; mm++) drop_outside<XT>(xr[p][mm], in_tile<RAGGED>(k, b < ntc ? b : b0, lane));
             }
-        }
-    }
-    for (int64_t b0 = wave; b0 < ntc; b0 += (int64_t)nwaves * P) {
-        X1Regs<XT> xr[P][M];
-        float4v gv[NORM ? P : 1];
-        typename Fmt::W wr[P][R];
-        go.touch();
-#pragma unroll
-        for (int p = 0; p < P; p++) {
-            const int64_t b = b0 + (int64_t)p * nwaves;
-#pragma unroll
-            for (int mm = 0; mm < M; mm++) xr[p][mm] = load_x1<XT, DT == TURQ_Q8_0>(xrow[mm], k, b < ntc ? b : b0, lane, go);
-            if constexpr (NORM) {
-                const int64_t bb = b < ntc ? b : b0;
-                const bool ok = DT != TURQ_Q8_0 || bb * 256 + 4 * lane < k;  // (Q8_0: k may end inside the tile; the columns are zeros then)
-                gv[p] = *(const float4v *)(gw + (ok ? bb * 256 + 4 * lane : 0));
-            }
-        }
-#pragma unroll
-        for (int p = 0; p < P; p++) {
-            const int64_t b = b0 + (int64_t)p * nwaves;
-#pragma unroll
-            for (int r = 0; r < R; r++) wr[p][r] = Fmt::load(wrow[r] + (b < ntc ? b : b0) * TB, go);
         }
 #pragma unroll
         for (int p = 0; p < P; p++)
@@ -495,7 +512,7 @@ __device__ __forceinline__ void row1_body(const uint8_t *__restrict__ w, void *_
                         const half2v a = as_half2(xr[p][mm].r[0]), c = as_half2(xr[p][mm].r[1]);
                         f[0] = (float)a.x, f[1] = (float)a.y, f[2] = (float)c.x, f[3] = (float)c.y;
                     }
-                    if (b0 + (int64_t)p * nwaves < ntc) ss += (f[0] * f[0] + f[1] * f[1]) + (f[2] * f[2] + f[3] * f[3]);  // (a tile past the end repeats another)
+                    if (b0 + (uint32_t)(p * nwaves) < ntc) ss += (f[0] * f[0] + f[1] * f[1]) + (f[2] * f[2] + f[3] * f[3]);  // (a tile past the end repeats another)
                     const half2v h01 = __builtin_convertvector(float2v{f[0] * gv[p].x, f[1] * gv[p].y}, half2v);
                     const half2v h23 = __builtin_convertvector(float2v{f[2] * gv[p].z, f[3] * gv[p].w}, half2v);
                     uint8_t *rg = region + p * PSTRIDE + mm * kRegion;
@@ -511,8 +528,22 @@ __device__ __forceinline__ void row1_body(const uint8_t *__restrict__ w, void *_
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
         for (int p = 0; p < P; p++) {
-            const int64_t b = b0 + (int64_t)p * nwaves;
-            if (b >= ntc) continue;  // uniform per wave
+            if (b0 + (uint32_t)(p * nwaves) >= ntc) continue;  // uniform per wave
+            if constexpr (R == 2 && M == 1 && P == 1) {
+                // two row tiles against one set of A operands: two independent chains, every operand read from the LDS once
+                float4v c[R];
+#pragma unroll
+                for (int r = 0; r < R; r++) c[r] = *(const float4v *)(region + kInit + 16 * g);
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    const half8v av = *(const half8v *)(region + Fmt::a_off(lc, i));
+#pragma unroll
+                    for (int r = 0; r < R; r++) c[r] = mfma16x16x32(av, Fmt::step(wr[p][r], i), c[r]);
+                }
+#pragma unroll
+                for (int r = 0; r < R; r++) acc[r][0] += Fmt::finish(Fmt::scales(wr[p][r], lc), c[r]);
+                continue;
+            }
 #pragma unroll
             for (int r = 0; r < R; r++) {
                 if constexpr (PK) {
@@ -530,8 +561,28 @@ __device__ __forceinline__ void row1_body(const uint8_t *__restrict__ w, void *_
                     }
                     continue;
                 }
+                // the A operands of one row are read ahead of the first look at the weights, which arrive last (read one by one next to their
+                // MFMAs, each of the eight waits for the LDS)
                 float4v c[M];
-                Fmt::template chain<M>(wr[p][r], region + p * PSTRIDE, lc, g, c);
+                const uint8_t *reg = region + p * PSTRIDE;
+                constexpr bool AHEAD = M == 1 && P == 1;  // (more tiles in flight leave no registers for it)
+#pragma unroll
+                for (int mm = 0; mm < M; mm++) c[mm] = *(const float4v *)(reg + mm * kRegion + kInit + 16 * g);
+                half8v av[8];
+                if constexpr (AHEAD) {
+#pragma unroll
+                    for (int i = 0; i < 8; i++) av[i] = *(const half8v *)(reg + Fmt::a_off(lc, i));
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    const half8v bop = Fmt::step(wr[p][r], i);
+#pragma unroll
+                    for (int mm = 0; mm < M; mm++) {
+                        if constexpr (!AHEAD) av[i] = *(const half8v *)(reg + mm * kRegion + Fmt::a_off(lc, i));
+                        c[mm] = mfma16x16x32(av[i], bop, c[mm]);
+                    }
+                }
                 // One tile after the other.  Left free, the scheduler interleaves the tiles' chains and scale arithmetic, the
                 // unpacked operands of several tiles are live at once and the 128 registers a wave of a 16-wave workgroup may
                 // use overflow (spills in the instantiations with four tiles per workgroup pass; the 510 MB LM head lost
@@ -546,67 +597,79 @@ __device__ __forceinline__ void row1_body(const uint8_t *__restrict__ w, void *_
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
+        b0 += (uint32_t)(nwaves * P);
+        if (b0 < ntc) request(b0);
     }
 
-    // y[mm][16 rt + n] = sum over lane groups and waves; wave i adds up the i-th (row tile, activation row) pair
+    // y[mm][16 rt + n] = sum over lane groups and waves; wave i adds up the i-th (row tile, activation row) pair (GU: pair of row tiles)
+    constexpr int RES = GU ? M : R * M;
+    const int n4 = lane >> 2, q = lane & 3;
+    // (where the first result goes, worked out while the others are still at it)
+    uint64_t y_first = (uint64_t)(uintptr_t)y + (uint64_t)((int64_t)mm1 * ldy + col_first) * ((yt & 0xFF) == TURQ_ACT_F32 ? 4 : 2);
+    bool ok_first = q == 0 && rt0 + r1 < nrt && col_first < n && (int)mm1 < m;
+    float kf = (float)k;
+    asm volatile("" : "+v"(y_first), "+v"(kf));
 #pragma unroll
     for (int r = 0; r < R; r++)
 #pragma unroll
         for (int mm = 0; mm < M; mm++) red[((r * M + mm) * nwaves + wave) * 64 + lane] = acc[r][mm];
-    if constexpr (NORM) {
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) ss += __shfl_xor(ss, off, 64);
-        if (lane == 0) red_ss[wave] = ss;
-    }
+    if constexpr (NORM) red_ss[wave * 64 + lane] = ss;
     __syncthreads();
+    if (wave >= RES) return;
+    // the sums of result i, and with the first the root of the row's mean square
     float inv_rms = 1.0f;
-    if constexpr (NORM) {
-        float tot = 0.0f;
-        for (int wv = 0; wv < nwaves; wv++) tot += red_ss[wv];
-        inv_rms = 1.0f / sqrtf(tot / (float)k + eps);
+    auto sums = [&](int i, auto first, float &s0, float &s1) {
+        constexpr bool SS = NORM && decltype(first)::value;
+        constexpr int N = 1 + (GU ? 1 : 0) + (SS ? 1 : 0);
+        const float *src[N];
+        float t[N];
+        src[0] = red + i * nwaves * 64 + n4 + 16 * q;
+        if constexpr (GU) src[1] = red + (M + i) * nwaves * 64 + n4 + 16 * q;
+        if constexpr (SS) src[N - 1] = red_ss + lane;
+        sum_waves<N>(src, nwaves, t);
+        if constexpr (SS) inv_rms = 1.0f / sqrtf(sum64(t[N - 1]) / kf + eps);
+        s0 = sum4(t[0]);
+        s1 = GU ? sum4(t[N > 1 ? 1 : 0]) : 0.0f;
+    };
+    auto value = [&](float s0, float s1, float b0, float b1) {
+        if constexpr (!GU) return s0 * inv_rms + b0;
+        const float gate = s0 * inv_rms + b0, up = s1 * inv_rms + b1;
+        return gate / (1.0f + expf(-gate)) * up;  // SiLU
+    };
+    float s0, s1;
+    sums(wave, std::true_type{}, s0, s1);
+    if (ok_first) {
+        const float out = value(s0, s1, bias_first, bias2_first);
+        void *at = (void *)(uintptr_t)y_first;
+        if constexpr (ACC) turq_store_any(at, yt & 0xFF, 0, out + out_value(old_bits, yt & 0xFF));  // (what y held was requested before the main loop)
+        else turq_store_any(at, yt, 0, out);
     }
-    const int n4 = lane >> 2, q = lane & 3;
-    if constexpr (GU) {
-        for (int mm = wave; mm < M; mm += nwaves) {
-            float sg = 0.0f, su = 0.0f;
-            for (int wv = 0; wv < nwaves; wv++) {
-                sg += red[(mm * nwaves + wv) * 64 + n4 + 16 * q];
-                su += red[((M + mm) * nwaves + wv) * 64 + n4 + 16 * q];
-            }
-            sg = sum4(sg);
-            su = sum4(su);
-            const int64_t col = rt0 * 16 + n4;
-            if (q == 0 && col < n && mm < m) {
-                const float gate = sg * inv_rms + (bias ? bias[col] : 0.0f), up = su * inv_rms + (bias2 ? bias2[col] : 0.0f);
-                const float out = gate / (1.0f + expf(-gate)) * up;  // SiLU
-                const int64_t at = (int64_t)mm * ldy + col;
-                turq_store_any(y, yt, at, out);
-            }
-        }
-        return;
-    }
-    for (int i = wave; i < R * M; i += nwaves) {
-        const int r = i / M, mm = i - r * M;
-        float s = 0.0f;
-        for (int wv = 0; wv < nwaves; wv++) s += red[(i * nwaves + wv) * 64 + n4 + 16 * q];
-        s = sum4(s);
-        const int64_t col = (rt0 + r) * 16 + n4;
-        if (q == 0 && rt0 + r < nrt && col < n && mm < m) {
-            const float out = s * inv_rms + (bias ? bias[col] : 0.0f);
-            const int64_t at = (int64_t)mm * ldy + col;
-            if (ACC && i == wave) turq_store_any(y, yt & 0xFF, at, out + old_first);  // (what y held was requested before the main loop)
-            else turq_store_any(y, yt, at, out);
-        }
+    for (int i = wave + nwaves; i < RES; i += nwaves) {  // (fewer waves than results)
+        sums(i, std::false_type{}, s0, s1);
+        const int r = GU ? 0 : i / M, mm = i - r * M;
+        const int64_t col = (int64_t)(rt0 + r) * 16 + n4;
+        if (q == 0 && rt0 + r < nrt && col < n && mm < m)
+            turq_store_any(y, yt, (int64_t)mm * ldy + col, value(s0, s1, bias ? bias[col] : 0.0f, GU && bias2 ? bias2[col] : 0.0f));
     }
 }
+
+// A launch's arguments are two hundred bytes that no cache holds when it starts.  Left to itself the compiler loads each where it is first used,
+// behind the branches that pick the weight: five scalar loads one after the other, each a round trip, before the first weight is
+// requested.  Naming them here makes them one.
+template <class... T> __device__ inline void load_together(T... v) { (void)std::initializer_list<int>{([](auto u) { asm volatile("" ::"s"(u)); }(v), 0)...}; }
 
 // which weight of the launch this workgroup works on
 struct Row1Pick { const uint8_t *w; void *y; const float *bias; int64_t n, ldy; int first; int index; };
 __device__ inline Row1Pick row1_pick(const Row1Args &a, int blk) {
     Row1Pick p{a.w[0], a.y[0], a.bias[0], a.n[0], a.ldy[0], 0, 0};
+    load_together(a.w[0], a.w[1], a.w[2], a.w[3], a.y[0], a.y[1], a.y[2], a.y[3], a.bias[0], a.bias[1], a.bias[2], a.bias[3], a.n[0], a.n[1], a.n[2], a.n[3],
+                  a.ldy[0], a.ldy[1], a.ldy[2], a.ldy[3], a.first[1], a.first[2], a.first[3], a.second);
 #pragma unroll
-    for (int i = 1; i < kMaxRow1; i++)
-        if (i < a.count && blk >= a.first[i]) p = Row1Pick{a.w[i], a.y[i], a.bias[i], a.n[i], a.ldy[i], a.first[i], i};
+    for (int i = 1; i < kMaxRow1; i++) {  // (selects, no branches; first of a weight that is not there: never reached)
+        const bool in = blk >= a.first[i];
+        p.w = in ? a.w[i] : p.w, p.y = in ? a.y[i] : p.y, p.bias = in ? a.bias[i] : p.bias;
+        p.n = in ? a.n[i] : p.n, p.ldy = in ? a.ldy[i] : p.ldy, p.first = in ? a.first[i] : p.first, p.index = in ? i : p.index;
+    }
     return p;
 }
 
@@ -614,8 +677,10 @@ __device__ inline Row1Pick row1_pick(const Row1Args &a, int blk) {
 template <int DT, int XT, int P, int R, int M, int MAXT, bool NORM = false, bool ACC = false>
 __global__ void __launch_bounds__(MAXT) gemv_row1_kernel(Row1Args a, int64_t k, const void *__restrict__ x, int64_t ldx, int m, int yt,
                                                          const float *__restrict__ gw, float eps) {
+    const int nwaves = blockDim.x >> 6;
+    load_together(k, x, ldx, m, yt, gw, eps, nwaves);
     const Row1Pick p = row1_pick(a, (int)blockIdx.x);
-    row1_body<DT, XT, P, R, M, false, NORM, ACC>(p.w, p.y, p.ldy, p.bias, p.n, (int64_t)((int)blockIdx.x - p.first), k, x, ldx, m, yt, nullptr,
+    row1_body<DT, XT, P, R, M, false, NORM, ACC>(p.w, p.y, p.ldy, p.bias, p.n, (int64_t)((int)blockIdx.x - p.first), k, x, ldx, m, yt, nwaves, nullptr,
                                             nullptr, gw, eps);
 }
 
@@ -627,7 +692,9 @@ __global__ void __launch_bounds__(MAXT) gemv_row1_gateup_kernel(const uint8_t *_
                                                                  int64_t k, const void *__restrict__ x, int64_t ldx, int m,
                                                                  void *__restrict__ y, int64_t ldy, int yt, const float *__restrict__ gw,
                                                                  float eps) {
-    row1_body<DT, XT, P, 2, M, true, NORM>(wg, y, ldy, bg, n, (int64_t)blockIdx.x, k, x, ldx, m, yt, wu, bu, gw, eps);
+    const int nwaves = blockDim.x >> 6;
+    load_together(wg, wu, bg, bu, n, k, x, ldx, m, y, ldy, yt, gw, eps, nwaves);
+    row1_body<DT, XT, P, 2, M, true, NORM>(wg, y, ldy, bg, n, (int64_t)blockIdx.x, k, x, ldx, m, yt, nwaves, wu, bu, gw, eps);
 }
 
 // weights of two formats that share an input (q, k Q4_K and v Q6_K of a Q4_K_M file) in one launch: the workgroup's weight
@@ -635,10 +702,12 @@ __global__ void __launch_bounds__(MAXT) gemv_row1_gateup_kernel(const uint8_t *_
 template <int DTA, int DTB, int XT, int P, int M, int MAXT, bool NORM = false>
 __global__ void __launch_bounds__(MAXT) gemv_row1_mixed_kernel(Row1Args a, int64_t k, const void *__restrict__ x, int64_t ldx, int m,
                                                                 int yt, const float *__restrict__ gw, float eps) {
+    const int nwaves = blockDim.x >> 6;
+    load_together(k, x, ldx, m, yt, gw, eps, nwaves);
     const Row1Pick p = row1_pick(a, (int)blockIdx.x);
     const int64_t rtb = (int64_t)((int)blockIdx.x - p.first);
-    if (p.index < a.second) row1_body<DTA, XT, P, 1, M, false, NORM>(p.w, p.y, p.ldy, p.bias, p.n, rtb, k, x, ldx, m, yt, nullptr, nullptr, gw, eps);
-    else row1_body<DTB, XT, P, 1, M, false, NORM>(p.w, p.y, p.ldy, p.bias, p.n, rtb, k, x, ldx, m, yt, nullptr, nullptr, gw, eps);
+    if (p.index < a.second) row1_body<DTA, XT, P, 1, M, false, NORM>(p.w, p.y, p.ldy, p.bias, p.n, rtb, k, x, ldx, m, yt, nwaves, nullptr, nullptr, gw, eps);
+    else row1_body<DTB, XT, P, 1, M, false, NORM>(p.w, p.y, p.ldy, p.bias, p.n, rtb, k, x, ldx, m, yt, nwaves, nullptr, nullptr, gw, eps);
 }
 
 struct Row1Launch {
@@ -656,7 +725,7 @@ struct Row1Launch {
 
 template <int DT, int P, int R, int M> size_t row1_lds(int nwaves) {
     const size_t tile = (Row1Fmt<DT>::kPacked && M > 1) ? (size_t)(M / 2) * kPairRegion : (size_t)M * kRegion;
-    return (size_t)nwaves * P * tile + (size_t)nwaves * R * M * 64 * sizeof(float) + 64;  // (+ a sum of squares per wave)
+    return (size_t)nwaves * P * tile + (size_t)nwaves * (R * M + 1) * 64 * sizeof(float) + kSumPad;  // (+ 1: the sums of squares)
 }
 
 template <int DT, int XT, int P, int R, int M, bool NORM, bool ACC>
@@ -773,8 +842,8 @@ bool row1_args(Row1Launch &l, int count, const void *const *w, const int64_t *n,
         l.a.first[i] = (int)blocks;
         blocks += (turq_tile_rows(n[i]) + row_tiles - 1) / row_tiles;
     }
-    l.a.count = count;
-    if (blocks > 0x7FFFFFFF) return false;
+    for (int i = count; i < kMaxRow1; i++) l.a.first[i] = INT_MAX;
+    if (blocks >= INT_MAX) return false;
     l.blocks = (int)blocks;
     return true;
 }
@@ -898,7 +967,8 @@ hipError_t launch_gateup_p(const GateUpLaunch &l) {
         if (l.gw) return hipErrorInvalidValue;  // (the norm inside the kernel: one activation row)
         return one ? launch_gateup_final<DT, XT, 1, 2, false>(l) : launch_gateup_final<DT, XT, 2, 2, false>(l);
     }
-    if (l.gw) return one ? launch_gateup_final<DT, XT, 1, 1, true>(l) : launch_gateup_final<DT, XT, 2, 1, true>(l);
+    constexpr int TWO = DT == TURQ_Q8_0 ? 1 : 2;  // (two tiles of two Q8_0 weights next to the norm weights do not fit the registers)
+    if (l.gw) return one ? launch_gateup_final<DT, XT, 1, 1, true>(l) : launch_gateup_final<DT, XT, TWO, 1, true>(l);
     return one ? launch_gateup_final<DT, XT, 1, 1, false>(l) : launch_gateup_final<DT, XT, 2, 1, false>(l);
 }
 

@@ -50,16 +50,24 @@ bool row1_takes(int64_t m, size_t weight_bytes, int dtype) {
     return weight_bytes <= ((size_t)(dtype == TURQ_Q4_K ? 64 : 128) << 20);
 }
 
-// Waves per workgroup of the one-row kernel: it is light on registers and on vector work, so what it wants is many waves
-// with few column tiles each (two by default), up to the largest workgroup.
-int pick_waves_row1(int64_t k) {
-    const int forced = turq_tuning().gemv_waves;
-    const int tpw_env = std::max(turq_tuning().row1_tpw, 0);
-    const int64_t col_tiles = turq_tile_cols(k);
-    // (up to four column tiles, K <= 1024: one per wave; the 3072 x 1024 Q8_0 matrix gains 5 %)
-    const int tpw = tpw_env ? tpw_env : (col_tiles <= 4 ? 1 : 2);
+// Waves per workgroup of the one-row kernels for a launch of `groups` workgroups of `rtiles` row tiles (2: two that share the staged
+// activations, or a gate and an up tile).  A launch of no more workgroups than compute units is a chain of memory round trips: as
+// many waves as there are column tiles, up to the largest workgroup (4096 x 12288 Q6_K at 8 / 12 / 16 waves 10.0 / 9.4 / 9.7 us,
+// 1024 x 2048 Q8_0 at 4 / 8 waves of 2 / 1 tiles 3.7 / 3.3).  Beyond that the workgroups of a unit should be resident together, and
+// it wants about ten waves in all: 384 workgroups (q, k and v of 4096 columns) at 4 / 6 / 8 / 16 waves 7.0 / 6.5 / 6.8 / 7.4 us, 640
+// (5120 columns) at 4 / 8 / 16 10.7 / 11.9 / 12.6, 2000 (32000 x 4096 Q4_K) 16.7 / 16.9 / 22.4; two tiles at a time keep eight (gate and up 12288
+// x 4096, 768 workgroups, at 4 / 8 / 16 11.9 / 11.6 / 13.5).
+int pick_waves_row1(const turq_ctx *ctx, int64_t k, int64_t groups, int rtiles) {
+    const int forced = turq_tuning().gemv_waves, tpw = turq_tuning().row1_tpw;
+    const int64_t col_tiles = turq_tile_cols(k), cus = ctx->compute_units > 0 ? ctx->compute_units : 256;
     if (forced >= 1 && forced <= 16) return (int)std::min<int64_t>(forced, col_tiles);
-    return (int)std::max<int64_t>(1, std::min<int64_t>((col_tiles + tpw - 1) / tpw, 16));
+    if (tpw > 0) return (int)std::max<int64_t>(1, std::min<int64_t>((col_tiles + tpw - 1) / tpw, 16));
+    if (groups <= cus) {
+        const int64_t turns = (col_tiles + 15) / 16;  // column tiles of a wave
+        return (int)std::max<int64_t>(1, (col_tiles + turns - 1) / turns);
+    }
+    const int64_t most = rtiles > 1 ? 8 : std::max<int64_t>(4, std::min<int64_t>(8, 10 * cus / groups));
+    return (int)std::max<int64_t>(1, std::min<int64_t>(col_tiles, most));
 }
 
 // Row tiles per workgroup of the one-row kernel (TURQ_ROW1_R forces it).
@@ -604,9 +612,10 @@ int turq_qmatmul_mfma(turq_ctx *ctx, const turq_weight *w, const void *x, int xt
             TURQ_HIP(ctx, turq_prof_next(ctx, &ev0, &ev1));
             const void *wp = w->dev;
             void *yv = yc;
+            const int64_t tiles = turq_tile_rows(w->n);
+            const int rtiles = mc == 1 ? pick_rows_row1(ctx, tiles) : 1;
             TURQ_HIP(ctx, turq_launch_gemv_row1(w->dtype, 1, &wp, &w->n, w->k, xc, xt, ldx, mc, &yv, yt, &ldy, bias ? &bias : nullptr,
-                                                pick_waves_row1(w->k), mc == 1 ? pick_rows_row1(ctx, turq_tile_rows(w->n)) : 1,
-                                                ctx->stream, ev0, ev1, norm ? norm->w : nullptr, norm ? norm->eps : 0.0f));
+                                                pick_waves_row1(ctx, w->k, (tiles + rtiles - 1) / rtiles, rtiles), rtiles, ctx->stream, ev0, ev1, norm ? norm->w : nullptr, norm ? norm->eps : 0.0f));
             continue;
         }
         if (use_fused(ctx, mc, turq_tile_rows(w->n), w->dev_bytes) && aligned && !no_fuse) {
@@ -706,11 +715,7 @@ int turq_qmatmul_gate_up_mfma(turq_ctx *ctx, const turq_weight *gate, const turq
         return TURQ_OK;
     }
     TURQ_HIP(ctx, turq_prof_next(ctx, &ev0, &ev1));
-    // a wave holds a tile of each weight per column tile: half as many column tiles per wave as in the plain launch, i.e. twice
-    // the waves (K = 4096: 16 waves of one column tile; 8 waves of two cost the MLP step 2.7 %)
-    const bool forced = turq_tuning().gemv_waves != 0;
-    int nwaves = pick_waves_row1(gate->k);
-    if (!forced) nwaves = (int)std::min<int64_t>({2 * (int64_t)nwaves, 16, turq_tile_cols(gate->k)});
+    const int nwaves = pick_waves_row1(ctx, gate->k, turq_tile_rows(gate->n), 2);
     TURQ_HIP(ctx, turq_launch_gemv_row1_gateup(gate->dtype, gate->dev, up->dev, gate->n, gate->k, x, xt, ldx, m, y, yt, ldy, bias_gate,
                                                bias_up, nwaves, ctx->stream, ev0, ev1, norm ? norm->w : nullptr, norm ? norm->eps : 0.0f));
     *taken = true;
@@ -791,15 +796,16 @@ int turq_qmatmul_multi_mfma(turq_ctx *ctx, int count, const turq_weight *const *
             while (j2 < count && w[j2]->dtype == w[j]->dtype) j2++;
             if (j2 - i <= 4) {
                 const void *wp[4];
-                int64_t nn[4];
+                int64_t nn[4], tiles = 0;
                 for (int t = i; t < j2; t++) {
                     wp[t - i] = w[t]->dev;
                     nn[t - i] = w[t]->n;
+                    tiles += turq_tile_rows(w[t]->n);
                 }
                 hipEvent_t ev0 = nullptr, ev1 = nullptr;
                 TURQ_HIP(ctx, turq_prof_next(ctx, &ev0, &ev1));
                 TURQ_HIP(ctx, turq_launch_gemv_row1_mixed(w[i]->dtype, w[j]->dtype, j2 - i, j - i, wp, nn, w[i]->k, x, xt, ldx, m, y + i,
-                                                          yt, ldy + i, bias ? bias + i : nullptr, pick_waves_row1(w[i]->k), ctx->stream,
+                                                          yt, ldy + i, bias ? bias + i : nullptr, pick_waves_row1(ctx, w[i]->k, tiles, 1), ctx->stream,
                                                           ev0, ev1, norm ? norm->w : nullptr, norm ? norm->eps : 0.0f));
                 i = j2;
                 continue;
@@ -830,17 +836,19 @@ int turq_qmatmul_multi_mfma(turq_ctx *ctx, int count, const turq_weight *const *
         if (row1_ok) {
             const void *wp[4];
             int64_t nn[4];
-            int64_t rows = 0;
+            int64_t rows = 0, tiles = 0;
             for (int t = i; t < j; t++) {
                 wp[t - i] = w[t]->dev;
                 nn[t - i] = w[t]->n;
                 rows += w[t]->n;
+                tiles += turq_tile_rows(w[t]->n);
             }
+            const int rtiles = m == 1 ? pick_rows_row1(ctx, turq_tile_rows(rows)) : 1;
             hipEvent_t ev0 = nullptr, ev1 = nullptr;
             TURQ_HIP(ctx, turq_prof_next(ctx, &ev0, &ev1));
             TURQ_HIP(ctx, turq_launch_gemv_row1(w[i]->dtype, j - i, wp, nn, w[i]->k, x, xt, ldx, m, y + i, yt, ldy + i,
-                                                bias ? bias + i : nullptr, pick_waves_row1(w[i]->k),
-                                                m == 1 ? pick_rows_row1(ctx, turq_tile_rows(rows)) : 1, ctx->stream, ev0, ev1,
+                                                bias ? bias + i : nullptr, pick_waves_row1(ctx, w[i]->k, (tiles + rtiles - 1) / rtiles, rtiles), rtiles,
+                                                ctx->stream, ev0, ev1,
                                                 norm ? norm->w : nullptr, norm ? norm->eps : 0.0f));
             i = j;
             continue;
