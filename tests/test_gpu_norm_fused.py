@@ -221,3 +221,29 @@ def test_errors_are_reported(gpu):
     assert L.turq_norm_mlp(ctx, w, w, None, capi.ptr(x), capi.ACT_F32, 1, 256, capi.ptr(nw), EPS, capi.ptr(y), capi.ACT_F32, 64, None, None, None,
                            0, capi.MEM_HOST) == capi.ERR_INVALID
     gpu.release(w)
+
+
+# 3 .. 8 rows of 1024 .. 4096 columns: the kernels that stage the rows apply the norm on the way, bit-equal to the separate calls.  One to eight waves
+# (pairs of column tiles), four and eight rows with and without rows that are not there, every activation type, one and two formats in the launch,
+# a row of zeros, tiny and huge rows (f32), weight rows that end inside a row tile, one weight (in the staged kernels from five rows on).  k = 512 (the norm of short rows adds up in another order) and 9
+# rows go through scratch.
+@pytest.mark.parametrize("x_dtype", [capi.ACT_F32, capi.ACT_BF16, capi.ACT_F16], ids=["f32", "bf16", "f16"])
+@pytest.mark.parametrize("k,m", [(512, 4), (1024, 3), (1024, 8), (1536, 5), (2048, 9), (2048, 8), (3072, 4), (4096, 3), (4096, 4)])
+@pytest.mark.parametrize("fmts", [(Q8_0, Q8_0), (Q4_K, Q4_K, Q6_K), (Q5_K, Q6_K), (Q6_K,)])
+def test_norm_in_the_staged_kernels(gpu, fmts, k, m, x_dtype):
+    ns = [200, 48, 96][:len(fmts)]
+    ws = [gpu.upload(dt, n, k, synth.random_weight(dt, n, k, seed=n + k), capi.LAYOUT_TILED) for dt, n in zip(fmts, ns)]
+    rng = np.random.default_rng(k + m)
+    x = synth.random_activation(m, k, seed=m + k, bf16=x_dtype == capi.ACT_BF16)
+    if x_dtype == capi.ACT_F32:
+        x[0] *= np.float32(1e-12)
+        x[1] *= np.float32(3e5)
+    x[2] = 0.0
+    nw = (1.0 + 0.3 * rng.standard_normal(k)).astype(np.float32)
+    biases = [rng.standard_normal(n).astype(np.float32) for n in ns]
+    got = norm_multi(gpu, ws, ns, x, nw, x_dtype=x_dtype, biases=biases)
+    want, _ = separate(gpu, ws, ns, x, nw, x_dtype=x_dtype, biases=biases)
+    for a, b in zip(got, want):
+        assert np.array_equal(a, b)
+    for w in ws:
+        gpu.release(w)

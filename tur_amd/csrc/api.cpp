@@ -1,5 +1,6 @@
 // C ABI of libturq: contexts, device memory helpers, weight upload/export, dequantize, forward.
 #include <algorithm>
+#include <utility>
 #include <cmath>
 #include <memory>
 #include <new>
@@ -811,9 +812,18 @@ static int impl_norm_qmatmul_multi(turq_ctx *ctx, int count, const turq_weight *
     }
     bool plain = !(yt & ~0xFF) && turq_act_bytes(yt) && count <= 16;
     for (int i = 0; i < count && plain; i++) plain = weights[i] && ys[i] && ldys[i] >= weights[i]->n;
+    // (results over the rows they come from: the kernels that apply the norm themselves read the rows until their last workgroup has started)
+    const auto span = [m](const void *p, int64_t ld, int64_t cols, int type) {
+        const uintptr_t lo = (uintptr_t)p;
+        return std::pair<uintptr_t, uintptr_t>(lo, lo + (uintptr_t)((m - 1) * ld + cols) * (uintptr_t)turq_act_bytes(type));
+    };
+    for (int i = 0; i < count && plain && m > 1 && m <= TURQ_GEMV_MAX_M; i++) {
+        const auto in = span(x, ldx, k, xt), out = span(ys[i], ldys[i], weights[i]->n, yt);
+        plain = in.second <= out.first || out.second <= in.first;
+    }
     if (plain && turq_norm_fuses(ctx, count, weights, x, xt, ldx, m)) {
         const TurqNorm nm{nw, eps};
-        if (m == 1) return turq_qmatmul_multi_mfma(ctx, count, weights, x, xt, m, ldx, ys, yt, ldys, biases, &nm);
+        if (m <= TURQ_GEMV_MAX_M) return turq_qmatmul_multi_mfma(ctx, count, weights, x, xt, m, ldx, ys, yt, ldys, biases, &nm);
         bool taken = false;
         rc = turq_qmatmul_multi_gemm(ctx, count, weights, x, xt, m, ldx, ys, yt, ldys, biases, &taken, &nm);
         if (rc != TURQ_OK || taken) return rc;
@@ -845,8 +855,8 @@ static int impl_norm_mlp(turq_ctx *ctx, const turq_weight *gate, const turq_weig
     if (y && ldy >= down->n && turq_norm_fuses(ctx, 2, gu, x, xt, ldx, m)) {
         const TurqNorm nm{nw, eps};
         bool taken = false;
-        if (m == 1 && gate->dtype == up->dtype) {
-            // as turq_mlp's one-row route: the f16 intermediate where down_proj rounds its input to f16 anyway
+        if (m <= TURQ_GEMV_MAX_M && gate->dtype == up->dtype) {
+            // as turq_mlp's route for so few rows: the f16 intermediate where down_proj rounds its input to f16 anyway
             const bool h16 = turq_dt_is_quant(down->dtype) && down->layout == TURQ_LAYOUT_TILED && n_ff % 8 == 0;
             const int ht = h16 ? TURQ_ACT_F16 : TURQ_ACT_F32;
             rc = turq_ctx_reserve(ctx, &ctx->mlp_h, &ctx->mlp_h_cap, (size_t)m * (size_t)n_ff * (h16 ? sizeof(uint16_t) : sizeof(float)) + 16);

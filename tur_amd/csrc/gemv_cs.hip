@@ -216,12 +216,25 @@ bool turq_gemv_cs_staged_takes(int dtype_a, int dtype_b, int x_dtype, int64_t k,
 
 int turq_gemv_cs_staged_second_rows(int row_tiles) { return staged_second_rows(row_tiles); }
 
+// Whether a launch of `groups` workgroups applies RmsNorm itself: 1024 .. 4096 columns, one pair of column tiles per wave (fewer columns: the norm's
+// own kernel adds their squares up in another order), while what a compute unit spends on it - its workgroups times rows (4 or 8) times columns -
+// is less than the norm's launch.  Norm and products, launch of its own / inside: q, k and v of 4096 columns at 3 / 8 rows 9.4 / 9.9 us against 9.0 / 10.7, of
+// 2048 at 8 rows 7.1 / 6.3, of 1024 at 4 / 8 rows 6.1 / 6.3 against 4.1 / 5.7; MLPs 12288 x 4096 at 3 rows 28.1 / 26.5, 3072 x 1024 at 8 13.4 / 11.8, but 512
+// workgroups (8192 x 3072 at 4 rows) 22.9 / 25.8; at 16 rows it never pays (2048 columns 7.4 / 9.1).  dtype: the first format
+bool turq_gemv_cs_staged_norm_takes(int dtype, int64_t k, int64_t m, int row_tiles, int64_t groups, int64_t units) {
+    if (m < 3 || m > 8 || k % 512 != 0 || k < 1024 || k > 4096) return false;
+    const int64_t mr = m <= 4 ? 4 : 8;
+    return staged_norm_takes(dtype, (int)mr, row_tiles) && std::max(groups, units) * mr * k <= units * 16384;
+}
+
 // count (1..4) tiled weights of one k against m (1..32) activation rows of stride ldx (rows 16-byte aligned); the first `second`
 // weights are of format dtype_a, the others of dtype_b (second = count and dtype_b = dtype_a: one format); row_tiles per
 // workgroup as turq_gemv_cs_staged_takes accepts (the weights of a second format: turq_gemv_cs_staged_second_rows of it)
 hipError_t turq_launch_gemv_cs_staged(int dtype_a, int dtype_b, int count, int second, const void *const *w, const int64_t *n, int64_t k,
                                       const void *x, int x_dtype, int64_t ldx, int64_t m, void *const *y, int y_dtype, const int64_t *ldy,
-                                      const float *const *bias, int row_tiles, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop) {
+                                      const float *const *bias, int row_tiles, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop,
+                                      const float *norm_weight, float norm_eps) {
+    if (norm_weight && (m > 8 || k > 4096)) return hipErrorInvalidValue;
     if (count < 1 || count > kMaxMulti || second < 1 || second > count || (second == count) != (dtype_a == dtype_b) ||
         !turq_gemv_cs_staged_takes(dtype_a, dtype_b, x_dtype, k, m, row_tiles))
         return hipErrorInvalidValue;
@@ -256,7 +269,9 @@ int turq_gemv_cs_staged_gateup_tiles(int dtype, int64_t n, int64_t k, int64_t m,
 // activation rows of stride ldx (rows 16-byte aligned); tiles as turq_gemv_cs_staged_gateup_tiles says
 hipError_t turq_launch_gemv_cs_staged_gateup(int dtype, const void *w_gate, const void *w_up, int64_t n, int64_t k, const void *x, int x_dtype,
                                              int64_t ldx, int64_t m, void *y, int y_dtype, int64_t ldy, const float *bias_gate,
-                                             const float *bias_up, int tiles, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop) {
+                                             const float *bias_up, int tiles, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop,
+                                             const float *norm_weight, float norm_eps) {
+    if (norm_weight && (m > 8 || k > 4096)) return hipErrorInvalidValue;
     if (!turq_gemv_cs_staged_waves(k) || m < 1 || m > 32 || (tiles != 2 && tiles != 6) ||
         (m > 16 && k > 4096))
         return hipErrorInvalidValue;

@@ -36,22 +36,29 @@ constexpr int kXRow = 512 + 16;  // bytes per staged activation row: 256 f16 and
 template <int XT, int MR> struct XRows {
     uint4v v[XT == TURQ_ACT_F32 ? MR : MR / 2];
 };
+// The rows of an instruction's 64 lanes as a scalar address and 32-bit lane offsets (ldx below 2^30, which the dispatch asks for): one 64-bit
+// address per lane and row was about eight vector instructions for each load, ahead of the first weight.
+template <int XT> struct XOff {
+    uint32_t one, two;  // 16-bit rows: the lane's 16 bytes with both halves of the wave on one row, on two neighbouring ones
+    __device__ XOff(int64_t ldx, int lane) {
+        one = XT == TURQ_ACT_F32 ? 16u * (uint32_t)lane : 16u * (uint32_t)(lane & 31);
+        two = one + (XT != TURQ_ACT_F32 && lane >= 32 ? 2u * (uint32_t)ldx : 0u);
+    }
+};
 // rows row0 .. row0 + MR - 1 (rows past m repeat row m - 1) of column tile b
 template <int XT, int MR>
-__device__ inline XRows<XT, MR> load_x_rows(const void *__restrict__ x, int64_t ldx, int64_t m, int row0, int64_t b, int lane) {
+__device__ inline XRows<XT, MR> load_x_rows(const void *__restrict__ x, int64_t ldx, int64_t m, int row0, int64_t b, XOff<XT> o) {
     XRows<XT, MR> raw;
-    if constexpr (XT == TURQ_ACT_F32) {
+    constexpr int ES = XT == TURQ_ACT_F32 ? 4 : 2;
+    const uint8_t *base = (const uint8_t *)x + b * (256 * ES);
+    const int top = (int)m - 1;
+    asm volatile("" : "+v"(o.one), "+v"(o.two));  // (32-bit offsets next to the loads: see GOff)
 #pragma unroll
-        for (int j = 0; j < MR; j++) {
-            const int64_t row = row0 + j < m ? row0 + j : m - 1;
-            raw.v[j] = *(const uint4v *)((const uint8_t *)x + (row * ldx + b * 256) * 4 + 16 * lane);
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < MR / 2; i++) {
-            const int64_t j = row0 + 2 * i + (lane >> 5), row = j < m ? j : m - 1;
-            raw.v[i] = *(const uint4v *)((const uint8_t *)x + (row * ldx + b * 256) * 2 + 16 * (lane & 31));
-        }
+    for (int j = 0; j < MR; j += XT == TURQ_ACT_F32 ? 1 : 2) {
+        const int row = row0 + j < top ? row0 + j : top;
+        const uint8_t *p = base + (uint64_t)(uint32_t)row * (uint64_t)ldx * ES;
+        if constexpr (XT == TURQ_ACT_F32) raw.v[j] = *(const uint4v *)(p + o.one);
+        else raw.v[j / 2] = *(const uint4v *)(p + (row0 + j < top ? o.two : o.one));
     }
     return raw;
 }
@@ -74,6 +81,118 @@ template <int XT, int MR> __device__ inline void stage_x_rows(const XRows<XT, MR
         }
     }
 }
+// ---- RmsNorm on the way (3 .. 8 rows, one pair of column tiles per wave): the rows are normalised between the load and the rounding to f16, with
+// the bits that rms_norm_kernel leaves.  Every workgroup then works out the roots of all its rows (4.5 instructions per value, a barrier
+// while the first weights are on their way), against a launch of about 3 us: turq_gemv_cs_staged_norm_takes has where that pays.
+
+// eight values of a row, as a lane of 16-bit rows holds them
+template <int XT> __device__ inline void x_values(const uint4v &u, float (&f)[8]) {
+    const uint32_t wd[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        if constexpr (XT == TURQ_ACT_BF16) f[2 * j] = __uint_as_float(wd[j] << 16), f[2 * j + 1] = __uint_as_float(wd[j] & 0xFFFF0000u);
+        else f[2 * j] = (float)as_half2(wd[j]).x, f[2 * j + 1] = (float)as_half2(wd[j]).y;
+    }
+}
+// The wave's share of the rows' sums of squares, tree by tree as sq4 says: part[row][PW floats of this wave], added up later as (0 + 1) + (2 + 3)
+// for 16-bit rows, whose column tile is two rows of 16 lanes, and as the same with pairs of pairs for f32, whose tile is four.
+template <int XT> constexpr int kNormPart = XT == TURQ_ACT_F32 ? 8 : 4;
+template <int XT, int MR>
+__device__ inline void norm_part(const XRows<XT, MR> (&raw)[2], float *__restrict__ part, int nwaves, int wave, int lane) {
+    constexpr int PW = kNormPart<XT>;
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+        if constexpr (XT == TURQ_ACT_F32) {
+#pragma unroll
+            for (int j = 0; j < MR; j++) {
+                const uint4v a = raw[t].v[j];
+                const float q = sum16(sq4(__uint_as_float(a.x), __uint_as_float(a.y), __uint_as_float(a.z), __uint_as_float(a.w)));
+                if ((lane & 15) == 0) part[(j * nwaves + wave) * PW + 4 * t + (lane >> 4)] = q;
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < MR / 2; i++) {
+                float f[8];
+                x_values<XT>(raw[t].v[i], f);
+                const float q = sum16(sq4(f[0], f[1], f[2], f[3]) + sq4(f[4], f[5], f[6], f[7]));
+                if ((lane & 15) == 0) part[((2 * i + (lane >> 5)) * nwaves + wave) * PW + 2 * t + ((lane >> 4) & 1)] = q;
+            }
+        }
+    }
+}
+// Lane r: the root of row r, as RowDiv (norm.hip) uses it: quotient q = v * inv, corrected by (v - q * rms) * fix to the correctly rounded one.  Rows
+// whose root is 0, an infinity, a NaN or outside 2^-40 .. 2^40 go without the correction (an ulp).
+struct NormRoot { float inv, rms, fix; };
+template <int XT, int MR>
+__device__ inline NormRoot norm_root(const float *__restrict__ part, int nwaves, int lane, int64_t k, float eps) {
+    constexpr int PW = kNormPart<XT>;
+    const float *p = part + (lane & (MR - 1)) * nwaves * PW;
+    float4v a[8][PW / 4];  // (all at once: at most eight waves, the last one's again past it)
+#pragma unroll
+    for (int wv = 0; wv < 8; wv++)
+#pragma unroll
+        for (int h = 0; h < PW / 4; h++) a[wv][h] = *(const float4v *)(p + PW * (wv < nwaves ? wv : nwaves - 1) + 4 * h);
+    float total = 0.0f;
+#pragma unroll
+    for (int wv = 0; wv < 8; wv++) {
+        float b = (a[wv][0][0] + a[wv][0][1]) + (a[wv][0][2] + a[wv][0][3]);
+        if constexpr (XT == TURQ_ACT_F32) b += (a[wv][1][0] + a[wv][1][1]) + (a[wv][1][2] + a[wv][1][3]);
+        total = wv == 0 ? b : wv < nwaves ? total + b : total;
+    }
+    const float rms = sqrtf(total / (float)k + eps);
+    const bool plain = !(rms > 0x1p-40f && rms < 0x1p40f);
+    const float inv = 1.0f / rms;
+    return NormRoot{inv, plain ? 0.0f : rms, plain ? 0.0f : inv};
+}
+__device__ inline float norm_value(float v, float w, float inv, float rms, float fix) {
+    const float q = v * inv;
+    return __builtin_fmaf(__builtin_fmaf(-q, rms, v), fix, q) * w;
+}
+__device__ inline float lane_value(float v, int lane) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane)); }
+// the norm weights of a lane's columns of column tile b
+template <int XT> struct NormW { float4v v[XT == TURQ_ACT_F32 ? 1 : 2]; };
+template <int XT> __device__ inline NormW<XT> load_norm_w(const float *__restrict__ gw, int64_t b, int lane) {
+    NormW<XT> r;
+    const uint8_t *p = (const uint8_t *)gw + b * 1024;
+    if constexpr (XT == TURQ_ACT_F32) {
+        r.v[0] = *(const float4v *)(p + 16u * (uint32_t)lane);
+    } else {
+        const uint32_t o = 32u * (uint32_t)(lane & 31);
+        r.v[0] = *(const float4v *)(p + o), r.v[1] = *(const float4v *)(p + o + 16u);
+    }
+    return r;
+}
+// stage_x_rows of the normalised rows
+template <int XT, int MR>
+__device__ inline void stage_norm_rows(const XRows<XT, MR> &raw, const NormW<XT> &w, const NormRoot &root, uint8_t *__restrict__ rows, int lane) {
+    if constexpr (XT == TURQ_ACT_F32) {
+#pragma unroll
+        for (int j = 0; j < MR; j++) {
+            const float inv = lane_value(root.inv, j), rms = lane_value(root.rms, j), fix = lane_value(root.fix, j);
+            float f[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) f[e] = norm_value(__uint_as_float(raw.v[j][e]), w.v[0][e], inv, rms, fix);
+            const half2v h0 = __builtin_convertvector(float2v{f[0], f[1]}, half2v), h1 = __builtin_convertvector(float2v{f[2], f[3]}, half2v);
+            *(uint2v *)(rows + j * kXRow + 8 * lane) = uint2v{__builtin_bit_cast(uint32_t, h0), __builtin_bit_cast(uint32_t, h1)};
+        }
+    } else {
+        const bool up = lane >= 32;
+#pragma unroll
+        for (int i = 0; i < MR / 2; i++) {
+            const float inv = up ? lane_value(root.inv, 2 * i + 1) : lane_value(root.inv, 2 * i);
+            const float rms = up ? lane_value(root.rms, 2 * i + 1) : lane_value(root.rms, 2 * i);
+            const float fix = up ? lane_value(root.fix, 2 * i + 1) : lane_value(root.fix, 2 * i);
+            float f[8];
+            x_values<XT>(raw.v[i], f);
+            uint32_t h[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                h[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(float2v{norm_value(f[2 * e], w.v[e >> 1][(2 * e) & 3], inv, rms, fix),
+                                                                                    norm_value(f[2 * e + 1], w.v[e >> 1][(2 * e + 1) & 3], inv, rms, fix)}, half2v));
+            *(uint4v *)(rows + (2 * i + (lane >> 5)) * kXRow + 16 * (lane & 31)) = uint4v{h[0], h[1], h[2], h[3]};
+        }
+    }
+}
 // the A fragments of the staged column tile: lane (r, g) holds row r (rows past m repeat row m - 1);
 // K-quants: step q = columns 64 g + 8 q .. + 7, step 8 = the (hi, lo) sums of its four 16-column groups; Q8_0: step q = columns 32 q + 8 g .. + 7
 template <int DT> __device__ inline void frags_from_staged(const uint8_t *__restrict__ rows, int m, int lane, half8v *__restrict__ out) {
@@ -93,12 +212,14 @@ template <int DT> __device__ inline void frags_from_staged(const uint8_t *__rest
 // is stored is silu(gate) * up (src/models/qwen3.rs:161-167).
 // CNT: pairs per wave when every wave has the same number and it is known at compile time (the loop is then written out, which
 // is 1 - 5 % faster on the 4096-column weights), 0: counted at run time.
-template <int DT, int XT, int MR, int RG, int D, int CNT, bool GU = false>
+// NORM (CNT 1, one pass): x stands for RmsNorm(x) with weight gw
+template <int DT, int XT, int MR, int RG, int D, int CNT, bool GU = false, bool NORM = false>
 __device__ __forceinline__ void cs_body_staged(const uint8_t *__restrict__ w, int64_t n, int64_t k, const void *__restrict__ x, int64_t ldx,
                                                int64_t m, void *__restrict__ y, int yt, int64_t ldy, const float *__restrict__ bias,
                                                int64_t grp, const uint8_t *__restrict__ w2 = nullptr,
-                                               const float *__restrict__ bias2 = nullptr) {
+                                               const float *__restrict__ bias2 = nullptr, const float *__restrict__ gw = nullptr, float eps = 0.0f) {
     static_assert(!GU || RG % 2 == 0, "gate and up tiles come in pairs");
+    static_assert(!NORM || (CNT == 1 && MR <= 8), "the norm inside the kernel: every wave holds its share of the rows at once");
     constexpr int RO = GU ? RG / 2 : RG;  // row tiles of the output per workgroup
     constexpr int HV = MR > 16 ? 2 : 1;   // passes of HR rows each
     constexpr int HR = MR / HV;
@@ -108,9 +229,9 @@ __device__ __forceinline__ void cs_body_staged(const uint8_t *__restrict__ w, in
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int nwaves = blockDim.x >> 6;  // at most ntc / 2
-    const int64_t ntc = turq_tile_cols(k), nrt = turq_tile_rows(n);
-    const int cnt = __builtin_amdgcn_readfirstlane((int)((ntc / 2 - wave + nwaves - 1) / nwaves));  // the wave's pairs
-    const int64_t rt0 = grp * RO;
+    const uint32_t ntc = (uint32_t)turq_tile_cols(k), nrt = (uint32_t)turq_tile_rows(n);
+    const int cnt = __builtin_amdgcn_readfirstlane(((int)(ntc / 2) - wave + nwaves - 1) / nwaves);  // the wave's pairs
+    const uint32_t rt0 = (uint32_t)grp * RO;
     float4v acc[RG][HV];
     const uint8_t *wrow[RG];  // row tiles past the weight's last one re-read it; their results are not stored
 #pragma unroll
@@ -118,29 +239,48 @@ __device__ __forceinline__ void cs_body_staged(const uint8_t *__restrict__ w, in
 #pragma unroll
         for (int h = 0; h < HV; h++) acc[r][h] = float4v{0.f, 0.f, 0.f, 0.f};
         const int ro = r < RO ? r : r - RO;
-        wrow[r] = (r < RO ? w : w2) + (rt0 + ro < nrt ? rt0 + ro : nrt - 1) * ntc * TB;
+        wrow[r] = (r < RO ? w : w2) + (uint64_t)((RO == 1 || rt0 + ro < nrt ? rt0 + ro : nrt - 1) * ntc) * TB;
     }
     GOff go = lane_offsets(lane, 16);
     int64_t p = wave;  // the current pair: column tiles 2 p and 2 p + 1
-    // the first column tile's rows go out first, the first D weight tiles right behind them
-    XRows<XT, HR> raw = load_x_rows<XT, HR>(x, ldx, m, 0, 2 * p, lane);
+    const XOff<XT> xo(ldx, lane);
+    // the first column tile's rows go out first (for the norm: those of both, and its weights), the first D weight tiles right behind them
+    XRows<XT, HR> raw = load_x_rows<XT, HR>(x, ldx, m, 0, 2 * p, xo);
+    [[maybe_unused]] XRows<XT, HR> raw2;
+    [[maybe_unused]] NormW<XT> nw[2];
+    if constexpr (NORM) {
+        raw2 = load_x_rows<XT, HR>(x, ldx, m, 0, 2 * p + 1, xo);
+        nw[0] = load_norm_w<XT>(gw, 2 * p, lane), nw[1] = load_norm_w<XT>(gw, 2 * p + 1, lane);
+    }
     WRegs<DT> wr[D];
 #pragma unroll
     for (int d = 0; d < D; d++) wr[d] = load_tile<DT>(wrow[d % RG] + (2 * p + d / RG) * TB, go);
     uint8_t *rows = smem + wave * (HR * kXRow);
     AFrags<DT, 1> f;
+    [[maybe_unused]] NormRoot root;
+    if constexpr (NORM) {
+        __builtin_amdgcn_sched_barrier(0);
+        float *part = (float *)(smem + (size_t)nwaves * (HR * kXRow));
+        const XRows<XT, HR> both[2] = {raw, raw2};
+        norm_part<XT, HR>(both, part, nwaves, wave, lane);
+        __syncthreads();
+        root = norm_root<XT, HR>(part, nwaves, lane, k, eps);
+    }
     auto pair = [&](auto last) {
         constexpr bool LAST = decltype(last)::value;
 #pragma unroll
         for (int cc = 0; cc < 2; cc++) {
 #pragma unroll
             for (int h = 0; h < HV; h++) {
-                stage_x_rows<XT, HR>(raw, rows, lane);
+                if constexpr (NORM) stage_norm_rows<XT, HR>(cc ? raw2 : raw, nw[cc], root, rows, lane);
+                else stage_x_rows<XT, HR>(raw, rows, lane);
                 __builtin_amdgcn_sched_barrier(0);
                 // the rows of the next pass: the other half of this column tile, the pair's second column tile, the next pair
-                if (h + 1 < HV) raw = load_x_rows<XT, HR>(x, ldx, m, HR * (h + 1), 2 * p + cc, lane);
-                else if (cc == 0) raw = load_x_rows<XT, HR>(x, ldx, m, 0, 2 * p + 1, lane);
-                else if (!LAST) raw = load_x_rows<XT, HR>(x, ldx, m, 0, 2 * (p + nwaves), lane);
+                if constexpr (!NORM) {
+                    if (h + 1 < HV) raw = load_x_rows<XT, HR>(x, ldx, m, HR * (h + 1), 2 * p + cc, xo);
+                    else if (cc == 0) raw = load_x_rows<XT, HR>(x, ldx, m, 0, 2 * p + 1, xo);
+                    else if (!LAST) raw = load_x_rows<XT, HR>(x, ldx, m, 0, 2 * (p + nwaves), xo);
+                }
                 __builtin_amdgcn_sched_barrier(0);
                 frags_from_staged<DT>(rows, (int)m - HR * h, lane, f.a[0]);
 #pragma unroll
@@ -196,7 +336,7 @@ __device__ __forceinline__ void cs_body_staged(const uint8_t *__restrict__ w, in
             s2 = red[(i2 * nwaves) * 64 + lane];
             for (int wv = 1; wv < nwaves; wv++) s2 += red[(i2 * nwaves + wv) * 64 + lane];
         }
-        const int64_t col = (rt0 + r) * 16 + nn;
+        const int64_t col = (int64_t)(rt0 + r) * 16 + nn;
         if (rt0 + r >= nrt || col >= n) continue;
         const float bv = bias ? bias[col] : 0.0f, bv2 = (GU && bias2) ? bias2[col] : 0.0f;
         if constexpr (GU) {
@@ -228,22 +368,27 @@ constexpr int staged_second_rows(int rg) { return (rg + 1) / 2; }
 
 // weights [0, a.second) are of format DTA with RG row tiles per workgroup, the others of DTB with staged_second_rows(RG)
 // (one format: DTA == DTB)
-template <int DTA, int DTB, int XT, int MR, int RG, int CNT>
-__global__ void __launch_bounds__(512) gemv_cs_staged_kernel(MultiArgs a, int64_t k, const void *__restrict__ x, int64_t ldx, int64_t m, int yt) {
+template <int DTA, int DTB, int XT, int MR, int RG, int CNT, bool NORM = false>
+__global__ void __launch_bounds__(512) gemv_cs_staged_kernel(MultiArgs a, int64_t k, const void *__restrict__ x, int64_t ldx, int64_t m, int yt,
+                                                             const float *__restrict__ gw, float eps) {
+    load_together(k, x, ldx, m, yt, gw, eps);
     const MultiPick p = multi_pick(a, (int)blockIdx.x);
     constexpr int RGB = staged_second_rows(RG);
     if (DTA == DTB || p.index < a.second)
-        cs_body_staged<DTA, XT, MR, RG, staged_ring(DTA, RG, MR, DTA != DTB), CNT>(p.w, p.n, k, x, ldx, m, p.y, yt, p.ldy, p.bias, (int64_t)p.block);
+        cs_body_staged<DTA, XT, MR, RG, staged_ring(DTA, RG, MR, DTA != DTB), CNT, false, NORM>(p.w, p.n, k, x, ldx, m, p.y, yt, p.ldy, p.bias,
+                                                                                               (int64_t)p.block, nullptr, nullptr, gw, eps);
     else
-        cs_body_staged<DTB, XT, MR, RGB, staged_ring(DTB, RGB, MR, DTA != DTB), CNT>(p.w, p.n, k, x, ldx, m, p.y, yt, p.ldy, p.bias, (int64_t)p.block);
+        cs_body_staged<DTB, XT, MR, RGB, staged_ring(DTB, RGB, MR, DTA != DTB), CNT, false, NORM>(p.w, p.n, k, x, ldx, m, p.y, yt, p.ldy, p.bias,
+                                                                                                 (int64_t)p.block, nullptr, nullptr, gw, eps);
 }
 
 // gate (a.w[0]) and up (a.w[1]) of one MLP, RG / 2 row tiles of each per workgroup, silu(gate) * up stored to a.y[0]
-template <int DT, int XT, int MR, int RG, int CNT>
+template <int DT, int XT, int MR, int RG, int CNT, bool NORM = false>
 __global__ void __launch_bounds__(512) gemv_cs_staged_gateup_kernel(MultiArgs a, int64_t k, const void *__restrict__ x, int64_t ldx, int64_t m,
-                                                                     int yt) {
-    cs_body_staged<DT, XT, MR, RG, staged_ring(DT, RG, MR), CNT, true>(a.w[0], a.n[0], k, x, ldx, m, a.y[0], yt, a.ldy[0], a.bias[0],
-                                                               (int64_t)blockIdx.x, a.w[1], a.bias[1]);
+                                                                     int yt, const float *__restrict__ gw, float eps) {
+    load_together(a.w[0], a.w[1], a.n[0], k, x, ldx, m, a.y[0], yt, a.ldy[0], a.bias[0], a.bias[1], gw, eps);
+    cs_body_staged<DT, XT, MR, RG, staged_ring(DT, RG, MR), CNT, true, NORM>(a.w[0], a.n[0], k, x, ldx, m, a.y[0], yt, a.ldy[0], a.bias[0],
+                                                                     (int64_t)blockIdx.x, a.w[1], a.bias[1], gw, eps);
 }
 
 // ---- 17 .. 32 rows, both 16-row tiles against ONE unpack of a weight tile ----
@@ -266,22 +411,23 @@ __device__ __forceinline__ void cs_body_staged_two(const uint8_t *__restrict__ w
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int nwaves = blockDim.x >> 6;  // at most ntc / 2
-    const int64_t ntc = turq_tile_cols(k), nrt = turq_tile_rows(n);
-    const int cnt = __builtin_amdgcn_readfirstlane((int)((ntc / 2 - wave + nwaves - 1) / nwaves));  // the wave's pairs
-    const int64_t rt0 = grp * RO;
+    const uint32_t ntc = (uint32_t)turq_tile_cols(k), nrt = (uint32_t)turq_tile_rows(n);
+    const int cnt = __builtin_amdgcn_readfirstlane(((int)(ntc / 2) - wave + nwaves - 1) / nwaves);  // the wave's pairs
+    const uint32_t rt0 = (uint32_t)grp * RO;
     float4v acc[RG][2];
     const uint8_t *wrow[RG];  // row tiles past the weight's last one re-read it; their results are not stored
 #pragma unroll
     for (int r = 0; r < RG; r++) {
         acc[r][0] = acc[r][1] = float4v{0.f, 0.f, 0.f, 0.f};
         const int ro = r < RO ? r : r - RO;
-        wrow[r] = (r < RO ? w : w2) + (rt0 + ro < nrt ? rt0 + ro : nrt - 1) * ntc * TB;
+        wrow[r] = (r < RO ? w : w2) + (uint64_t)((rt0 + ro < nrt ? rt0 + ro : nrt - 1) * ntc) * TB;
     }
     GOff go = lane_offsets(lane, 16);
     int64_t p = wave;
+    const XOff<XT> xo(ldx, lane);
     XRows<XT, 16> raw[2];
 #pragma unroll
-    for (int mt = 0; mt < 2; mt++) raw[mt] = load_x_rows<XT, 16>(x, ldx, m, 16 * mt, 2 * p, lane);
+    for (int mt = 0; mt < 2; mt++) raw[mt] = load_x_rows<XT, 16>(x, ldx, m, 16 * mt, 2 * p, xo);
     WRegs<DT> wr[D];
 #pragma unroll
     for (int d = 0; d < D; d++) wr[d] = load_tile<DT>(wrow[d % RG] + (2 * p + d / RG) * TB, go);
@@ -297,7 +443,7 @@ __device__ __forceinline__ void cs_body_staged_two(const uint8_t *__restrict__ w
             if (cc == 0 || !LAST) {
                 const int64_t b = cc == 0 ? 2 * p + 1 : 2 * (p + nwaves);
 #pragma unroll
-                for (int mt = 0; mt < 2; mt++) raw[mt] = load_x_rows<XT, 16>(x, ldx, m, 16 * mt, b, lane);
+                for (int mt = 0; mt < 2; mt++) raw[mt] = load_x_rows<XT, 16>(x, ldx, m, 16 * mt, b, xo);
             }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -344,7 +490,7 @@ __device__ __forceinline__ void cs_body_staged_two(const uint8_t *__restrict__ w
             s2 = red[(i2 * nwaves) * 64 + lane];
             for (int wv = 1; wv < nwaves; wv++) s2 += red[(i2 * nwaves + wv) * 64 + lane];
         }
-        const int64_t col = (rt0 + r) * 16 + nn;
+        const int64_t col = (int64_t)(rt0 + r) * 16 + nn;
         if (rt0 + r >= nrt || col >= n) continue;
         const float bv = bias ? bias[col] : 0.0f, bv2 = (GU && bias2) ? bias2[col] : 0.0f;
         if constexpr (GU) {
@@ -364,7 +510,8 @@ __device__ __forceinline__ void cs_body_staged_two(const uint8_t *__restrict__ w
 // four waves; weights [0, a.second) of format DTA, the others of DTB with staged_second_rows(6) row tiles per workgroup
 template <int DTA, int DTB, int XT, int CNT>
 __global__ void __launch_bounds__(256) gemv_cs_staged_two_kernel(MultiArgs a, int64_t k, const void *__restrict__ x, int64_t ldx, int64_t m,
-                                                                  int yt) {
+                                                                  int yt, const float *, float) {
+    load_together(k, x, ldx, m, yt);
     const MultiPick p = multi_pick(a, (int)blockIdx.x);
     constexpr int RGB = staged_second_rows(6);
     if (DTA == DTB || p.index < a.second) cs_body_staged_two<DTA, XT, 6, 3, CNT>(p.w, p.n, k, x, ldx, m, p.y, yt, p.ldy, p.bias, (int64_t)p.block);
@@ -374,7 +521,8 @@ __global__ void __launch_bounds__(256) gemv_cs_staged_two_kernel(MultiArgs a, in
 // ... gate (a.w[0]) and up (a.w[1]) of one MLP, three row tiles of each per workgroup, silu(gate) * up stored to a.y[0]
 template <int DT, int XT, int CNT>
 __global__ void __launch_bounds__(256) gemv_cs_staged_two_gateup_kernel(MultiArgs a, int64_t k, const void *__restrict__ x, int64_t ldx,
-                                                                         int64_t m, int yt) {
+                                                                         int64_t m, int yt, const float *, float) {
+    load_together(a.w[0], a.w[1], a.n[0], k, x, ldx, m, a.y[0], yt, a.ldy[0], a.bias[0], a.bias[1]);
     cs_body_staged_two<DT, XT, 6, 3, CNT, true>(a.w[0], a.n[0], k, x, ldx, m, a.y[0], yt, a.ldy[0], a.bias[0], (int64_t)blockIdx.x, a.w[1],
                                            a.bias[1]);
 }
@@ -390,7 +538,12 @@ struct StagedLaunch {
     hipEvent_t ev0, ev1;
     bool two;  // the four-wave form for 17 .. 32 rows
     int cnt;   // pairs of column tiles per wave if that is the same number for every wave, else 0
+    const float *gw;  // RmsNorm weight (null: the rows are taken as they are) and eps
+    float eps;
 };
+
+// the kernels that apply the norm themselves: up to 8 rows (six row tiles of Q8_0, the largest, do not fit the registers next to two column tiles of rows)
+constexpr bool staged_norm_takes(int dt, int mr, int rg) { return mr <= 8 && (dt != TURQ_Q8_0 || rg <= 3); }
 
 // launches `kernel` with lds bytes of dynamic LDS (more than 64 KiB: raised once per kernel)
 template <auto kernel>
@@ -401,24 +554,30 @@ hipError_t staged_go(size_t lds, const StagedLaunch &l) {
     }
     const dim3 grid((unsigned)l.blocks), block((unsigned)(64 * l.nwaves));
     if (l.ev0) {
-        hipExtLaunchKernelGGL(kernel, grid, block, (unsigned)lds, l.s, l.ev0, l.ev1, 0, l.a, l.k, l.x, l.ldx, l.m, l.yt);
+        hipExtLaunchKernelGGL(kernel, grid, block, (unsigned)lds, l.s, l.ev0, l.ev1, 0, l.a, l.k, l.x, l.ldx, l.m, l.yt, l.gw, l.eps);
         return hipGetLastError();
     }
-    kernel<<<grid, block, lds, l.s>>>(l.a, l.k, l.x, l.ldx, l.m, l.yt);
+    kernel<<<grid, block, lds, l.s>>>(l.a, l.k, l.x, l.ldx, l.m, l.yt, l.gw, l.eps);
     return hipGetLastError();
 }
 
-template <int MR, int RG> size_t staged_lds(int nwaves) {
+template <int MR, int RG> size_t staged_lds(int nwaves, bool norm) {
     constexpr int HV = MR > 16 ? 2 : 1;
-    return std::max((size_t)nwaves * (MR / HV) * kXRow, (size_t)nwaves * RG * HV * 64 * sizeof(float4v));
+    return std::max((size_t)nwaves * (MR / HV) * (kXRow + (norm ? 32 : 0)), (size_t)nwaves * RG * HV * 64 * sizeof(float4v));  // (norm: kNormPart floats a row)
 }
 
 // one pair per wave (up to 4096 columns) written out, anything else counted at run time; more than 16 rows of f32 are only taken on
 // up to 4096 columns (turq_gemv_cs_staged_takes)
 template <int DTA, int DTB, int XT, int MR, int RG>
 hipError_t staged_count(const StagedLaunch &l) {
-    if (l.cnt == 1) return staged_go<gemv_cs_staged_kernel<DTA, DTB, XT, MR, RG, 1>>(staged_lds<MR, RG>(l.nwaves), l);
-    if constexpr (MR <= 16 || XT != TURQ_ACT_F32) return staged_go<gemv_cs_staged_kernel<DTA, DTB, XT, MR, RG, 0>>(staged_lds<MR, RG>(l.nwaves), l);
+    if (l.gw) {
+        if constexpr (staged_norm_takes(DTA, MR, RG)) {
+            if (l.cnt == 1) return staged_go<gemv_cs_staged_kernel<DTA, DTB, XT, MR, RG, 1, true>>(staged_lds<MR, RG>(l.nwaves, true), l);
+        }
+        return hipErrorInvalidValue;
+    }
+    if (l.cnt == 1) return staged_go<gemv_cs_staged_kernel<DTA, DTB, XT, MR, RG, 1>>(staged_lds<MR, RG>(l.nwaves, false), l);
+    if constexpr (MR <= 16 || XT != TURQ_ACT_F32) return staged_go<gemv_cs_staged_kernel<DTA, DTB, XT, MR, RG, 0>>(staged_lds<MR, RG>(l.nwaves, false), l);
     return hipErrorInvalidValue;
 }
 
@@ -441,7 +600,7 @@ template <int DTA, int DTB, int XT>
 hipError_t staged_rows(int rg, const StagedLaunch &l) {
     if (l.two) {
         const size_t lds = std::max((size_t)l.nwaves * 32 * kXRow, (size_t)l.nwaves * 12 * 1024);
-        if (rg != 6) return hipErrorInvalidValue;
+        if (rg != 6 || l.gw) return hipErrorInvalidValue;
         return l.cnt == 2 ? staged_go<gemv_cs_staged_two_kernel<DTA, DTB, XT, 2>>(lds, l) : staged_go<gemv_cs_staged_two_kernel<DTA, DTB, XT, 0>>(lds, l);
     }
     if (l.m <= 4) return staged_shape<DTA, DTB, XT, 4>(rg, l);
@@ -452,8 +611,14 @@ hipError_t staged_rows(int rg, const StagedLaunch &l) {
 
 template <int DT, int XT, int MR, int RG>
 hipError_t staged_gateup_count(const StagedLaunch &l) {
-    if (l.cnt == 1) return staged_go<gemv_cs_staged_gateup_kernel<DT, XT, MR, RG, 1>>(staged_lds<MR, RG>(l.nwaves), l);
-    if constexpr (MR <= 16) return staged_go<gemv_cs_staged_gateup_kernel<DT, XT, MR, RG, 0>>(staged_lds<MR, RG>(l.nwaves), l);
+    if (l.gw) {
+        if constexpr (staged_norm_takes(DT, MR, RG)) {
+            if (l.cnt == 1) return staged_go<gemv_cs_staged_gateup_kernel<DT, XT, MR, RG, 1, true>>(staged_lds<MR, RG>(l.nwaves, true), l);
+        }
+        return hipErrorInvalidValue;
+    }
+    if (l.cnt == 1) return staged_go<gemv_cs_staged_gateup_kernel<DT, XT, MR, RG, 1>>(staged_lds<MR, RG>(l.nwaves, false), l);
+    if constexpr (MR <= 16) return staged_go<gemv_cs_staged_gateup_kernel<DT, XT, MR, RG, 0>>(staged_lds<MR, RG>(l.nwaves, false), l);
     return hipErrorInvalidValue;
 }
 
@@ -462,7 +627,7 @@ template <int DT, int XT>
 hipError_t staged_gateup_shape(int rg, const StagedLaunch &l) {
     if (l.two) {
         const size_t lds = std::max((size_t)l.nwaves * 32 * kXRow, (size_t)l.nwaves * 12 * 1024);
-        if (rg != 6) return hipErrorInvalidValue;
+        if (rg != 6 || l.gw) return hipErrorInvalidValue;
         return l.cnt == 2 ? staged_go<gemv_cs_staged_two_gateup_kernel<DT, XT, 2>>(lds, l) : staged_go<gemv_cs_staged_two_gateup_kernel<DT, XT, 0>>(lds, l);
     }
     if (rg == 2)
@@ -493,7 +658,7 @@ inline int turq_gemv_cs_staged_two_waves(int64_t k, int64_t m, int row_tiles) {
 template <int XT>
 hipError_t staged_launch(int dtype_a, int dtype_b, int count, int second, const void *const *w, const int64_t *n, int64_t k, const void *x,
                          int64_t ldx, int64_t m, void *const *y, int y_dtype, const int64_t *ldy, const float *const *bias, int row_tiles,
-                         hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop) {
+                         hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop, const float *norm_weight, float norm_eps) {
     const int two = turq_gemv_cs_staged_two_waves(k, m, row_tiles);
     StagedLaunch l{};
     l.two = two != 0;
@@ -515,7 +680,7 @@ hipError_t staged_launch(int dtype_a, int dtype_b, int count, int second, const 
     if (blocks == 0) return hipSuccess;
     if (blocks > 0x7FFFFFFF) return hipErrorInvalidValue;
     l.blocks = (int)blocks, l.k = k, l.x = x, l.ldx = ldx, l.m = m, l.yt = y_dtype;
-    l.s = stream, l.ev0 = ev_start, l.ev1 = ev_stop;
+    l.s = stream, l.ev0 = ev_start, l.ev1 = ev_stop, l.gw = norm_weight, l.eps = norm_eps;
     if (dtype_a == TURQ_Q4_K && dtype_b == TURQ_Q6_K) return staged_rows<TURQ_Q4_K, TURQ_Q6_K, XT>(row_tiles, l);
     if (dtype_a == TURQ_Q5_K && dtype_b == TURQ_Q6_K) return staged_rows<TURQ_Q5_K, TURQ_Q6_K, XT>(row_tiles, l);
     switch (dtype_a) {
@@ -531,7 +696,7 @@ hipError_t staged_launch(int dtype_a, int dtype_b, int count, int second, const 
 template <int XT>
 hipError_t staged_gateup_launch(int dtype, const void *w_gate, const void *w_up, int64_t n, int64_t k, const void *x, int64_t ldx, int64_t m,
                                 void *y, int y_dtype, int64_t ldy, const float *bias_gate, const float *bias_up, int tiles,
-                                hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop) {
+                                hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop, const float *norm_weight, float norm_eps) {
     const int two = turq_gemv_cs_staged_two_waves(k, m, tiles);
     StagedLaunch l{};
     l.two = two != 0;
@@ -544,7 +709,7 @@ hipError_t staged_gateup_launch(int dtype, const void *w_gate, const void *w_up,
     if (blocks == 0) return hipSuccess;
     if (blocks > 0x7FFFFFFF) return hipErrorInvalidValue;
     l.blocks = (int)blocks, l.k = k, l.x = x, l.ldx = ldx, l.m = m, l.yt = y_dtype;
-    l.s = stream, l.ev0 = ev_start, l.ev1 = ev_stop;
+    l.s = stream, l.ev0 = ev_start, l.ev1 = ev_stop, l.gw = norm_weight, l.eps = norm_eps;
     switch (dtype) {
     case TURQ_Q4_K: return staged_gateup_shape<TURQ_Q4_K, XT>(tiles, l);
     case TURQ_Q5_K: return staged_gateup_shape<TURQ_Q5_K, XT>(tiles, l);
@@ -556,11 +721,12 @@ hipError_t staged_gateup_launch(int dtype, const void *w_gate, const void *w_up,
 
 #define TURQ_STAGED_GATEUP_ARGS                                                                                                          \
     int dtype, const void *w_gate, const void *w_up, int64_t n, int64_t k, const void *x, int64_t ldx, int64_t m, void *y, int y_dtype,  \
-        int64_t ldy, const float *bias_gate, const float *bias_up, int tiles, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop
-#define TURQ_STAGED_GATEUP_PASS dtype, w_gate, w_up, n, k, x, ldx, m, y, y_dtype, ldy, bias_gate, bias_up, tiles, stream, ev_start, ev_stop
+        int64_t ldy, const float *bias_gate, const float *bias_up, int tiles, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop,    \
+        const float *norm_weight, float norm_eps
+#define TURQ_STAGED_GATEUP_PASS dtype, w_gate, w_up, n, k, x, ldx, m, y, y_dtype, ldy, bias_gate, bias_up, tiles, stream, ev_start, ev_stop, norm_weight, norm_eps
 
 #define TURQ_STAGED_LAUNCH_ARGS                                                                                                          \
     int dtype_a, int dtype_b, int count, int second, const void *const *w, const int64_t *n, int64_t k, const void *x, int64_t ldx,      \
         int64_t m, void *const *y, int y_dtype, const int64_t *ldy, const float *const *bias, int row_tiles, hipStream_t stream,         \
-        hipEvent_t ev_start, hipEvent_t ev_stop
-#define TURQ_STAGED_LAUNCH_PASS dtype_a, dtype_b, count, second, w, n, k, x, ldx, m, y, y_dtype, ldy, bias, row_tiles, stream, ev_start, ev_stop
+        hipEvent_t ev_start, hipEvent_t ev_stop, const float *norm_weight, float norm_eps
+#define TURQ_STAGED_LAUNCH_PASS dtype_a, dtype_b, count, second, w, n, k, x, ldx, m, y, y_dtype, ldy, bias, row_tiles, stream, ev_start, ev_stop, norm_weight, norm_eps

@@ -31,7 +31,6 @@
 
 #include <algorithm>
 #include <climits>
-#include <initializer_list>
 
 #include "layout.h"
 #include "mfma_common.h"
@@ -48,23 +47,6 @@ constexpr int kX = 0, kInit = 512, kZero = 576, kRegion = 640;
 // LDS region of one (wave, tile in flight, PAIR of activation rows) in the packed form, where the sixteen A rows of an MFMA are
 // eight sub-blocks x two activation rows: 2 x 256 f16 of x, 16 start values, 16 sums of x (for the mins), 64 bytes of zeros
 constexpr int kPX = 0, kPInit = 1024, kPSum = 1088, kPZero = 1152, kPairRegion = 1216;
-
-// v + (the same value from the lane `CTRL` points at), inside a row of 16 lanes
-template <int CTRL> __device__ inline float dpp_add(float v) {
-    const int o = __builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false);
-    return v + __int_as_float(o);
-}
-__device__ inline float sum4(float v) {
-    v = dpp_add<0xB1>(v);  // quad_perm [1, 0, 3, 2]
-    return dpp_add<0x4E>(v);  // quad_perm [2, 3, 0, 1]
-}
-// row_half_mirror: lane i <- lane 7 - i of its half row.  The result is pinned here: the callers store it from one lane in eight,
-// and an add that the compiler sinks into that branch no longer merges with its DPP move.
-__device__ inline float sum8(float v) {
-    float r = dpp_add<0x141>(sum4(v));
-    asm volatile("" : "+v"(r));
-    return r;
-}
 
 __device__ inline float dot2(half2v a, _Float16 b0, float c) { return __builtin_amdgcn_fdot2(a, splat2(b0), c, false); }
 
@@ -335,13 +317,6 @@ __device__ inline void stage_x1(const X1Regs<XT> &v, uint8_t *region, int lane) 
     Row1Fmt<DT>::sums(h01, h23, region, lane);
 }
 
-// the sum over the 64 lanes, in every lane
-__device__ inline float sum64(float v) {
-    float r = dpp_add<0x140>(sum8(v));  // row_mirror: lane i <- lane 15 - i of its row
-    asm volatile("" : "+v"(r));
-    auto row = [&](int i) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r), 16 * i)); };
-    return (row(0) + row(1)) + (row(2) + row(3));
-}
 // The sums over the waves of what each has left 64 floats apart from the next, in wave order, for N such runs together.  Eight reads of each at a
 // time, those past the last wave dropped: a wait per read, as a loop over the waves makes it, was half of what the end of a small launch took.
 template <int N> __device__ inline void sum_waves(const float *const (&p)[N], int nwaves, float (&s)[N]) {
@@ -652,11 +627,6 @@ __device__ __forceinline__ void row1_body(const uint8_t *__restrict__ w, void *_
             turq_store_any(y, yt, (int64_t)mm * ldy + col, value(s0, s1, bias ? bias[col] : 0.0f, GU && bias2 ? bias2[col] : 0.0f));
     }
 }
-
-// A launch's arguments are two hundred bytes that no cache holds when it starts.  Left to itself the compiler loads each where it is first used,
-// behind the branches that pick the weight: five scalar loads one after the other, each a round trip, before the first weight is
-// requested.  Naming them here makes them one.
-template <class... T> __device__ inline void load_together(T... v) { (void)std::initializer_list<int>{([](auto u) { asm volatile("" ::"s"(u)); }(v), 0)...}; }
 
 // which weight of the launch this workgroup works on
 struct Row1Pick { const uint8_t *w; void *y; const float *bias; int64_t n, ldy; int first; int index; };

@@ -374,9 +374,14 @@ struct MultiArgs {
 struct MultiPick { const uint8_t *w; void *y; const float *bias; int64_t n, ldy; int block; int index; };
 __device__ inline MultiPick multi_pick(const MultiArgs &a, int blk) {
     MultiPick p{a.w[0], a.y[0], a.bias[0], a.n[0], a.ldy[0], blk, 0};
+    load_together(a.w[0], a.w[1], a.w[2], a.w[3], a.y[0], a.y[1], a.y[2], a.y[3], a.bias[0], a.bias[1], a.bias[2], a.bias[3], a.n[0], a.n[1], a.n[2], a.n[3],
+                  a.ldy[0], a.ldy[1], a.ldy[2], a.ldy[3], a.first[1], a.first[2], a.first[3], a.count, a.second);
 #pragma unroll
-    for (int i = 1; i < kMaxMulti; i++)
-        if (i < a.count && blk >= a.first[i]) p = MultiPick{a.w[i], a.y[i], a.bias[i], a.n[i], a.ldy[i], blk - a.first[i], i};
+    for (int i = 1; i < kMaxMulti; i++) {  // (selects, no branches)
+        const bool in = i < a.count && blk >= a.first[i];
+        p.w = in ? a.w[i] : p.w, p.y = in ? a.y[i] : p.y, p.bias = in ? a.bias[i] : p.bias;
+        p.n = in ? a.n[i] : p.n, p.ldy = in ? a.ldy[i] : p.ldy, p.block = in ? blk - a.first[i] : p.block, p.index = in ? i : p.index;
+    }
     return p;
 }
 

@@ -24,6 +24,7 @@
 // mpad is the m-tile height rounded up to 1, 2, 4, 8 or 16; rows beyond m are zero.
 #pragma once
 
+#include <initializer_list>
 #include <mutex>
 #include <set>
 #include <utility>
@@ -107,6 +108,45 @@ __device__ inline half8v make_half8(half2v a, half2v b, half2v c, half2v d) {
 __device__ inline float4v mfma16x16x32(half8v a, half8v b, float4v c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
+
+// v + (the same value from the lane `CTRL` points at), inside a row of 16 lanes
+template <int CTRL> __device__ inline float dpp_add(float v) {
+    const int o = __builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false);
+    return v + __int_as_float(o);
+}
+__device__ inline float sum4(float v) {
+    v = dpp_add<0xB1>(v);  // quad_perm [1, 0, 3, 2]
+    return dpp_add<0x4E>(v);  // quad_perm [2, 3, 0, 1]
+}
+// row_half_mirror: lane i <- lane 7 - i of its half row.  The result is pinned here: the callers store it from one lane in eight,
+// and an add that the compiler sinks into that branch no longer merges with its DPP move.
+__device__ inline float sum8(float v) {
+    float r = dpp_add<0x141>(sum4(v));
+    asm volatile("" : "+v"(r));
+    return r;
+}
+
+// row_mirror: lane i <- lane 15 - i of its row of 16
+__device__ inline float sum16(float v) {
+    float r = dpp_add<0x140>(sum8(v));
+    asm volatile("" : "+v"(r));
+    return r;
+}
+// the sum over the 64 lanes, in every lane: rows (0 + 1) + (2 + 3)
+__device__ inline float sum64(float v) {
+    const float r = sum16(v);
+    auto row = [&](int i) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r), 16 * i)); };
+    return (row(0) + row(1)) + (row(2) + row(3));
+}
+// What RmsNorm adds up of four neighbouring columns; the order of the whole sum of squares of a row of 1024 columns and more, the same in every
+// kernel that takes it, so that they agree to the bit: eight columns are sq4 + sq4, 64 such pieces (512 columns) a tree over the lanes (sum64), the
+// blocks of 512 columns one after the other.
+__device__ inline float sq4(float a, float b, float c, float d) { return __builtin_fmaf(d, d, __builtin_fmaf(c, c, __builtin_fmaf(b, b, a * a))); }
+
+// A launch's arguments are two hundred bytes that no cache holds when it starts.  Left to itself the compiler loads each where it is first used,
+// behind the branches that pick the weight: five scalar loads one after the other, each a round trip, before the first weight is
+// requested.  Naming them here makes them one.
+template <class... T> __device__ inline void load_together(T... v) { (void)std::initializer_list<int>{([](auto u) { asm volatile("" ::"s"(u)); }(v), 0)...}; }
 
 // 32-bit per-lane byte offsets of the global loads.  An offset computed (and widened to 64 bits) outside the loop reaches
 // the loads as a register pair and costs a 64-bit vector add per load; one that is widened next to the load folds into the
@@ -299,15 +339,16 @@ hipError_t turq_launch_gemv_cs(int dtype, int count, const void *const *w_tiled,
                                int nwaves, int row_tiles, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop);
 bool turq_gemv_cs_staged_takes(int dtype_a, int dtype_b, int x_dtype, int64_t k, int64_t m, int row_tiles);
 int turq_gemv_cs_staged_second_rows(int row_tiles);
+bool turq_gemv_cs_staged_norm_takes(int dtype, int64_t k, int64_t m, int row_tiles, int64_t groups, int64_t units);
 hipError_t turq_launch_gemv_cs_staged(int dtype_a, int dtype_b, int count, int second, const void *const *w_tiled, const int64_t *n,
                                       int64_t k, const void *x, int x_dtype, int64_t ldx, int64_t m, void *const *y, int y_dtype,
-                                      const int64_t *ldy, const float *const *bias, int row_tiles, hipStream_t stream,
-                                      hipEvent_t ev_start, hipEvent_t ev_stop);
+                                      const int64_t *ldy, const float *const *bias, int row_tiles, hipStream_t stream, hipEvent_t ev_start,
+                                      hipEvent_t ev_stop, const float *norm_weight = nullptr, float norm_eps = 0.0f);
 int turq_gemv_cs_staged_gateup_tiles(int dtype, int64_t n, int64_t k, int64_t m, int64_t units);
 hipError_t turq_launch_gemv_cs_staged_gateup(int dtype, const void *w_gate, const void *w_up, int64_t n, int64_t k, const void *x,
                                              int x_dtype, int64_t ldx, int64_t m, void *y, int y_dtype, int64_t ldy,
                                              const float *bias_gate, const float *bias_up, int tiles, hipStream_t stream,
-                                             hipEvent_t ev_start, hipEvent_t ev_stop);
+                                             hipEvent_t ev_start, hipEvent_t ev_stop, const float *norm_weight = nullptr, float norm_eps = 0.0f);
 bool turq_gemv_multi_mixed_supports(int dtype_a, int dtype_b);
 hipError_t turq_launch_gemv_multi_mixed(int dtype_a, int dtype_b, int count, int second, const void *const *w_tiled, const int64_t *n,
                                         int64_t k, const void *frags, int64_t m, void *const *y, int y_dtype, const int64_t *ldy,

@@ -131,6 +131,41 @@ int staged_row_tiles(const turq_ctx *ctx, int dtype_a, int dtype_b, int xt, int6
     return turq_gemv_cs_staged_takes(dtype_a, dtype_b, xt, k, m, rg) ? rg : 0;
 }
 
+// activation rows that the staged kernels can load: 16 bytes at a time, two neighbouring ones from one address and a 32-bit offset
+bool staged_rows_ok(const void *x, int xt, int64_t ldx) {
+    return (uintptr_t)x % 16 == 0 && ((size_t)ldx * turq_act_bytes(xt)) % 16 == 0 && ldx < (1 << 30);
+}
+
+// The staged launch that the first weights of a call go out in (rg 0: none): a run of one format, with one of a second format behind it
+// where the kernel has the pair.
+struct StagedRun {
+    int count, second;  // weights, and those of the first format
+    int dtype_b, rg;    // the second format (the first again: there is none), row tiles per workgroup
+    bool as_f16;        // the rows are rounded to f16 rows first
+};
+StagedRun staged_run(const turq_ctx *ctx, int left, const turq_weight *const *w, int xt, int64_t m, bool rows_ok) {
+    int j = 1;
+    while (j < left && j < 4 && w[j]->dtype == w[0]->dtype) j++;
+    int j2 = j;
+    if (!turq_tuning().gemv_no_mixed && j < left) {
+        j2 = j + 1;
+        while (j2 < left && w[j2]->dtype == w[j]->dtype) j2++;
+        if (j2 > 4) j2 = j;
+    }
+    // (more than 16 wide rows of f32, or rows that cannot be loaded 16 bytes at a time: as f16 first, so that a call gives
+    // the same bits whatever type and alignment its rows have)
+    const bool as_f16 = m > 16 && w[0]->k > 4096 && (xt == TURQ_ACT_F32 || !rows_ok);
+    for (int end = j2; end >= j; end = (end == j ? -1 : j)) {
+        int64_t tiles = 0, tiles_b = 0;
+        for (int t = 0; t < end; t++) tiles += turq_tile_rows(w[t]->n);
+        for (int t = j; t < end; t++) tiles_b += turq_tile_rows(w[t]->n);
+        const int dtb = end > j ? w[j]->dtype : w[0]->dtype;
+        const int rg = staged_row_tiles(ctx, w[0]->dtype, dtb, as_f16 ? (int)TURQ_ACT_F16 : xt, w[0]->k, m, tiles, tiles_b, rows_ok || as_f16);
+        if (rg) return StagedRun{end, end > j ? j : end, dtb, rg, as_f16};
+    }
+    return StagedRun{0, 0, 0, 0, false};
+}
+
 // whether the prefill GEMM can take this weight (its largest packed value must fit f16), and the power of two by which the
 // kernel multiplies the block scales
 bool gemm_takes(const turq_weight *w, float *wscale) {
@@ -513,7 +548,22 @@ bool turq_norm_fuses(const turq_ctx *ctx, int count, const turq_weight *const *w
             if (!use_row1(w[i]->dtype)) return false;
         return aligned && !no_fuse;
     }
-    if (m <= TURQ_GEMV_MAX_M) return false;
+    if (m <= TURQ_GEMV_MAX_M) {  // the staged kernels, where they take every weight of the call
+        // (one weight at up to four rows: turq_qmatmul's other kernels)
+        if (no_fuse || !staged_rows_ok(x, xt, ldx) || (count == 1 && m <= TURQ_ROW1_MAX_M)) return false;
+        for (int i = 0; i < count;) {
+            const StagedRun run = staged_run(ctx, count - i, w + i, xt, m, true);
+            if (!run.rg) return false;
+            int64_t groups = 0;
+            for (int t = 0; t < run.count; t++) {
+                const int rt = t < run.second ? run.rg : turq_gemv_cs_staged_second_rows(run.rg);
+                groups += (turq_tile_rows(w[i + t]->n) + rt - 1) / rt;
+            }
+            if (!turq_gemv_cs_staged_norm_takes(w[i]->dtype, w[0]->k, m, run.rg, groups, ctx->compute_units > 0 ? ctx->compute_units : 256)) return false;
+            i += run.count;
+        }
+        return true;
+    }
     if (w[0]->k % 256 != 0 || w[0]->k > 16384 || turq_rows_in_chunks(ctx, count, w, x, xt, ldx, m)) return false;
     for (int i = 0; i < count; i++)
         if (!gemm_takes(w[i], &ws)) return false;
@@ -643,7 +693,7 @@ int turq_qmatmul_mfma(turq_ctx *ctx, const turq_weight *w, const void *x, int xt
 bool turq_rows_in_chunks(const turq_ctx *ctx, int count, const turq_weight *const *w, const void *x, int xt, int64_t ldx, int64_t m) {
     const bool off = turq_tuning().rows_in_chunks_off;
     if (off || m <= TURQ_GEMV_MAX_M || m > 2 * TURQ_GEMV_MAX_M || count < 1 || count > 4) return false;
-    const bool aligned = ((uintptr_t)x % 16 == 0) && ((size_t)ldx * turq_act_bytes(xt)) % 16 == 0;
+    const bool aligned = staged_rows_ok(x, xt, ldx);
     const int64_t cus = ctx->compute_units > 0 ? ctx->compute_units : 256;
     int64_t row_tiles = 0;
     for (int i = 0; i < count; i++) {
@@ -661,7 +711,6 @@ int turq_qmatmul_gate_up_mfma(turq_ctx *ctx, const turq_weight *gate, const turq
                               const TurqNorm *norm) {
     const bool no_fuse = turq_tuning().gemv_no_fuse;
     *taken = false;
-    if (norm && m != 1) return TURQ_OK;  // (the caller normalises into scratch first)
     {
         const turq_weight *pair[2] = {gate, up};
         if (m > TURQ_GEMV_MAX_M && gate->n == up->n && turq_rows_in_chunks(ctx, 2, pair, x, xt, ldx, m) &&
@@ -688,12 +737,15 @@ int turq_qmatmul_gate_up_mfma(turq_ctx *ctx, const turq_weight *gate, const turq
     {
         const int staged = turq_tuning().cs_staged;
         const int64_t cus = ctx->compute_units > 0 ? ctx->compute_units : 256;
-        const int tiles = (staged != 0 && aligned && m >= 3 && gate->n == up->n && gate->k == up->k)
+        const int tiles = (staged != 0 && staged_rows_ok(x, xt, ldx) && m >= 3 && gate->n == up->n && gate->k == up->k)
                               ? turq_gemv_cs_staged_gateup_tiles(gate->dtype, gate->n, gate->k, m, cus) : 0;
+        if (norm && m != 1 && (!tiles || !turq_gemv_cs_staged_norm_takes(gate->dtype, gate->k, m, tiles, (turq_tile_rows(gate->n) + tiles / 2 - 1) / (tiles / 2), cus)))
+            return TURQ_OK;  // (the caller normalises into scratch first)
         if (tiles) {
             TURQ_HIP(ctx, turq_prof_next(ctx, &ev0, &ev1));
             TURQ_HIP(ctx, turq_launch_gemv_cs_staged_gateup(gate->dtype, gate->dev, up->dev, gate->n, gate->k, x, xt, ldx, m, y, yt, ldy,
-                                                            bias_gate, bias_up, tiles, ctx->stream, ev0, ev1));
+                                                            bias_gate, bias_up, tiles, ctx->stream, ev0, ev1, norm ? norm->w : nullptr,
+                                                            norm ? norm->eps : 0.0f));
             *taken = true;
             return TURQ_OK;
         }
@@ -729,7 +781,7 @@ int turq_qmatmul_gate_up_mfma(turq_ctx *ctx, const turq_weight *gate, const turq
 int turq_qmatmul_multi_mfma(turq_ctx *ctx, int count, const turq_weight *const *w, const void *x, int xt, int64_t m,
                             int64_t ldx, void *const *y, int yt, const int64_t *ldy, const float *const *bias, const TurqNorm *norm) {
     const bool no_fuse = turq_tuning().gemv_no_fuse;
-    if (norm && !(m == 1 && turq_norm_fuses(ctx, count, w, x, xt, ldx, m)))
+    if (norm && !(m <= TURQ_GEMV_MAX_M && turq_norm_fuses(ctx, count, w, x, xt, ldx, m)))
         return turq_fail(ctx, TURQ_ERR_INVALID, "turq_qmatmul_multi: no kernel applies the norm for this call (internal)");
     const bool aligned = ((uintptr_t)x % 16 == 0) && ((size_t)ldx * turq_act_bytes(xt)) % 16 == 0;
     int64_t all_tiles = 0;
@@ -748,44 +800,28 @@ int turq_qmatmul_multi_mfma(turq_ctx *ctx, int count, const turq_weight *const *
         const bool no_mixed = turq_tuning().gemv_no_mixed;
         // 3 .. 32 rows: fragments made in the kernel from the rows themselves (staged through the LDS), a second format in the
         // same launch where the kernel has the pair
-        {
-            int j2 = j;
-            if (!no_mixed && j < count) {
-                j2 = j + 1;
-                while (j2 < count && w[j2]->dtype == w[j]->dtype) j2++;
-                if (j2 - i > 4) j2 = j;
+        const StagedRun run = staged_run(ctx, count - i, w + i, xt, m, staged_rows_ok(x, xt, ldx));
+        if (run.rg) {
+            if (run.as_f16 && prepared != 3) {
+                const int rc = turq_ctx_reserve(ctx, &ctx->act_prep, &ctx->act_prep_cap, turq_act_prep_bytes(w[i]->dtype, m, w[i]->k));
+                if (rc != TURQ_OK) return rc;
+                TURQ_HIP(ctx, turq_launch_act_rows_f16(x, xt, m, w[i]->k, ldx, ctx->act_prep, ctx->stream));
+                prepared = 3;
             }
-            for (int end = j2; end >= j; end = (end == j ? -1 : j)) {
-                int64_t tiles = 0, tiles_b = 0;
-                for (int t = i; t < end; t++) tiles += turq_tile_rows(w[t]->n);
-                for (int t = j; t < end; t++) tiles_b += turq_tile_rows(w[t]->n);
-                const int dtb = end > j ? w[j]->dtype : w[i]->dtype;
-                // (more than 16 wide rows of f32, or rows that cannot be loaded 16 bytes at a time: as f16 first, so that a call gives
-                // the same bits whatever type and alignment its rows have)
-                const bool as_f16 = m > 16 && w[i]->k > 4096 && (xt == TURQ_ACT_F32 || !aligned);
-                const int rg = staged_row_tiles(ctx, w[i]->dtype, dtb, as_f16 ? (int)TURQ_ACT_F16 : xt, w[i]->k, m, tiles, tiles_b, aligned || as_f16);
-                if (!rg) continue;
-                if (as_f16 && prepared != 3) {
-                    const int rc = turq_ctx_reserve(ctx, &ctx->act_prep, &ctx->act_prep_cap, turq_act_prep_bytes(w[i]->dtype, m, w[i]->k));
-                    if (rc != TURQ_OK) return rc;
-                    TURQ_HIP(ctx, turq_launch_act_rows_f16(x, xt, m, w[i]->k, ldx, ctx->act_prep, ctx->stream));
-                    prepared = 3;
-                }
-                const void *wp[4];
-                int64_t nn[4];
-                for (int t = i; t < end; t++) {
-                    wp[t - i] = w[t]->dev;
-                    nn[t - i] = w[t]->n;
-                }
-                hipEvent_t ev0 = nullptr, ev1 = nullptr;
-                TURQ_HIP(ctx, turq_prof_next(ctx, &ev0, &ev1));
-                TURQ_HIP(ctx, turq_launch_gemv_cs_staged(w[i]->dtype, dtb, end - i, end > j ? j - i : end - i, wp, nn, w[i]->k, as_f16 ? ctx->act_prep : x,
-                                                         as_f16 ? (int)TURQ_ACT_F16 : xt, as_f16 ? w[i]->k : ldx, m,
-                                                         y + i, yt, ldy + i, bias ? bias + i : nullptr, rg, ctx->stream, ev0, ev1));
-                i = end;
-                break;
+            const void *wp[4];
+            int64_t nn[4];
+            for (int t = 0; t < run.count; t++) {
+                wp[t] = w[i + t]->dev;
+                nn[t] = w[i + t]->n;
             }
-            if (i >= j) continue;
+            hipEvent_t ev0 = nullptr, ev1 = nullptr;
+            TURQ_HIP(ctx, turq_prof_next(ctx, &ev0, &ev1));
+            TURQ_HIP(ctx, turq_launch_gemv_cs_staged(w[i]->dtype, run.dtype_b, run.count, run.second, wp, nn, w[i]->k, run.as_f16 ? ctx->act_prep : x,
+                                                     run.as_f16 ? (int)TURQ_ACT_F16 : xt, run.as_f16 ? w[i]->k : ldx, m, y + i, yt, ldy + i,
+                                                     bias ? bias + i : nullptr, run.rg, ctx->stream, ev0, ev1, norm ? norm->w : nullptr,
+                                                     norm ? norm->eps : 0.0f));
+            i += run.count;
+            continue;
         }
         // (more than two rows: only a call of one format, which would otherwise lose the launch it shares with a second one)
         const bool row1_ok = aligned && !no_fuse && use_row1(w[i]->dtype) && row1_takes(m, all_bytes, w[i]->dtype) &&

@@ -104,17 +104,24 @@ __device__ inline bool vec_row(const void *p, int64_t ld, int elem_bytes) {
     return ((uintptr_t)p & 15) == 0 && ((ld * elem_bytes) & 15) == 0;
 }
 
-// sqrt(mean(x^2) + eps) of the row that a group of four waves holds: s = what a thread added up of the squares of its columns
-// (explicit fused multiply-adds, piece by piece), then the waves their lanes and the group its four waves - one fixed order, shared
-// by the kernels below so that they agree to the bit.  part: four floats of the row's group.  Every thread of the workgroup calls it.
-__device__ inline float rms_of(float s, int64_t k, float eps, float *part) {
+// sqrt(mean(x^2) + eps) of the row that a workgroup of four waves holds: s[j] = what a thread has of the squares of its piece j, summed up over
+// the lanes of each wave and then over the blocks 4 j + wave in order - one fixed order, shared by the kernels below so that they
+// agree to the bit (as sq4 says).  part: 4 PER floats, or `blocks` of which those from 4 PER on are there.  Every thread of the workgroup calls it.
+template <int PER> __device__ inline float rms_of(const float (&s)[PER], int64_t k, float eps, float *part, int blocks = 0) {
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) s += __shfl_xor(s, off, 64);
-    if ((threadIdx.x & 63) == 0) part[(threadIdx.x >> 6) & 3] = s;
+    for (int j = 0; j < PER; j++) {
+        const float t = sum64(s[j]);
+        if ((threadIdx.x & 63) == 0) part[4 * j + ((threadIdx.x >> 6) & 3)] = t;
+    }
     __syncthreads();
-    const float total = (part[0] + part[1]) + (part[2] + part[3]);
+    float total = part[0];
+#pragma unroll
+    for (int b = 1; b < 4 * PER; b++) total += part[b];
+    for (int b = 4 * PER; b < blocks; b++) total += part[b];
     return sqrtf(total / (float)k + eps);
 }
+// the squares of a piece of eight columns
+__device__ inline float sq8(const float (&v)[8]) { return sq4(v[0], v[1], v[2], v[3]) + sq4(v[4], v[5], v[6], v[7]); }
 
 // v / rms for many v against one rms, to the last bit: with r = 1 / rms correctly rounded, q = v * r corrected once by its own
 // remainder is the correctly rounded quotient (P. Markstein, "Computation of elementary functions on the IBM RISC System/6000",
@@ -163,7 +170,8 @@ __global__ void __launch_bounds__(256) rms_norm_short_kernel(const void *__restr
     const int tid = threadIdx.x;
     const int64_t row = blockIdx.x;
     float v[2];
-    const float rms = rms_of(short_square_sum<XT>(x, row * ldx, k, tid, v), k, eps, part);
+    const float sq[1] = {short_square_sum<XT>(x, row * ldx, k, tid, v)};
+    const float rms = rms_of(sq, k, eps, part);
 #pragma unroll
     for (int j = 0; j < 2; j++) {
         const int64_t c = (int64_t)j * 256 + tid;
@@ -176,26 +184,31 @@ __global__ void __launch_bounds__(256) rms_norm_short_kernel(const void *__restr
 template <int XT, int YT, int PER>
 __global__ void __launch_bounds__(256) rms_norm_kernel(const void *__restrict__ x, int64_t k, int64_t ldx, const float *__restrict__ w,
                                                        float eps, void *__restrict__ y, int64_t ldy) {
-    __shared__ float part[4];
+    __shared__ float part[PER == 3 ? 32 : 4 * PER];
     const int tid = threadIdx.x;
     const int64_t row = blockIdx.x;
     const int64_t xo = row * ldx, yo = row * ldy;
     const bool vx = vec_row(x, ldx, XT == TURQ_ACT_F32 ? 4 : 2), vy = vec_row(y, ldy, YT == TURQ_ACT_F32 ? 4 : 2);
     const bool vw = ((uintptr_t)w & 15) == 0;
     float v[PER][8], wv[PER][8];
-    float s = 0.0f;
     ld_pieces<XT, PER, PER>(x, xo, k, true, vx, w, vw, tid, v, wv);
+    float s[PER];
 #pragma unroll
-    for (int j = 0; j < PER; j++)
-#pragma unroll
-        for (int e = 0; e < 8; e++) s = __builtin_fmaf(v[j][e], v[j][e], s);  // (columns past k add +0: the sum is that of the columns that exist)
-    for (int64_t col0 = ((int64_t)PER * 256 + tid) * 8; PER == 3 && col0 < k; col0 += 2048) {
+    for (int j = 0; j < PER; j++) s[j] = sq8(v[j]);  // (columns past k add +0: the sum is that of the columns that exist)
+    // longer rows: blocks of 512 columns of their own up to 16384 columns, what lies behind is added to the first
+    int j = PER;
+    for (; PER == 3 && (int64_t)j * 2048 < k && j < 8; j++) {
+        float t[8];
+        ld_piece<XT>(x, xo, ((int64_t)j * 256 + tid) * 8, k, vx, t);
+        const float b = sum64(sq8(t));
+        if ((tid & 63) == 0) part[4 * j + (tid >> 6)] = b;
+    }
+    for (int64_t col0 = ((int64_t)j * 256 + tid) * 8; PER == 3 && col0 < k; col0 += 2048) {
         float t[8];
         ld_piece<XT>(x, xo, col0, k, vx, t);
-#pragma unroll
-        for (int e = 0; e < 8; e++) s = __builtin_fmaf(t[e], t[e], s);
+        s[0] += sq8(t);
     }
-    const RowDiv div(rms_of(s, k, eps, part));
+    const RowDiv div(rms_of(s, k, eps, part, 4 * j));
     auto store = [&](int64_t col0, const float (&t)[8], const float (&tw)[8]) {
         if (col0 >= k) return;
         float o[8];
@@ -243,7 +256,7 @@ __global__ void __launch_bounds__(256) rms_norm_kernel(const void *__restrict__ 
 template <int XT, bool Q8, int PER>
 __global__ void __launch_bounds__(256) rms_norm_prep32_kernel(const void *__restrict__ x, int64_t m, int64_t k, int64_t ldx, const float *__restrict__ w,
                                                               float eps, int64_t ntc, half8v *__restrict__ frags) {
-    __shared__ float part[4];
+    __shared__ float part[4 * PER];
     const int tid = threadIdx.x;
     // workgroups of one XCD (blockIdx % 8) take neighbouring rows (the grid: a multiple of 32)
     const int64_t row = (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
@@ -254,16 +267,14 @@ __global__ void __launch_bounds__(256) rms_norm_prep32_kernel(const void *__rest
     const bool vx = vec_row(x, ldx, XT == TURQ_ACT_F32 ? 4 : 2), vw = ((uintptr_t)w & 15) == 0;
     constexpr int WPER = PER <= 2 ? PER : 1;  // (longer rows: eight waves share a SIMD up to 64 registers)
     float v[PER][8], wv[WPER][8];
-    float s = 0.0f;
+    float s[PER];
     ld_pieces<XT, PER, WPER>(x, xo, k, live, vx, w, vw, tid, v, wv);
     if (PER == 1 && k <= kShort) {  // (the order of rms_norm_short_kernel)
         float sq[2];
-        s = short_square_sum<XT>(x, xo, live ? k : 0, tid, sq);
+        s[0] = short_square_sum<XT>(x, xo, live ? k : 0, tid, sq);
     } else {
 #pragma unroll
-        for (int j = 0; j < PER; j++)
-#pragma unroll
-            for (int e = 0; e < 8; e++) s = __builtin_fmaf(v[j][e], v[j][e], s);
+        for (int j = 0; j < PER; j++) s[j] = sq8(v[j]);
     }
     const RowDiv div(rms_of(s, k, eps, part));
 #pragma unroll
