@@ -144,10 +144,12 @@ template <int XT, bool Q8, bool GU = false>
 __global__ void __launch_bounds__(256) act_prep32_kernel(const void *__restrict__ x, int64_t m, int64_t k, int64_t ldx,
                                                          int64_t ntc, half8v *__restrict__ frags, const float *__restrict__ up = nullptr) {
     const int tid = threadIdx.x;
-    const int64_t wg = blockIdx.x;  // (mt * ntc + b) * 4 + quarter
+    load_together(x, m, k, ldx, ntc, frags, up);
+    const uint32_t wg = blockIdx.x;  // (mt * ntc + b) * 4 + quarter
     const int quarter = (int)(wg & 3);
-    const int64_t tb = wg >> 2;
-    const int64_t b = tb % ntc, mt = tb / ntc;
+    // (32-bit: the quotient of 64-bit values was a hundred instructions ahead of the load)
+    const uint32_t tb32 = wg >> 2, mt32 = tb32 / (uint32_t)ntc;
+    const int64_t tb = tb32, b = tb32 - mt32 * (uint32_t)ntc, mt = mt32;
     const int r = tid >> 3, pc = tid & 7;
     const int cc = 8 * quarter + pc;  // piece of 8 columns inside the 256-column tile
     const int64_t row = mt * 32 + r, col0 = b * 256 + 8 * cc;
@@ -194,10 +196,10 @@ __global__ void __launch_bounds__(256) act_prep32_kernel(const void *__restrict_
     float sum = 0.0f;
 #pragma unroll
     for (int j = 0; j < 8; j++) {
-        turq_note_result<TURQ_ACT_F16>(v[j]);
         h[j] = (_Float16)v[j];
         sum += (float)h[j];
     }
+    turq_note_results<TURQ_ACT_F16>(v);
     half8v *dst = frags + tb * (17 * 64);
     const int g32 = Q8 ? (cc >> 1) & 1 : cc >> 4, q = Q8 ? 2 * (cc >> 2) + (cc & 1) : cc & 15;
     dst[q * 64 + r + 32 * g32] = h;

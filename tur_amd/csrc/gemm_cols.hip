@@ -22,6 +22,7 @@
 #include <hip/hip_ext.h>
 
 #include <algorithm>
+#include <climits>
 
 #include "gemm_formats.h"
 #include "tuning.h"
@@ -35,8 +36,17 @@ struct ColsGroup {
     const float *bias[kMaxGroup];
     int64_t n[kMaxGroup], ldy[kMaxGroup];
     float wscale[kMaxGroup];
-    int first[kMaxGroup];  // first n-block of the weight
-    int count, second;     // weights from `second` on are of the kernel's second format
+    int first[kMaxGroup];  // first n-block of the weight (INT_MAX: there is none)
+    int second;            // weights from `second` on are of the kernel's second format
+};
+// the weight of a workgroup
+struct ColsPick {
+    const uint8_t *w;
+    void *y;
+    const float *bias;
+    int64_t n, ldy;
+    float wscale;
+    int index, first;
 };
 
 // a lane's packed weights of one 32-row tile and one super-block, as the loads deliver them: the header, and the four stages in order;
@@ -114,14 +124,14 @@ template <int MT, int NT> struct Meet {
 // 5 us launch between it and down_proj: whole MLPs Q8_0 1024 x 3072 at 34 / 300 rows 19.3 / 30.3 -> 16.5 / 25.0 us, Q5_K / Q6_K
 // 4096 x 12288 at 77 rows 66.6 -> 62.2, at 180 rows 108 -> 96; nowhere slower (4096 x 12288 .. 5120 x 15360, 34 - 600 rows, every format).
 template <int DT, int MT, int NT, bool TIGHT, bool PAIR>
-__device__ __forceinline__ void cols_body(const ColsGroup &grp, int wi, int nb, int mb, int64_t k, const uint8_t *__restrict__ frags, int64_t m,
+__device__ __forceinline__ void cols_body(const ColsGroup &grp, const ColsPick &pick, int nb, int mb, int64_t k, const uint8_t *__restrict__ frags, int64_t m,
                                           int yt, int vec_out, uint8_t *lds) {
     using Fm = GFmt<DT>;
     using Wb = WBlk<DT>;
     constexpr int TB = TiledFmt<DT>::kTileBytes;
     constexpr bool SUMS = Fm::SUMS;
-    const uint8_t *__restrict__ w = grp.w[wi];
-    const int64_t n = grp.n[wi];
+    const uint8_t *__restrict__ w = pick.w;
+    const int64_t n = pick.n;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n32 = lane & 31, g32 = lane >> 5, r16 = n32 & 15, tsel = n32 >> 4;
@@ -152,7 +162,7 @@ __device__ __forceinline__ void cols_body(const ColsGroup &grp, int wi, int nb, 
     auto w_at = [&](int b, int j) { return (PAIR ? w_lane[j] : w_src) + (size_t)b * TB; };
     uint32_t lane16 = 16u * (uint32_t)lane;
     const uint32_t slot = (uint32_t)(r16 + 32 * g32);
-    const _Float16 ws = (_Float16)(PAIR ? (tsel ? grp.wscale[1] : grp.wscale[0]) : grp.wscale[wi]);
+    const _Float16 ws = (_Float16)(PAIR ? (tsel ? grp.wscale[1] : grp.wscale[0]) : pick.wscale);
 
     float16v acc[MT][NT];
 #pragma unroll
@@ -354,10 +364,10 @@ __device__ __forceinline__ void cols_body(const ColsGroup &grp, int wi, int nb, 
         turq_note_flush(bad);
         return;
     }
-    const float inv_ws = 1.0f / grp.wscale[wi];  // (a power of two: exact)
-    const float *bias = grp.bias[wi];
-    void *y = grp.y[wi];
-    const int64_t ldy = grp.ldy[wi];
+    const float inv_ws = 1.0f / pick.wscale;  // (a power of two: exact)
+    const float *bias = pick.bias;
+    void *y = pick.y;
+    const int64_t ldy = pick.ldy;
     const int ytb = yt & 0xFF;
     const float lim = turq_finite_limit(ytb);
     uint32_t bad = 0;
@@ -442,19 +452,29 @@ template <int DTA, int DTB, int MT, int NT, bool TIGHT, int MINB, bool PAIR>
 __global__ void __launch_bounds__(64 * W, MINB) gemm_cols_kernel(ColsGroup grp, int64_t k, const uint8_t *__restrict__ frags, int64_t m, int yt,
                                                            int nblocks_n, int nblocks_m, int vec_out) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    load_together(k, frags, m, yt, nblocks_n, nblocks_m, vec_out);
+    load_together(grp.w[0], grp.w[1], grp.n[0], grp.wscale[0], grp.wscale[1], grp.y[0], grp.bias[0], grp.bias[1], grp.ldy[0]);
+    if constexpr (!PAIR)
+        load_together(grp.w[2], grp.w[3], grp.n[1], grp.n[2], grp.n[3], grp.wscale[2], grp.wscale[3], grp.y[1], grp.y[2], grp.y[3], grp.bias[2], grp.bias[3],
+                      grp.ldy[1], grp.ldy[2], grp.ldy[3], grp.first[1], grp.first[2], grp.first[3], grp.second);
     // consecutive logical ids run on one XCD (blockIdx % 8): the m-blocks of one n-block share its packed weights in that XCD's L2.  Also where
     // the workgroups are no multiple of 8 (the first XCDs have one more): with ids as they come there, Q8_0 18944 x 1024 at 300 rows (990
     // workgroups) took 47.3 us instead of 41.3
     const int nwg = nblocks_n * nblocks_m, xcd = (int)blockIdx.x & 7, extra = nwg & 7;
     const int lid = xcd * (nwg >> 3) + (xcd < extra ? xcd : extra) + ((int)blockIdx.x >> 3);
     const int mb = lid % nblocks_m, nb_all = lid / nblocks_m;
-    int wi = 0;
+    ColsPick p{grp.w[0], grp.y[0], grp.bias[0], grp.n[0], grp.ldy[0], grp.wscale[0], 0, 0};
+    if constexpr (!PAIR) {
 #pragma unroll
-    for (int i = 1; i < kMaxGroup; i++)
-        if (!PAIR && i < grp.count && nb_all >= grp.first[i]) wi = i;
-    const int nb = nb_all - grp.first[wi];
-    if (DTA == DTB || wi < grp.second) cols_body<DTA, MT, NT, TIGHT, PAIR>(grp, wi, nb, mb, k, frags, m, yt, vec_out, lds);
-    else cols_body<DTB, MT, NT, TIGHT, PAIR>(grp, wi, nb, mb, k, frags, m, yt, vec_out, lds);
+        for (int i = 1; i < kMaxGroup; i++) {  // (selects, no branches)
+            const bool in = nb_all >= grp.first[i];
+            p.w = in ? grp.w[i] : p.w, p.y = in ? grp.y[i] : p.y, p.bias = in ? grp.bias[i] : p.bias, p.n = in ? grp.n[i] : p.n;
+            p.ldy = in ? grp.ldy[i] : p.ldy, p.wscale = in ? grp.wscale[i] : p.wscale, p.index = in ? i : p.index, p.first = in ? grp.first[i] : p.first;
+        }
+    }
+    const int nb = nb_all - p.first;
+    if (DTA == DTB || p.index < grp.second) cols_body<DTA, MT, NT, TIGHT, PAIR>(grp, p, nb, mb, k, frags, m, yt, vec_out, lds);
+    else cols_body<DTB, MT, NT, TIGHT, PAIR>(grp, p, nb, mb, k, frags, m, yt, vec_out, lds);
 }
 
 template <int DTA, int DTB, int MT, int NT, bool TIGHT = false, int MINB = 1, bool PAIR = false>
@@ -464,8 +484,8 @@ hipError_t launch_cols(const TurqGemmWeights &ws, int second, int64_t k, const v
     constexpr int LDS_BYTES = Meet<MT, NT>::LDS;
     static_assert(LDS_BYTES <= 64 * 1024, "no raised LDS limit");
     ColsGroup grp{};
-    grp.count = ws.count;
     grp.second = second;
+    for (int i = ws.count; i < kMaxGroup; i++) grp.first[i] = INT_MAX;
     const int es = (yt & 0xFF) == TURQ_ACT_F32 ? 4 : 2;
     int nbn = 0, vec_out = 1;  // rows of y can be written four aligned columns at a time (every weight of the launch, or none)
     for (int i = 0; i < ws.count; i++) {
@@ -495,12 +515,20 @@ int64_t cols_workgroups(int tile, int count, const int64_t *n, int64_t m) {
     return nbn * ((m + 32 * (tile / 10) - 1) / (32 * (tile / 10)));
 }
 
+// Whether a launch of 32 x 32 tiles that is more than one round over the CUs goes out as one of 64 x 32, two of them one under the other: the same sums
+// in the same order, and one round instead of a second for half of the CUs.  By the estimates, which for these two are right to a few percent:
+// Q6_K 4096 x 12288 at 65 - 96 rows 34.4 -> 27.4 us, 2048 x 6144 at 150 18.7 -> 17.0, Q5_K / Q4_K 4096 x 4096 at 77 13.4 / 11.9 -> 12.2 / 11.2; not of Q8_0, of which
+// three workgroups on a CU lose less (1024 x 2048 at 300 rows 8.1 -> 8.3).
+bool two_under_another(int dtype_a, int dtype_b, const TurqGemmWeights &ws, int64_t k, int64_t m, int64_t cus);
+
 template <int DTA, int DTB>
 hipError_t launch_tile(int tile, const TurqGemmWeights &ws, int second, int64_t k, const void *frags, int64_t m, int yt, int64_t cus,
                        hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop) {
     switch (tile) {
 #define TURQ_COLS(MT, NT, ...) launch_cols<DTA, DTB, MT, NT, ##__VA_ARGS__>(ws, second, k, frags, m, yt, stream, ev_start, ev_stop)
-    case 11: return TURQ_COLS(1, 1);
+    case 11:
+        if (two_under_another(DTA, DTB, ws, k, m, cus)) return TURQ_COLS(2, 1);
+        return TURQ_COLS(1, 1);
     case 21: return TURQ_COLS(2, 1);
     case 31: return TURQ_COLS(3, 1);
     case 22:  // (more than one workgroup per CU: two of them at a time)
@@ -580,6 +608,14 @@ static double cols_us(int tile, int dtype_a, int dtype_b, int count, const int64
     return std::max(turq_launch_model_us(c->base, std::max(c->per[fmt(dtype_a)], c->per[fmt(dtype_b)]) * (double)(k / 256), c->again, c->more, c->fill, x),
                     cols_frag_us(tile, wgs / ((m + 32 * (tile / 10) - 1) / (32 * (tile / 10))), k, m, cus, x));
 }
+
+namespace {
+bool two_under_another(int dtype_a, int dtype_b, const TurqGemmWeights &ws, int64_t k, int64_t m, int64_t cus) {
+    if (dtype_a == TURQ_Q8_0 || turq_tuning().gemm_cols > 0) return false;  // (a forced tile is that tile)
+    if (cols_workgroups(11, ws.count, ws.n, m) <= cus || cols_workgroups(21, ws.count, ws.n, m) > cus) return false;
+    return cols_us(21, dtype_a, dtype_b, ws.count, ws.n, k, m, cus) < cols_us(11, dtype_a, dtype_b, ws.count, ws.n, k, m, cus);
+}
+}  // namespace
 
 // The tile with which one weight goes through this kernel as far as single rounds over the CUs decide, 0: gemm_kq_kernel.
 // A launch of one round takes about base + per_sb * super-blocks, one line for every format; a further round costs as much again without the
