@@ -240,3 +240,35 @@ def test_mlp_intermediate_outside_f16_is_counted_and_wide_handles_it(m):
             g.release(w)
     finally:
         g.close()
+
+
+# A call on host pointers goes through pinned memory of the context that the scaling kernels read and write, or, with more than 8 MiB of rows and results,
+# through copies; both are the device call with the switch on, bit for bit.  Rows in one piece and with strides, added to what y holds, Q8_0 rows that end
+# inside a column tile, rows that a workgroup keeps in registers (up to 4096 and to 12288 columns) and longer ones, rows that are not aligned.
+@pytest.mark.parametrize("dt,n,k,m,pad", [(Q4_K, 96, 512, 3, 0), (Q8_0, 40, 4128, 2, 0), (Q6_K, 48, 12544, 2, 0), (Q5_K, 64, 1024, 40, 8), (Q8_0, 33, 96, 5, 3),
+                                          (Q4_K, 16, 12288, 33, 0), (Q4_K, 64, 8192, 300, 0)])
+@pytest.mark.parametrize("x_dtype", [capi.ACT_F32, capi.ACT_BF16], ids=["f32", "bf16"])
+def test_host_calls_are_the_wide_device_calls(gpu, dt, n, k, m, pad, x_dtype):
+    L, ctx = gpu.L, gpu.ctx
+    w = gpu.upload(dt, n, k, synth.random_weight(dt, n, k, seed=n + k), capi.LAYOUT_TILED)
+    x = np.zeros((m, k + pad), np.float32)
+    x[:, :k] = rows_of_mixed_magnitude(m, k, seed=m + k)
+    xs = synth.to_bf16_bits(x).reshape(x.shape) if x_dtype == capi.ACT_BF16 else x
+    y0 = np.random.default_rng(n).standard_normal((m, n + pad)).astype(np.float32)
+    bias = np.random.default_rng(k).standard_normal(n).astype(np.float32)
+    for flag in (0, capi.OUT_ACCUMULATE):
+        host = y0.copy()
+        capi.check(L.turq_qmatmul(ctx, w, capi.ptr(xs), x_dtype, m, k + pad, capi.ptr(host), capi.ACT_F32 | flag, n + pad, capi.ptr(bias), capi.MEM_HOST,
+                                  capi.ALGO_AUTO), ctx)
+        ps = [gpu.dev_buffer(a) for a in (np.ascontiguousarray(xs[:, :k]), np.ascontiguousarray(y0[:, :n]), bias)]
+        capi.check(L.turq_ctx_set_wide_activations(ctx, 1), ctx)
+        try:
+            capi.check(L.turq_qmatmul(ctx, w, ps[0], x_dtype, m, k, ps[1], capi.ACT_F32 | flag, n, ps[2], capi.MEM_DEVICE, capi.ALGO_AUTO), ctx)
+            dev = gpu.read_back(ps[1], (m, n), np.float32)
+        finally:
+            capi.check(L.turq_ctx_set_wide_activations(ctx, 0), ctx)
+            for p in ps:
+                gpu.dev_free(p)
+        assert np.array_equal(host[:, :n], dev)
+        assert np.array_equal(host[:, n:], y0[:, n:])
+    gpu.release(w)

@@ -176,6 +176,7 @@ void turq_ctx_destroy(turq_ctx *ctx) {
     if (ctx->wide_s) (void)hipFree(ctx->wide_s);
     if (ctx->wide_y) (void)hipFree(ctx->wide_y);
     if (ctx->stage_b) (void)hipFree(ctx->stage_b);
+    if (ctx->host_map) (void)hipHostFree(ctx->host_map);
     if (ctx->stage_w) (void)hipFree(ctx->stage_w);
     for (void *p : ctx->retired) (void)hipFree(p);  // graphs that still refer to them can no longer be launched: that needs the context
     for (auto &p : ctx->prof_events) { (void)hipEventDestroy(p.first); (void)hipEventDestroy(p.second); }
@@ -519,15 +520,33 @@ static int impl_rms_norm(turq_ctx *ctx, const void *x, int xt, int64_t m, int64_
 
 // ---- forward ----
 
-// wide: activations of any finite f32 magnitude (wide.hip) where the kernel would round them to f16
+// the context's pinned memory, made on first use (not during a capture, whose calls on host pointers fail as they did)
+static bool host_map_ready(turq_ctx *ctx) {
+    if (ctx->capturing) return false;
+    if (!ctx->host_map) {
+        void *p = nullptr, *d = nullptr;
+        if (hipHostMalloc(&p, turq_ctx::kHostMapBytes, hipHostMallocMapped) != hipSuccess) { (void)hipGetLastError(); return false; }
+        if (hipHostGetDevicePointer(&d, p, 0) != hipSuccess) { (void)hipGetLastError(); (void)hipHostFree(p); return false; }
+        ctx->host_map = p, ctx->host_map_dev = d;
+    }
+    return true;
+}
+
+// whether a wide call goes through the scaling kernels, which read x and the bias once and write y once
+static bool wide_scales(const turq_ctx *ctx, const turq_weight *w, int xt, int algo) {
+    return !ctx->fixed_scratch && xt != TURQ_ACT_F16 && (algo == TURQ_ALGO_AUTO || algo == TURQ_ALGO_GEMV || algo == TURQ_ALGO_GEMM) &&
+           w->layout == TURQ_LAYOUT_TILED;
+}
+
+// wide: activations of any finite f32 magnitude (wide.hip) where the kernel would round them to f16; y_far: y is not in device memory (the
+// products are kept there until they are scaled back)
 static int qmatmul_device(turq_ctx *ctx, const turq_weight *w, const void *x, int xt, int64_t m, int64_t ldx, void *y,
-                          int yt, int64_t ldy, const float *bias, int algo, bool wide) {
+                          int yt, int64_t ldy, const float *bias, int algo, bool wide, bool y_far = false) {
     if (algo == TURQ_ALGO_AUTO) {
         if (w->layout == TURQ_LAYOUT_NATIVE) algo = TURQ_ALGO_SIMPLE;
         else algo = (m <= TURQ_GEMV_MAX_M || turq_rows_in_chunks(ctx, 1, &w, x, xt, ldx, m)) ? TURQ_ALGO_GEMV : TURQ_ALGO_GEMM;
     }
-    if (wide && !ctx->fixed_scratch && xt != TURQ_ACT_F16 && (algo == TURQ_ALGO_GEMV || algo == TURQ_ALGO_GEMM) &&
-        w->layout == TURQ_LAYOUT_TILED) {
+    if (wide && wide_scales(ctx, w, xt, algo)) {
         // rows scaled by powers of two into the f16 range, the plain call on the f16 copy, rows scaled back (+ bias)
         int rc = turq_ctx_reserve(ctx, &ctx->wide_x, &ctx->wide_x_cap, (size_t)m * (size_t)w->k * 2);
         if (rc != TURQ_OK) return rc;
@@ -535,7 +554,7 @@ static int qmatmul_device(turq_ctx *ctx, const turq_weight *w, const void *x, in
         if (rc != TURQ_OK) return rc;
         float *y32 = (float *)y;
         int64_t ld32 = ldy;
-        if (yt != TURQ_ACT_F32) {  // (also an f32 output that is added to: the product must not land on the residual stream)
+        if (yt != TURQ_ACT_F32 || y_far) {  // (also an f32 output that is added to: the product must not land on the residual stream)
             rc = turq_ctx_reserve(ctx, &ctx->wide_y, &ctx->wide_y_cap, (size_t)m * (size_t)w->n * sizeof(float));
             if (rc != TURQ_OK) return rc;
             y32 = (float *)ctx->wide_y;
@@ -583,8 +602,29 @@ static int impl_qmatmul(turq_ctx *ctx, const turq_weight *w, const void *x, int 
     if (mem == TURQ_MEM_DEVICE) return qmatmul_device(ctx, w, x, xt, m, ldx, y, yt, ldy, bias, algo, ctx->wide);
     if (mem != TURQ_MEM_HOST) return turq_fail(ctx, TURQ_ERR_INVALID, "turq_qmatmul: bad mem %d", mem);
 
-    // host pointers: stage rows densely (ld = k / n on the device side), run, copy back
     const size_t xrow = (size_t)w->k * xb, yrow = (size_t)w->n * yb;
+    if (wide_scales(ctx, w, xt, algo) && xrow * (size_t)m + yrow * (size_t)m + (size_t)w->n * sizeof(float) + 64 <= turq_ctx::kHostMapBytes && host_map_ready(ctx)) {
+        // through pinned memory that the scaling kernels read and write themselves, without the runtime's copies from and to pageable memory: Q8_0
+        // 3072 x 1024 at one row 48 -> 32 us a call, Q4_K 12288 x 4096 at 16 rows 346 -> 86, 12288 x 12288 at 64 (6 MB of rows and results) 1300 -> 335
+        const auto up = [](size_t n) { return (n + 15) & ~(size_t)15; };
+        const size_t at_b = up(xrow * (size_t)m), at_y = at_b + up((size_t)w->n * sizeof(float));
+        uint8_t *host = (uint8_t *)ctx->host_map, *dev = (uint8_t *)ctx->host_map_dev;
+        const auto rows = [m](uint8_t *dst, size_t dst_ld, const uint8_t *src, size_t src_ld, size_t row) {
+            if (dst_ld == row && src_ld == row) memcpy(dst, src, row * (size_t)m);
+            else for (int64_t r = 0; r < m; r++) memcpy(dst + (size_t)r * dst_ld, src + (size_t)r * src_ld, row);
+        };
+        rows(host, xrow, (const uint8_t *)x, (size_t)ldx * xb, xrow);
+        if (bias) memcpy(host + at_b, bias, (size_t)w->n * sizeof(float));
+        if (yt & TURQ_OUT_ACCUMULATE) rows(host + at_y, yrow, (const uint8_t *)y, (size_t)ldy * yb, yrow);
+        const int rc = qmatmul_device(ctx, w, dev, xt, m, w->k, dev + at_y, yt, w->n, bias ? (const float *)(dev + at_b) : nullptr, algo, true, true);
+        // (waited for also where a launch failed: the next call writes into the same memory)
+        const hipError_t done = hipStreamSynchronize(ctx->stream);
+        if (rc != TURQ_OK) return rc;
+        TURQ_HIP(ctx, done);
+        rows((uint8_t *)y, (size_t)ldy * yb, host + at_y, yrow, yrow);
+        return TURQ_OK;
+    }
+    // host pointers: stage rows densely (ld = k / n on the device side), run, copy back
     int rc = turq_ctx_reserve(ctx, &ctx->stage_x, &ctx->stage_x_cap, xrow * (size_t)m);
     if (rc != TURQ_OK) return rc;
     rc = turq_ctx_reserve(ctx, &ctx->stage_y, &ctx->stage_y_cap, yrow * (size_t)m);

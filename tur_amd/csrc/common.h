@@ -87,6 +87,9 @@ struct turq_ctx {
     void *stage_x = nullptr;  size_t stage_x_cap = 0;
     void *stage_y = nullptr;  size_t stage_y_cap = 0;
     void *stage_b = nullptr;  size_t stage_b_cap = 0;
+    // pinned memory of TURQ_MEM_HOST calls that the scaling kernels read and write over the bus (one size, made by the first such call)
+    static constexpr size_t kHostMapBytes = (size_t)8 << 20;
+    void *host_map = nullptr, *host_map_dev = nullptr;
     void *stage_w = nullptr;  // turq_weight_upload: a fixed size, held by one upload at a time (stage_w_mu: uploads may come from several threads)
     std::mutex stage_w_mu;
     void *act_prep = nullptr; size_t act_prep_cap = 0;

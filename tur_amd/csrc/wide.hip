@@ -16,20 +16,46 @@ template <int XT> __device__ inline float ld_x(const void *x, int64_t i) {
     return __uint_as_float((uint32_t)((const uint16_t *)x)[i] << 16);  // bf16
 }
 
-// one workgroup of 256 threads per row: the row's largest magnitude, then the scaled f16 copy
-template <int XT>
+// one workgroup of 256 threads per row: the row's largest magnitude, then the scaled f16 copy.  Bound by latency: host calls read their rows over
+// the bus, where a load takes over a microsecond, so with VEC (rows aligned to 16 bytes, k a multiple of 4) a thread requests its first
+// PER pieces of four columns together and keeps them for the second pass; what lies behind them is read again.
+template <int XT, int PER, bool VEC>
 __global__ void __launch_bounds__(256) wide_scale_kernel(const void *__restrict__ x, int64_t k, int64_t ldx, _Float16 *__restrict__ x16,
                                                          float *__restrict__ inv) {
     __shared__ float part[4];
     const int tid = threadIdx.x;
-    const int64_t row = blockIdx.x;
+    const int64_t row = blockIdx.x, xo = row * ldx;
     float amax = 0.0f;
     bool finite = true;
-    for (int64_t c = tid; c < k; c += 256) {
-        const float v = fabsf(ld_x<XT>(x, row * ldx + c));
+    auto see = [&](float f) {
+        const float v = fabsf(f);
         finite = finite && v <= 3.4028234e38f;  // false for an infinity and for a NaN
         amax = fmaxf(amax, v);
+    };
+    constexpr int KEEP = VEC ? PER : 1;
+    uint4v raw[KEEP];
+    float v[KEEP][4];
+    if constexpr (VEC) {
+#pragma unroll
+        for (int j = 0; j < PER; j++) {  // (pieces past the row: its first one, not looked at)
+            const int64_t c = 4 * ((int64_t)j * 256 + tid);
+            if constexpr (XT == TURQ_ACT_F32) {
+                raw[j] = *(const uint4v *)((const float *)x + xo + (c < k ? c : 0));
+            } else {
+                const uint2v u = *(const uint2v *)((const uint16_t *)x + xo + (c < k ? c : 0));
+                raw[j] = uint4v{u.x << 16, u.x & 0xFFFF0000u, u.y << 16, u.y & 0xFFFF0000u};
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < PER; j++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                v[j][e] = 4 * ((int64_t)j * 256 + tid) < k ? __uint_as_float(raw[j][e]) : 0.0f;
+                see(v[j][e]);
+            }
     }
+    const int64_t rest = VEC ? (int64_t)PER * 1024 : 0;
+    for (int64_t c = rest + tid; c < k; c += 256) see(ld_x<XT>(x, xo + c));
     if (!finite) amax = __uint_as_float(0x7F800000u);
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
@@ -46,7 +72,15 @@ __global__ void __launch_bounds__(256) wide_scale_kernel(const void *__restrict_
     }
     const float s = ldexpf(1.0f, e);
     if (tid == 0) inv[row] = ldexpf(1.0f, -e);
-    for (int64_t c = tid; c < k; c += 256) x16[row * k + c] = (_Float16)(ld_x<XT>(x, row * ldx + c) * s);
+    if constexpr (VEC) {
+#pragma unroll
+        for (int j = 0; j < PER; j++) {
+            const int64_t c = 4 * ((int64_t)j * 256 + tid);
+            const half2v a = {(_Float16)(v[j][0] * s), (_Float16)(v[j][1] * s)}, b = {(_Float16)(v[j][2] * s), (_Float16)(v[j][3] * s)};
+            if (c < k) *(uint2v *)(x16 + row * k + c) = uint2v{as_u32(a), as_u32(b)};
+        }
+    }
+    for (int64_t c = rest + tid; c < k; c += 256) x16[row * k + c] = (_Float16)(ld_x<XT>(x, xo + c) * s);
 }
 
 // y[r][c] = y32[r][c] * inv[r] + bias[c]
@@ -68,9 +102,15 @@ __global__ void __launch_bounds__(256) wide_rescale_kernel(const float *__restri
 hipError_t turq_launch_wide_scale(const void *x, int x_dtype, int64_t m, int64_t k, int64_t ldx, void *x16, float *inv, hipStream_t stream) {
     if (m == 0 || k == 0) return hipSuccess;
     if (m > 0x7FFFFFFF) return hipErrorInvalidValue;
-    if (x_dtype == TURQ_ACT_F32) wide_scale_kernel<TURQ_ACT_F32><<<(unsigned)m, 256, 0, stream>>>(x, k, ldx, (_Float16 *)x16, inv);
-    else if (x_dtype == TURQ_ACT_BF16) wide_scale_kernel<TURQ_ACT_BF16><<<(unsigned)m, 256, 0, stream>>>(x, k, ldx, (_Float16 *)x16, inv);
+    const bool vec = (uintptr_t)x % 16 == 0 && ldx % 8 == 0 && k % 4 == 0;
+#define TURQ_WIDE_SCALE(XT)                                                                                                              \
+    if (!vec) wide_scale_kernel<XT, 1, false><<<(unsigned)m, 256, 0, stream>>>(x, k, ldx, (_Float16 *)x16, inv);                         \
+    else if (k <= 4096) wide_scale_kernel<XT, 4, true><<<(unsigned)m, 256, 0, stream>>>(x, k, ldx, (_Float16 *)x16, inv);                \
+    else wide_scale_kernel<XT, 12, true><<<(unsigned)m, 256, 0, stream>>>(x, k, ldx, (_Float16 *)x16, inv)
+    if (x_dtype == TURQ_ACT_F32) { TURQ_WIDE_SCALE(TURQ_ACT_F32); }
+    else if (x_dtype == TURQ_ACT_BF16) { TURQ_WIDE_SCALE(TURQ_ACT_BF16); }
     else return hipErrorInvalidValue;
+#undef TURQ_WIDE_SCALE
     return hipGetLastError();
 }
 
