@@ -203,6 +203,44 @@ template <int DT> __device__ inline void frags_from_staged(const uint8_t *__rest
     if constexpr (DT != TURQ_Q8_0) out[8] = kq_group_sums(out);
 }
 
+// What the first result of a wave is added to (TURQ_OUT_ACCUMULATE): the bits of y's four rows of the lane's column, requested behind the first weights
+// so that they have long arrived when the sums are done.  Always requested, whatever the flag says: a load behind a condition would make the
+// compiler wait for the weights in front of it.  (Places outside y: the last one inside it.)
+struct OldBits { uint32_t v[4]; };
+__device__ inline OldBits old_request(const void *__restrict__ y, int yt, int64_t row0, int64_t m, int64_t ldy, int64_t col, int64_t n) {
+    OldBits o;
+    const int64_t c = col < n ? col : n - 1;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int64_t at = (row0 + j < m ? row0 + j : m - 1) * ldy + c;
+        if ((yt & 0xFF) == TURQ_ACT_F32) o.v[j] = ((const uint32_t *)y)[at];
+        else o.v[j] = ((const uint16_t *)y)[at];
+    }
+    return o;
+}
+__device__ inline void store_col4(void *y, int yt, int64_t row0, int64_t m, int64_t ldy, int64_t col, float4v v, const OldBits &o) {
+    const int base = yt & 0xFF;
+    if (yt & TURQ_OUT_ACCUMULATE)
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] += out_value(o.v[j], base);
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+        if (row0 + j < m) turq_store_any(y, base, (row0 + j) * ldy + col, v[j]);
+}
+// the waves' parts of a result in wave order, four reads at a time (those past the last wave: its own again, dropped)
+__device__ inline float4v sum_parts(const float4v *__restrict__ red, int nwaves, int lane) {
+    float4v s = red[lane];
+    for (int wv = 1; wv < nwaves; wv += 4) {
+        float4v t[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) t[i] = red[(wv + i < nwaves ? wv + i : nwaves - 1) * 64 + lane];
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (wv + i < nwaves) s += t[i];
+    }
+    return s;
+}
+
 // m <= MR rows (4, 8, 16 or 32), k a multiple of 512.  More than 16 rows are taken as two halves of 16, one after the other against
 // the same weight tiles (HV = 2): the tiles of a column tile stay in their registers for both passes and are unpacked once per
 // pass, which for these launches costs less than what holding the fragments of 32 rows next to the rows in flight would
@@ -255,6 +293,13 @@ __device__ __forceinline__ void cs_body_staged(const uint8_t *__restrict__ w, in
     WRegs<DT> wr[D];
 #pragma unroll
     for (int d = 0; d < D; d++) wr[d] = load_tile<DT>(wrow[d % RG] + (2 * p + d / RG) * TB, go);
+    [[maybe_unused]] const int i1 = wave < RO * HV ? wave : 0;
+    [[maybe_unused]] OldBits old;
+    constexpr bool EARLY = !GU && RG <= 3;  // (six row tiles leave no registers for it)
+    if constexpr (EARLY) {
+        const uint32_t rt1 = rt0 + i1 / HV < nrt ? rt0 + i1 / HV : nrt - 1;
+        old = old_request(y, yt, HR * (i1 % HV) + 4 * (lane >> 4), m, ldy, (int64_t)rt1 * 16 + (lane & 15), n);
+    }
     uint8_t *rows = smem + wave * (HR * kXRow);
     AFrags<DT, 1> f;
     [[maybe_unused]] NormRoot root;
@@ -328,14 +373,9 @@ __device__ __forceinline__ void cs_body_staged(const uint8_t *__restrict__ w, in
     const int nn = lane & 15, g = lane >> 4;
     for (int i = wave; i < RO * HV; i += nwaves) {
         const int r = i / HV, h = i - r * HV;
-        float4v s = red[(i * nwaves) * 64 + lane];
-        for (int wv = 1; wv < nwaves; wv++) s += red[(i * nwaves + wv) * 64 + lane];
+        const float4v s = sum_parts(red + i * nwaves * 64, nwaves, lane);
         float4v s2 = float4v{0.f, 0.f, 0.f, 0.f};
-        if constexpr (GU) {
-            const int i2 = i + RO * HV;  // the up tile of the pair
-            s2 = red[(i2 * nwaves) * 64 + lane];
-            for (int wv = 1; wv < nwaves; wv++) s2 += red[(i2 * nwaves + wv) * 64 + lane];
-        }
+        if constexpr (GU) s2 = sum_parts(red + (i + RO * HV) * nwaves * 64, nwaves, lane);  // the up tile of the pair
         const int64_t col = (int64_t)(rt0 + r) * 16 + nn;
         if (rt0 + r >= nrt || col >= n) continue;
         const float bv = bias ? bias[col] : 0.0f, bv2 = (GU && bias2) ? bias2[col] : 0.0f;
@@ -348,7 +388,8 @@ __device__ __forceinline__ void cs_body_staged(const uint8_t *__restrict__ w, in
                 turq_store_any(y, yt, row * ldy + col, gate / (1.0f + expf(-gate)) * up);
             }
         } else {
-            turq_store_col4(y, yt, HR * h + 4 * g, m, ldy, col, s + float4v{bv, bv, bv, bv});
+            if (EARLY && i == wave) store_col4(y, yt, HR * h + 4 * g, m, ldy, col, s + float4v{bv, bv, bv, bv}, old);
+            else turq_store_col4(y, yt, HR * h + 4 * g, m, ldy, col, s + float4v{bv, bv, bv, bv});
         }
     }
 }
@@ -482,14 +523,9 @@ __device__ __forceinline__ void cs_body_staged_two(const uint8_t *__restrict__ w
     const int nn = lane & 15, g = lane >> 4;
     for (int i = wave; i < RO * 2; i += nwaves) {
         const int r = i / 2, mt = i - 2 * r;
-        float4v s = red[(i * nwaves) * 64 + lane];
-        for (int wv = 1; wv < nwaves; wv++) s += red[(i * nwaves + wv) * 64 + lane];
+        const float4v s = sum_parts(red + i * nwaves * 64, nwaves, lane);
         float4v s2 = float4v{0.f, 0.f, 0.f, 0.f};
-        if constexpr (GU) {
-            const int i2 = i + RO * 2;  // the up tile of the pair
-            s2 = red[(i2 * nwaves) * 64 + lane];
-            for (int wv = 1; wv < nwaves; wv++) s2 += red[(i2 * nwaves + wv) * 64 + lane];
-        }
+        if constexpr (GU) s2 = sum_parts(red + (i + RO * 2) * nwaves * 64, nwaves, lane);  // the up tile of the pair
         const int64_t col = (int64_t)(rt0 + r) * 16 + nn;
         if (rt0 + r >= nrt || col >= n) continue;
         const float bv = bias ? bias[col] : 0.0f, bv2 = (GU && bias2) ? bias2[col] : 0.0f;

@@ -335,11 +335,6 @@ template <int N> __device__ inline void sum_waves(const float *const (&p)[N], in
     }
 }
 constexpr int kSumPad = 7 * 64 * 4;  // bytes of LDS that sum_waves may read past the last wave's floats
-// an element of y as it lies in memory
-__device__ inline float out_value(uint32_t bits, int yt) {
-    return yt == TURQ_ACT_F32 ? __uint_as_float(bits) : yt == TURQ_ACT_BF16 ? __uint_as_float(bits << 16) : (float)as_half2(bits).x;
-}
-
 constexpr int kMaxRow1 = 4;
 struct Row1Args {
     const uint8_t *w[kMaxRow1];

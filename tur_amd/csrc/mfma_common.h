@@ -248,6 +248,10 @@ template <int YT> __device__ inline float turq_load_out(const void *y, int64_t i
     __builtin_memcpy(&h, &b, 2);
     return (float)h;
 }
+// an element of y as it lies in memory
+__device__ inline float out_value(uint32_t bits, int yt) {
+    return yt == TURQ_ACT_F32 ? __uint_as_float(bits) : yt == TURQ_ACT_BF16 ? __uint_as_float(bits << 16) : (float)as_half2(bits).x;
+}
 // the store of a result element whose type is only known at run time; with TURQ_OUT_ACCUMULATE in yt the value is added to
 // what y holds (the residual stream), in f32, and rounded once
 __device__ inline void turq_store_any(void *y, int yt, int64_t i, float v) {
