@@ -620,8 +620,7 @@ bool two_under_another(int dtype_a, int dtype_b, const TurqGemmWeights &ws, int6
 // The tile with which one weight goes through this kernel as far as single rounds over the CUs decide, 0: gemm_kq_kernel.
 // A launch of one round takes about base + per_sb * super-blocks, one line for every format; a further round costs as much again without the
 // launch itself, of the smallest tile, of which three workgroups share a CU, three fifths of it.  So the smallest tile that makes the launch one
-// round is taken, and the smallest of all up to one and a half (which at 1.5 is behind the one-round tile: Q6_K 4096 x 12288 at 65 - 96 rows 34.6 us against 27.5 of
-// 64 x 32, Q5_K 4096 x 4096 14.1 against 12.9).  Against gemm_kq_kernel:
+// round is taken, and the smallest of all up to one and a half (K-quants: two of them per workgroup where that makes one round, two_under_another).  Against gemm_kq_kernel:
 //   one or two MFMA tiles: Q4_K 1024 x 4096 at 40 / 300 / 512 rows 13.0 / 19.0 / 19.1 -> 6.6 / 9.3 / 10.7 us, 4096 x 4096 at 40 / 100 rows 19.2 /
 //   22.6 -> 8.7 / 11.3, Q6_K 4096 x 12288 33 / 43 -> 23 / 29, Q8_0 2048 x 2048 15 -> 5.4 / 5.5;
 //   three or four: K-quants from two super-blocks on (Q4_K 12288 x 256 at 48 rows 8.4 -> 9.4); Q8_0 2048 x 2048 at 300 / 512 rows 15.4 -> 8.5 / 10.2, Q4_K 4096 x 4096 at 256 24 -> 15;
