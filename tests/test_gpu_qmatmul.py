@@ -890,3 +890,20 @@ def test_columns_over_waves_two_workgroups_per_cu(gpu, dt, k):
     assert rel_l2(got, orc.matmul_dequant(dt, x, raw, n, k)) <= 1e-3
     assert np.array_equal(got[:64], gpu.qmatmul(w, x[:64], n, k))
     gpu.release(w)
+
+
+# K-quant launches of 32 x 32 tiles between one and one and a half rounds over the CUs go out with two tiles one under the other per workgroup: 97
+# n-blocks of three m-tiles (291 workgroups, 194 of two), the last block's second m-tile empty or ragged, weight rows that end inside a tile, bias; the
+# rows of a smaller call, which keeps one tile per workgroup, are the same to the bit.
+@pytest.mark.parametrize("dt", [Q4_K, Q5_K, Q6_K])
+@pytest.mark.parametrize("m", [65, 96])
+def test_two_tiles_per_workgroup_between_rounds(gpu, dt, m):
+    n, k = 3100, 2048
+    raw = synth.random_weight(dt, n, k, seed=dt + m)
+    w = gpu.upload(dt, n, k, raw, capi.LAYOUT_TILED)
+    x = synth.random_activation(m, k, seed=m, bf16=True)
+    bias = np.random.default_rng(m).standard_normal(n).astype(np.float32)
+    y = gpu.qmatmul(w, x, n, k, x_dtype=capi.ACT_BF16, bias=bias)
+    assert rel_l2(y - bias, orc.matmul_dequant(dt, x, raw, n, k)) <= 1e-3
+    assert np.array_equal(y[:40], gpu.qmatmul(w, x[:40], n, k, x_dtype=capi.ACT_BF16, bias=bias))
+    gpu.release(w)
