@@ -452,11 +452,6 @@ template <int DTA, int DTB, int MT, int NT, bool TIGHT, int MINB, bool PAIR>
 __global__ void __launch_bounds__(64 * W, MINB) gemm_cols_kernel(ColsGroup grp, int64_t k, const uint8_t *__restrict__ frags, int64_t m, int yt,
                                                            int nblocks_n, int nblocks_m, int vec_out) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    load_together(k, frags, m, yt, nblocks_n, nblocks_m, vec_out);
-    load_together(grp.w[0], grp.w[1], grp.n[0], grp.wscale[0], grp.wscale[1], grp.y[0], grp.bias[0], grp.bias[1], grp.ldy[0]);
-    if constexpr (!PAIR)
-        load_together(grp.w[2], grp.w[3], grp.n[1], grp.n[2], grp.n[3], grp.wscale[2], grp.wscale[3], grp.y[1], grp.y[2], grp.y[3], grp.bias[2], grp.bias[3],
-                      grp.ldy[1], grp.ldy[2], grp.ldy[3], grp.first[1], grp.first[2], grp.first[3], grp.second);
     // consecutive logical ids run on one XCD (blockIdx % 8): the m-blocks of one n-block share its packed weights in that XCD's L2.  Also where
     // the workgroups are no multiple of 8 (the first XCDs have one more): with ids as they come there, Q8_0 18944 x 1024 at 300 rows (990
     // workgroups) took 47.3 us instead of 41.3
