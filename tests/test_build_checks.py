@@ -4,9 +4,16 @@ import importlib.util
 import os
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-spec = importlib.util.spec_from_file_location("check_lds_waits", os.path.join(HERE, "..", "tur_amd", "csrc", "check_lds_waits.py"))
-chk = importlib.util.module_from_spec(spec)
-spec.loader.exec_module(chk)
+
+
+def load(name):
+    spec = importlib.util.spec_from_file_location(name, os.path.join(HERE, "..", "tur_amd", "csrc", name + ".py"))
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    return mod
+
+
+chk = load("check_lds_waits")
 
 
 def run(body):
@@ -59,3 +66,20 @@ def test_resource_remarks(tmp_path):
     p.write_text("x.hip:1:1: remark: Function Name: _Z4kernv [-Rpass]\nx.hip:1:1: remark:     ScratchSize [bytes/lane]: 16 [-R]\n"
                  "x.hip:1:1: remark:     VGPRs Spill: 3 [-R]\n")
     assert len(chk.check_resources(str(p), "kern")) == 2
+
+
+def test_spill_check(tmp_path):
+    """kernels that use scratch memory or keep scalar registers in vector ones are refused, but for those that are listed"""
+    spills = load("check_spills")
+    p = tmp_path / "r.remarks"
+
+    def status(name, scratch, sgprs):
+        p.write_text(f"x.hip:1:1: remark: Function Name: {name} [-Rpass]\nx.hip:1:1: remark:     ScratchSize [bytes/lane]: {scratch} [-R]\n"
+                     f"x.hip:1:1: remark:     SGPRs Spill: {sgprs} [-R]\nx.hip:1:1: remark:     VGPRs Spill: 0 [-R]\n")
+        return spills.main([str(p)])
+
+    staged, frag = "_Z15gemv_cs_stagedILi1EEvv", "_Z16gemv_mfma_kernelILi1EEvv"  # void gemv_cs_staged<1>(), void gemv_mfma_kernel<1>()
+    assert status(staged, 0, 0) == 0 and status(frag, 0, 0) == 0
+    assert status(staged, 16, 0) == 1 and status(frag, 16, 0) == 1
+    assert status(staged, 0, 2) == 1
+    assert status(frag, 0, 245) == 0 and status(frag, 0, 251) == 1

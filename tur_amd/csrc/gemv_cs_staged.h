@@ -45,20 +45,35 @@ template <int XT> struct XOff {
         two = one + (XT != TURQ_ACT_F32 && lane >= 32 ? 2u * (uint32_t)ldx : 0u);
     }
 };
-// rows row0 .. row0 + MR - 1 (rows past m repeat row m - 1) of column tile b
-template <int XT, int MR>
-__device__ inline XRows<XT, MR> load_x_rows(const void *__restrict__ x, int64_t ldx, int64_t m, int row0, int64_t b, XOff<XT> o) {
+// What the rows' addresses are worked out from.  Left alone the compiler keeps those of every row from pass to pass, which in the loops over pairs
+// overran the scalar registers (up to 198 of them kept in vector lanes, a write and its reads each): renew() makes new values of them where a
+// loop comes round, so that nothing behind it uses what was worked out before.
+struct XFrom {
+    int64_t ldx;
+    int last;  // the last row
+    __device__ XFrom(int64_t l, int64_t m) : ldx(l), last((int)m - 1) {}
+    __device__ void renew() { asm volatile("" : "+s"(ldx), "+s"(last)); }
+};
+// Rows row0 .. row0 + MR - 1 of column tile b (past the last row one that is there, of which nothing is read back from the LDS).  CHAIN: one scalar
+// address that steps from load to load, by a stride that becomes 0 behind the last row, which takes the fewest registers; otherwise a product per
+// row, whose instructions do not wait for each other.  In us, kept from pass to pass / products / chain: Q4_K 2048 x 6144 at 24 f16 rows 9.9 / 9.8 / 9.4, 8192 x
+// 8192 at 32 bf16 rows 20.3 / - / 19.4, Q6_K 4096 x 12288 at 32 f16 rows 19.5 / 19.7 / 19.1, at 16 f32 rows 18.1 / 18.3 / 18.3; Q5_K 4096 x 4096, written out, at 20
+// bf16 rows 9.7 / 10.4 / 9.7; but Q4_K 4096 x 4096 at 32 f32 rows 10.1 / 10.05 / 10.3, Q8_0 2048 x 6144 at 8 rows 7.44 / 7.44 / 7.50.
+template <int XT, int MR, bool CHAIN>
+__device__ inline XRows<XT, MR> load_x_rows(const void *__restrict__ x, const XFrom &from, int row0, int64_t b, XOff<XT> o) {
     XRows<XT, MR> raw;
-    constexpr int ES = XT == TURQ_ACT_F32 ? 4 : 2;
-    const uint8_t *base = (const uint8_t *)x + b * (256 * ES);
-    const int top = (int)m - 1;
+    constexpr int ES = XT == TURQ_ACT_F32 ? 4 : 2, STEP = XT == TURQ_ACT_F32 ? 1 : 2;
+    const uint64_t stride = (uint64_t)from.ldx * ES;
+    const int left = from.last - row0;  // rows behind the first
     asm volatile("" : "+v"(o.one), "+v"(o.two));  // (32-bit offsets next to the loads: see GOff)
+    const uint32_t past = CHAIN && (left & 1) ? o.two : o.one;
+    const uint8_t *base = (const uint8_t *)x + b * (256 * ES), *p = base + (uint64_t)row0 * stride;
 #pragma unroll
-    for (int j = 0; j < MR; j += XT == TURQ_ACT_F32 ? 1 : 2) {
-        const int row = row0 + j < top ? row0 + j : top;
-        const uint8_t *p = base + (uint64_t)(uint32_t)row * (uint64_t)ldx * ES;
+    for (int j = 0; j < MR; j += STEP) {
+        if constexpr (!CHAIN) p = base + (uint64_t)(uint32_t)(row0 + j < from.last ? row0 + j : from.last) * stride;
         if constexpr (XT == TURQ_ACT_F32) raw.v[j] = *(const uint4v *)(p + o.one);
-        else raw.v[j / 2] = *(const uint4v *)(p + (row0 + j < top ? o.two : o.one));
+        else raw.v[j / 2] = *(const uint4v *)(p + (j < left ? o.two : past));
+        if constexpr (CHAIN) p += j + STEP <= left ? STEP * stride : 0;
     }
     return raw;
 }
@@ -261,6 +276,7 @@ __device__ __forceinline__ void cs_body_staged(const uint8_t *__restrict__ w, in
     constexpr int RO = GU ? RG / 2 : RG;  // row tiles of the output per workgroup
     constexpr int HV = MR > 16 ? 2 : 1;   // passes of HR rows each
     constexpr int HR = MR / HV;
+    constexpr bool CHAIN = HR == 16 && (CNT == 0 || (HV == 2 && XT != TURQ_ACT_F32)), RENEW = HV == 2 && CNT > 0 && CHAIN;  // (RENEW: for every column tile)
     static_assert(D >= 1 && D <= 2 * RG && (2 * RG) % D == 0 && (HV == 1 || D >= RG), "ring of weight tiles");
     extern __shared__ uint8_t smem[];
     constexpr int TB = TiledFmt<DT>::kTileBytes;
@@ -282,12 +298,13 @@ __device__ __forceinline__ void cs_body_staged(const uint8_t *__restrict__ w, in
     GOff go = lane_offsets(lane, 16);
     int64_t p = wave;  // the current pair: column tiles 2 p and 2 p + 1
     const XOff<XT> xo(ldx, lane);
+    XFrom from(ldx, m);
     // the first column tile's rows go out first (for the norm: those of both, and its weights), the first D weight tiles right behind them
-    XRows<XT, HR> raw = load_x_rows<XT, HR>(x, ldx, m, 0, 2 * p, xo);
+    XRows<XT, HR> raw = load_x_rows<XT, HR, CHAIN>(x, from, 0, 2 * p, xo);
     [[maybe_unused]] XRows<XT, HR> raw2;
     [[maybe_unused]] NormW<XT> nw[2];
     if constexpr (NORM) {
-        raw2 = load_x_rows<XT, HR>(x, ldx, m, 0, 2 * p + 1, xo);
+        raw2 = load_x_rows<XT, HR, CHAIN>(x, from, 0, 2 * p + 1, xo);
         nw[0] = load_norm_w<XT>(gw, 2 * p, lane), nw[1] = load_norm_w<XT>(gw, 2 * p + 1, lane);
     }
     WRegs<DT> wr[D];
@@ -322,9 +339,10 @@ __device__ __forceinline__ void cs_body_staged(const uint8_t *__restrict__ w, in
                 __builtin_amdgcn_sched_barrier(0);
                 // the rows of the next pass: the other half of this column tile, the pair's second column tile, the next pair
                 if constexpr (!NORM) {
-                    if (h + 1 < HV) raw = load_x_rows<XT, HR>(x, ldx, m, HR * (h + 1), 2 * p + cc, xo);
-                    else if (cc == 0) raw = load_x_rows<XT, HR>(x, ldx, m, 0, 2 * p + 1, xo);
-                    else if (!LAST) raw = load_x_rows<XT, HR>(x, ldx, m, 0, 2 * (p + nwaves), xo);
+                    if (h + 1 == HV && (cc == 1 || RENEW)) from.renew();
+                    if (h + 1 < HV) raw = load_x_rows<XT, HR, CHAIN>(x, from, HR * (h + 1), 2 * p + cc, xo);
+                    else if (cc == 0) raw = load_x_rows<XT, HR, CHAIN>(x, from, 0, 2 * p + 1, xo);
+                    else if (!LAST) raw = load_x_rows<XT, HR, CHAIN>(x, from, 0, 2 * (p + nwaves), xo);
                 }
                 __builtin_amdgcn_sched_barrier(0);
                 frags_from_staged<DT>(rows, (int)m - HR * h, lane, f.a[0]);
@@ -466,9 +484,13 @@ __device__ __forceinline__ void cs_body_staged_two(const uint8_t *__restrict__ w
     GOff go = lane_offsets(lane, 16);
     int64_t p = wave;
     const XOff<XT> xo(ldx, lane);
+    XFrom from(ldx, m);
     XRows<XT, 16> raw[2];
 #pragma unroll
-    for (int mt = 0; mt < 2; mt++) raw[mt] = load_x_rows<XT, 16>(x, ldx, m, 16 * mt, 2 * p, xo);
+    for (int mt = 0; mt < 2; mt++) {
+        raw[mt] = load_x_rows<XT, 16, true>(x, from, 16 * mt, 2 * p, xo);
+        if (CNT == 0) from.renew();
+    }
     WRegs<DT> wr[D];
 #pragma unroll
     for (int d = 0; d < D; d++) wr[d] = load_tile<DT>(wrow[d % RG] + (2 * p + d / RG) * TB, go);
@@ -484,7 +506,10 @@ __device__ __forceinline__ void cs_body_staged_two(const uint8_t *__restrict__ w
             if (cc == 0 || !LAST) {
                 const int64_t b = cc == 0 ? 2 * p + 1 : 2 * (p + nwaves);
 #pragma unroll
-                for (int mt = 0; mt < 2; mt++) raw[mt] = load_x_rows<XT, 16>(x, ldx, m, 16 * mt, b, xo);
+                for (int mt = 0; mt < 2; mt++) {
+                    if (mt == 0 || CNT == 0) from.renew();
+                    raw[mt] = load_x_rows<XT, 16, true>(x, from, 16 * mt, b, xo);
+                }
             }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
