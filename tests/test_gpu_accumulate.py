@@ -112,6 +112,22 @@ def test_results_are_added_to_the_output(gpu, dt, n, k, ms, yt):
     gpu.release(w)
 
 
+# launches of several row tiles per workgroup in the kernels that stage the rows (263 row tiles: two, 513: three), whose waves request what y held ahead of
+# their sums: every row count's instantiation, one pair of column tiles per wave (1024) and several (5120), a last row tile that ends inside
+@pytest.mark.parametrize("yt", [capi.ACT_F32, capi.ACT_BF16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("dt,n,k", [(Q4_K, 4200, 1024), (Q6_K, 8202, 1024), (Q8_0, 4200, 5120), (Q5_K, 8202, 5120), (Q8_0, 130, 5120)])
+def test_results_are_added_by_the_staged_kernels(gpu, dt, n, k, yt):
+    w = gpu.upload(dt, n, k, synth.random_weight(dt, n, k, seed=n + k), capi.LAYOUT_TILED)
+    rng = np.random.default_rng(n)
+    for m in (3, 8, 13, 32):
+        for xt in (capi.ACT_F32, capi.ACT_BF16):
+            x = synth.random_activation(m, k, seed=m, bf16=True)
+            y0 = to_type(rng.standard_normal((m, n)).astype(np.float32) * 50.0, yt)
+            plain = run(gpu, w, x, n, k, np.zeros((m, n), np.float32), capi.ACT_F32, 0, x_dtype=xt)
+            assert np.array_equal(run(gpu, w, x, n, k, y0, yt, ACC, x_dtype=xt), to_type(plain + y0, yt)), (m, xt)
+    gpu.release(w)
+
+
 # the matrices above are small, so the rules give them the smallest tile: once more with every tile of gemm_kq_kernel (o_proj and
 # down_proj of long prompts), and with the tiles of the column-splitting kernel whose waves meet in several rounds
 @pytest.mark.parametrize("switch,value", [("TURQ_GEMM_COLS", "0"), ("TURQ_GEMM_WIDE", "1"), ("TURQ_GEMM_LOW", "0"), ("TURQ_GEMM_KGROUPS", "1"),

@@ -218,9 +218,10 @@ template <int DT> __device__ inline void frags_from_staged(const uint8_t *__rest
     if constexpr (DT != TURQ_Q8_0) out[8] = kq_group_sums(out);
 }
 
-// What the first result of a wave is added to (TURQ_OUT_ACCUMULATE): the bits of y's four rows of the lane's column, requested behind the first weights
-// so that they have long arrived when the sums are done.  Always requested, whatever the flag says: a load behind a condition would make the
-// compiler wait for the weights in front of it.  (Places outside y: the last one inside it.)
+// What the first result of a wave is added to (TURQ_OUT_ACCUMULATE, an instantiation of its own: a load behind a condition would make the compiler wait
+// for the weights in front of it, and one that is always made costs the launches that add nothing 0.3 - 0.6 us, q, k and v of 4096 columns at 8 rows 7.9
+// for 7.35): the bits of y's four rows of the lane's column, requested behind the first weights so that they have long arrived when the
+// sums are done.  (Places outside y: the last one inside it.)
 struct OldBits { uint32_t v[4]; };
 __device__ inline OldBits old_request(const void *__restrict__ y, int yt, int64_t row0, int64_t m, int64_t ldy, int64_t col, int64_t n) {
     OldBits o;
@@ -233,14 +234,11 @@ __device__ inline OldBits old_request(const void *__restrict__ y, int yt, int64_
     }
     return o;
 }
-__device__ inline void store_col4(void *y, int yt, int64_t row0, int64_t m, int64_t ldy, int64_t col, float4v v, const OldBits &o) {
+__device__ inline void add_col4(void *y, int yt, int64_t row0, int64_t m, int64_t ldy, int64_t col, float4v v, const OldBits &o) {
     const int base = yt & 0xFF;
-    if (yt & TURQ_OUT_ACCUMULATE)
-#pragma unroll
-        for (int j = 0; j < 4; j++) v[j] += out_value(o.v[j], base);
 #pragma unroll
     for (int j = 0; j < 4; j++)
-        if (row0 + j < m) turq_store_any(y, base, (row0 + j) * ldy + col, v[j]);
+        if (row0 + j < m) turq_store_any(y, base, (row0 + j) * ldy + col, v[j] + out_value(o.v[j], base));
 }
 // the waves' parts of a result in wave order, four reads at a time (those past the last wave: its own again, dropped)
 __device__ inline float4v sum_parts(const float4v *__restrict__ red, int nwaves, int lane) {
@@ -265,8 +263,8 @@ __device__ inline float4v sum_parts(const float4v *__restrict__ red, int nwaves,
 // is stored is silu(gate) * up (src/models/qwen3.rs:161-167).
 // CNT: pairs per wave when every wave has the same number and it is known at compile time (the loop is then written out, which
 // is 1 - 5 % faster on the 4096-column weights), 0: counted at run time.
-// NORM (CNT 1, one pass): x stands for RmsNorm(x) with weight gw
-template <int DT, int XT, int MR, int RG, int D, int CNT, bool GU = false, bool NORM = false>
+// NORM (CNT 1, one pass): x stands for RmsNorm(x) with weight gw.  ACC: yt has TURQ_OUT_ACCUMULATE
+template <int DT, int XT, int MR, int RG, int D, int CNT, bool GU = false, bool NORM = false, bool ACC = false>
 __device__ __forceinline__ void cs_body_staged(const uint8_t *__restrict__ w, int64_t n, int64_t k, const void *__restrict__ x, int64_t ldx,
                                                int64_t m, void *__restrict__ y, int yt, int64_t ldy, const float *__restrict__ bias,
                                                int64_t grp, const uint8_t *__restrict__ w2 = nullptr,
@@ -312,7 +310,7 @@ __device__ __forceinline__ void cs_body_staged(const uint8_t *__restrict__ w, in
     for (int d = 0; d < D; d++) wr[d] = load_tile<DT>(wrow[d % RG] + (2 * p + d / RG) * TB, go);
     [[maybe_unused]] const int i1 = wave < RO * HV ? wave : 0;
     [[maybe_unused]] OldBits old;
-    constexpr bool EARLY = !GU && RG <= 3;  // (six row tiles leave no registers for it)
+    constexpr bool EARLY = ACC && !GU && RG <= 3;  // (six row tiles leave no registers for it)
     if constexpr (EARLY) {
         const uint32_t rt1 = rt0 + i1 / HV < nrt ? rt0 + i1 / HV : nrt - 1;
         old = old_request(y, yt, HR * (i1 % HV) + 4 * (lane >> 4), m, ldy, (int64_t)rt1 * 16 + (lane & 15), n);
@@ -406,7 +404,7 @@ __device__ __forceinline__ void cs_body_staged(const uint8_t *__restrict__ w, in
                 turq_store_any(y, yt, row * ldy + col, gate / (1.0f + expf(-gate)) * up);
             }
         } else {
-            if (EARLY && i == wave) store_col4(y, yt, HR * h + 4 * g, m, ldy, col, s + float4v{bv, bv, bv, bv}, old);
+            if (EARLY && i == wave) add_col4(y, yt, HR * h + 4 * g, m, ldy, col, s + float4v{bv, bv, bv, bv}, old);
             else turq_store_col4(y, yt, HR * h + 4 * g, m, ldy, col, s + float4v{bv, bv, bv, bv});
         }
     }
@@ -427,17 +425,16 @@ constexpr int staged_second_rows(int rg) { return (rg + 1) / 2; }
 
 // weights [0, a.second) are of format DTA with RG row tiles per workgroup, the others of DTB with staged_second_rows(RG)
 // (one format: DTA == DTB)
-template <int DTA, int DTB, int XT, int MR, int RG, int CNT, bool NORM = false>
+template <int DTA, int DTB, int XT, int MR, int RG, int CNT, bool NORM = false, bool ACC = false>
 __global__ void __launch_bounds__(512) gemv_cs_staged_kernel(MultiArgs a, int64_t k, const void *__restrict__ x, int64_t ldx, int64_t m, int yt,
                                                              const float *__restrict__ gw, float eps) {
-    load_together(k, x, ldx, m, yt, gw, eps);
     const MultiPick p = multi_pick(a, (int)blockIdx.x);
     constexpr int RGB = staged_second_rows(RG);
     if (DTA == DTB || p.index < a.second)
-        cs_body_staged<DTA, XT, MR, RG, staged_ring(DTA, RG, MR, DTA != DTB), CNT, false, NORM>(p.w, p.n, k, x, ldx, m, p.y, yt, p.ldy, p.bias,
+        cs_body_staged<DTA, XT, MR, RG, staged_ring(DTA, RG, MR, DTA != DTB), CNT, false, NORM, ACC>(p.w, p.n, k, x, ldx, m, p.y, yt, p.ldy, p.bias,
                                                                                                (int64_t)p.block, nullptr, nullptr, gw, eps);
     else
-        cs_body_staged<DTB, XT, MR, RGB, staged_ring(DTB, RGB, MR, DTA != DTB), CNT, false, NORM>(p.w, p.n, k, x, ldx, m, p.y, yt, p.ldy, p.bias,
+        cs_body_staged<DTB, XT, MR, RGB, staged_ring(DTB, RGB, MR, DTA != DTB), CNT, false, NORM, ACC>(p.w, p.n, k, x, ldx, m, p.y, yt, p.ldy, p.bias,
                                                                                                  (int64_t)p.block, nullptr, nullptr, gw, eps);
 }
 
@@ -572,7 +569,6 @@ __device__ __forceinline__ void cs_body_staged_two(const uint8_t *__restrict__ w
 template <int DTA, int DTB, int XT, int CNT>
 __global__ void __launch_bounds__(256) gemv_cs_staged_two_kernel(MultiArgs a, int64_t k, const void *__restrict__ x, int64_t ldx, int64_t m,
                                                                   int yt, const float *, float) {
-    load_together(k, x, ldx, m, yt);
     const MultiPick p = multi_pick(a, (int)blockIdx.x);
     constexpr int RGB = staged_second_rows(6);
     if (DTA == DTB || p.index < a.second) cs_body_staged_two<DTA, XT, 6, 3, CNT>(p.w, p.n, k, x, ldx, m, p.y, yt, p.ldy, p.bias, (int64_t)p.block);
@@ -636,6 +632,12 @@ hipError_t staged_count(const StagedLaunch &l) {
             if (l.cnt == 1) return staged_go<gemv_cs_staged_kernel<DTA, DTB, XT, MR, RG, 1, true>>(staged_lds<MR, RG>(l.nwaves, true), l);
         }
         return hipErrorInvalidValue;
+    }
+    if constexpr (DTA == DTB && RG <= 3) {  // (the residual additions behind o_proj and down_proj, each a weight alone; others add through the store)
+        if (l.yt & TURQ_OUT_ACCUMULATE) {
+            if (l.cnt == 1) return staged_go<gemv_cs_staged_kernel<DTA, DTB, XT, MR, RG, 1, false, true>>(staged_lds<MR, RG>(l.nwaves, false), l);
+            if constexpr (MR <= 16 || XT != TURQ_ACT_F32) return staged_go<gemv_cs_staged_kernel<DTA, DTB, XT, MR, RG, 0, false, true>>(staged_lds<MR, RG>(l.nwaves, false), l);
+        }
     }
     if (l.cnt == 1) return staged_go<gemv_cs_staged_kernel<DTA, DTB, XT, MR, RG, 1>>(staged_lds<MR, RG>(l.nwaves, false), l);
     if constexpr (MR <= 16 || XT != TURQ_ACT_F32) return staged_go<gemv_cs_staged_kernel<DTA, DTB, XT, MR, RG, 0>>(staged_lds<MR, RG>(l.nwaves, false), l);
