@@ -247,3 +247,49 @@ def test_norm_in_the_staged_kernels(gpu, fmts, k, m, x_dtype):
         assert np.array_equal(a, b)
     for w in ws:
         gpu.release(w)
+
+
+@pytest.mark.parametrize("mlp", [False, True], ids=["multi", "mlp"])
+def test_scratch_of_more_rows_serves_a_capture_of_fewer(mlp):
+    """8 rows are normalised inside the kernels, 2 rows in scratch memory first: the call of 8 leaves enough for a capture of the call of 2, in
+    which nothing may be allocated"""
+    gpu = Gpu()
+    L, ctx = gpu.L, gpu.ctx
+    k, n = (2048, 4096) if mlp else (1024, 200)
+    shapes = [(n, k), (n, k), (k, n)] if mlp else [(n, k), (48, k)]
+    ws = [gpu.upload(Q8_0, a, b, synth.random_weight(Q8_0, a, b, seed=i), capi.LAYOUT_TILED) for i, (a, b) in enumerate(shapes)]
+    x = synth.random_activation(8, k, seed=2)
+    ns = [k] if mlp else [n, 48]
+    d = Dev(gpu)
+    xp, nwp, yps = d.put(x), d.put(np.full(k, 0.02, np.float32)), [d.put(np.zeros((8, c), np.float32)) for c in ns]
+    warr = (ctypes.c_void_p * len(ws))(*[w.value for w in ws])
+    yarr, ldys = (ctypes.c_void_p * len(ns))(*[p.value for p in yps]), (ctypes.c_int64 * len(ns))(*ns)
+
+    def call(m):
+        if mlp:
+            rc = L.turq_norm_mlp(ctx, *ws, xp, capi.ACT_F32, m, k, nwp, EPS, yps[0], capi.ACT_F32, k, None, None, None, 0, capi.MEM_DEVICE)
+        else:
+            rc = L.turq_norm_qmatmul_multi(ctx, len(ws), warr, xp, capi.ACT_F32, m, k, nwp, EPS, yarr, capi.ACT_F32, ldys, None, capi.MEM_DEVICE)
+        capi.check(rc, ctx)
+
+    call(8)
+    capi.check(L.turq_sync(ctx), ctx)
+    capi.check(L.turq_graph_begin(ctx), ctx)
+    call(2)
+    g = ctypes.c_void_p()
+    capi.check(L.turq_graph_end(ctx, ctypes.byref(g)), ctx)
+    call(2)
+    want = [gpu.read_back(p, (2, c), np.float32) for p, c in zip(yps, ns)]
+    for _ in range(3):
+        call(8)
+        for p, c in zip(yps, ns):
+            capi.check(L.turq_memcpy_h2d(ctx, p, capi.ptr(np.zeros((2, c), np.float32)), 8 * c), ctx)
+        capi.check(L.turq_graph_launch(ctx, g), ctx)
+        capi.check(L.turq_sync(ctx), ctx)
+        for p, c, t in zip(yps, ns, want):
+            assert np.array_equal(gpu.read_back(p, (2, c), np.float32), t)
+    L.turq_graph_destroy(g)
+    d.free()
+    for w in ws:
+        gpu.release(w)
+    gpu.close()

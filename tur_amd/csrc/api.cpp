@@ -815,12 +815,21 @@ static int impl_mlp(turq_ctx *ctx, const turq_weight *gate, const turq_weight *u
 
 // the normalised rows in scratch memory of the context, for the calls whose kernels do not apply the norm themselves: f16 where
 // the matmul kernels would round them to f16 first thing (the same values, half the bytes), f32 with wide activations
+static int norm_reserve(turq_ctx *ctx, int64_t m, int64_t k, int ht) {
+    return turq_ctx_reserve(ctx, &ctx->norm_x, &ctx->norm_x_cap, (size_t)m * (size_t)k * (size_t)turq_act_bytes(ht) + 16);
+}
 static int norm_to_scratch(turq_ctx *ctx, const void *x, int xt, int64_t m, int64_t k, int64_t ldx, const float *nw, float eps, int *ht) {
     *ht = ctx->wide ? TURQ_ACT_F32 : TURQ_ACT_F16;
-    int rc = turq_ctx_reserve(ctx, &ctx->norm_x, &ctx->norm_x_cap, (size_t)m * (size_t)k * (size_t)turq_act_bytes(*ht) + 16);
+    const int rc = norm_reserve(ctx, m, k, *ht);
     if (rc != TURQ_OK) return rc;
     TURQ_HIP(ctx, turq_launch_rms_norm(x, xt, m, k, ldx, nw, eps, ctx->norm_x, *ht, k, ctx->stream));
     return TURQ_OK;
+}
+
+// A call of several rows whose kernels apply the norm leaves that scratch behind all the same: one of fewer rows, which may need it, then finds it in a
+// capture, where nothing may be allocated.  (Inside a capture, which cannot make any, the call goes without.)
+static int norm_for_fewer_rows(turq_ctx *ctx, int64_t m, int64_t k) {
+    return m > 1 && !ctx->capturing ? norm_reserve(ctx, m, k, TURQ_ACT_F16) : TURQ_OK;
 }
 
 static int norm_args(turq_ctx *ctx, const char *fn, const void *x, int xt, int64_t m, int64_t k, int64_t ldx, const float *nw) {
@@ -863,7 +872,11 @@ static int impl_norm_qmatmul_multi(turq_ctx *ctx, int count, const turq_weight *
     }
     if (plain && turq_norm_fuses(ctx, count, weights, x, xt, ldx, m)) {
         const TurqNorm nm{nw, eps};
-        if (m <= TURQ_GEMV_MAX_M) return turq_qmatmul_multi_mfma(ctx, count, weights, x, xt, m, ldx, ys, yt, ldys, biases, &nm);
+        if (m <= TURQ_GEMV_MAX_M) {
+            rc = norm_for_fewer_rows(ctx, m, k);
+            if (rc != TURQ_OK) return rc;
+            return turq_qmatmul_multi_mfma(ctx, count, weights, x, xt, m, ldx, ys, yt, ldys, biases, &nm);
+        }
         bool taken = false;
         rc = turq_qmatmul_multi_gemm(ctx, count, weights, x, xt, m, ldx, ys, yt, ldys, biases, &taken, &nm);
         if (rc != TURQ_OK || taken) return rc;
@@ -900,6 +913,8 @@ static int impl_norm_mlp(turq_ctx *ctx, const turq_weight *gate, const turq_weig
             const bool h16 = turq_dt_is_quant(down->dtype) && down->layout == TURQ_LAYOUT_TILED && n_ff % 8 == 0;
             const int ht = h16 ? TURQ_ACT_F16 : TURQ_ACT_F32;
             rc = turq_ctx_reserve(ctx, &ctx->mlp_h, &ctx->mlp_h_cap, (size_t)m * (size_t)n_ff * (h16 ? sizeof(uint16_t) : sizeof(float)) + 16);
+            if (rc != TURQ_OK) return rc;
+            rc = norm_for_fewer_rows(ctx, m, k);
             if (rc != TURQ_OK) return rc;
             rc = turq_qmatmul_gate_up_mfma(ctx, gate, up, x, xt, m, ldx, ctx->mlp_h, ht, n_ff, bias_gate, bias_up, &taken, &nm);
             if (rc != TURQ_OK) return rc;
