@@ -293,3 +293,34 @@ def test_scratch_of_more_rows_serves_a_capture_of_fewer(mlp):
     for w in ws:
         gpu.release(w)
     gpu.close()
+
+
+# results over the rows they come from: the kernels that normalise on the way read x until their last workgroup has started, so the norm goes to
+# scratch memory first, which gives the bits of the separate calls at one row too (40 rows: the norm's fragments are written before the products)
+@pytest.mark.parametrize("m", [1, 2, 3, 8, 32, 40])
+def test_results_over_the_activations(gpu, m):
+    L, ctx = gpu.L, gpu.ctx
+    k, ns = 1024, [1024, 48]
+    ws = [gpu.upload(dt, n, k, synth.random_weight(dt, n, k, seed=n), capi.LAYOUT_TILED) for dt, n in zip((Q4_K, Q6_K), ns)]
+    x = synth.random_activation(m, k, seed=m)
+    nw = (1.0 + 0.3 * np.random.default_rng(m).standard_normal(k)).astype(np.float32)
+    want, normed = separate(gpu, ws, ns, x, nw)
+    alone = gpu.qmatmul_multi(ws[1:], normed, ns[1:], k)[0]
+    d = Dev(gpu)
+    xp, nwp, yp = d.put(x), d.put(nw), d.put(np.zeros((m, 48), np.float32))
+
+    def call(weights, outs, lds):
+        cnt = len(weights)
+        capi.check(L.turq_memcpy_h2d(ctx, xp, capi.ptr(x), x.nbytes), ctx)
+        capi.check(L.turq_norm_qmatmul_multi(ctx, cnt, (ctypes.c_void_p * cnt)(*[w.value for w in weights]), xp, capi.ACT_F32, m, k, nwp, EPS,
+                                             (ctypes.c_void_p * cnt)(*[p.value for p in outs]), capi.ACT_F32, (ctypes.c_int64 * cnt)(*lds), None,
+                                             capi.MEM_DEVICE), ctx)
+        return gpu.read_back(xp, (m, k), np.float32)
+
+    assert np.array_equal(call(ws, [xp, yp], [k, 48]), want[0])
+    assert np.array_equal(gpu.read_back(yp, (m, 48), np.float32), want[1])
+    over = call(ws[1:], [xp], [k])  # one weight, fewer columns than x has
+    assert np.array_equal(over[:, :48], alone) and np.array_equal(over[:, 48:], x[:, 48:])
+    d.free()
+    for w in ws:
+        gpu.release(w)

@@ -866,7 +866,7 @@ static int impl_norm_qmatmul_multi(turq_ctx *ctx, int count, const turq_weight *
         const uintptr_t lo = (uintptr_t)p;
         return std::pair<uintptr_t, uintptr_t>(lo, lo + (uintptr_t)((m - 1) * ld + cols) * (uintptr_t)turq_act_bytes(type));
     };
-    for (int i = 0; i < count && plain && m > 1 && m <= TURQ_GEMV_MAX_M; i++) {
+    for (int i = 0; i < count && plain && m <= TURQ_GEMV_MAX_M; i++) {
         const auto in = span(x, ldx, k, xt), out = span(ys[i], ldys[i], weights[i]->n, yt);
         plain = in.second <= out.first || out.second <= in.first;
     }
