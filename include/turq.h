@@ -295,7 +295,7 @@ int turq_mlp(turq_ctx *ctx, const turq_weight *gate, const turq_weight *up, cons
  * where the separate calls round the normalised value: within 5e-4 relative L2 of them, inside the 1e-3 bar against an f64 norm
  * followed by the f32 matmul); for MORE THAN 32 rows the norm writes the fragments of the prefill GEMM directly (the results of turq_rms_norm into f32
  * followed by turq_qmatmul_multi, bit for bit); for 3 - 8 rows of 1024 - 4096 columns against few weight rows the kernels that stage the rows
- * normalise them on the way (bit for bit too, but for rows whose root is outside 2^-40 .. 2^40).  Every other case, and any call of up to 32 rows whose
+ * normalise them on the way (bit for bit too).  Every other case, and any call of up to 32 rows whose
  * results lie over x, runs the norm into scratch memory of the context - as f16 where the matmul kernels would round its output to f16
  * anyway: the same values, half the bytes for them to read - and then
  * the plain call (also bit-equal to the separate calls).  Range: the one-row route rounds x * norm_weight, not the normalised

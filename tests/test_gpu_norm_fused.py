@@ -324,3 +324,19 @@ def test_results_over_the_activations(gpu, m):
     d.free()
     for w in ws:
         gpu.release(w)
+
+
+@pytest.mark.parametrize("x_dtype", [capi.ACT_F32, capi.ACT_BF16], ids=["f32", "bf16"])
+def test_rows_with_very_large_roots_in_the_staged_kernels(gpu, x_dtype):
+    """roots above 2^40, where the norm divides instead of correcting a product: the bits of the separate calls (a quotient an ulp off moves one f16
+    rounding in 2^13, so it takes some rows to see it)"""
+    k, m, n = 2048, 8, 48
+    w = gpu.upload(Q8_0, n, k, synth.random_weight(Q8_0, n, k, seed=1), capi.LAYOUT_TILED)
+    for seed in range(24):
+        x = synth.random_activation(m, k, seed=seed, bf16=x_dtype == capi.ACT_BF16) * np.float32(2.0 ** 46)
+        x[seed % m] *= np.float32(2.0 ** -50)  # (one row of the usual kind among them)
+        nw = np.ones(k, np.float32)
+        got = norm_multi(gpu, [w, w], [n, n], x, nw, x_dtype=x_dtype)
+        want, _ = separate(gpu, [w, w], [n, n], x, nw, x_dtype=x_dtype)
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1]), seed
+    gpu.release(w)

@@ -135,9 +135,10 @@ __device__ inline void norm_part(const XRows<XT, MR> (&raw)[2], float *__restric
         }
     }
 }
-// Lane r: the root of row r, as RowDiv (norm.hip) uses it: quotient q = v * inv, corrected by (v - q * rms) * fix to the correctly rounded one.  Rows
-// whose root is 0, an infinity, a NaN or outside 2^-40 .. 2^40 go without the correction (an ulp).
-struct NormRoot { float inv, rms, fix; };
+// Lane r: the root of row r, as RowDiv (norm.hip) uses it: quotient q = v * inv, corrected by (v - q * rms) * inv to the correctly rounded one.  plain: one of
+// the rows has a root that is 0, an infinity, a NaN or outside 2^-40 .. 2^40: the wave divides.  (An element below 2^-60, which RowDiv divides as
+// well, has a quotient that is corrected exactly or too small for f16.)
+struct NormRoot { float inv, rms; bool plain; };
 template <int XT, int MR>
 __device__ inline NormRoot norm_root(const float *__restrict__ part, int nwaves, int lane, int64_t k, float eps) {
     constexpr int PW = kNormPart<XT>;
@@ -155,13 +156,12 @@ __device__ inline NormRoot norm_root(const float *__restrict__ part, int nwaves,
         total = wv == 0 ? b : wv < nwaves ? total + b : total;
     }
     const float rms = sqrtf(total / (float)k + eps);
-    const bool plain = !(rms > 0x1p-40f && rms < 0x1p40f);
-    const float inv = 1.0f / rms;
-    return NormRoot{inv, plain ? 0.0f : rms, plain ? 0.0f : inv};
+    return NormRoot{1.0f / rms, rms, __builtin_amdgcn_ballot_w64(!(rms > 0x1p-40f && rms < 0x1p40f)) != 0};
 }
-__device__ inline float norm_value(float v, float w, float inv, float rms, float fix) {
+template <bool PLAIN> __device__ inline float norm_value(float v, float w, float inv, float rms) {
+    if constexpr (PLAIN) return v / rms * w;
     const float q = v * inv;
-    return __builtin_fmaf(__builtin_fmaf(-q, rms, v), fix, q) * w;
+    return __builtin_fmaf(__builtin_fmaf(-q, rms, v), inv, q) * w;
 }
 __device__ inline float lane_value(float v, int lane) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane)); }
 // the norm weights of a lane's columns of column tile b
@@ -178,15 +178,15 @@ template <int XT> __device__ inline NormW<XT> load_norm_w(const float *__restric
     return r;
 }
 // stage_x_rows of the normalised rows
-template <int XT, int MR>
-__device__ inline void stage_norm_rows(const XRows<XT, MR> &raw, const NormW<XT> &w, const NormRoot &root, uint8_t *__restrict__ rows, int lane) {
+template <int XT, int MR, bool PLAIN>
+__device__ inline void stage_norm_rows_as(const XRows<XT, MR> &raw, const NormW<XT> &w, const NormRoot &root, uint8_t *__restrict__ rows, int lane) {
     if constexpr (XT == TURQ_ACT_F32) {
 #pragma unroll
         for (int j = 0; j < MR; j++) {
-            const float inv = lane_value(root.inv, j), rms = lane_value(root.rms, j), fix = lane_value(root.fix, j);
+            const float inv = lane_value(root.inv, j), rms = lane_value(root.rms, j);
             float f[4];
 #pragma unroll
-            for (int e = 0; e < 4; e++) f[e] = norm_value(__uint_as_float(raw.v[j][e]), w.v[0][e], inv, rms, fix);
+            for (int e = 0; e < 4; e++) f[e] = norm_value<PLAIN>(__uint_as_float(raw.v[j][e]), w.v[0][e], inv, rms);
             const half2v h0 = __builtin_convertvector(float2v{f[0], f[1]}, half2v), h1 = __builtin_convertvector(float2v{f[2], f[3]}, half2v);
             *(uint2v *)(rows + j * kXRow + 8 * lane) = uint2v{__builtin_bit_cast(uint32_t, h0), __builtin_bit_cast(uint32_t, h1)};
         }
@@ -196,17 +196,21 @@ __device__ inline void stage_norm_rows(const XRows<XT, MR> &raw, const NormW<XT>
         for (int i = 0; i < MR / 2; i++) {
             const float inv = up ? lane_value(root.inv, 2 * i + 1) : lane_value(root.inv, 2 * i);
             const float rms = up ? lane_value(root.rms, 2 * i + 1) : lane_value(root.rms, 2 * i);
-            const float fix = up ? lane_value(root.fix, 2 * i + 1) : lane_value(root.fix, 2 * i);
             float f[8];
             x_values<XT>(raw.v[i], f);
             uint32_t h[4];
 #pragma unroll
             for (int e = 0; e < 4; e++)
-                h[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(float2v{norm_value(f[2 * e], w.v[e >> 1][(2 * e) & 3], inv, rms, fix),
-                                                                                    norm_value(f[2 * e + 1], w.v[e >> 1][(2 * e + 1) & 3], inv, rms, fix)}, half2v));
+                h[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(float2v{norm_value<PLAIN>(f[2 * e], w.v[e >> 1][(2 * e) & 3], inv, rms),
+                                                                                    norm_value<PLAIN>(f[2 * e + 1], w.v[e >> 1][(2 * e + 1) & 3], inv, rms)}, half2v));
             *(uint4v *)(rows + (2 * i + (lane >> 5)) * kXRow + 16 * (lane & 31)) = uint4v{h[0], h[1], h[2], h[3]};
         }
     }
+}
+template <int XT, int MR>
+__device__ inline void stage_norm_rows(const XRows<XT, MR> &raw, const NormW<XT> &w, const NormRoot &root, uint8_t *__restrict__ rows, int lane) {
+    if (root.plain) stage_norm_rows_as<XT, MR, true>(raw, w, root, rows, lane);
+    else stage_norm_rows_as<XT, MR, false>(raw, w, root, rows, lane);
 }
 // the A fragments of the staged column tile: lane (r, g) holds row r (rows past m repeat row m - 1);
 // K-quants: step q = columns 64 g + 8 q .. + 7, step 8 = the (hi, lo) sums of its four 16-column groups; Q8_0: step q = columns 32 q + 8 g .. + 7
