@@ -372,8 +372,7 @@ int turq_read_yardstick(turq_ctx *ctx, const void *dev_ptr, size_t nbytes);
 /* Which launch the rules for prompt chunks (more than 32 rows, K-quant or Q8_0 weights in the tiled layout) make for a weight of
  * n rows and k columns on a device with `compute_units` CUs; no GPU is needed and nothing is launched.  tile: 1 = 128 x 128,
  * 2 = 128 x 192 (Q8_0: 128 x 64), 3 = 128 x 256, 4 = 64 x 128 of the LDS-staged GEMM; 11, 21, 31, 22, 32, 23, 42, 33: 10 r + c = 32 r x 32 c of
- * the kernel whose waves split the columns, which launches of few tiles go through (11, K-quants, between one and one and a half rounds over
- * the CUs: two of the tiles one under the other per workgroup where that is one round); split: workgroups that share the columns of
+ * the kernel whose waves split the columns, which launches of few tiles go through; split: workgroups that share the columns of
  * every tile (1: none); wave_groups: 2 where the 64 x 128 tile runs eight waves as two groups on alternate super-blocks.  Not part of the
  * path, no counterpart in the reference: for tests of the rules and for tuning them on another device. */
 int turq_prefill_plan(int dtype, int64_t n, int64_t k, int64_t m, int compute_units, int *tile, int *split, int *wave_groups);

@@ -898,7 +898,11 @@ def test_columns_over_waves_two_workgroups_per_cu(gpu, dt, k):
 @pytest.mark.parametrize("dt", [Q4_K, Q5_K, Q6_K])
 @pytest.mark.parametrize("m", [65, 96])
 def test_two_tiles_per_workgroup_between_rounds(gpu, dt, m):
-    n, k = 3100, 2048
+    n, k = 3100, 4096
+    tile = ctypes.c_int()
+    for rows, want in ((m, 21), (40, 11)):
+        capi.check(gpu.L.turq_prefill_plan(dt, n, k, rows, 256, ctypes.byref(tile), None, None))
+        assert tile.value == want
     raw = synth.random_weight(dt, n, k, seed=dt + m)
     w = gpu.upload(dt, n, k, raw, capi.LAYOUT_TILED)
     x = synth.random_activation(m, k, seed=m, bf16=True)

@@ -510,20 +510,12 @@ int64_t cols_workgroups(int tile, int count, const int64_t *n, int64_t m) {
     return nbn * ((m + 32 * (tile / 10) - 1) / (32 * (tile / 10)));
 }
 
-// Whether a launch of 32 x 32 tiles that is more than one round over the CUs goes out as one of 64 x 32, two of them one under the other: the same sums
-// in the same order, and one round instead of a second for half of the CUs.  By the estimates, which for these two are right to a few percent:
-// Q6_K 4096 x 12288 at 65 - 96 rows 34.4 -> 27.4 us, 2048 x 6144 at 150 18.7 -> 17.0, Q5_K / Q4_K 4096 x 4096 at 77 13.4 / 11.9 -> 12.2 / 11.2; not of Q8_0, of which
-// three workgroups on a CU lose less (1024 x 2048 at 300 rows 8.1 -> 8.3).
-bool two_under_another(int dtype_a, int dtype_b, const TurqGemmWeights &ws, int64_t k, int64_t m, int64_t cus);
-
 template <int DTA, int DTB>
 hipError_t launch_tile(int tile, const TurqGemmWeights &ws, int second, int64_t k, const void *frags, int64_t m, int yt, int64_t cus,
                        hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop) {
     switch (tile) {
 #define TURQ_COLS(MT, NT, ...) launch_cols<DTA, DTB, MT, NT, ##__VA_ARGS__>(ws, second, k, frags, m, yt, stream, ev_start, ev_stop)
-    case 11:
-        if (two_under_another(DTA, DTB, ws, k, m, cus)) return TURQ_COLS(2, 1);
-        return TURQ_COLS(1, 1);
+    case 11: return TURQ_COLS(1, 1);
     case 21: return TURQ_COLS(2, 1);
     case 31: return TURQ_COLS(3, 1);
     case 22:  // (more than one workgroup per CU: two of them at a time)
@@ -604,13 +596,14 @@ static double cols_us(int tile, int dtype_a, int dtype_b, int count, const int64
                     cols_frag_us(tile, wgs / ((m + 32 * (tile / 10) - 1) / (32 * (tile / 10))), k, m, cus, x));
 }
 
-namespace {
-bool two_under_another(int dtype_a, int dtype_b, const TurqGemmWeights &ws, int64_t k, int64_t m, int64_t cus) {
-    if (dtype_a == TURQ_Q8_0 || turq_tuning().gemm_cols > 0) return false;  // (a forced tile is that tile)
-    if (cols_workgroups(11, ws.count, ws.n, m) <= cus || cols_workgroups(21, ws.count, ws.n, m) > cus) return false;
-    return cols_us(21, dtype_a, dtype_b, ws.count, ws.n, k, m, cus) < cols_us(11, dtype_a, dtype_b, ws.count, ws.n, k, m, cus);
+// Whether a launch of one weight in 32 x 32 tiles that is more than one round over the CUs goes out as one of 64 x 32, two of them one under the other:
+// the same sums in the same order, and one round instead of a second for half of the CUs.  By the estimates, which for these two are right to a few
+// percent: Q6_K 4096 x 12288 at 65 - 96 rows 34.4 -> 27.4 us, 2048 x 6144 at 150 18.7 -> 17.0, Q5_K / Q4_K 4096 x 4096 at 77 13.4 / 11.9 -> 12.2 / 11.2; not of
+// Q8_0, of which three workgroups on a CU lose less (1024 x 2048 at 300 rows 8.1 -> 8.3).
+static bool two_under_another(int dtype, const int64_t *n, int64_t k, int64_t m, int64_t cus) {
+    if (dtype == TURQ_Q8_0 || cols_workgroups(11, 1, n, m) <= cus || cols_workgroups(21, 1, n, m) > cus) return false;
+    return cols_us(21, dtype, dtype, 1, n, k, m, cus) < cols_us(11, dtype, dtype, 1, n, k, m, cus);
 }
-}  // namespace
 
 // The tile with which one weight goes through this kernel as far as single rounds over the CUs decide, 0: gemm_kq_kernel.
 // A launch of one round takes about base + per_sb * super-blocks, one line for every format; a further round costs as much again without the
@@ -696,6 +689,9 @@ int turq_gemm_cols_tile(int dtype_a, int dtype_b, int count, const int64_t *n, i
         }
     }
     if (us && best) *us = best_us;
+    // (The time stays that of 32 x 32, what several weights together are held against: of 60000 calls of two or three weights 19 change with the other, and
+    // eight of those, some of which went out together only so, took 0.87 - 1.19 of the time.)
+    if (count == 1 && best == 11 && two_under_another(dtype_a, n, k, m, cus)) best = 21;
     return best;
 }
 
