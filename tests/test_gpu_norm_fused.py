@@ -223,6 +223,13 @@ def test_errors_are_reported(gpu):
     gpu.release(w)
 
 
+def norm_plan(fmts, ns, k, m, gate_up=False):
+    """row tiles per workgroup with which the call's rules take the norm into the staged kernels, 0: it has a launch of its own"""
+    f = capi.lib().turq_norm_plan
+    f.argtypes = [ctypes.c_int, ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_int64), ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_int]
+    return f(len(ns), (ctypes.c_int * len(ns))(*fmts), (ctypes.c_int64 * len(ns))(*ns), k, m, int(gate_up), 256)
+
+
 # 3 .. 8 rows of 1024 .. 4096 columns: the kernels that stage the rows apply the norm on the way, bit-equal to the separate calls.  One to eight waves
 # (pairs of column tiles), four and eight rows with and without rows that are not there, every activation type, one and two formats in the launch,
 # a row of zeros, tiny and huge rows (f32), weight rows that end inside a row tile, one weight (in the staged kernels from five rows on).  k = 512 (the norm of short rows adds up in another order) and 9
@@ -232,6 +239,8 @@ def test_errors_are_reported(gpu):
 @pytest.mark.parametrize("fmts", [(Q8_0, Q8_0), (Q4_K, Q4_K, Q6_K), (Q5_K, Q6_K), (Q6_K,)])
 def test_norm_in_the_staged_kernels(gpu, fmts, k, m, x_dtype):
     ns = [200, 48, 96][:len(fmts)]
+    # (one weight at 3 and 4 rows: the kernels of turq_qmatmul, with the norm in scratch)
+    assert norm_plan(fmts, ns, k, m) == (1 if k >= 1024 and m <= 8 and (len(fmts) > 1 or m > 4) else 0)
     ws = [gpu.upload(dt, n, k, synth.random_weight(dt, n, k, seed=n + k), capi.LAYOUT_TILED) for dt, n in zip(fmts, ns)]
     rng = np.random.default_rng(k + m)
     x = synth.random_activation(m, k, seed=m + k, bf16=x_dtype == capi.ACT_BF16)
@@ -340,3 +349,52 @@ def test_rows_with_very_large_roots_in_the_staged_kernels(gpu, x_dtype):
         want, _ = separate(gpu, [w, w], [n, n], x, nw, x_dtype=x_dtype)
         assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1]), seed
     gpu.release(w)
+
+
+# launches of more weight rows: two, three and six row tiles per workgroup (of a second format half of them), q, k and v of an 8B model at three rows
+@pytest.mark.parametrize("x_dtype", [capi.ACT_F32, capi.ACT_BF16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("fmts,ns,k,m,tiles", [
+    ((Q4_K, Q4_K, Q6_K), (4096, 1024, 1000), 4096, 3, 2), ((Q5_K, Q6_K), (4200, 1048), 1024, 8, 2), ((Q8_0, Q8_0), (4200, 216), 1024, 7, 2),
+    ((Q5_K, Q5_K), (8000, 216), 1024, 6, 3), ((Q4_K, Q6_K), (8000, 216), 1024, 4, 3), ((Q8_0, Q8_0), (8000, 216), 1024, 8, 3),
+    ((Q4_K, Q4_K), (20600, 48), 1024, 4, 6), ((Q5_K, Q6_K), (20600, 48), 1024, 8, 6), ((Q6_K,), (20600,), 1024, 5, 6)])
+def test_norm_in_the_staged_kernels_of_several_row_tiles(gpu, fmts, ns, k, m, tiles, x_dtype):
+    assert norm_plan(fmts, ns, k, m) == tiles
+    ws = [gpu.upload(dt, n, k, synth.random_weight(dt, n, k, seed=n + k), capi.LAYOUT_TILED) for dt, n in zip(fmts, ns)]
+    rng = np.random.default_rng(k + m)
+    x = synth.random_activation(m, k, seed=m + k, bf16=x_dtype == capi.ACT_BF16)
+    nw = (1.0 + 0.3 * rng.standard_normal(k)).astype(np.float32)
+    got = norm_multi(gpu, ws, list(ns), x, nw, x_dtype=x_dtype)
+    want, _ = separate(gpu, ws, list(ns), x, nw, x_dtype=x_dtype)
+    for a, b in zip(got, want):
+        assert np.array_equal(a, b)
+    for w in ws:
+        gpu.release(w)
+
+
+# gate and up of an MLP: one row tile of each per workgroup, and three (more than two tiles of each per CU; an 8B model's at three rows is the last
+# that the rule takes), for rows that fill the four or eight that the kernels hold and rows that do not; Q8_0 takes no six
+@pytest.mark.parametrize("x_dtype", [capi.ACT_F32, capi.ACT_BF16, capi.ACT_F16], ids=["f32", "bf16", "f16"])
+@pytest.mark.parametrize("dt,n_ff,k,m,tiles", [
+    (Q4_K, 3072, 1024, 8, 2), (Q5_K, 3072, 1024, 5, 2), (Q6_K, 1536, 1024, 3, 2), (Q8_0, 3072, 1024, 8, 2), (Q8_0, 1536, 2048, 4, 2),
+    (Q4_K, 8448, 1024, 7, 6), (Q5_K, 8448, 1024, 8, 6), (Q6_K, 8448, 1024, 4, 6), (Q8_0, 8448, 1024, 4, 0), (Q4_K, 12288, 4096, 3, 6), (Q4_K, 12288, 4096, 5, 0)])
+def test_norm_in_the_gate_up_kernels(gpu, dt, n_ff, k, m, tiles, x_dtype):
+    assert norm_plan((dt, dt), (n_ff, n_ff), k, m, gate_up=True) == tiles
+    n_out, down = 256, Q8_0
+    shapes = [(dt, n_ff, k), (dt, n_ff, k), (down, n_out, n_ff)]
+    ws = [gpu.upload(d, n, c, synth.random_weight(d, n, c, seed=i), capi.LAYOUT_TILED) for i, (d, n, c) in enumerate(shapes)]
+    L, ctx = gpu.L, gpu.ctx
+    x = synth.random_activation(m, k, seed=m + k, bf16=x_dtype == capi.ACT_BF16)
+    nw = (0.02 * (1.0 + 0.3 * np.random.default_rng(m).standard_normal(k))).astype(np.float32)
+    d = Dev(gpu)
+    try:
+        xp, nwp, yp, xn = d.put(send(x, x_dtype)), d.put(nw), d.put(np.zeros((m, n_out), np.float32)), d.put(np.zeros((m, k), np.float32))
+        capi.check(L.turq_norm_mlp(ctx, *ws, xp, x_dtype, m, k, nwp, EPS, yp, capi.ACT_F32, n_out, None, None, None, 0, capi.MEM_DEVICE), ctx)
+        got = gpu.read_back(yp, (m, n_out), np.float32)
+        capi.check(L.turq_rms_norm(ctx, xp, x_dtype, m, k, k, nwp, EPS, xn, capi.ACT_F32, k, capi.MEM_DEVICE), ctx)
+        normed = gpu.read_back(xn, (m, k), np.float32)
+    finally:
+        d.free()
+    assert np.isfinite(got).all() and np.abs(got).max() > 0
+    assert np.array_equal(got, gpu.mlp(*ws, normed, n_ff, k, n_out))
+    for w in ws:
+        gpu.release(w)

@@ -706,6 +706,15 @@ bool turq_rows_in_chunks(const turq_ctx *ctx, int count, const turq_weight *cons
     return staged_row_tiles(ctx, w[0]->dtype, w[0]->dtype, xt, w[0]->k, TURQ_GEMV_MAX_M, row_tiles, 0, aligned) == 6;
 }
 
+// the row tiles per workgroup (gate's and up's together) with which the staged kernel normalises the rows on the way to gate and up, 0: it does not
+static int gateup_norm_tiles(const turq_ctx *ctx, const turq_weight *gate, const turq_weight *up, int64_t m) {
+    const int64_t cus = ctx->compute_units > 0 ? ctx->compute_units : 256;
+    if (turq_tuning().cs_staged == 0 || m < 3 || gate->dtype != up->dtype || gate->n != up->n || gate->k != up->k) return 0;
+    const int tiles = turq_gemv_cs_staged_gateup_tiles(gate->dtype, gate->n, gate->k, m, cus);
+    if (!tiles || !turq_gemv_cs_staged_norm_takes(gate->dtype, gate->k, m, tiles, (turq_tile_rows(gate->n) + tiles / 2 - 1) / (tiles / 2), cus)) return 0;
+    return tiles;
+}
+
 int turq_qmatmul_gate_up_mfma(turq_ctx *ctx, const turq_weight *gate, const turq_weight *up, const void *x, int xt, int64_t m,
                               int64_t ldx, void *y, int yt, int64_t ldy, const float *bias_gate, const float *bias_up, bool *taken,
                               const TurqNorm *norm) {
@@ -739,8 +748,7 @@ int turq_qmatmul_gate_up_mfma(turq_ctx *ctx, const turq_weight *gate, const turq
         const int64_t cus = ctx->compute_units > 0 ? ctx->compute_units : 256;
         const int tiles = (staged != 0 && staged_rows_ok(x, xt, ldx) && m >= 3 && gate->n == up->n && gate->k == up->k)
                               ? turq_gemv_cs_staged_gateup_tiles(gate->dtype, gate->n, gate->k, m, cus) : 0;
-        if (norm && m != 1 && (!tiles || !turq_gemv_cs_staged_norm_takes(gate->dtype, gate->k, m, tiles, (turq_tile_rows(gate->n) + tiles / 2 - 1) / (tiles / 2), cus)))
-            return TURQ_OK;  // (the caller normalises into scratch first)
+        if (norm && m != 1 && (!tiles || !gateup_norm_tiles(ctx, gate, up, m))) return TURQ_OK;  // (the caller normalises into scratch first)
         if (tiles) {
             TURQ_HIP(ctx, turq_prof_next(ctx, &ev0, &ev1));
             TURQ_HIP(ctx, turq_launch_gemv_cs_staged_gateup(gate->dtype, gate->dev, up->dev, gate->n, gate->k, x, xt, ldx, m, y, yt, ldy,
@@ -984,6 +992,24 @@ extern "C" int turq_mlp_pair_plan(int dtype, int down_dtype, int64_t n_ff, int64
     const turq_weight *const gu[2] = {&one, &one};
     const int pair = gemm_pair(&ctx, gu, down_dtype, m);
     return pair == kGemmPairKq ? -turq_gemm_form(dtype, 2 * n_ff, k, m, compute_units) : pair;
+}
+
+// For tests of the rules (not part of the C ABI): the row tiles per workgroup with which the staged kernels normalise 2 - 32 aligned f32 rows of stride k on
+// the way to `count` weights (of the first launch), or (gate_up, two weights of one shape) to gate and up, on a device of that many CUs; 0: the norm
+// has a launch of its own
+extern "C" int turq_norm_plan(int count, const int *dtypes, const int64_t *n, int64_t k, int64_t m, int gate_up, int compute_units) {
+    if (count < 1 || count > 4 || m < 2 || m > TURQ_GEMV_MAX_M || compute_units <= 0) return 0;
+    turq_ctx ctx;
+    ctx.compute_units = compute_units;
+    turq_weight held[4];
+    const turq_weight *w[4];
+    for (int i = 0; i < count; i++) {
+        held[i].dtype = dtypes[i], held[i].layout = TURQ_LAYOUT_TILED, held[i].n = n[i], held[i].k = k;
+        w[i] = &held[i];
+    }
+    if (!turq_norm_fuses(&ctx, count, w, nullptr, TURQ_ACT_F32, k, m)) return 0;
+    if (!gate_up) return staged_run(&ctx, count, w, TURQ_ACT_F32, m, true).rg;
+    return count == 2 ? gateup_norm_tiles(&ctx, w[0], w[1], m) : 0;
 }
 
 // which launch the rules above, in gemm_cols.hip and in gemm_mfma.hip make for a prompt chunk (no GPU needed)
