@@ -911,3 +911,35 @@ def test_two_tiles_per_workgroup_between_rounds(gpu, dt, m):
     assert rel_l2(y - bias, orc.matmul_dequant(dt, x, raw, n, k)) <= 1e-3
     assert np.array_equal(y[:40], gpu.qmatmul(w, x[:40], n, k, x_dtype=capi.ACT_BF16, bias=bias))
     gpu.release(w)
+
+
+# rows a very long stride apart (4 GiB of f32; of 16-bit rows 2 GiB and a little, whose second row lies past a signed 32-bit offset): the kernels that
+# stage them take them, in a capture on a new context, where nothing can be allocated, and with the bits of dense rows
+@pytest.mark.parametrize("x_dtype,ldx", [(capi.ACT_F32, 1 << 30), (capi.ACT_BF16, (1 << 30) + 8)], ids=["f32", "bf16"])
+def test_rows_a_long_stride_apart(x_dtype, ldx):
+    gpu = Gpu()
+    L, ctx = gpu.L, gpu.ctx
+    n, k, m, es = 200, 1024, 5, 4 if x_dtype == capi.ACT_F32 else 2
+    w = gpu.upload(Q4_K, n, k, synth.random_weight(Q4_K, n, k, seed=1), capi.LAYOUT_TILED)
+    x = synth.random_activation(m, k, seed=2, bf16=True)
+    rows = x if x_dtype == capi.ACT_F32 else synth.to_bf16_bits(x).reshape(m, k)
+    xd, yd = ctypes.c_void_p(), gpu.dev_buffer(np.zeros((m, n), np.float32))
+    capi.check(L.turq_dev_alloc(ctx, ((m - 1) * ldx + k) * es, ctypes.byref(xd)), ctx)
+    for r in range(m):
+        row = np.ascontiguousarray(rows[r])
+        capi.check(L.turq_memcpy_h2d(ctx, ctypes.c_void_p(xd.value + r * ldx * es), capi.ptr(row), row.nbytes), ctx)
+    capi.check(L.turq_graph_begin(ctx), ctx)
+    capi.check(L.turq_qmatmul(ctx, w, xd, x_dtype, m, ldx, yd, capi.ACT_F32, n, None, capi.MEM_DEVICE, capi.ALGO_AUTO), ctx)
+    g = ctypes.c_void_p()
+    capi.check(L.turq_graph_end(ctx, ctypes.byref(g)), ctx)
+    want = gpu.qmatmul(w, x, n, k, x_dtype=x_dtype)
+    for _ in range(3):
+        capi.check(L.turq_memcpy_h2d(ctx, yd, capi.ptr(np.zeros((m, n), np.float32)), 4 * m * n), ctx)
+        capi.check(L.turq_graph_launch(ctx, g), ctx)
+        capi.check(L.turq_sync(ctx), ctx)
+        assert np.array_equal(gpu.read_back(yd, (m, n), np.float32), want)
+    L.turq_graph_destroy(g)
+    for p in (xd, yd):
+        gpu.dev_free(p)
+    gpu.release(w)
+    gpu.close()

@@ -36,8 +36,8 @@ constexpr int kXRow = 512 + 16;  // bytes per staged activation row: 256 f16 and
 template <int XT, int MR> struct XRows {
     uint4v v[XT == TURQ_ACT_F32 ? MR : MR / 2];
 };
-// The rows of an instruction's 64 lanes as a scalar address and 32-bit lane offsets (ldx below 2^30, which the dispatch asks for): one 64-bit
-// address per lane and row was about eight vector instructions for each load, ahead of the first weight.
+// The rows of an instruction's 64 lanes as a scalar address and 32-bit lane offsets (16-bit rows: 2 ldx + 512 below 2^32, which the dispatch asks for): one
+// 64-bit address per lane and row was about eight vector instructions for each load, ahead of the first weight.
 template <int XT> struct XOff {
     uint32_t one, two;  // 16-bit rows: the lane's 16 bytes with both halves of the wave on one row, on two neighbouring ones
     __device__ XOff(int64_t ldx, int lane) {

@@ -131,9 +131,10 @@ int staged_row_tiles(const turq_ctx *ctx, int dtype_a, int dtype_b, int xt, int6
     return turq_gemv_cs_staged_takes(dtype_a, dtype_b, xt, k, m, rg) ? rg : 0;
 }
 
-// activation rows that the staged kernels can load: 16 bytes at a time, two neighbouring ones from one address and a 32-bit offset
+// activation rows that the staged kernels can load: 16 bytes at a time, of 16-bit rows two neighbouring ones from one address and a 32-bit offset (a
+// stride of up to 4 GiB)
 bool staged_rows_ok(const void *x, int xt, int64_t ldx) {
-    return (uintptr_t)x % 16 == 0 && ((size_t)ldx * turq_act_bytes(xt)) % 16 == 0 && ldx < (1 << 30);
+    return (uintptr_t)x % 16 == 0 && ((size_t)ldx * turq_act_bytes(xt)) % 16 == 0 && (xt == TURQ_ACT_F32 || ldx <= (1ll << 31) - 256);
 }
 
 // The staged launch that the first weights of a call go out in (rg 0: none): a run of one format, with one of a second format behind it
