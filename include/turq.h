@@ -108,7 +108,8 @@ void *turq_ctx_stream(turq_ctx *ctx);
  * propagate.  It costs two launches per call and the grouped launches of turq_qmatmul_multi / turq_qmatmul_gate_up.  Default:
  * off, for engines whose activations are known to be bounded (after an RmsNorm, say); turq_ctx_nonfinite_count tells a host
  * that left it off whether a call overflowed.  Calls on HOST pointers always take the wide path: they are the reference's own
- * contract, and the staging copies dominate them anyway.  turq_qmatmul_noalloc cannot take it (it has no scratch for the
+ * contract.  The first of them takes 8 MiB of page-locked memory for the life of the context, through which f32 and bf16 rows against
+ * tiled weights go (larger calls are copied in and out).  turq_qmatmul_noalloc cannot take it (it has no scratch for the
  * scaled rows) and refuses f32 / bf16 activations with TURQ_ERR_INVALID while the switch is on. */
 int turq_ctx_set_wide_activations(turq_ctx *ctx, int on);
 /* Whether a forward call left the number range of its kernels.  Every kernel that stores results (the matmuls, turq_rms_norm,
@@ -309,8 +310,8 @@ int turq_norm_qmatmul_multi(turq_ctx *ctx, int count, const turq_weight *const *
 
 /* turq_mlp on RmsNorm(x), the second half of the reference's decoder layer: with y_dtype | TURQ_OUT_ACCUMULATE and y = the
  * residual stream it is `x + mlp(ln2(x))` in one call (src/models/qwen3.rs:637-640).  norm_weight and eps as above, everything
- * else as in turq_mlp; the norm is taken into the kernels in the same two cases (one row: into the gate / up kernel; more than
- * 32 rows: the norm writes the fragments of the gate / up GEMMs) and runs into scratch memory otherwise. */
+ * else as in turq_mlp; the norm is taken into the kernels in the same three cases (one row, and 3 - 8 rows where that pays: into the
+ * gate / up kernel; more than 32 rows: the norm writes the fragments of the gate / up GEMMs) and runs into scratch memory otherwise. */
 int turq_norm_mlp(turq_ctx *ctx, const turq_weight *gate, const turq_weight *up, const turq_weight *down, const void *x, int x_dtype,
                   int64_t m, int64_t ldx, const float *norm_weight, float eps, void *y, int y_dtype, int64_t ldy, const float *bias_gate,
                   const float *bias_up, const float *bias_down, int act, int mem);

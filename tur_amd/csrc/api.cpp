@@ -532,7 +532,8 @@ static bool host_map_ready(turq_ctx *ctx) {
     return true;
 }
 
-// whether a wide call goes through the scaling kernels, which read x and the bias once and write y once
+// whether a wide call goes through the scaling kernels, which read x once (twice past 12288 columns, and rows that they cannot load four columns at a
+// time) and write y once; the bias, which they read for every row, costs host calls 1 - 3 us at any number of rows
 static bool wide_scales(const turq_ctx *ctx, const turq_weight *w, int xt, int algo) {
     return !ctx->fixed_scratch && xt != TURQ_ACT_F16 && (algo == TURQ_ALGO_AUTO || algo == TURQ_ALGO_GEMV || algo == TURQ_ALGO_GEMM) &&
            w->layout == TURQ_LAYOUT_TILED;
@@ -605,7 +606,8 @@ static int impl_qmatmul(turq_ctx *ctx, const turq_weight *w, const void *x, int 
     const size_t xrow = (size_t)w->k * xb, yrow = (size_t)w->n * yb;
     if (wide_scales(ctx, w, xt, algo) && xrow * (size_t)m + yrow * (size_t)m + (size_t)w->n * sizeof(float) + 64 <= turq_ctx::kHostMapBytes && host_map_ready(ctx)) {
         // through pinned memory that the scaling kernels read and write themselves, without the runtime's copies from and to pageable memory: Q8_0
-        // 3072 x 1024 at one row 48 -> 32 us a call, Q4_K 12288 x 4096 at 16 rows 346 -> 86, 12288 x 12288 at 64 (6 MB of rows and results) 1300 -> 335
+        // 3072 x 1024 with bias at one / 16 rows 45 / 282 -> 24.5 / 34 us a call (from the C ABI), Q4_K 12288 x 4096 at 16 / 64 342 / 1258 -> 72 / 256, 4096 x 12288 at 33
+        // 634 -> 118, Q8_0 512 x 32768 at 16, whose rows are read twice, 397 -> 209
         const auto up = [](size_t n) { return (n + 15) & ~(size_t)15; };
         const size_t at_b = up(xrow * (size_t)m), at_y = at_b + up((size_t)w->n * sizeof(float));
         uint8_t *host = (uint8_t *)ctx->host_map, *dev = (uint8_t *)ctx->host_map_dev;

@@ -218,9 +218,10 @@ int turq_gemv_cs_staged_second_rows(int row_tiles) { return staged_second_rows(r
 
 // Whether a launch of `groups` workgroups applies RmsNorm itself: 1024 .. 4096 columns, one pair of column tiles per wave (fewer columns: the norm's
 // own kernel adds their squares up in another order), while what a compute unit spends on it - its workgroups times rows (4 or 8) times columns -
-// is less than the norm's launch.  Norm and products, launch of its own / inside: q, k and v of 4096 columns at 3 / 8 rows 9.4 / 9.9 us against 9.0 / 10.7, of
-// 2048 at 8 rows 7.1 / 6.3, of 1024 at 4 / 8 rows 6.1 / 6.3 against 4.1 / 5.7; MLPs 12288 x 4096 at 3 rows 28.1 / 26.5, 3072 x 1024 at 8 13.4 / 11.8, but 512
-// workgroups (8192 x 3072 at 4 rows) 22.9 / 25.8; at 16 rows it never pays (2048 columns 7.4 / 9.1).  dtype: the first format
+// is less than the norm's launch.  Norm and products, launch of its own / inside: q, k and v of 4096 columns at 3 f32 rows 9.4 / 9.4 us, at 4
+// bf16 rows 9.7 / 8.9, of 2048 at 8 rows 6.9 / 6.0, of 1024 at 4 / 8 rows 5.9 / 6.0 against 4.1 / 5.1; MLPs 12288 x 4096 at 3 rows 27.5 / 26.3, 3072 x 1024 at 8 13.5 /
+// 13.0.  Behind when it was tried without the line: 4096 columns at 8 rows 9.9 / 10.7, 512 workgroups (8192 x 3072 at 4 rows) 22.9 / 25.8, 2048 columns at 16 rows
+// 7.4 / 9.1.  dtype: the first format
 bool turq_gemv_cs_staged_norm_takes(int dtype, int64_t k, int64_t m, int row_tiles, int64_t groups, int64_t units) {
     if (m < 3 || m > 8 || k % 512 != 0 || k < 1024 || k > 4096) return false;
     const int64_t mr = m <= 4 ? 4 : 8;

@@ -145,7 +145,7 @@ __device__ inline float sq4(float a, float b, float c, float d) { return __built
 
 // A launch's arguments are two hundred bytes that no cache holds when it starts.  Left to itself the compiler loads each where it is first used,
 // behind the branches that pick the weight: five scalar loads one after the other, each a round trip, before the first weight is
-// requested.  Naming them here makes them one.
+// requested.  Naming them here makes them one: ahead in the one-row kernels, and behind where several rows are (multi_pick, gemm_cols.hip).
 template <class... T> __device__ inline void load_together(T... v) { (void)std::initializer_list<int>{([](auto u) { asm volatile("" ::"s"(u)); }(v), 0)...}; }
 
 // 32-bit per-lane byte offsets of the global loads.  An offset computed (and widened to 64 bits) outside the loop reaches

@@ -56,7 +56,8 @@ bool row1_takes(int64_t m, size_t weight_bytes, int dtype) {
 // 1024 x 2048 Q8_0 at 4 / 8 waves of 2 / 1 tiles 3.7 / 3.3).  Beyond that the workgroups of a unit should be resident together, and
 // it wants about ten waves in all: 384 workgroups (q, k and v of 4096 columns) at 4 / 6 / 8 / 16 waves 7.0 / 6.5 / 6.8 / 7.4 us, 640
 // (5120 columns) at 4 / 8 / 16 10.7 / 11.9 / 12.6, 2000 (32000 x 4096 Q4_K) 16.7 / 16.9 / 22.4; two tiles at a time keep eight (gate and up 12288
-// x 4096, 768 workgroups, at 4 / 8 / 16 11.9 / 11.6 / 13.5).
+// x 4096, 768 workgroups, at 4 / 8 / 16 11.9 / 11.6 / 13.5).  Wide columns on more than 256 row tiles, which had 16 waves, at 5 - 8: Q6_K 4608 x 12288 14.4 -> 13.5,
+// 5120 x 13824 15.6 -> 15.4, 6144 x 16384 19.1 -> 18.3, Q8_0 5120 x 15360 20.6 -> 19.4, Q4_K 5120 x 13824 12.9 -> 11.6, 8192 x 8192 10.2 -> 9.8, 12288 x 12288 16.1 -> 16.2.
 int pick_waves_row1(const turq_ctx *ctx, int64_t k, int64_t groups, int rtiles) {
     const int forced = turq_tuning().gemv_waves, tpw = turq_tuning().row1_tpw;
     const int64_t col_tiles = turq_tile_cols(k), cus = ctx->compute_units > 0 ? ctx->compute_units : 256;

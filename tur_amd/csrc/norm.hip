@@ -106,7 +106,8 @@ __device__ inline bool vec_row(const void *p, int64_t ld, int elem_bytes) {
 
 // sqrt(mean(x^2) + eps) of the row that a workgroup of four waves holds: s[j] = what a thread has of the squares of its piece j, summed up over
 // the lanes of each wave and then over the blocks 4 j + wave in order - one fixed order, shared by the kernels below so that they
-// agree to the bit (as sq4 says).  part: 4 PER floats, or `blocks` of which those from 4 PER on are there.  Every thread of the workgroup calls it.
+// agree to the bit (as sq4 says).  part: 4 PER floats, which it fills; of a row with more than 4 PER blocks `blocks` floats, those behind the first 4 PER
+// already filled by the caller (part[b]: the sum of block b).  Every thread of the workgroup calls it.
 template <int PER> __device__ inline float rms_of(const float (&s)[PER], int64_t k, float eps, float *part, int blocks = 0) {
 #pragma unroll
     for (int j = 0; j < PER; j++) {
