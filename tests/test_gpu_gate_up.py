@@ -67,6 +67,23 @@ def test_gate_up_matches_the_two_calls(gpu, dt, m):
     gpu.release(wu)
 
 
+# one and two rows, as many waves as the launch's size asks for: eight that take three column tiles each (24 column tiles on no more workgroups than
+# compute units; 17 leave seven of the waves one tile short), twelve with one or two (16 column tiles on 272 workgroups), eight again (10 column tiles).  Two rows
+# of these sizes are 8 MB and more.
+@pytest.mark.parametrize("dt,n,k", [(Q4_K, 3000, 6144), (Q8_0, 2100, 4352 + 32), (Q5_K, 4352, 4096), (Q6_K, 4352, 3072), (Q8_0, 4352, 2560)])
+def test_gate_up_waves(gpu, dt, n, k):
+    raw_g = synth.random_weight(dt, n, k, seed=dt + n)
+    raw_u = synth.random_weight(dt, n, k, seed=dt + k)
+    wg = gpu.upload(dt, n, k, raw_g, capi.LAYOUT_TILED)
+    wu = gpu.upload(dt, n, k, raw_u, capi.LAYOUT_TILED)
+    for m in (1, 2):
+        x = synth.random_activation(m, k, seed=m)
+        y = gpu.gate_up(wg, wu, x, n, k)
+        assert rel_l2(y, expected(dt, f16_round(x), raw_g, raw_u, n, k)) <= 5e-5
+    gpu.release(wg)
+    gpu.release(wu)
+
+
 # 17 .. 32 rows, staged in the kernel: one row tile of each weight per workgroup (200 rows end inside one; 4096 rows are 256 workgroups) or
 # three (8240 rows: more than two row tiles per compute unit); 512 columns are one pair of column tiles for one wave, 2048 one for each of
 # four, 4096 for each of eight.  The kernel rounds f32 rows to f16 as the caller would.  Tolerance as above.

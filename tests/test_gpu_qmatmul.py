@@ -943,3 +943,15 @@ def test_rows_a_long_stride_apart(x_dtype, ldx):
         gpu.dev_free(p)
     gpu.release(w)
     gpu.close()
+
+
+# one row on one and two thirds to two row tiles per compute unit (438: eight waves, of which four have a second column tile of 12; 512), and on 513 (four waves)
+@pytest.mark.parametrize("dt", [Q4_K, Q6_K, Q8_0])
+@pytest.mark.parametrize("n", [7000, 8192, 8200])
+def test_one_row_waves(gpu, dt, n):
+    k = 3072
+    raw = synth.random_weight(dt, n, k, seed=dt + n)
+    w = gpu.upload(dt, n, k, raw, capi.LAYOUT_TILED)
+    x = synth.random_activation(1, k, seed=n).astype(np.float16).astype(np.float32)
+    assert rel_l2(gpu.qmatmul(w, x, n, k), orc.matmul_dequant(dt, x, raw, n, k)) <= 5e-5
+    gpu.release(w)

@@ -51,23 +51,36 @@ bool row1_takes(int64_t m, size_t weight_bytes, int dtype) {
 }
 
 // Waves per workgroup of the one-row kernels for a launch of `groups` workgroups of `rtiles` row tiles (2: two that share the staged
-// activations, or a gate and an up tile).  A launch of no more workgroups than compute units is a chain of memory round trips: as
-// many waves as there are column tiles, up to the largest workgroup (4096 x 12288 Q6_K at 8 / 12 / 16 waves 10.0 / 9.4 / 9.7 us,
-// 1024 x 2048 Q8_0 at 4 / 8 waves of 2 / 1 tiles 3.7 / 3.3).  Beyond that the workgroups of a unit should be resident together, and
-// it wants about ten waves in all: 384 workgroups (q, k and v of 4096 columns) at 4 / 6 / 8 / 16 waves 7.0 / 6.5 / 6.8 / 7.4 us, 640
-// (5120 columns) at 4 / 8 / 16 10.7 / 11.9 / 12.6, 2000 (32000 x 4096 Q4_K) 16.7 / 16.9 / 22.4; two tiles at a time keep eight (gate and up 12288
-// x 4096, 768 workgroups, at 4 / 8 / 16 11.9 / 11.6 / 13.5).  Wide columns on more than 256 row tiles, which had 16 waves, at 5 - 8: Q6_K 4608 x 12288 14.4 -> 13.5,
-// 5120 x 13824 15.6 -> 15.4, 6144 x 16384 19.1 -> 18.3, Q8_0 5120 x 15360 20.6 -> 19.4, Q4_K 5120 x 13824 12.9 -> 11.6, 8192 x 8192 10.2 -> 9.8, 12288 x 12288 16.1 -> 16.2.
+// activations, or a gate and an up tile).
+// A launch of no more workgroups than compute units is a chain of memory round trips: as many waves as there are column tiles, up to the
+// largest workgroup (4096 x 12288 Q6_K at 8 / 12 / 16 waves 10.0 / 9.4 / 9.7 us, 1024 x 2048 Q8_0 at 4 / 8 waves of 2 / 1 tiles 3.7 / 3.3); but
+// eight where two row tiles have more column tiles than that (gate and up 4064 x 6144 Q4_K at 8 / 12 / 16 7.1 / 7.4 / 7.1, 3072 x 5120 Q6_K at 8 / 10 / 16 7.5 /
+// 8.2 / 7.9, 4096 x 12288 Q5_K at 8 / 16 14.0 / 14.7).
+// Beyond that the workgroups of a unit should be resident together.  One row tile: three and more on a unit four waves (640 workgroups of 8192 columns at 4 /
+// 8 / 16 13.5 / 16.5 / 15.9, 625 of 4096 6.9 / 7.2 / 8.8), two eight (464 of 5120 at 4 / 5 / 8 / 16 8.3 / 8.0 / 7.6 / 8.7, 501 of 4096 7.0 / 6.9 / 6.0 / 7.3, 512 of 2048 4.9 / 5.0 /
+// 4.8 / 4.8), and towards one and a half, where half of the units have one, about ten waves in all (384, q, k and v of 4096 columns with the norm, at 4 /
+// 6 / 8 / 16 7.0 / 6.5 / 6.9 / 7.5).  Two row tiles: up to two on a unit twelve (5120 x 4096 Q4_K / Q6_K at 8 / 12 / 16 7.9 / 7.7 / 8.6 and 10.2 / 9.7 / 10.8), unless
+// that is more than the column tiles (8192 x 2560 Q8_0 at 8 / 10 9.4 / 10.3); otherwise eight (12288 x 4096, 768 workgroups, at 4 / 8 / 12 / 16 11.9 / 11.6 / 12.0 / 13.6).
+// Wide columns on more than 256 row tiles, which once had 16 waves: Q6_K 4608 x 12288 14.4 -> 13.5, 6144 x 16384 19.1 -> 18.3, Q8_0 5120 x 15360 20.6 -> 19.4,
+// Q4_K 5120 x 13824 12.9 -> 11.6, 8192 x 8192 10.2 -> 9.8, 12288 x 12288 16.1 -> 16.2.
 int pick_waves_row1(const turq_ctx *ctx, int64_t k, int64_t groups, int rtiles) {
     const int forced = turq_tuning().gemv_waves, tpw = turq_tuning().row1_tpw;
     const int64_t col_tiles = turq_tile_cols(k), cus = ctx->compute_units > 0 ? ctx->compute_units : 256;
     if (forced >= 1 && forced <= 16) return (int)std::min<int64_t>(forced, col_tiles);
     if (tpw > 0) return (int)std::max<int64_t>(1, std::min<int64_t>((col_tiles + tpw - 1) / tpw, 16));
+    int64_t most = 8;
     if (groups <= cus) {
-        const int64_t turns = (col_tiles + 15) / 16;  // column tiles of a wave
-        return (int)std::max<int64_t>(1, (col_tiles + turns - 1) / turns);
+        if (rtiles == 1 || col_tiles <= 16) {
+            const int64_t turns = (col_tiles + 15) / 16;  // column tiles of a wave
+            most = (col_tiles + turns - 1) / turns;
+        }
+    } else if (rtiles > 1) {
+        if (groups <= 2 * cus && col_tiles >= 12) most = 12;
+    } else if (groups > 2 * cus) {
+        most = 4;
+    } else if (3 * groups < 5 * cus) {
+        most = std::min<int64_t>(8, 10 * cus / groups);
     }
-    const int64_t most = rtiles > 1 ? 8 : std::max<int64_t>(4, std::min<int64_t>(8, 10 * cus / groups));
     return (int)std::max<int64_t>(1, std::min<int64_t>(col_tiles, most));
 }
 
