@@ -20,7 +20,7 @@ ALLOWED = [
     ("ScratchSize [bytes/lane]", r"\bgather_tiled_kernel<", 256, "the same private block, for embedding rows of a table kept in the tiled layout"),
     ("SGPRs Spill", r"\bgemv_(mfma|multi_frag|gateup_frag|multi_frag_mixed)_kernel<", 250,
      "prepared fragments with several row tiles or column tiles in flight: the addresses of two m-tiles' fragments; accepted as it is"),
-    ("SGPRs Spill", r"\bgemv_cs_staged_kernel<\d+, \d+, \d+, (8, 6, 0|16, 3, 1|32, [12], [01]), false, (true|false)>", 48,
+    ("SGPRs Spill", r"\bgemv_cs_staged_kernel<\d+, \d+, \d+, 32, 2, 0, false, (true|false)>", 8,
      "row addresses that a pair of column tiles shares: worked out for every column tile instead, the launches take 1 - 2 % longer (load_x_rows)"),
 ]
 UNITS = {"ScratchSize [bytes/lane]": "bytes of scratch per lane", "SGPRs Spill": "scalar registers that are kept elsewhere"}

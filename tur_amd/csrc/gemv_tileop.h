@@ -371,17 +371,14 @@ struct MultiArgs {
 };
 
 // the weight a workgroup of such a launch works on, and its index among the weight's workgroups
-// (Without load_together: its round trip for every weight's arguments pays in the one-row kernels, not in front of several rows, Q8_0 2048 x 1024 at 16 rows
-// 4.4 us with it, 4.1 without.)
+// (Branches, and the arguments where they are used: with every weight's arguments loaded together in front Q8_0 2048 x 1024 at 16 rows takes 4.4 us for
+// 4.1, and selects instead of the branches keep them all in scalar registers: Q8_0 and Q5_K 8000 x 3072 at 16 rows 10.0 and 10.1 us for 9.1 and 9.2.)
 struct MultiPick { const uint8_t *w; void *y; const float *bias; int64_t n, ldy; int block; int index; };
 __device__ inline MultiPick multi_pick(const MultiArgs &a, int blk) {
     MultiPick p{a.w[0], a.y[0], a.bias[0], a.n[0], a.ldy[0], blk, 0};
 #pragma unroll
-    for (int i = 1; i < kMaxMulti; i++) {  // (selects, no branches)
-        const bool in = i < a.count && blk >= a.first[i];
-        p.w = in ? a.w[i] : p.w, p.y = in ? a.y[i] : p.y, p.bias = in ? a.bias[i] : p.bias;
-        p.n = in ? a.n[i] : p.n, p.ldy = in ? a.ldy[i] : p.ldy, p.block = in ? blk - a.first[i] : p.block, p.index = in ? i : p.index;
-    }
+    for (int i = 1; i < kMaxMulti; i++)
+        if (i < a.count && blk >= a.first[i]) p = MultiPick{a.w[i], a.y[i], a.bias[i], a.n[i], a.ldy[i], blk - a.first[i], i};
     return p;
 }
 
