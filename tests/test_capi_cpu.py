@@ -233,6 +233,8 @@ def test_prefill_launch_rules_on_a_256_cu_device():
     assert [plan(Q6_K, 4096, 12288, m) for m in (33, 64, 96, 128, 256, 300, 512)] == [(t, 1, 1) for t in (11, 11, 21, 21, 22, 32, 42)]
     # ... also where the smallest tile would be up to one and a half rounds
     assert [plan(dt, 3100, 4096, m)[0] for dt in (Q4_K, capi.Q5_K, Q6_K) for m in (40, 65, 96)] == [11, 21, 21] * 3
+    # (260 and 272 workgroups of the smallest: a handful beyond the round does not count)
+    assert [plan(Q6_K, n, 4096, 46)[0] for n in (4144, 4352)] == [11, 21]
     assert plan(Q6_K, 4096, 12288, 1024) == (1, 1, 1)
     # o_proj / q_proj 4096 x 4096 and k_proj 1024 x 4096: eight MFMA tiles not at 16 super-blocks; there the low tile, with eight waves
     # while there is at most one workgroup per CU

@@ -599,9 +599,11 @@ static double cols_us(int tile, int dtype_a, int dtype_b, int count, const int64
 // Whether a launch of one weight in 32 x 32 tiles that is more than one round over the CUs goes out as one of 64 x 32, two of them one under the other:
 // the same sums in the same order, and one round instead of a second for half of the CUs.  By the estimates, which for these two are right to a few
 // percent: Q6_K 4096 x 12288 at 65 - 96 rows 34.4 -> 27.4 us, 2048 x 6144 at 150 18.7 -> 17.0, Q5_K / Q4_K 4096 x 4096 at 77 13.4 / 11.9 -> 12.2 / 11.2; not of
-// Q8_0, of which three workgroups on a CU lose less (1024 x 2048 at 300 rows 8.1 -> 8.3).
+// Q8_0, of which three workgroups on a CU lose less (1024 x 2048 at 300 rows 8.1 -> 8.3), nor for a handful of workgroups beyond the round, which the
+// estimates do not see: 4096 columns at 46 rows, 32 x 32 / 64 x 32, 260 workgroups Q4_K 12.8 / 14.2, Q5_K 14.0 / 14.7, Q6_K 14.7 / 15.0, but 272 14.0 / 14.0, 15.7 / 14.6 and
+// 16.5 / 15.1.
 static bool two_under_another(int dtype, const int64_t *n, int64_t k, int64_t m, int64_t cus) {
-    if (dtype == TURQ_Q8_0 || cols_workgroups(11, 1, n, m) <= cus || cols_workgroups(21, 1, n, m) > cus) return false;
+    if (dtype == TURQ_Q8_0 || cols_workgroups(11, 1, n, m) <= cus + cus / 32 || cols_workgroups(21, 1, n, m) > cus) return false;
     return cols_us(21, dtype, dtype, 1, n, k, m, cus) < cols_us(11, dtype, dtype, 1, n, k, m, cus);
 }
 
