@@ -428,11 +428,11 @@ constexpr int staged_ring(int dt, int rg, int mr, bool two_formats = false) {
 constexpr int staged_second_rows(int rg) { return (rg + 1) / 2; }
 
 // weights [0, a.second) are of format DTA with RG row tiles per workgroup, the others of DTB with staged_second_rows(RG)
-// (one format: DTA == DTB)
+// (one format: DTA == DTB; ACC: one weight)
 template <int DTA, int DTB, int XT, int MR, int RG, int CNT, bool NORM = false, bool ACC = false>
 __global__ void __launch_bounds__(512) gemv_cs_staged_kernel(MultiArgs a, int64_t k, const void *__restrict__ x, int64_t ldx, int64_t m, int yt,
                                                              const float *__restrict__ gw, float eps) {
-    const MultiPick p = multi_pick(a, (int)blockIdx.x);
+    const MultiPick p = ACC ? MultiPick{a.w[0], a.y[0], a.bias[0], a.n[0], a.ldy[0], (int)blockIdx.x, 0} : multi_pick(a, (int)blockIdx.x);
     constexpr int RGB = staged_second_rows(RG);
     if (DTA == DTB || p.index < a.second)
         cs_body_staged<DTA, XT, MR, RG, staged_ring(DTA, RG, MR, DTA != DTB), CNT, false, NORM, ACC>(p.w, p.n, k, x, ldx, m, p.y, yt, p.ldy, p.bias,
@@ -638,7 +638,7 @@ hipError_t staged_count(const StagedLaunch &l) {
         return hipErrorInvalidValue;
     }
     if constexpr (DTA == DTB && RG <= 3) {  // (the residual additions behind o_proj and down_proj, each a weight alone; others add through the store)
-        if (l.yt & TURQ_OUT_ACCUMULATE) {
+        if (l.a.count == 1 && (l.yt & TURQ_OUT_ACCUMULATE)) {
             if (l.cnt == 1) return staged_go<gemv_cs_staged_kernel<DTA, DTB, XT, MR, RG, 1, false, true>>(staged_lds<MR, RG>(l.nwaves, false), l);
             if constexpr (MR <= 16 || XT != TURQ_ACT_F32) return staged_go<gemv_cs_staged_kernel<DTA, DTB, XT, MR, RG, 0, false, true>>(staged_lds<MR, RG>(l.nwaves, false), l);
         }
